@@ -24,14 +24,48 @@ DevSystem &atrip_amd::get_sys(atrip_hip_ctx *ctx, int sys) {
 
 namespace {
 void *dev_bytes(DevSystem &s, size_t bytes, const char *what);
-// Zeroed tiled bf16x3 copy (and row-swapped copy) of geometry g.
+// Tiled bf16x3 copy (and row-swapped copy) of geometry g; its fill writes
+// every element, padding included.
 void alloc_tri(DevSystem &s, TriOp &o, const TriGeom &g, const char *what) {
   const size_t bytes = (size_t)tri_parts(g) * 2;
   o.p = (uint16_t *)dev_bytes(s, bytes, what);
-  check(hipMemset(o.p, 0, bytes), what);
-  if (g.swapped) {
-    o.sw = (uint16_t *)dev_bytes(s, bytes, what);
-    check(hipMemset(o.sw, 0, bytes), what);
+  if (g.swapped) o.sw = (uint16_t *)dev_bytes(s, bytes, what);
+}
+
+// Copies of a system's operands that a failure part-way gives back whole.
+struct CopyGuard {
+  DevSystem &s;
+  size_t n;
+  uint64_t bytes;
+  bool done = false;
+  explicit CopyGuard(DevSystem &s_)
+      : s(s_), n(s_.allocations.size()), bytes(s_.bytes) {}
+  ~CopyGuard() {
+    if (done) return;
+    for (size_t q = n; q < s.allocations.size(); q++)
+      (void)hipFree(s.allocations[q]);
+    s.allocations.resize(n);
+    s.bytes = bytes;
+  }
+};
+
+// FP64 operand x of a system in its split form, or its bf16x3 form with the
+// row-swapped copy.
+void convert_split(const DevSystem &s, const double *x, const TriGeom &g,
+                   const DevSystem::Split &o, hipStream_t st) {
+  OpSink k;
+  k.h = o.h;
+  k.l = o.l;
+  check(launch_convert(x, g, k, g, false, s.No, st), "split conversion");
+}
+void convert_tri(const DevSystem &s, const double *x, const TriGeom &gx,
+                 const TriOp &o, const TriGeom &g, hipStream_t st) {
+  for (uint16_t *p : {o.p, o.sw}) {
+    if (!p) continue;
+    OpSink k;
+    k.t = p;
+    check(launch_convert(x, gx, k, g, p == o.sw, s.No, st),
+          "bf16x3 conversion");
   }
 }
 }
@@ -40,21 +74,26 @@ void alloc_tri(DevSystem &s, TriOp &o, const TriGeom &g, const char *what) {
 // mixed-precision run.
 void atrip_amd::ensure_split(atrip_hip_ctx *ctx, DevSystem &s) {
   if (s.split_ready) return;
-  const int64_t No = s.No, Nv = s.Nv, N2 = No * No, Nv2 = Nv * Nv;
-  auto make = [&](const double *x, DevSystem::Split &o, int64_t n) {
+  const int64_t No = s.No, Nv = s.Nv;
+  const TriGeom ga = f64_geom_a(No, Nv, s.Kv), gb = f64_geom_b(No, Nv, s.Kv),
+                gh = f64_geom_a(No, Nv, s.Ko), gt = f64_geom_b(No, Nv, s.Ko);
+  CopyGuard guard(s);
+  auto make = [&](const double *x, DevSystem::Split &o, const TriGeom &g) {
     if (!x) return;
-    o.h = (float *)dev_bytes(s, (size_t)n * sizeof(float), "alloc split");
-    o.l = (uint16_t *)dev_bytes(s, (size_t)n * 2, "alloc split");
-    check(launch_split(x, o, n, ctx->stream), "split conversion");
+    const size_t n = (size_t)(g.no * g.nr * g.K);
+    o.h = (float *)dev_bytes(s, n * sizeof(float), "alloc split");
+    o.l = (uint16_t *)dev_bytes(s, n * 2, "alloc split");
+    convert_split(s, x, g, o, ctx->stream);
   };
-  make(s.T3, s.sT3, Nv * N2 * s.Kv);
-  make(s.V3, s.sV3, Nv2 * No * s.Kv);
-  make(s.H3, s.sH3, Nv * N2 * s.Ko);
-  make(s.T2N, s.sT2N, Nv2 * No * s.Ko);
-  make(s.T2TN, s.sT2TN, Nv2 * No * s.Ko);
-  make(s.V3J, s.sV3J, Nv2 * No * s.Kv);
-  make(s.H3J, s.sH3J, Nv * N2 * s.Ko);
+  make(s.T3, s.sT3, ga);
+  make(s.V3, s.sV3, gb);
+  make(s.H3, s.sH3, gh);
+  make(s.T2N, s.sT2N, gt);
+  make(s.T2TN, s.sT2TN, gt);
+  make(s.V3J, s.sV3J, gb);
+  make(s.H3J, s.sH3J, gh);
   check(hipStreamSynchronize(ctx->stream), "split conversion");
+  guard.done = true;
   s.split_ready = true;
 }
 
@@ -81,21 +120,23 @@ void atrip_amd::check_precision(const DevSystem &s, int precision) {
 void atrip_amd::ensure_tri(atrip_hip_ctx *ctx, DevSystem &s) {
   if (s.tri_ready) return;
   const int64_t No = s.No, Nv = s.Nv;
-  const TriGeom ga = tri_geom_a(No, Nv, s.Kv), gb = tri_geom_b(No, Nv, s.Kv),
-                gh = tri_geom_a(No, Nv, s.Ko), gt = tri_geom_b(No, Nv, s.Ko);
-  auto make = [&](const double *x, TriOp &o, const TriGeom &g) {
+  CopyGuard guard(s);
+  auto make = [&](const double *x, TriOp &o, bool a, int64_t K) {
     if (!x) return;
+    const TriGeom g = a ? tri_geom_a(No, Nv, K) : tri_geom_b(No, Nv, K);
     alloc_tri(s, o, g, "alloc bf16x3");
-    check(launch_tri(x, o, g, No, ctx->stream), "bf16x3 conversion");
+    convert_tri(s, x, a ? f64_geom_a(No, Nv, K) : f64_geom_b(No, Nv, K), o, g,
+                ctx->stream);
   };
-  make(s.T3, s.tT3, ga);
-  make(s.V3, s.tV3, gb);
-  make(s.H3, s.tH3, gh);
-  make(s.T2N, s.tT2N, gt);
-  make(s.T2TN, s.tT2TN, gt);
-  make(s.V3J, s.tV3J, gb);
-  make(s.H3J, s.tH3J, gh);
+  make(s.T3, s.tT3, true, s.Kv);
+  make(s.V3, s.tV3, false, s.Kv);
+  make(s.H3, s.tH3, true, s.Ko);
+  make(s.T2N, s.tT2N, false, s.Ko);
+  make(s.T2TN, s.tT2TN, false, s.Ko);
+  make(s.V3J, s.tV3J, false, s.Kv);
+  make(s.H3J, s.tH3J, true, s.Ko);
   check(hipStreamSynchronize(ctx->stream), "bf16x3 conversion");
+  guard.done = true;
   s.tri_ready = true;
 }
 
@@ -107,8 +148,63 @@ double *dev_alloc(DevSystem &s, int64_t n, const char *what) {
   check(hipMalloc(&p, bytes), what);
   s.allocations.push_back(p);
   s.bytes += bytes;
-  check(hipMemset(p, 0, bytes), what);
   return (double *)p;
+}
+
+// The row-swapped copies of a system's FP64 A operands and the copies they
+// belong to, with their contraction lengths.
+struct SwapCopy {
+  double **copy, *from;
+  int64_t K;
+};
+std::vector<SwapCopy> swap_copies(DevSystem &s) {
+  std::vector<SwapCopy> v;
+  auto add = [&](double *&copy, double *from, int64_t K) {
+    if (from) v.push_back({&copy, from, K});
+  };
+  add(s.T3s, s.T3, s.Kv);
+  add(s.H3s, s.H3, s.Ko);
+  add(s.H3Js, s.H3J, s.Ko);
+  add(s.T3is, s.T3i, s.Kv);
+  add(s.H3is, s.H3i, s.Ko);
+  add(s.H3Jis, s.H3Ji, s.Ko);
+  add(s.T3ins, s.T3in, s.Kv);
+  add(s.H3ins, s.H3in, s.Ko);
+  add(s.H3Jins, s.H3Jin, s.Ko);
+  return v;
+}
+
+// Allocates the row-swapped copies that fit; one that finds no memory stays
+// null and the kernels read the swapped rows from the straight array.
+void alloc_swaps(DevSystem &s) {
+  for (const SwapCopy &c : swap_copies(s)) {
+    const size_t bytes =
+        (size_t)f64_elems(f64_geom_a(s.No, s.Nv, c.K)) * sizeof(double);
+    void *p = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      continue;
+    }
+    s.allocations.push_back(p);
+    s.bytes += bytes;
+    *c.copy = (double *)p;
+  }
+}
+
+// Zeroes the FP64 operands of a system whose upload leaves their padding
+// unwritten.
+void clear_operands(DevSystem &s, hipStream_t st) {
+  auto zero = [&](double *x, bool a, int64_t K) {
+    if (!x) return;
+    const TriGeom g = a ? f64_geom_a(s.No, s.Nv, K) : f64_geom_b(s.No, s.Nv, K);
+    check(hipMemsetAsync(x, 0, (size_t)f64_elems(g) * sizeof(double), st),
+          "clear operands");
+  };
+  for (double *x : {s.T3, s.T3s, s.T3i, s.T3is}) zero(x, true, s.Kv);
+  for (double *x : {s.H3, s.H3s, s.H3J, s.H3Js, s.H3i, s.H3is, s.H3Ji, s.H3Jis})
+    zero(x, true, s.Ko);
+  for (double *x : {s.V3, s.V3J, s.V3i, s.V3Ji}) zero(x, false, s.Kv);
+  for (double *x : {s.T2N, s.T2TN, s.T2Ni, s.T2TNi}) zero(x, false, s.Ko);
 }
 
 void *dev_bytes(DevSystem &s, size_t bytes, const char *what) {
@@ -126,10 +222,28 @@ void free_system(DevSystem &s) {
 
 }  // namespace
 
+bool atrip_amd::drop_swap_copies(atrip_hip_ctx *ctx) {
+  bool any = false;
+  if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
+  for (auto &kv : ctx->systems) {
+    DevSystem &s = kv.second;
+    for (const SwapCopy &c : swap_copies(s)) {
+      if (!*c.copy) continue;
+      s.allocations.erase(std::find(s.allocations.begin(), s.allocations.end(),
+                                    (void *)*c.copy));
+      (void)hipFree(*c.copy);
+      *c.copy = nullptr;
+      s.bytes -= (uint64_t)f64_elems(f64_geom_a(s.No, s.Nv, c.K)) * sizeof(double);
+      any = true;
+    }
+  }
+  return any;
+}
+
 // Device bytes alloc_system takes for a system (the arrays below, the
 // packed point table and the canonical-index prefix).
 uint64_t atrip_amd::system_bytes(int64_t No, int64_t Nv, bool with_j,
-                                 int store) {
+                                 int store, bool swaps) {
   const uint64_t Kv = pad16(Nv), Ko = pad16(No), N2 = No * No, Nv2 = Nv * Nv;
   const auto d = [](uint64_t n) { return std::max<uint64_t>(n, 1) * 8; };
   // doubles operands: 8 bytes per element as FP64, 6 as split (4 + 2), 4
@@ -143,6 +257,12 @@ uint64_t atrip_amd::system_bytes(int64_t No, int64_t Nv, bool with_j,
          tri_bytes(tri_geom_a(No, Nv, Ko)) + 2 * tri_bytes(tri_geom_b(No, Nv, Ko));
     if (with_j)
       b += tri_bytes(tri_geom_b(No, Nv, Kv)) + tri_bytes(tri_geom_a(No, Nv, Ko));
+  } else if (store == 0) {
+    const auto f = [&](const TriGeom &g) { return d((uint64_t)f64_elems(g)); };
+    const uint64_t t3 = f(f64_geom_a(No, Nv, Kv)), h3 = f(f64_geom_a(No, Nv, Ko)),
+                   v3 = f(f64_geom_b(No, Nv, Kv));
+    b += t3 + v3 + h3 + 2 * f(f64_geom_b(No, Nv, Ko)) + (swaps ? t3 + h3 : 0);
+    if (with_j) b += v3 + h3 + (swaps ? h3 : 0);
   } else {
     b += o(Nv * N2 * Kv) + o(Nv2 * No * Kv) + o(Nv * N2 * Ko) +
          2 * o(Nv2 * No * Ko);
@@ -172,11 +292,12 @@ void alloc_system(atrip_hip_ctx *ctx, DevSystem &s, int64_t No, int64_t Nv,
                      const TriGeom &g, const char *what) {
     const int64_t n = g.no * g.nr * g.K;
     if (s.store == 0) {
-      x = dev_alloc(s, n, what);
+      x = dev_alloc(s, f64_elems(g), what);
       return;
     }
     if (s.store == 3) {
-      alloc_tri(s, tp, g, what);
+      alloc_tri(s, tp, g.swapped ? tri_geom_a(No, Nv, g.K) : tri_geom_b(No, Nv, g.K),
+                what);
       return;
     }
     sp.h = (float *)dev_bytes(s, (size_t)n * sizeof(float), what);
@@ -184,8 +305,8 @@ void alloc_system(atrip_hip_ctx *ctx, DevSystem &s, int64_t No, int64_t Nv,
       sp.l = (uint16_t *)dev_bytes(s, (size_t)n * 2, what);
     }
   };
-  const TriGeom ga = tri_geom_a(No, Nv, s.Kv), gb = tri_geom_b(No, Nv, s.Kv),
-                gh = tri_geom_a(No, Nv, s.Ko), gt = tri_geom_b(No, Nv, s.Ko);
+  const TriGeom ga = f64_geom_a(No, Nv, s.Kv), gb = f64_geom_b(No, Nv, s.Kv),
+                gh = f64_geom_a(No, Nv, s.Ko), gt = f64_geom_b(No, Nv, s.Ko);
   operand(s.T3, s.sT3, s.tT3, ga, "alloc T3");
   operand(s.V3, s.sV3, s.tV3, gb, "alloc V3");
   operand(s.H3, s.sH3, s.tH3, gh, "alloc H3");
@@ -204,23 +325,24 @@ void alloc_system(atrip_hip_ctx *ctx, DevSystem &s, int64_t No, int64_t Nv,
   }
   s.cplx = cplx;
   if (cplx) {
-    s.T3i = dev_alloc(s, Nv * N2 * s.Kv, "alloc T3 (im)");
-    s.V3i = dev_alloc(s, Nv2 * No * s.Kv, "alloc V3 (im)");
-    s.H3i = dev_alloc(s, Nv * N2 * s.Ko, "alloc H3 (im)");
-    s.T2Ni = dev_alloc(s, Nv2 * No * s.Ko, "alloc T2N (im)");
-    s.T2TNi = dev_alloc(s, Nv2 * No * s.Ko, "alloc T2TN (im)");
+    s.T3i = dev_alloc(s, f64_elems(ga), "alloc T3 (im)");
+    s.V3i = dev_alloc(s, f64_elems(gb), "alloc V3 (im)");
+    s.H3i = dev_alloc(s, f64_elems(gh), "alloc H3 (im)");
+    s.T2Ni = dev_alloc(s, f64_elems(gt), "alloc T2N (im)");
+    s.T2TNi = dev_alloc(s, f64_elems(gt), "alloc T2TN (im)");
     s.VHHi = dev_alloc(s, Nv2 * N2, "alloc VHH (im)");
     s.Taii = dev_alloc(s, Nv * No, "alloc Tai (im)");
     s.eii = dev_alloc(s, No, "alloc ei (im)");
     s.eai = dev_alloc(s, Nv, "alloc ea (im)");
-    s.T3in = dev_alloc(s, Nv * N2 * s.Kv, "alloc -T3 (im)");
-    s.H3in = dev_alloc(s, Nv * N2 * s.Ko, "alloc -H3 (im)");
+    s.T3in = dev_alloc(s, f64_elems(ga), "alloc -T3 (im)");
+    s.H3in = dev_alloc(s, f64_elems(gh), "alloc -H3 (im)");
     if (with_j) {
-      s.V3Ji = dev_alloc(s, Nv2 * No * s.Kv, "alloc V3J (im)");
-      s.H3Ji = dev_alloc(s, Nv * N2 * s.Ko, "alloc H3J (im)");
-      s.H3Jin = dev_alloc(s, Nv * N2 * s.Ko, "alloc -H3J (im)");
+      s.V3Ji = dev_alloc(s, f64_elems(gb), "alloc V3J (im)");
+      s.H3Ji = dev_alloc(s, f64_elems(gh), "alloc H3J (im)");
+      s.H3Jin = dev_alloc(s, f64_elems(gh), "alloc -H3J (im)");
     }
   }
+  if (s.store == 0 && ctx->operand_swaps) alloc_swaps(s);
   // i >= j >= k points of the energy loops, packed 10 bits per index
   std::vector<uint32_t> pts;
   for (int64_t k = 0; k < No; k++)
@@ -389,44 +511,41 @@ void staged(atrip_hip_ctx *ctx, Source &src, int t, int64_t slab,
 struct TempOperands {
   DevSystem &s;
   hipStream_t st;
-  std::vector<std::pair<double **, DevSystem::Split *>> items;
-  std::vector<std::pair<TriOp *, TriGeom>> tris;
-  std::vector<int64_t> sizes;
+  struct Item {
+    double **x;
+    DevSystem::Split *sp;
+    TriOp *tp;
+    TriGeom g;  // of the FP64 array
+  };
+  std::vector<Item> items;
   void add(double *&x, DevSystem::Split &sp, TriOp &tp, const TriGeom &g) {
-    const int64_t n = g.no * g.nr * g.K;
     if (s.store == 0) return;
+    const size_t bytes = (size_t)f64_elems(g) * sizeof(double);
     void *p = nullptr;
-    check(hipMalloc(&p, (size_t)std::max<int64_t>(n, 1) * sizeof(double)),
-          "alloc temporary operand");
-    check(hipMemsetAsync(p, 0, (size_t)std::max<int64_t>(n, 1) * sizeof(double),
-                         st),
-          "clear temporary operand");
+    check(hipMalloc(&p, bytes), "alloc temporary operand");
     x = (double *)p;
-    items.push_back({&x, &sp});
-    tris.push_back({&tp, g});
-    sizes.push_back(n);
+    items.push_back({&x, &sp, &tp, g});
+    check(hipMemsetAsync(p, 0, bytes, st), "clear temporary operand");
   }
   void convert() {
-    for (size_t q = 0; q < items.size(); q++) {
+    for (Item &it : items) {
       if (s.store == 3)
-        check(launch_tri(*items[q].first, *tris[q].first, tris[q].second,
-                         s.No, st),
-              "bf16x3 conversion");
+        convert_tri(s, *it.x, it.g, *it.tp,
+                    it.g.swapped ? tri_geom_a(s.No, s.Nv, it.g.K)
+                                 : tri_geom_b(s.No, s.Nv, it.g.K),
+                    st);
       else
-        check(launch_split(*items[q].first, *items[q].second, sizes[q], st),
-              "split conversion");
-      check(hipStreamSynchronize(st), "split conversion");
-      (void)hipFree(*items[q].first);
-      *items[q].first = nullptr;
+        convert_split(s, *it.x, it.g, *it.sp, st);
+      check(hipStreamSynchronize(st), "operand conversion");
+      (void)hipFree(*it.x);
+      *it.x = nullptr;
     }
     items.clear();
-    tris.clear();
-    sizes.clear();
   }
   ~TempOperands() {
-    for (auto &it : items) {
-      (void)hipFree(*it.first);
-      *it.first = nullptr;
+    for (Item &it : items) {
+      (void)hipFree(*it.x);
+      *it.x = nullptr;
     }
   }
 };
@@ -444,29 +563,45 @@ void upload_tensors(atrip_hip_ctx *ctx, DevSystem &s, DevSystem *im,
   if ((m == 2) != (im != nullptr)) throw Fail{"internal: complex parts"};
   DevSystem *dst[2] = {&s, im};
   hipStream_t st = ctx->stream;
-  TempOperands tmp{s, st, {}, {}};
-  tmp.add(s.T3, s.sT3, s.tT3, tri_geom_a(No, Nv, Kv));
-  tmp.add(s.T2N, s.sT2N, s.tT2N, tri_geom_b(No, Nv, Ko));
-  tmp.add(s.T2TN, s.sT2TN, s.tT2TN, tri_geom_b(No, Nv, Ko));
+  clear_operands(s, st);
+  TempOperands tmp{s, st, {}};
+  tmp.add(s.T3, s.sT3, s.tT3, f64_geom_a(No, Nv, Kv));
+  tmp.add(s.T2N, s.sT2N, s.tT2N, f64_geom_b(No, Nv, Ko));
+  tmp.add(s.T2TN, s.sT2TN, s.tT2TN, f64_geom_b(No, Nv, Ko));
+  const int64_t N2p = pad16(N2);
+  // straight array, then its row-swapped copy when there is one
+  auto both = [&](double *x, double *xs, const double *c, int64_t no,
+                  int64_t na, int64_t nb, int64_t so, int64_t sa, int64_t sb,
+                  TileMap straight, TileMap swapped, const char *what) {
+    check(launch_transpose_tiled(c, x, no, na, nb, so, sa, sb, straight, 1.0, st),
+          what);
+    if (xs)
+      check(launch_transpose_tiled(c, xs, no, na, nb, so, sa, sb, swapped, 1.0, st),
+            what);
+  };
   // Tabij {Nv,Nv,No,No}: slowest index j
   staged(ctx, src, ATRIP_TENSOR_TABIJ, Nv2 * No, No,
          [&](const double *c, int64_t j0, int64_t cj) {
            for (int part = 0; part < m; part++) {
              DevSystem &d = *dst[part];
              // T3[x][p + No q][E] = T[x,E,p,q], rows of this chunk: q = j
-             check(launch_transpose(c + part, d.T3 + j0 * No * Kv, No * cj, Nv,
-                                    Nv, m * Nv2, m * Nv, m, Kv, 1, N2 * Kv,
-                                    1.0, st),
-                   "relayout T3");
+             TileMap t, w;
+             t.R0 = j0 * No; t.Ro = 1; t.Rb = N2p; t.ka = 1; t.K = Kv;
+             w = t;
+             w.R0 = w.Ro = 0; w.swap = 1; w.row0 = j0 * No; w.No = No;
+             both(d.T3, d.T3s, c + part, No * cj, Nv, Nv, m * Nv2, m * Nv, m,
+                  t, w, "relayout T3");
              // T2N[pair][n][L] = -T[pair,L,n], n = j
-             check(launch_transpose(c + part, d.T2N + j0 * Ko, cj, No, Nv2,
-                                    m * Nv2 * No, m * Nv2, m, Ko, 1, No * Ko,
-                                    -1.0, st),
+             TileMap n;
+             n.R0 = j0; n.Ro = 1; n.Rb = No; n.ka = 1; n.K = Ko;
+             check(launch_transpose_tiled(c + part, d.T2N, cj, No, Nv2,
+                                          m * Nv2 * No, m * Nv2, m, n, -1.0, st),
                    "relayout T2N");
              // T2TN[pair][n][L] = -T[pair,n,L], L = j
-             check(launch_transpose(c + part, d.T2TN + j0, cj, No, Nv2,
-                                    m * Nv2 * No, m * Nv2, m, 1, Ko, No * Ko,
-                                    -1.0, st),
+             TileMap l;
+             l.Ra = 1; l.Rb = No; l.k0 = j0; l.ko = 1; l.K = Ko;
+             check(launch_transpose_tiled(c + part, d.T2TN, cj, No, Nv2,
+                                          m * Nv2 * No, m * Nv2, m, l, -1.0, st),
                    "relayout T2TN");
            }
          });
@@ -480,39 +615,45 @@ void upload_tensors(atrip_hip_ctx *ctx, DevSystem &s, DevSystem *im,
                    "relayout VHH");
          });
   // Vijka {No,No,No,Nv}: H3[x][row][L] = V[row,L,x]
-  auto hhh = [&](int t, double *DevSystem::*arr) {
+  auto hhh = [&](int t, double *DevSystem::*arr, double *DevSystem::*arrs) {
     staged(ctx, src, t, N2 * No, Nv,
            [&](const double *c, int64_t x0, int64_t cx) {
-             for (int part = 0; part < m; part++)
-               check(launch_transpose(c + part, dst[part]->*arr + x0 * N2 * Ko,
-                                      cx, No, N2, m * N2 * No, m * N2, m,
-                                      N2 * Ko, 1, Ko, 1.0, st),
-                     "relayout H3");
+             for (int part = 0; part < m; part++) {
+               TileMap t, w;
+               t.R0 = x0 * N2p; t.Ro = N2p; t.Rb = 1; t.ka = 1; t.K = Ko;
+               w = t;
+               w.Rb = 0; w.swap = 2; w.No = No;
+               both(dst[part]->*arr, dst[part]->*arrs, c + part, cx, No, N2,
+                    m * N2 * No, m * N2, m, t, w, "relayout H3");
+             }
            });
   };
   // Vabci {Nv,Nv,Nv,No}: V3[pair][r][E] = V[pair,E,r]
   auto ppph = [&](int t, double *DevSystem::*arr) {
     staged(ctx, src, t, Nv2 * Nv, No,
            [&](const double *c, int64_t r0, int64_t cr) {
-             for (int part = 0; part < m; part++)
-               check(launch_transpose(c + part, dst[part]->*arr + r0 * Kv, cr,
-                                      Nv, Nv2, m * Nv2 * Nv, m * Nv2, m, Kv, 1,
-                                      No * Kv, 1.0, st),
+             for (int part = 0; part < m; part++) {
+               TileMap t;
+               t.R0 = r0; t.Ro = 1; t.Rb = No; t.ka = 1; t.K = Kv;
+               check(launch_transpose_tiled(c + part, dst[part]->*arr, cr, Nv,
+                                            Nv2, m * Nv2 * Nv, m * Nv2, m, t,
+                                            1.0, st),
                      "relayout V3");
+             }
            });
   };
   tmp.convert();
-  tmp.add(s.H3, s.sH3, s.tH3, tri_geom_a(No, Nv, Ko));
-  hhh(ATRIP_TENSOR_VIJKA, &DevSystem::H3);
+  tmp.add(s.H3, s.sH3, s.tH3, f64_geom_a(No, Nv, Ko));
+  hhh(ATRIP_TENSOR_VIJKA, &DevSystem::H3, &DevSystem::H3s);
   tmp.convert();
-  tmp.add(s.V3, s.sV3, s.tV3, tri_geom_b(No, Nv, Kv));
+  tmp.add(s.V3, s.sV3, s.tV3, f64_geom_b(No, Nv, Kv));
   ppph(ATRIP_TENSOR_VABCI, &DevSystem::V3);
   tmp.convert();
   if (s.has_j) {
-    tmp.add(s.H3J, s.sH3J, s.tH3J, tri_geom_a(No, Nv, Ko));
-    hhh(ATRIP_TENSOR_JIJKA, &DevSystem::H3J);
+    tmp.add(s.H3J, s.sH3J, s.tH3J, f64_geom_a(No, Nv, Ko));
+    hhh(ATRIP_TENSOR_JIJKA, &DevSystem::H3J, &DevSystem::H3Js);
     tmp.convert();
-    tmp.add(s.V3J, s.sV3J, s.tV3J, tri_geom_b(No, Nv, Kv));
+    tmp.add(s.V3J, s.sV3J, s.tV3J, f64_geom_b(No, Nv, Kv));
     ppph(ATRIP_TENSOR_JABCI, &DevSystem::V3J);
     tmp.convert();
   }
@@ -541,20 +682,29 @@ DevSystem imag_view(const DevSystem &s) {
   v.T3 = s.T3i; v.V3 = s.V3i; v.H3 = s.H3i; v.T2N = s.T2Ni;
   v.T2TN = s.T2TNi; v.VHH = s.VHHi; v.Tai = s.Taii; v.ei = s.eii;
   v.ea = s.eai; v.V3J = s.V3Ji; v.H3J = s.H3Ji;
+  v.T3s = s.T3is; v.H3s = s.H3is; v.H3Js = s.H3Jis;
   v.aprefix = s.aprefix;
   return v;
 }
 
 // Negated imaginary planes of T3 and the hole integrals.
 void complex_negations(atrip_hip_ctx *ctx, DevSystem &s) {
-  const int64_t N2 = s.No * s.No;
-  check(launch_scale(s.T3i, s.T3in, s.Nv * N2 * s.Kv, -1.0, ctx->stream),
-        "negate T3 (im)");
-  check(launch_scale(s.H3i, s.H3in, s.Nv * N2 * s.Ko, -1.0, ctx->stream),
-        "negate H3 (im)");
-  if (s.has_j)
-    check(launch_scale(s.H3Ji, s.H3Jin, s.Nv * N2 * s.Ko, -1.0, ctx->stream),
-          "negate H3J (im)");
+  const int64_t nt = f64_elems(f64_geom_a(s.No, s.Nv, s.Kv)),
+                nh = f64_elems(f64_geom_a(s.No, s.Nv, s.Ko));
+  auto neg = [&](const double *x, double *y, int64_t n) {
+    if (x && y)
+      check(launch_scale(x, y, n, -1.0, ctx->stream), "negate imaginary plane");
+  };
+  // a swapped negated copy needs its swapped source
+  auto pair = [&](const double *x, double *y, const double *xs, double *&ys,
+                  int64_t n) {
+    neg(x, y, n);
+    if (!xs) ys = nullptr;
+    neg(xs, ys, n);
+  };
+  pair(s.T3i, s.T3in, s.T3is, s.T3ins, nt);
+  pair(s.H3i, s.H3in, s.H3is, s.H3ins, nh);
+  pair(s.H3Ji, s.H3Jin, s.H3Jis, s.H3Jins, nh);
   check(hipStreamSynchronize(ctx->stream), "negations");
 }
 
@@ -578,6 +728,10 @@ void complex_passes(const DevSystem &s, DevSystem v[4]) {
   v[2].T2TN = s.T2TNi; v[2].V3J = s.V3Ji; v[2].H3J = s.H3J;
   v[3].T3 = s.T3i;  v[3].V3 = s.V3;  v[3].H3 = s.H3in; v[3].T2N = s.T2N;
   v[3].T2TN = s.T2TN;  v[3].V3J = s.V3J;  v[3].H3J = s.H3Jin;
+  v[0].T3s = s.T3s;   v[0].H3s = s.H3s;   v[0].H3Js = s.H3Js;
+  v[1].T3s = s.T3ins; v[1].H3s = s.H3is;  v[1].H3Js = s.H3Jis;
+  v[2].T3s = s.T3s;   v[2].H3s = s.H3s;   v[2].H3Js = s.H3Js;
+  v[3].T3s = s.T3is;  v[3].H3s = s.H3ins; v[3].H3Js = s.H3Jins;
 }
 
 // Host-side canonical index, identical to the device one.
@@ -1128,7 +1282,7 @@ const char *atrip_hip_last_error(atrip_hip_ctx *ctx) {
 
 int atrip_hip_upload(atrip_hip_ctx *ctx, const atrip_sys_desc *desc,
                      int *sys) {
-  return guarded(ctx, [&] {
+  return guarded_memory(ctx, [&] {
     if (!desc || !sys) throw Fail{"null argument"};
     if (!desc->ei || !desc->ea || !desc->Tai || !desc->Tabij ||
         !desc->Vabij || !desc->Vijka || !desc->Vabci)
@@ -1160,7 +1314,7 @@ int atrip_hip_upload_synthetic(atrip_hip_ctx *ctx, int64_t No, int64_t Nv,
 int atrip_hip_upload_synthetic_scaled(atrip_hip_ctx *ctx, int64_t No,
                                       int64_t Nv, uint64_t seed, int with_j,
                                       double scale, int *sys) {
-  return guarded(ctx, [&] {
+  return guarded_memory(ctx, [&] {
     if (!sys) throw Fail{"null argument"};
     if (!std::isfinite(scale)) throw Fail{"scale must be finite"};
     check(hipSetDevice(ctx->device), "hipSetDevice");
@@ -1182,7 +1336,7 @@ int atrip_hip_upload_synthetic_scaled(atrip_hip_ctx *ctx, int64_t No,
 
 int atrip_hip_upload_complex(atrip_hip_ctx *ctx, const atrip_sys_desc *desc,
                              int *sys) {
-  return guarded(ctx, [&] {
+  return guarded_memory(ctx, [&] {
     if (!desc || !sys) throw Fail{"null argument"};
     if (!desc->ei || !desc->ea || !desc->Tai || !desc->Tabij ||
         !desc->Vabij || !desc->Vijka || !desc->Vabci)
@@ -1211,7 +1365,7 @@ int atrip_hip_upload_complex(atrip_hip_ctx *ctx, const atrip_sys_desc *desc,
 int atrip_hip_upload_stream(atrip_hip_ctx *ctx, int64_t No, int64_t Nv,
                             int flags, atrip_read_fn read, void *user,
                             int *sys) {
-  return guarded(ctx, [&] {
+  return guarded_memory(ctx, [&] {
     if (!read || !sys) throw Fail{"null argument"};
     if (flags & ~(ATRIP_STREAM_WITH_J | ATRIP_STREAM_COMPLEX))
       throw Fail{"unknown upload flags"};
@@ -1244,7 +1398,7 @@ int atrip_hip_upload_stream(atrip_hip_ctx *ctx, int64_t No, int64_t Nv,
 int atrip_hip_upload_synthetic_complex(atrip_hip_ctx *ctx, int64_t No,
                                        int64_t Nv, uint64_t seed, int with_j,
                                        int *sys) {
-  return guarded(ctx, [&] {
+  return guarded_memory(ctx, [&] {
     if (!sys) throw Fail{"null argument"};
     check(hipSetDevice(ctx->device), "hipSetDevice");
     DevSystem s;
@@ -1279,7 +1433,7 @@ int atrip_hip_release(atrip_hip_ctx *ctx, int sys) {
 int atrip_hip_run(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
                   uint64_t first, uint64_t count, double *energy,
                   double *ct_energy) {
-  return guarded(ctx, [&] {
+  return guarded_memory(ctx, [&] {
     if (!energy) throw Fail{"null energy pointer"};
     check(hipSetDevice(ctx->device), "hipSetDevice");
     const uint64_t last =
@@ -1295,7 +1449,7 @@ int atrip_hip_run_windows(atrip_hip_ctx *ctx, int sys, int precision,
                           int ijkabc, uint64_t stride, uint64_t offset,
                           double *energy, double *ct_energy,
                           uint64_t *tuples) {
-  return guarded(ctx, [&] {
+  return guarded_memory(ctx, [&] {
     if (!energy) throw Fail{"null energy pointer"};
     if (stride == 0) throw Fail{"stride must be positive"};
     check(hipSetDevice(ctx->device), "hipSetDevice");
@@ -1312,7 +1466,7 @@ int atrip_hip_run_windows(atrip_hip_ctx *ctx, int sys, int precision,
 int atrip_hip_tuple_energies(atrip_hip_ctx *ctx, int sys, int precision,
                              int ijkabc, uint64_t first, uint64_t count,
                              double *e, double *e_ct) {
-  return guarded(ctx, [&] {
+  return guarded_memory(ctx, [&] {
     if (!e) throw Fail{"null output pointer"};
     check(hipSetDevice(ctx->device), "hipSetDevice");
     DevSystem &s = get_sys(ctx, sys);

@@ -161,6 +161,7 @@ BSys make_bsys(atrip_hip_ctx *ctx, DevSystem &s, const BatchTune &p,
   if (precision != ATRIP_FP64) ensure_split(ctx, s);
   BSys b;
   b.T3 = s.T3; b.V3 = s.V3; b.H3 = s.H3; b.T2N = s.T2N; b.T2TN = s.T2TN;
+  b.T3s = s.T3s; b.H3s = s.H3s;
   b.VHH = s.VHH; b.Tai = s.Tai; b.ei = s.ei; b.ea = s.ea;
   b.points = s.points;
   b.No = s.No; b.Nv = s.Nv; b.Kv = s.Kv; b.Ko = s.Ko; b.npoints = s.npoints;
@@ -321,7 +322,7 @@ int atrip_hip_batch_plan(atrip_hip_ctx *ctx, int sys, int precision, int *nb,
 
 int atrip_hip_batch_run(atrip_hip_ctx *ctx, const int *systems, int nsys,
                         int precision, double *energies) {
-  return guarded(ctx, [&] {
+  return guarded_memory(ctx, [&] {
     if (nsys < 0 || (nsys > 0 && (!systems || !energies)))
       throw Fail{"bad system list"};
     check_batched_precision(precision);
@@ -381,7 +382,7 @@ int atrip_hip_batch_run(atrip_hip_ctx *ctx, const int *systems, int nsys,
 
 int atrip_hip_batch_tune(atrip_hip_ctx *ctx, const int *systems, int nsys,
                          int precision, int mode) {
-  return guarded(ctx, [&] {
+  return guarded_memory(ctx, [&] {
     if (nsys < 0 || (nsys > 0 && !systems)) throw Fail{"bad system list"};
     if (mode != 0 && mode != 1) throw Fail{"mode must be 0 or 1"};
     check_batched_precision(precision);

@@ -27,6 +27,7 @@ namespace atrip_amd {
 namespace {
 
 typedef double d4 __attribute__((ext_vector_type(4)));
+typedef double d2 __attribute__((ext_vector_type(2)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
@@ -48,13 +49,13 @@ __device__ inline double wave_sum(double v) {
   return v;
 }
 
-// B operand base of segment sg for column tuple (a,b,c) of class cl.
+// B operand row of segment sg at index rr of column tuple (a,b,c), class cl.
 __device__ __forceinline__ const double *bbase(const BSys &S, int cl, int sg, int64_t a,
-                                      int64_t b, int64_t c) {
+                                      int64_t b, int64_t c, int64_t rr) {
   int64_t u, v;
   const int which = b_pair(cl, sg, a, b, c, u, v);
   const double *Bt = which == 0 ? S.V3 : which == 1 ? S.T2N : S.T2TN;
-  return Bt + (u + S.Nv * v) * S.No * (sg < 2 ? S.Kv : S.Ko);
+  return Bt + f64_row((u + S.Nv * v) * S.No + rr, sg < 2 ? S.Kv : S.Ko);
 }
 
 // Adds one wave tile into W (order i + No j + No^2 k).  Class u's column
@@ -198,49 +199,51 @@ __device__ __forceinline__ void wave_tile(const BSys &S, int cl, int al,
 #pragma unroll
     for (int g = 0; g < FN; g++) acc[f][g] = d4{0.0, 0.0, 0.0, 0.0};
   const double *ap[FM], *bp[FN];
-  d4 a0[FM], b0[FN], a1[FM], b1[FN];
-#define LOAD(AV, BV, KOFF)                                              \
+  d2 a0[FM], b0[FN], a1[FM], b1[FN];
+#define LOAD(AV, BV, C)                                                 \
   {                                                                     \
     _Pragma("unroll") for (int f = 0; f < FM; f++) AV[f] =              \
-        *(const d4 *)(ap[f] + (KOFF));                                  \
+        *(const d2 *)(ap[f] + 128 * (C));                               \
     _Pragma("unroll") for (int g = 0; g < FN; g++) BV[g] =              \
-        *(const d4 *)(bp[g] + (KOFF));                                  \
+        *(const d2 *)(bp[g] + 128 * (C));                               \
     __builtin_amdgcn_sched_barrier(0);                                  \
   }
 #define COMPUTE(AV, BV)                                                   \
   {                                                                       \
-    _Pragma("unroll") for (int s = 0; s < 4; s++)                         \
+    _Pragma("unroll") for (int s = 0; s < 2; s++)                         \
         _Pragma("unroll") for (int f = 0; f < FM; f++)                    \
             _Pragma("unroll") for (int g = 0; g < FN; g++) acc[f][g] =    \
                 __builtin_amdgcn_mfma_f64_16x16x4f64(AV[f][s], BV[g][s],  \
                                                      acc[f][g], 0, 0, 0); \
   }
   // segments: 0 T3[x1] straight, 1 T3[x2] swapped, 2 H3[x2] straight,
-  //           3 H3[x1] swapped; K runs are multiples of 16.  Each segment
-  // has its own two-stage pipeline: one pipeline through all four keeps the
-  // next segment's pointers live as well and costs the kernel its second
-  // wave per SIMD.
+  //           3 H3[x1] swapped, in 8-deep chunks (one operand tile each).
+  // Each segment has its own two-stage pipeline: one pipeline through all
+  // four keeps the next segment's pointers live as well and costs the kernel
+  // its second wave per SIMD.
+  const int64_t N2p = pad16(N2);
 #pragma unroll 1
   for (int sg = 0; sg < 4; sg++) {
     const int64_t K_ = sg < 2 ? Kv : Ko;
-    const double *Ab = sg < 2 ? S.T3 + (sg == 0 ? x1 : x2) * N2 * Kv
-                              : S.H3 + (sg == 2 ? x2 : x1) * N2 * Ko;
+    const double *As = sg < 2 ? S.T3s : S.H3s;  // null: the straight array
+    const bool sw = (sg & 1) && As;
+    const double *Ab = sw ? As : sg < 2 ? S.T3 : S.H3;
+    const int64_t xr = (sg == 0 || sg == 3 ? x1 : x2) * N2p;
 #pragma unroll
     for (int f = 0; f < FM; f++)
-      ap[f] = Ab + (int64_t)((sg & 1) ? rowW[f] : rowS[f]) * K_ + 4 * kk;
+      ap[f] = Ab + f64_row(xr + ((sg & 1) && !sw ? rowW[f] : rowS[f]), K_) + 32 * kk;
 #pragma unroll
     for (int g = 0; g < FN; g++)
-      bp[g] = bbase(S, cl, sg, ca[g], cb[g], cc[g]) + (int64_t)crr[g] * K_ +
-              4 * kk;
-    const int64_t last = K_ - KCHUNK;
+      bp[g] = bbase(S, cl, sg, ca[g], cb[g], cc[g], crr[g]) + 32 * kk;
+    const int last = (int)(((sg < 2 ? Nv : No) + 7) / 8) - 1;
     LOAD(a0, b0, 0);
-    for (int64_t k0 = 0;; k0 += 2 * KCHUNK) {
-      LOAD(a1, b1, k0 + KCHUNK < last ? k0 + KCHUNK : last);
+    for (int c = 0;; c += 2) {
+      LOAD(a1, b1, c + 1 < last ? c + 1 : last);
       COMPUTE(a0, b0);
-      if (k0 + KCHUNK > last) break;
-      LOAD(a0, b0, k0 + 2 * KCHUNK < last ? k0 + 2 * KCHUNK : last);
+      if (c + 1 > last) break;
+      LOAD(a0, b0, c + 2 < last ? c + 2 : last);
       COMPUTE(a1, b1);
-      if (k0 + 2 * KCHUNK > last) break;
+      if (c + 2 > last) break;
     }
   }
 #undef LOAD

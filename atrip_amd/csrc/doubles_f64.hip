@@ -16,13 +16,16 @@
 // in the W layout W[i + No j + No^2 k]; the energy kernel sums the three.
 //
 // MFMA v_mfma_f64_16x16x4f64, operands straight from global memory (L2/MALL
-// resident) into registers.  A K chunk of 16 is split over the lane groups
-// q = lane/16 as kappa = k0 + 2q + {0, 1} (k-steps 0, 1) and
-// k0 + 8 + 2q + {0, 1} (k-steps 2, 3): each of a lane's two 16-byte loads
-// then sits next to those of the other lane groups, so one load instruction
-// covers 64 contiguous bytes of each of its 16 rows (two whole 32-byte
-// sectors) and the L1 serves half the sector requests of a 32-byte-per-lane
-// split.
+// resident) into registers.  Operands are 16-row x 8-kappa tiles in lane
+// order (f64_at): lane group q = lane/16 feeds kappa k0 + 2q (k-step 0) and
+// k0 + 2q + 1 (k-step 1) of an 8-deep chunk, one 16-byte load per lane and
+// fragment over 1 KiB of consecutive addresses.  Read from rows K apart, as
+// before, the same load touched 64 lines, one L1 tag access each, and the
+// texture units were 80 % busy with them at 5x5 and the bound of every
+// smaller tile (No=16, Nv=120 with 4x4: 290 -> 245 us per launch of 2048
+// slots; 5x5 at No=40: 10.42 -> 10.25 ms).  An 8-deep chunk needs half the
+// operand registers of a 16-deep one, so tiles up to 4x4 run two waves per
+// SIMD.
 #include "doubles_common.hpp"
 
 namespace atrip_amd {
@@ -31,34 +34,33 @@ namespace {
 typedef double d4 __attribute__((ext_vector_type(4)));
 typedef double d2 __attribute__((ext_vector_type(2)));
 
-// A lane's four doubles of a chunk: 2q, 2q+1 and 8+2q, 9+2q past p.
-__device__ __forceinline__ d4 load_chunk(const double *p) {
-  const d2 lo = *(const d2 *)p, hi = *(const d2 *)(p + 8);
-  return __builtin_shufflevector(lo, hi, 0, 1, 2, 3);
-}
+constexpr int KC = 8;     // kappa per chunk: one operand tile
+constexpr int TILE = 128;  // doubles per operand tile
 
 struct DoublesParams {
-  const double *T3, *V3, *H3, *T2N, *T2TN;
+  // T3s, H3s: row-swapped copies (null: read the swapped rows of T3, H3)
+  const double *T3, *T3s, *V3, *H3, *H3s, *T2N, *T2TN;
   const int32_t *windows;
   const uint64_t *aprefix;
   double *G;
-  int64_t No, Nv, Kv, Ko, N2, W3, NoP, slots;
+  int64_t No, Nv, Kv, Ko, N2, N2p, W3, NoP, slots;
   uint64_t first, last;
   int nb, mtiles, ntiles;
   int64_t total, per_xcd;
 };
 
-// B operand base of segment sg for a column tuple.
+// B operand of segment sg at column (tuple (a, b, c), index rr): its row.
 __device__ inline const double *b_base(const DoublesParams &P, int cl, int sg,
-                                       int64_t a, int64_t b, int64_t c) {
+                                       int64_t a, int64_t b, int64_t c,
+                                       int64_t rr) {
   int64_t u, v;
   const int which = b_pair(cl, sg, a, b, c, u, v);
   const double *Bt = which == 0 ? P.V3 : which == 1 ? P.T2N : P.T2TN;
-  return Bt + (u + P.Nv * v) * P.No * (sg < 2 ? P.Kv : P.Ko);
+  return Bt + f64_row((u + P.Nv * v) * P.No + rr, sg < 2 ? P.Kv : P.Ko);
 }
 
 template <int FM, int FN>
-__global__ __launch_bounds__(256) void doubles_f64_kernel(DoublesParams P) {
+__global__ __launch_bounds__(256, FM *FN <= 16 ? 2 : 1) void doubles_f64_kernel(DoublesParams P) {
   constexpr int MT = 32 * FM, NT = 32 * FN;
   const int64_t bid = blockIdx.x;
   const int64_t logical = (bid % 8) * P.per_xcd + bid / 8;  // XCD-aware
@@ -126,12 +128,15 @@ __global__ __launch_bounds__(256) void doubles_f64_kernel(DoublesParams P) {
 #define SET_PTRS(SG)                                                        \
   {                                                                         \
     const int64_t K_ = (SG) < 2 ? Kv : Ko;                                  \
-    const double *Ab_ = (SG) < 2 ? P.T3 + ((SG) == 0 ? x1 : x2) * N2 * Kv   \
-                                 : P.H3 + ((SG) == 2 ? x2 : x1) * N2 * Ko;  \
+    const int64_t xr_ = ((SG) == 0 || (SG) == 3 ? x1 : x2) * P.N2p;         \
+    const double *As_ = (SG) < 2 ? P.T3s : P.H3s;                           \
+    const bool sw_ = ((SG)&1) && As_;                                       \
+    const double *Ab_ = sw_ ? As_ : (SG) < 2 ? P.T3 : P.H3;                 \
     _Pragma("unroll") for (int f = 0; f < FM; f++) ap[f] =                  \
-        Ab_ + (((SG)&1) ? rowW[f] : rowS[f]) * K_ + 2 * kk;                 \
+        Ab_ + f64_row(xr_ + (((SG)&1) && !sw_ ? rowW[f] : rowS[f]), K_) +   \
+        32 * kk;                                                            \
     _Pragma("unroll") for (int g = 0; g < FN; g++) bp[g] =                  \
-        b_base(P, cl, (SG), ca[g], cb[g], cc[g]) + crr[g] * K_ + 2 * kk;    \
+        b_base(P, cl, (SG), ca[g], cb[g], cc[g], crr[g]) + 32 * kk;         \
   }
   d4 acc[FM][FN];
 #pragma unroll
@@ -143,76 +148,59 @@ __global__ __launch_bounds__(256) void doubles_f64_kernel(DoublesParams P) {
   // chunk are in flight while the MFMAs of the other run (no register
   // copies between the sets, hence no wait on the in-flight loads).
   const double *ap[FM], *bp[FN];
-#define LOAD(AV, BV, KOFF)                                              \
+#define LOAD(AV, BV, C)                                                 \
   {                                                                     \
     _Pragma("unroll") for (int f = 0; f < FM; f++) AV[f] =              \
-        load_chunk(ap[f] + (KOFF));                                     \
+        *(const d2 *)(ap[f] + TILE * (C));                              \
     _Pragma("unroll") for (int g = 0; g < FN; g++) BV[g] =              \
-        load_chunk(bp[g] + (KOFF));                                     \
+        *(const d2 *)(bp[g] + TILE * (C));                              \
     __builtin_amdgcn_sched_barrier(0);                                  \
   }
-  // k-steps 0, 1 hold kappa k0 .. k0 + 7 and steps 2, 3 kappa k0 + 8 ..
-  // k0 + 15: a last chunk with at most 8 occupied kappa (the rest zero
-  // padding, which adds exact zeros) skips steps 2, 3
-#define STEPS(AV, BV, S0, S1)                                           \
-  _Pragma("unroll") for (int s = S0; s < S1; s++)                       \
+#define COMPUTE(AV, BV)                                                 \
+  _Pragma("unroll") for (int s = 0; s < 2; s++)                         \
       _Pragma("unroll") for (int f = 0; f < FM; f++)                    \
           _Pragma("unroll") for (int g = 0; g < FN; g++) acc[f][g] =    \
               __builtin_amdgcn_mfma_f64_16x16x4f64(AV[f][s], BV[g][s],  \
                                                    acc[f][g], 0, 0, 0);
-#define COMPUTE(AV, BV, HALF)                                           \
-  {                                                                     \
-    STEPS(AV, BV, 0, 2)                                                 \
-    if (!(HALF)) { STEPS(AV, BV, 2, 4) }                                \
-  }
-  d4 a0[FM], b0[FN], a1[FM], b1[FN];
+  d2 a0[FM], b0[FN], a1[FM], b1[FN];
   // One pipeline through the four segments: (sg, c) is the next chunk to
   // load, and past a segment's end the pointers move to the next segment's
   // chunk 0 in place, so every segment but the first starts with its first
   // chunk in flight (3 % faster at No=40 than a pipeline restarted per
-  // segment).  The prefetch is issued unconditionally (after the last chunk
-  // it re-reads it, a load never used) so every path into a COMPUTE has the
-  // same loads outstanding.  h0 / h1: the chunk in set 0 / 1 is a segment's
-  // last and holds at most 8 occupied kappa.
+  // segment).  A segment ends at the last chunk that holds an occupied
+  // kappa.  The prefetch is issued unconditionally (after the last chunk it
+  // re-reads it, a load never used) so every path into a COMPUTE has the
+  // same loads outstanding.
   int sg = 0;
-  int64_t nch = Kv / KCHUNK, c = 0;
-  bool t8 = P.Nv - (Kv - KCHUNK) <= 8;  // tail rule of segment sg
+  int nch = (int)((P.Nv + KC - 1) / KC), c = 0;
   SET_PTRS(0);
 #define ADVANCE()                                                            \
   {                                                                          \
     if (++c == nch && ++sg < 4) {                                            \
       SET_PTRS(sg);                                                          \
-      const int64_t K_ = sg < 2 ? Kv : Ko;                                   \
-      nch = K_ / KCHUNK;                                                     \
-      t8 = (sg < 2 ? P.Nv : No) - (K_ - KCHUNK) <= 8;                        \
+      nch = (int)(((sg < 2 ? P.Nv : No) + KC - 1) / KC);                     \
       c = 0;                                                                 \
     }                                                                        \
   }
-#define NEXT_OFF() (KCHUNK * (sg < 4 ? c : nch - 1))
-#define HALF_NEXT() (sg < 4 && t8 && c == nch - 1)
-  bool h0 = HALF_NEXT(), h1 = false;
+#define NEXT() ((int64_t)(sg < 4 ? c : nch - 1))
   LOAD(a0, b0, 0);
   ADVANCE();
 #pragma unroll 1
   for (;;) {
     const bool v1 = sg < 4;
-    h1 = HALF_NEXT();
-    LOAD(a1, b1, NEXT_OFF());
+    LOAD(a1, b1, NEXT());
     if (v1) ADVANCE();
-    COMPUTE(a0, b0, h0);
+    COMPUTE(a0, b0);
     if (!v1) break;
     const bool v2 = sg < 4;
-    h0 = HALF_NEXT();
-    LOAD(a0, b0, NEXT_OFF());
+    LOAD(a0, b0, NEXT());
     if (v2) ADVANCE();
-    COMPUTE(a1, b1, h1);
+    COMPUTE(a1, b1);
     if (!v2) break;
   }
 #undef ADVANCE
-#undef NEXT_OFF
-#undef HALF_NEXT
+#undef NEXT
 #undef LOAD
-#undef STEPS
 #undef COMPUTE
 
 #undef SET_PTRS
@@ -244,8 +232,10 @@ hipError_t launch_doubles_f64(const DevSystem &s, const BatchArgs &b,
                               hipStream_t st) {
   DoublesParams P;
   P.T3 = s.T3;
+  P.T3s = s.T3s;
   P.V3 = use_j ? s.V3J : s.V3;
   P.H3 = use_j ? s.H3J : s.H3;
+  P.H3s = use_j ? s.H3Js : s.H3s;
   P.T2N = s.T2N;
   P.T2TN = s.T2TN;
   P.windows = b.windows;
@@ -256,6 +246,7 @@ hipError_t launch_doubles_f64(const DevSystem &s, const BatchArgs &b,
   P.Kv = s.Kv;
   P.Ko = s.Ko;
   P.N2 = s.No * s.No;
+  P.N2p = pad16(P.N2);
   P.NoP = g_pitch(s.No, false);
   P.W3 = g_elems(s.No, false);
   P.slots = b.slots;

@@ -237,27 +237,7 @@ __global__ __launch_bounds__(256) void doubles_split_kernel(SplitParams P) {
   }
 }
 
-// x -> hi = (float)x, l = bf16(x - hi); bf16 by round to nearest even on
-// the float bits.
-__global__ __launch_bounds__(256) void split_kernel(const double *x, float *h,
-                                                    uint16_t *l, int64_t n) {
-  for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n;
-       q += (int64_t)gridDim.x * blockDim.x) {
-    split_store(x[q], h, l, q);
-  }
-}
-
 }  // namespace
-
-hipError_t launch_split(const double *x, DevSystem::Split &out, int64_t n,
-                        hipStream_t st) {
-  if (n <= 0) return hipSuccess;
-  int64_t blocks = (n + 255) / 256;
-  if (blocks > 65536L * 16) blocks = 65536L * 16;
-  hipLaunchKernelGGL(split_kernel, dim3((unsigned)blocks), dim3(256), 0, st, x,
-                     out.h, out.l, n);
-  return hipGetLastError();
-}
 
 hipError_t launch_doubles_split(const DevSystem &s, const BatchArgs &b,
                                 bool use_j, float *G, bool corrections,

@@ -233,28 +233,7 @@ __global__ __launch_bounds__(256) void doubles_tri_kernel(TriParams P) {
   }
 }
 
-// FP64 operand -> its tiled bf16x3 copy (and row-swapped copy).
-__global__ __launch_bounds__(256) void tri_kernel(const double *x, TriOp out,
-                                                  TriGeom g, int64_t No,
-                                                  int64_t n) {
-  for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n;
-       q += (int64_t)gridDim.x * blockDim.x)
-    tri_store(x[q], out, g, No, q);
-}
-
 }  // namespace
-
-hipError_t launch_tri(const double *x, const TriOp &out, const TriGeom &g,
-                      int64_t No, hipStream_t st) {
-  const int64_t n = g.no * g.nr * g.K;
-  if (n <= 0) return hipSuccess;
-  if (g.K % 16 || (g.swapped && g.nr != No * No)) return hipErrorInvalidValue;
-  int64_t blocks = (n + 255) / 256;
-  if (blocks > 65536L * 16) blocks = 65536L * 16;
-  hipLaunchKernelGGL(tri_kernel, dim3((unsigned)blocks), dim3(256), 0, st, x,
-                     out, g, No, n);
-  return hipGetLastError();
-}
 
 hipError_t launch_doubles_tri(const DevSystem &s, const BatchArgs &b,
                               bool use_j, float *G, int tile, hipStream_t st) {

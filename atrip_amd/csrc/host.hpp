@@ -56,7 +56,37 @@ void check_precision(const DevSystem &s, int precision);
 
 // Device bytes of the resident arrays of a system uploaded with operand
 // store mode `store` (what admission charges).
-uint64_t system_bytes(int64_t No, int64_t Nv, bool with_j, int store);
+// (`swaps`: with the row-swapped copies of the FP64 store).
+uint64_t system_bytes(int64_t No, int64_t Nv, bool with_j, int store,
+                      bool swaps = true);
+// Frees the row-swapped copies of a context's FP64 systems (the kernels then
+// read the straight arrays); whether there were any.
+bool drop_swap_copies(atrip_hip_ctx *ctx);
+// f(), again without the row-swapped copies (of the resident systems and of
+// the one an upload is making) when the device ran out of memory: they are a
+// convenience and never cost a call its memory.  f leaves nothing behind when
+// it throws.
+template <typename F>
+auto retry_memory(atrip_hip_ctx *ctx, F &&f) {
+  try {
+    return f();
+  } catch (const Fail &x) {
+    if (x.msg.find("out of memory") == std::string::npos) throw;
+    (void)hipGetLastError();
+    drop_swap_copies(ctx);
+  }
+  struct Without {
+    atrip_hip_ctx *ctx;
+    bool was;
+    ~Without() { ctx->operand_swaps = was; }
+  } w{ctx, ctx->operand_swaps};
+  ctx->operand_swaps = false;
+  return f();
+}
+template <typename F>
+int guarded_memory(atrip_hip_ctx *ctx, F &&f) {
+  return guarded(ctx, [&] { retry_memory(ctx, f); });
+}
 
 // atrip_hip_run over [first, first + count) with every piece of device
 // scratch (class buffers, W cubes, slot energies, batch partials, window

@@ -50,6 +50,25 @@ __host__ __device__ inline int tri_lane(int64_t R, int64_t k) {
   return (int)((R & 31) + 32 * ((k & 15) >> 3));
 }
 
+// FP64 operands: the same rows R and contraction index k in tiles of 16 rows
+// x 8 k, 128 doubles (1 KiB) each, tile (R / 16, k / 8) at
+// ((R / 16) (K / 8) + k / 8) * 128; inside it (R, k) sits at
+// 32 ((k % 8) / 2) + 2 (R % 16) + k % 2: lane (R % 16) + 16 ((k % 8) / 2) of
+// a 16x16x4 MFMA fragment owns the two k of its 16 bytes, so a fragment's
+// 8-deep K step is one 16-byte load per lane over 1 KiB of consecutive
+// addresses (8 lines of 128 bytes; rows K apart cost 64 lines).  The A
+// operands (rows (p, q), padded to whole tiles per o) keep a row-swapped
+// copy like the bf16x3 ones.
+__host__ __device__ inline int64_t f64_row(int64_t R, int64_t K) {
+  return (R >> 4) * (K >> 3) * 128 + 2 * (R & 15);
+}
+__host__ __device__ inline int64_t f64_at(int64_t R, int64_t k, int64_t K) {
+  return f64_row(R, K) + (k >> 3) * 128 + 32 * ((k & 7) >> 1) + (k & 1);
+}
+__host__ __device__ inline int64_t f64_elems(const TriGeom &g) {
+  return pad16(g.no * g.nrp) * g.K;
+}
+
 // Layout of the per-tuple class buffers written by the doubles kernels and
 // read by the energy kernels: each class keeps its GEMM output order,
 // element (row m, column index r) at m * P + r with the row pitch
@@ -90,21 +109,26 @@ __host__ __device__ inline int64_t n_triples(int64_t nbk) {
 }
 
 // Device-resident system.  Pair-indexed arrays use the CTF pair order
-// p(x,y) = x + Nv*y.  Layouts (all row-major with the last index fastest):
+// p(x,y) = x + Nv*y.  The doubles operands, as rows times contraction index:
 //   T3  [x][p + No q][E < Kv]    = Tpphh[x,E,p,q]          (T(x) slices)
 //   V3  [p(x,y)][r][E < Kv]      = Vppph[x,y,E,r]          (V(xy) slices)
 //   H3  [x][p + No q][L < Ko]    = Vhhhp[p,q,L,x]          (Vhhh(x) slices)
 //   T2N [p(x,y)][n][L < Ko]      = -Tpphh[x,y,L,n]         (-T(xy)[L,n])
 //   T2TN[p(x,y)][n][L < Ko]      = -Tpphh[x,y,n,L]         (-T(xy)[n,L])
+// in FP64 as 16 x 8 tiles (f64_at); T3s, H3s hold row q + No p in row
+// p + No q (null when they found no memory: the kernels then read the
+// swapped rows from T3, H3).  The other arrays, last index fastest:
 //   VHH [p(x,y)][i + No j]       = Vpphh[x,y,i,j]          (V(xy)ij)
 //   Tai [a + Nv i], ei[i], ea[a] as in CTF.
-// Padding entries (E >= Nv, L >= No) are zero.
+// Padding entries (E >= Nv, L >= No, rows past No^2) are zero.
 struct DevSystem {
   int64_t No = 0, Nv = 0, Kv = 0, Ko = 0;
   double *T3 = nullptr, *V3 = nullptr, *H3 = nullptr, *T2N = nullptr,
          *T2TN = nullptr, *VHH = nullptr, *Tai = nullptr, *ei = nullptr,
          *ea = nullptr;
+  double *T3s = nullptr, *H3s = nullptr;  // row-swapped copies of T3, H3
   double *V3J = nullptr, *H3J = nullptr;  // (cT) integrals, may be null
+  double *H3Js = nullptr;
   bool has_j = false;                     // (cT) integrals present
   // Complex systems: the arrays above hold the real parts, these the
   // imaginary parts (same layouts), and the *n arrays the negated imaginary
@@ -113,7 +137,9 @@ struct DevSystem {
   double *T3i = nullptr, *V3i = nullptr, *H3i = nullptr, *T2Ni = nullptr,
          *T2TNi = nullptr, *VHHi = nullptr, *Taii = nullptr, *eii = nullptr,
          *eai = nullptr, *V3Ji = nullptr, *H3Ji = nullptr;
+  double *T3is = nullptr, *H3is = nullptr, *H3Jis = nullptr;
   double *T3in = nullptr, *H3in = nullptr, *H3Jin = nullptr;
+  double *T3ins = nullptr, *H3ins = nullptr, *H3Jins = nullptr;
   // Split-FP32 copies of the GEMM operands, made on the first mixed run:
   // h = (float)x and l = bf16(x - h), same layouts as above (bf16(h), the
   // other factor of the correction products, is formed in registers).
@@ -147,40 +173,71 @@ __device__ inline uint16_t to_bf16(float v) {
   return (uint16_t)(u >> 16);
 }
 
-// Split-FP32 element q of x: h = (float)x, l = bf16(x - h); l may be null
-// (FP32-only store).
-__device__ inline void split_store(double x, float *h, uint16_t *l,
-                                   int64_t q) {
-  const float hi = (float)x;
-  h[q] = hi;
-  if (l) l[q] = to_bf16((float)(x - (double)hi));
-}
-
-// bf16x3 parts of x into element (R, k) of a tiled copy: b0 = bf16(x),
-// b1 = bf16(x - b0), b2 = bf16(x - b0 - b1), each residual formed in FP64,
-// so b0 + b1 + b2 is x within 2^-27 |x|.
-__device__ inline void tri_put(double x, uint16_t *out, int64_t R, int64_t k,
-                               int64_t K) {
-  const uint16_t p0 = to_bf16((float)x);
-  const double r1 = x - (double)__uint_as_float((uint32_t)p0 << 16);
-  const uint16_t p1 = to_bf16((float)r1);
-  const double r2 = r1 - (double)__uint_as_float((uint32_t)p1 << 16);
-  const int64_t at = tri_tile(R, k, K) + 8 * tri_lane(R, k) + (k & 7);
-  out[at] = p0;
-  out[at + 512] = p1;
-  out[at + 1024] = to_bf16((float)r2);
-}
-
-// Element q of FP64 operand [o][r][k] into its tiled copy (and the
-// row-swapped one when the geometry keeps it; No = sqrt(nr) there).
-__device__ inline void tri_store(double x, const TriOp &t, const TriGeom &g,
-                                 int64_t No, int64_t q) {
-  const int64_t k = q % g.K, row = q / g.K, r = row % g.nr, o = row / g.nr;
-  tri_put(x, t.p, o * g.nrp + r, k, g.K);
-  if (g.swapped) {
-    const int64_t rs = r / No + No * (r % No);
-    tri_put(x, t.sw, o * g.nrp + rs, k, g.K);
+// A conversion works on octets: the eight k of one row that share an FP64
+// tile (and one lane slot of a bf16x3 tile).
+//
+// bf16x3 parts of the octet v into row R, k = k8 of a tiled copy:
+// b0 = bf16(x), b1 = bf16(x - b0), b2 = bf16(x - b0 - b1), each residual
+// formed in FP64, so b0 + b1 + b2 is x within 2^-27 |x|.
+__device__ inline void tri_put8(const double (&v)[8], uint16_t *out, int64_t R,
+                                int64_t k8, int64_t K) {
+  typedef uint16_t u8 __attribute__((ext_vector_type(8)));
+  u8 p0, p1, p2;
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    p0[e] = to_bf16((float)v[e]);
+    const double r1 = v[e] - (double)__uint_as_float((uint32_t)p0[e] << 16);
+    p1[e] = to_bf16((float)r1);
+    const double r2 = r1 - (double)__uint_as_float((uint32_t)p1[e] << 16);
+    p2[e] = to_bf16((float)r2);
   }
+  uint16_t *at = out + tri_tile(R, k8, K) + 8 * tri_lane(R, k8);
+  *(u8 *)at = p0;
+  *(u8 *)(at + 512) = p1;
+  *(u8 *)(at + 1024) = p2;
+}
+
+// Split-FP32 octet: h = (float)x, l = bf16(x - h), row-major at element q;
+// l may be null (FP32-only store).
+__device__ inline void split_put8(const double (&v)[8], float *h, uint16_t *l,
+                                  int64_t q) {
+  typedef uint16_t u8 __attribute__((ext_vector_type(8)));
+  typedef float f8 __attribute__((ext_vector_type(8)));
+  f8 hi;
+  u8 lo;
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    hi[e] = (float)v[e];
+    lo[e] = to_bf16((float)(v[e] - (double)hi[e]));
+  }
+  *(f8 *)(h + q) = hi;
+  if (l) *(u8 *)(l + q) = lo;
+}
+
+// FP64 octet into row R, k = k8 of a tiled operand.
+__device__ inline void f64_put8(const double (&v)[8], double *out, int64_t R,
+                                int64_t k8, int64_t K) {
+  typedef double d2 __attribute__((ext_vector_type(2)));
+  double *at = out + f64_at(R, k8, K);
+#pragma unroll
+  for (int q = 0; q < 4; q++) *(d2 *)(at + 32 * q) = d2{v[2 * q], v[2 * q + 1]};
+}
+
+// One form of a doubles operand being filled: FP64 tiles, split FP32 rows
+// and / or bf16x3 tiles (null: not kept).
+struct OpSink {
+  double *d = nullptr;
+  float *h = nullptr;
+  uint16_t *l = nullptr, *t = nullptr;
+};
+__device__ inline void sink_put8(const double (&v)[8], const OpSink &s,
+                                 const TriGeom &g, int64_t o, int64_t r,
+                                 int64_t k8) {
+  const int64_t R = o * g.nrp + r;
+  if (s.d) f64_put8(v, s.d, R, k8, g.K);
+  if (s.h && r < g.nr && o < g.no)
+    split_put8(v, s.h, s.l, (o * g.nr + r) * g.K + k8);
+  if (s.t) tri_put8(v, s.t, R, k8, g.K);
 }
 
 // Tuple windows: block triples (alpha <= beta <= gamma) of edge nb.
@@ -222,6 +279,7 @@ struct atrip_hip_ctx {
   int timing = 0;
   int tile = -1;  // -1: chosen per system shape
   int operand_store = 0;  // store mode of the next uploads (DevSystem::store)
+  bool operand_swaps = true;  // uploads keep row-swapped copies (FP64 store)
   int epilogue = 0;  // 0: fused class sums + energy, 1: W cubes first
   int serve_plain_no = 16;  // served requests with No >= this: plain path
   int64_t stage_kb = 4 << 20;  // device staging of host uploads (KiB)
@@ -328,6 +386,20 @@ hipError_t launch_transpose(const double *src, double *dst, int64_t n_outer,
                             int64_t src_a, int64_t src_b, int64_t dst_o,
                             int64_t dst_a, int64_t dst_b, double scale,
                             hipStream_t st);
+// The same copy into an FP64 operand's tiles: element (o, a, b) goes to row
+// R0 + o Ro + a Ra + b Rb at contraction index k0 + o ko + a ka.  swap 1:
+// the row part of R is row0 + o, swap 2: it is b, and the element goes to
+// the swapped row q + No p instead of p + No q (R: the other parts).
+struct TileMap {
+  int64_t R0 = 0, Ro = 0, Ra = 0, Rb = 0, k0 = 0, ko = 0, ka = 0, K = 0;
+  int swap = 0;
+  int64_t row0 = 0, No = 1;
+};
+hipError_t launch_transpose_tiled(const double *src, double *dst,
+                                  int64_t n_outer, int64_t n_a, int64_t n_b,
+                                  int64_t src_o, int64_t src_a, int64_t src_b,
+                                  const TileMap &m, double scale,
+                                  hipStream_t st);
 // Generate a synthetic system in place; tensor_flag is or-ed into every
 // tensor id (ATRIP_SYN_IMAG fills the imaginary parts of a complex system,
 // given a DevSystem whose arrays are its imaginary planes).
@@ -339,13 +411,19 @@ hipError_t launch_synth(DevSystem &s, uint64_t seed, bool with_j,
 // dst[q] = scale * src[q], q < n.
 hipError_t launch_scale(const double *src, double *dst, int64_t n,
                         double scale, hipStream_t st);
-// Fill a Split copy of n doubles.
-hipError_t launch_split(const double *x, DevSystem::Split &out, int64_t n,
-                        hipStream_t st);
-// Fill the bf16x3 copy (and row-swapped copy) of FP64 operand x of
-// geometry g (No: occupied indices, for the swap).
-hipError_t launch_tri(const double *x, const TriOp &out, const TriGeom &g,
-                      int64_t No, hipStream_t st);
+// Fill another form of FP64 operand x (geometry gx) of geometry g, in g's
+// row order or, swapped, with row q + No p in row p + No q.
+hipError_t launch_convert(const double *x, const TriGeom &gx,
+                          const OpSink &out, const TriGeom &g, bool swapped,
+                          int64_t No, hipStream_t st);
+// Geometry of a system's FP64 operands: A (T3, H3 and H3J, rows padded to
+// whole tiles) and the pair-indexed B arrays (V3, T2N, T2TN, V3J).
+inline TriGeom f64_geom_a(int64_t No, int64_t Nv, int64_t K) {
+  return TriGeom{Nv, No * No, pad16(No * No), K, true};
+}
+inline TriGeom f64_geom_b(int64_t No, int64_t Nv, int64_t K) {
+  return TriGeom{Nv * Nv, No, No, K, false};
+}
 // Geometry of a system's bf16x3 operands: A (T3, H3 and H3J) and the
 // pair-indexed B arrays (V3, T2N, T2TN, V3J), for contraction length K.
 inline TriGeom tri_geom_a(int64_t No, int64_t Nv, int64_t K) {
@@ -364,7 +442,7 @@ inline uint64_t tri_bytes(const TriGeom &g) {
 // chosen for it.  Tile variant v is the wave tile of (16*bfm(v)) x
 // (16*bfn(v)) outputs.
 struct BSys {
-  const double *T3, *V3, *H3, *T2N, *T2TN, *VHH, *Tai, *ei, *ea;
+  const double *T3, *T3s, *V3, *H3, *H3s, *T2N, *T2TN, *VHH, *Tai, *ei, *ea;
   const uint32_t *points;
   int64_t No, Nv, Kv, Ko, npoints;
   int32_t nb, tile;

@@ -10,6 +10,8 @@
 #include "../../include/atrip_synth.h"
 #include "internal.hpp"
 
+#include <algorithm>
+
 namespace atrip_amd {
 namespace {
 
@@ -40,84 +42,167 @@ __global__ __launch_bounds__(256) void transpose_kernel(
   }
 }
 
-enum SynthTarget { S_T3, S_V3, S_H3, S_T2N, S_T2TN, S_VHH, S_PLAIN };
-
-// Fill one device array from the generator; element q of the destination is
-// mapped back to the CTF linear index of the tensor it holds.
-__global__ __launch_bounds__(256) void synth_kernel(double *dst, float *sh,
-                                                    uint16_t *sl, TriOp tri,
-                                                    TriGeom tg, int64_t n,
-                                                    int target, int tensor,
-                                                    uint64_t stream, int64_t No,
-                                                    int64_t Nv, int64_t Kv,
-                                                    int64_t Ko, double scale) {
-  const int64_t N2 = No * No, Nv2 = Nv * Nv;
-  for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n;
-       q += (int64_t)gridDim.x * blockDim.x) {
-    int64_t idx = -1;
-    double sign = 1.0;
-    switch (target) {
-    case S_T3: {  // [x][row][E<Kv] = Tpphh[x,E,row]
-      const int64_t E = q % Kv, r = q / Kv, row = r % N2, x = r / N2;
-      if (E < Nv) idx = x + Nv * E + Nv2 * row;
-      break;
+// The same through the tile addresses of an FP64 operand (f64_at).  A row's
+// consecutive k are 16-byte pairs 256 bytes apart, so the writes are 16-byte
+// pieces; uploads are bound by the host link, not by them.
+__global__ __launch_bounds__(256) void transpose_tiled_kernel(
+    const double *__restrict__ src, double *__restrict__ dst, int64_t n_a,
+    int64_t n_b, int64_t tiles_a, int64_t o_first, int64_t src_o,
+    int64_t src_a, int64_t src_b, TileMap m, double scale) {
+  __shared__ double tile[TT][TT + 1];
+  const int64_t o = blockIdx.y + o_first;
+  const int64_t ta = blockIdx.x % tiles_a, tb = blockIdx.x / tiles_a;
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  const double *s = src + o * src_o;
+#pragma unroll
+  for (int r = 0; r < TT; r += 8) {
+    const int64_t a = ta * TT + ty + r, b = tb * TT + tx;
+    if (a < n_a && b < n_b) tile[ty + r][tx] = s[a * src_a + b * src_b];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < TT; r += 8) {
+    const int64_t b = tb * TT + ty + r, a = ta * TT + tx;
+    if (a >= n_a || b >= n_b) continue;
+    int64_t R = m.R0 + o * m.Ro + a * m.Ra + b * m.Rb;
+    if (m.swap) {
+      const int64_t row = m.swap == 1 ? m.row0 + o : b;
+      R += row / m.No + m.No * (row % m.No);
     }
-    case S_V3: {  // [pair][r][E<Kv] = Vppph[pair,E,r]
-      const int64_t E = q % Kv, t = q / Kv, r = t % No, pair = t / No;
-      if (E < Nv) idx = pair + Nv2 * E + Nv2 * Nv * r;
-      break;
-    }
-    case S_H3: {  // [x][row][L<Ko] = Vhhhp[row,L,x]
-      const int64_t L = q % Ko, t = q / Ko, row = t % N2, x = t / N2;
-      if (L < No) idx = row + N2 * L + N2 * No * x;
-      break;
-    }
-    case S_T2N: {  // [pair][n][L<Ko] = -Tpphh[pair,L,n]
-      const int64_t L = q % Ko, t = q / Ko, nn = t % No, pair = t / No;
-      if (L < No) idx = pair + Nv2 * L + Nv2 * No * nn;
-      sign = -1.0;
-      break;
-    }
-    case S_T2TN: {  // [pair][n][L<Ko] = -Tpphh[pair,n,L]
-      const int64_t L = q % Ko, t = q / Ko, nn = t % No, pair = t / No;
-      if (L < No) idx = pair + Nv2 * nn + Nv2 * No * L;
-      sign = -1.0;
-      break;
-    }
-    case S_VHH: {  // [pair][ij] = Vpphh[pair,ij]
-      const int64_t ij = q % N2, pair = q / N2;
-      idx = pair + Nv2 * ij;
-      break;
-    }
-    default: idx = q;
-    }
-    double v = 0.0;
-    if (idx >= 0)
-      v = sign * atrip_synth_value(stream, tensor, (uint64_t)No, (uint64_t)Nv,
-                                   (uint64_t)idx) * scale;
-    if (dst) dst[q] = v;
-    if (sh) split_store(v, sh, sl, q);
-    if (tri.p) tri_store(v, tri, tg, No, q);
+    dst[f64_at(R, m.k0 + o * m.ko + a * m.ka, m.K)] = scale * tile[tx][ty + r];
   }
 }
 
-// Fill n elements of a target layout into dst (FP64), the split arrays o
-// (o.h null: none) and/or the bf16x3 copy tri of geometry tg (tri.p null:
-// none).
-hipError_t synth_fill(double *dst, const DevSystem::Split &o, const TriOp &tri,
-                      const TriGeom &tg, int64_t n, SynthTarget target,
-                      int tensor, uint64_t seed, const DevSystem &s,
-                      double scale, hipStream_t st) {
+enum SynthTarget { S_T3, S_V3, S_H3, S_T2N, S_T2TN };
+
+// Fill the forms `out` of a doubles operand of geometry g from the generator,
+// one octet (eight k of a row) per thread, consecutive threads on the
+// consecutive rows of a 16-row tile, so FP64 and bf16x3 tiles are written in
+// whole lines and the index divisions are paid once per eight values.  Bound
+// by the generator's FP64 arithmetic; at No=40, Nv=400 all operands take 30 ms
+// in bf16x3 (48 ms with one element per thread and scattered 2-byte stores)
+// and 30 ms in FP64 with the row-swapped copies (32 ms without them before).
+// swapped: row p + No q holds the values of row q + No p.
+__global__ __launch_bounds__(256) void synth_operand_kernel(
+    OpSink out, TriGeom g, int64_t n, int target, int tensor, uint64_t stream,
+    int64_t No, int64_t Nv, bool swapped, double scale) {
+  const int64_t N2 = No * No, Nv2 = Nv * Nv, K8 = g.K >> 3;
+  for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n;
+       q += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t t = q >> 4, R = t / K8 * 16 + (q & 15), k8 = t % K8 * 8;
+    const int64_t o = R / g.nrp;
+    int64_t r = R - o * g.nrp, base = 0, step = 0, kmax = 0;
+    const int64_t row = r;
+    double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (o < g.no && r < g.nr) {
+      if (swapped) r = r / No + No * (r % No);
+      double sign = 1.0;
+      switch (target) {
+      case S_T3:  // [x][row][E] = Tpphh[x,E,row]
+        base = o + Nv2 * r; step = Nv; kmax = Nv;
+        break;
+      case S_V3:  // [pair][r][E] = Vppph[pair,E,r]
+        base = o + Nv2 * Nv * r; step = Nv2; kmax = Nv;
+        break;
+      case S_H3:  // [x][row][L] = Vhhhp[row,L,x]
+        base = r + N2 * No * o; step = N2; kmax = No;
+        break;
+      case S_T2N:  // [pair][n][L] = -Tpphh[pair,L,n]
+        base = o + Nv2 * No * r; step = Nv2; kmax = No; sign = -1.0;
+        break;
+      default:  // S_T2TN: [pair][n][L] = -Tpphh[pair,n,L]
+        base = o + Nv2 * r; step = Nv2 * No; kmax = No; sign = -1.0;
+      }
+#pragma unroll 1
+      for (int e = 0; e < 8; e++) {
+        const int64_t k = k8 + e;
+        if (k >= kmax) break;
+        const double x = sign * atrip_synth_value(stream, tensor, (uint64_t)No,
+                                                  (uint64_t)Nv,
+                                                  (uint64_t)(base + k * step)) *
+                         scale;
+        // a run-time index into v would put it in scratch memory
+#pragma unroll
+        for (int z = 0; z < 8; z++)
+          if (z == e) v[z] = x;
+      }
+    }
+    sink_put8(v, out, g, o, row, k8);
+  }
+}
+
+// Fill a plain array of n elements: element q is the tensor's element q, or
+// with nij > 0 (VHH) [pair][ij] = Vpphh[pair,ij], nij = No^2.
+__global__ __launch_bounds__(256) void synth_plain_kernel(
+    double *dst, int64_t n, int64_t nij, int tensor, uint64_t stream,
+    int64_t No, int64_t Nv, double scale) {
+  for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n;
+       q += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t idx = nij ? q / nij + Nv * Nv * (q % nij) : q;
+    dst[q] = atrip_synth_value(stream, tensor, (uint64_t)No, (uint64_t)Nv,
+                               (uint64_t)idx) * scale;
+  }
+}
+
+// FP64 operand to another form, one octet per thread in the order of the
+// destination's tiles.
+__global__ __launch_bounds__(256) void convert_kernel(const double *x,
+                                                      TriGeom gx, OpSink out,
+                                                      TriGeom g, bool swapped,
+                                                      int64_t No, int64_t n) {
+  typedef double d2 __attribute__((ext_vector_type(2)));
+  const int64_t K8 = g.K >> 3;
+  for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n;
+       q += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t t = q >> 4, R = t / K8 * 16 + (q & 15), k8 = t % K8 * 8;
+    const int64_t o = R / g.nrp, r = R - o * g.nrp;
+    double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (o < g.no && r < g.nr) {
+      const int64_t rs = swapped ? r / No + No * (r % No) : r;
+      const double *at = x + f64_at(o * gx.nrp + rs, k8, gx.K);
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const d2 y = *(const d2 *)(at + 32 * e);
+        v[2 * e] = y[0];
+        v[2 * e + 1] = y[1];
+      }
+    }
+    sink_put8(v, out, g, o, r, k8);
+  }
+}
+
+unsigned fill_blocks(int64_t n) {
+  return (unsigned)std::min<int64_t>((n + 255) / 256, 65536L * 16);
+}
+
+// Rows of a form's arrays, whole tiles of 32 (bf16x3) or 16 rows.
+int64_t fill_rows(const OpSink &out, const TriGeom &g) {
+  return out.t ? pad32(g.no * g.nrp) : pad16(g.no * g.nrp);
+}
+
+hipError_t synth_operand(const OpSink &out, const TriGeom &g,
+                         SynthTarget target, int tensor, uint64_t seed,
+                         const DevSystem &s, bool swapped, double scale,
+                         hipStream_t st) {
+  const int64_t n = fill_rows(out, g) * (g.K >> 3);
   if (n <= 0) return hipSuccess;
-  const uint64_t stream = atrip_synth_stream(seed, tensor);
+  hipLaunchKernelGGL(synth_operand_kernel, dim3(fill_blocks(n)), dim3(256), 0,
+                     st, out, g, n, (int)target, tensor,
+                     atrip_synth_stream(seed, tensor), s.No, s.Nv, swapped,
+                     scale);
+  return hipGetLastError();
+}
+
+hipError_t synth_plain(double *dst, int64_t n, int64_t nij, int tensor,
+                       uint64_t seed, const DevSystem &s, double scale,
+                       hipStream_t st) {
+  if (n <= 0) return hipSuccess;
   // amplitudes and integrals carry the scale, orbital energies do not
   const int base = tensor & 15;
   if (base == ATRIP_SYN_EI || base == ATRIP_SYN_EA) scale = 1.0;
-  int64_t blocks = (n + 255) / 256;
-  if (blocks > 65536L * 16) blocks = 65536L * 16;
-  hipLaunchKernelGGL(synth_kernel, dim3((unsigned)blocks), dim3(256), 0, st,
-                     dst, o.h, o.l, tri, tg, n, (int)target, tensor, stream, s.No,
-                     s.Nv, s.Kv, s.Ko, scale);
+  hipLaunchKernelGGL(synth_plain_kernel, dim3(fill_blocks(n)), dim3(256), 0,
+                     st, dst, n, nij, tensor, atrip_synth_stream(seed, tensor),
+                     s.No, s.Nv, scale);
   return hipGetLastError();
 }
 
@@ -144,43 +229,75 @@ hipError_t launch_transpose(const double *src, double *dst, int64_t n_outer,
   return hipSuccess;
 }
 
+hipError_t launch_transpose_tiled(const double *src, double *dst,
+                                  int64_t n_outer, int64_t n_a, int64_t n_b,
+                                  int64_t src_o, int64_t src_a, int64_t src_b,
+                                  const TileMap &m, double scale,
+                                  hipStream_t st) {
+  if (n_outer <= 0 || n_a <= 0 || n_b <= 0) return hipSuccess;
+  const int64_t tiles_a = (n_a + TT - 1) / TT, tiles_b = (n_b + TT - 1) / TT;
+  for (int64_t o0 = 0; o0 < n_outer; o0 += 65535) {
+    const int64_t no = n_outer - o0 < 65535 ? n_outer - o0 : 65535;
+    hipLaunchKernelGGL(transpose_tiled_kernel,
+                       dim3((unsigned)(tiles_a * tiles_b), (unsigned)no),
+                       dim3(256), 0, st, src, dst, n_a, n_b, tiles_a, o0,
+                       src_o, src_a, src_b, m, scale);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+hipError_t launch_convert(const double *x, const TriGeom &gx,
+                          const OpSink &out, const TriGeom &g, bool swapped,
+                          int64_t No, hipStream_t st) {
+  const int64_t n = fill_rows(out, g) * (g.K >> 3);
+  if (n <= 0) return hipSuccess;
+  if (g.K % 16 || g.K != gx.K || (swapped && g.nr != No * No))
+    return hipErrorInvalidValue;
+  hipLaunchKernelGGL(convert_kernel, dim3(fill_blocks(n)), dim3(256), 0, st, x,
+                     gx, out, g, swapped, No, n);
+  return hipGetLastError();
+}
+
 hipError_t launch_synth(DevSystem &s, uint64_t seed, bool with_j,
                         hipStream_t st, int tensor_flag, double scale) {
   const int64_t No = s.No, Nv = s.Nv, N2 = No * No, Nv2 = Nv * Nv;
-  hipError_t e;
-  const DevSystem::Split none;
-  const TriOp tnone;
-  const TriGeom ga = tri_geom_a(No, Nv, s.Kv), gb = tri_geom_b(No, Nv, s.Kv),
-                gh = tri_geom_a(No, Nv, s.Ko), gt = tri_geom_b(No, Nv, s.Ko);
-  // doubles operands: FP64 array, or straight into the split arrays or the
-  // bf16x3 copy when the system keeps no FP64 copy
-#define SYN(ptr, sp, tp, g, tgt, tensor)                                    \
-  if ((e = synth_fill(s.store == 0 ? ptr : nullptr,                         \
-                      s.store == 1 || s.store == 2 ? sp : none,             \
-                      s.store == 3 ? tp : tnone, g, (g).no * (g).nr * (g).K, \
-                      tgt, (tensor) | tensor_flag, seed, s, scale, st)) !=  \
-      hipSuccess)                                                           \
-    return e;
-#define SYN64(ptr, n, tgt, tensor)                                         \
-  if ((e = synth_fill(ptr, none, tnone, ga, n, tgt, (tensor) | tensor_flag, \
-                      seed, s, scale, st)) != hipSuccess)                   \
-    return e;
-  SYN(s.T3, s.sT3, s.tT3, ga, S_T3, ATRIP_SYN_TABIJ);
-  SYN(s.V3, s.sV3, s.tV3, gb, S_V3, ATRIP_SYN_VABCI);
-  SYN(s.H3, s.sH3, s.tH3, gh, S_H3, ATRIP_SYN_VIJKA);
-  SYN(s.T2N, s.sT2N, s.tT2N, gt, S_T2N, ATRIP_SYN_TABIJ);
-  SYN(s.T2TN, s.sT2TN, s.tT2TN, gt, S_T2TN, ATRIP_SYN_TABIJ);
-  SYN64(s.VHH, Nv2 * N2, S_VHH, ATRIP_SYN_VABIJ);
-  SYN64(s.Tai, Nv * No, S_PLAIN, ATRIP_SYN_TAI);
-  SYN64(s.ei, No, S_PLAIN, ATRIP_SYN_EI);
-  SYN64(s.ea, Nv, S_PLAIN, ATRIP_SYN_EA);
+  hipError_t e = hipSuccess;
+  // a doubles operand in the form the system keeps, with its row-swapped
+  // copy (xs, tp.sw)
+  auto op = [&](double *x, double *xs, const DevSystem::Split &sp,
+                const TriOp &tp, bool a, int64_t K, SynthTarget target,
+                int tensor) {
+    const TriGeom g = s.store == 3 ? (a ? tri_geom_a(No, Nv, K) : tri_geom_b(No, Nv, K))
+                                   : (a ? f64_geom_a(No, Nv, K) : f64_geom_b(No, Nv, K));
+    for (int sw = 0; sw < 2 && e == hipSuccess; sw++) {
+      OpSink k;
+      if (s.store == 0) k.d = sw ? xs : x;
+      else if (s.store == 3) k.t = sw ? tp.sw : tp.p;
+      else if (!sw) { k.h = sp.h; k.l = sp.l; }
+      if (!k.d && !k.h && !k.t) continue;
+      e = synth_operand(k, g, target, tensor | tensor_flag, seed, s, sw, scale, st);
+    }
+  };
+  auto plain = [&](double *x, int64_t n, int64_t nij, int tensor) {
+    if (e == hipSuccess)
+      e = synth_plain(x, n, nij, tensor | tensor_flag, seed, s, scale, st);
+  };
+  op(s.T3, s.T3s, s.sT3, s.tT3, true, s.Kv, S_T3, ATRIP_SYN_TABIJ);
+  op(s.V3, nullptr, s.sV3, s.tV3, false, s.Kv, S_V3, ATRIP_SYN_VABCI);
+  op(s.H3, s.H3s, s.sH3, s.tH3, true, s.Ko, S_H3, ATRIP_SYN_VIJKA);
+  op(s.T2N, nullptr, s.sT2N, s.tT2N, false, s.Ko, S_T2N, ATRIP_SYN_TABIJ);
+  op(s.T2TN, nullptr, s.sT2TN, s.tT2TN, false, s.Ko, S_T2TN, ATRIP_SYN_TABIJ);
+  plain(s.VHH, Nv2 * N2, N2, ATRIP_SYN_VABIJ);
+  plain(s.Tai, Nv * No, 0, ATRIP_SYN_TAI);
+  plain(s.ei, No, 0, ATRIP_SYN_EI);
+  plain(s.ea, Nv, 0, ATRIP_SYN_EA);
   if (with_j) {
-    SYN(s.V3J, s.sV3J, s.tV3J, gb, S_V3, ATRIP_SYN_JABCI);
-    SYN(s.H3J, s.sH3J, s.tH3J, gh, S_H3, ATRIP_SYN_JIJKA);
+    op(s.V3J, nullptr, s.sV3J, s.tV3J, false, s.Kv, S_V3, ATRIP_SYN_JABCI);
+    op(s.H3J, s.H3Js, s.sH3J, s.tH3J, true, s.Ko, S_H3, ATRIP_SYN_JIJKA);
   }
-#undef SYN
-#undef SYN64
-  return hipSuccess;
+  return e;
 }
 
 __global__ __launch_bounds__(256) void scale_kernel(const double *src,

@@ -144,7 +144,13 @@ void admit(atrip_hip_server *srv, int grid) {
                       : srv->precision == ATRIP_SPLIT_FP32 ? 1
                       : srv->precision == ATRIP_FP32       ? 2
                                                            : 3;
-    r.bytes = system_bytes(r.No, r.Nv, false, store);
+    // the row-swapped operand copies are kept only where they fit the budget
+    bool swaps = true;
+    r.bytes = system_bytes(r.No, r.Nv, false, store, swaps);
+    if (srv->resident + r.bytes > srv->budget) {
+      swaps = false;
+      r.bytes = system_bytes(r.No, r.Nv, false, store, swaps);
+    }
     if (r.bytes > srv->budget) {
       fail_request(srv, r, "system larger than the HBM budget");
       srv->queue.pop_front();
@@ -153,12 +159,15 @@ void admit(atrip_hip_server *srv, int grid) {
     if (srv->resident + r.bytes > srv->budget) break;  // wait for memory
     int sys = 0;
     const int store_before = ctx->operand_store;
+    const bool swaps_before = ctx->operand_swaps;
     ctx->operand_store = store;
+    ctx->operand_swaps = swaps;
     const int rc =
         r.synthetic
             ? atrip_hip_upload_synthetic(ctx, r.No, r.Nv, r.seed, 0, &sys)
             : atrip_hip_upload(ctx, &r.desc, &sys);
     ctx->operand_store = store_before;
+    ctx->operand_swaps = swaps_before;
     if (rc != 0) {
       // out of device memory with other requests resident: wait for them
       if (!srv->active.empty() &&
@@ -233,8 +242,8 @@ int step(atrip_hip_server *srv) {
                      [&](int64_t x, int64_t y) { return remaining(x) < remaining(y); });
   const double target = srv->iter_ms * 1e-3 * grid;
   double left = target;
-  std::vector<BSys> sys;
-  std::vector<BSplit> split;
+  std::vector<DevSystem *> owners;  // systems of the batched launch
+  std::vector<BatchTune> plans;
   std::vector<BTask> tasks;
   std::vector<double> cost;
   std::vector<std::pair<int64_t, size_t>> took;   // batched: request, windows
@@ -253,10 +262,9 @@ int step(atrip_hip_server *srv) {
       plain.push_back({id, k});
       continue;
     }
-    const int si = (int)sys.size();
-    DevSystem &ds = get_sys(ctx, r.sys);
-    sys.push_back(make_bsys(ctx, ds, r.plan, srv->precision));
-    split.push_back(make_bsplit(ds));
+    const int si = (int)owners.size();
+    owners.push_back(&get_sys(ctx, r.sys));
+    plans.push_back(r.plan);
     const double nb3 = (double)r.plan.nb * r.plan.nb * r.plan.nb;
     for (size_t q = 0; q < k; q++) {
       const Win &w = r.wins[r.cursor + q];
@@ -270,8 +278,15 @@ int step(atrip_hip_server *srv) {
     std::iota(order.begin(), order.end(), 0);
     std::stable_sort(order.begin(), order.end(),
                      [&](int32_t x, int32_t y) { return cost[x] > cost[y]; });
-    const LaunchOut out =
-        run_tasks(ctx, srv->precision, sys, split, tasks, order, grid, true);
+    const LaunchOut out = retry_memory(ctx, [&] {
+      std::vector<BSys> sys;
+      std::vector<BSplit> split;
+      for (size_t q = 0; q < owners.size(); q++) {
+        sys.push_back(make_bsys(ctx, *owners[q], plans[q], srv->precision));
+        split.push_back(make_bsplit(*owners[q]));
+      }
+      return run_tasks(ctx, srv->precision, sys, split, tasks, order, grid, true);
+    });
     srv->busy_ms += out.ms;
     srv->launches++;
     // accumulate in canonical window order
@@ -290,9 +305,10 @@ int step(atrip_hip_server *srv) {
   for (auto &pk : plain) {
     Request &r = srv->reqs.at(pk.first);
     const Clock::time_point t0 = Clock::now();
-    run_plan_windows(ctx, r.sys, srv->precision, r.plan.nb, r.cursor,
-                     r.cursor + pk.second,
-                     wsum);
+    retry_memory(ctx, [&] {
+      run_plan_windows(ctx, r.sys, srv->precision, r.plan.nb, r.cursor,
+                       r.cursor + pk.second, wsum);
+    });
     const double ms =
         std::chrono::duration<double, std::milli>(Clock::now() - t0).count();
     if (wsum.size() != 2 * pk.second) throw Fail{"plain-path window count"};
