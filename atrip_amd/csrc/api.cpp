@@ -902,7 +902,7 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
           }
     }
     if (!cnt) continue;
-    sel.insert(sel.end(), {(int32_t)al, (int32_t)be, (int32_t)ga});
+    sel.insert(sel.end(), {(int32_t)al * nb, (int32_t)be * nb, (int32_t)ga * nb});
     counts.push_back(cnt);
     res.tuples += cnt;
   }
@@ -1038,7 +1038,8 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
     const int w0 = bi * bw;
     b.nw = std::min(bw, nsel - w0);
     b.windows = (const int32_t *)d_sel + 3 * w0;
-    b.nb = nb;
+    b.aprefix = s.aprefix;
+    b.ea = b.eb = b.ec = nb;
     b.first = full ? 0 : first;
     b.last = full ? ~0ULL : last;
     b.slots = (int64_t)b.nw * nb3;
@@ -1486,9 +1487,9 @@ int atrip_hip_tuple_energies(atrip_hip_ctx *ctx, int sys, int precision,
         const int64_t nb3 = (int64_t)nb * nb * nb;
         for (int w = 0; w < nw; w++)
           for (int64_t q = 0; q < nb3; q++) {
-            const uint64_t a = (uint64_t)win[3 * w] * nb + q / (nb * nb);
-            const uint64_t b = (uint64_t)win[3 * w + 1] * nb + (q / nb) % nb;
-            const uint64_t c = (uint64_t)win[3 * w + 2] * nb + q % nb;
+            const uint64_t a = (uint64_t)win[3 * w] + q / (nb * nb);
+            const uint64_t b = (uint64_t)win[3 * w + 1] + (q / nb) % nb;
+            const uint64_t c = (uint64_t)win[3 * w + 2] + q % nb;
             if (!tuple_ok(Nv, a, b, c)) continue;
             const uint64_t idx = (*h)(a, b, c);
             if (idx < first || idx >= last) continue;

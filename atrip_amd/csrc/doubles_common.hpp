@@ -2,6 +2,8 @@
 // the class/segment table of the regrouped doubles contractions.
 #pragma once
 
+#include <algorithm>
+
 #include "internal.hpp"
 
 namespace atrip_amd {
@@ -57,6 +59,113 @@ __device__ inline void class_pair(int cl, int64_t al, int64_t be, int64_t ga,
   if (cl == 0) { x1 = al * nb + o1; x2 = be * nb + o2; }
   else if (cl == 1) { x1 = al * nb + o1; x2 = ga * nb + o2; }
   else { x1 = be * nb + o1; x2 = ga * nb + o2; }
+}
+
+// One workgroup's share of a launch over windows of eb x ec columns (see
+// BatchArgs): a class, an A-pair of its window and one tile of that pair's
+// GEMM.  The GEMM's columns are only those of valid tuples: the valid third
+// indices of a pair are consecutive (the tuples of a pair are ordered along
+// the third index, so a tuple range cuts them at the ends), so column n is
+// index n % No of third index y0 + n / No, n < ncols.  Column tuple slot:
+// slot0 + (n / No) slot_step.
+struct TileWork {
+  int cl, mt, nt, w;
+  int32_t x1, x2;  // A-pair: w (a,b), v (a,c), u (b,c)
+  int32_t y0;      // first valid third index
+  int ncols;
+  int slot0, slot_step;
+};
+
+// Work of this workgroup; false when its tile holds no column.  Units
+// (window, class, pair) go round the eight XCDs (workgroup b runs on XCD
+// b % 8) and a unit's tiles stay on one, so they share the pair's A rows and
+// columns in its L2, and the units that hold few columns (windows on the
+// diagonal, ends of a range) spread evenly: with one contiguous eighth of the
+// launch per XCD the XCDs that got the diagonal windows ran out of work.
+__device__ __forceinline__ bool tile_work(const WindowArgs &W, uint64_t Nv,
+                                          int No, int ntile_cols,
+                                          TileWork &T) {
+  const uint32_t bid = blockIdx.x, j = bid >> 3;
+  const uint32_t tiles = (uint32_t)(W.mtiles * W.ntiles);
+  const uint32_t uq = j / tiles, tile = j - uq * tiles;
+  const uint32_t unit = 8 * uq + (bid & 7);
+  const uint32_t units =
+      (uint32_t)(W.ea * W.eb + W.ea * W.ec + W.eb * W.ec);
+  if (unit >= units * (uint32_t)W.nw) return false;
+  T.mt = (int)(tile / (uint32_t)W.ntiles);
+  T.nt = (int)(tile - (uint32_t)T.mt * (uint32_t)W.ntiles);
+  T.w = (int)(unit / units);
+  int u = (int)(unit - (uint32_t)T.w * units);
+  const int32_t a0 = W.windows[3 * T.w], b0 = W.windows[3 * T.w + 1],
+                c0 = W.windows[3 * T.w + 2];
+  int edge;
+  int32_t y;
+  if (u < W.ea * W.eb) {
+    const int o1 = u / W.eb, o2 = u - o1 * W.eb;
+    T.cl = 0; T.x1 = a0 + o1; T.x2 = b0 + o2;
+    y = c0; edge = W.ec;
+    T.slot0 = u * W.ec; T.slot_step = 1;
+  } else if ((u -= W.ea * W.eb) < W.ea * W.ec) {
+    const int o1 = u / W.ec, o2 = u - o1 * W.ec;
+    T.cl = 1; T.x1 = a0 + o1; T.x2 = c0 + o2;
+    y = b0; edge = W.eb;
+    T.slot0 = o1 * W.eb * W.ec + o2; T.slot_step = W.ec;
+  } else {
+    u -= W.ea * W.ec;
+    const int o1 = u / W.ec, o2 = u - o1 * W.ec;
+    T.cl = 2; T.x1 = b0 + o1; T.x2 = c0 + o2;
+    y = a0; edge = W.ea;
+    T.slot0 = u; T.slot_step = W.eb * W.ec;
+  }
+  const int lane = threadIdx.x & 63;
+  const int64_t yl = y + lane;
+  const uint64_t a = T.cl == 2 ? yl : T.x1,
+                 b = T.cl == 0 ? T.x2 : T.cl == 1 ? yl : T.x1,
+                 c = T.cl == 0 ? yl : T.x2;
+  bool ok = lane < edge && tuple_ok(Nv, a, b, c);
+  if (ok && (W.first > 0 || W.last != ~0ULL)) {
+    const uint64_t idx = tuple_index(W.aprefix, Nv, a, b, c);
+    ok = idx >= W.first && idx < W.last;
+  }
+  const uint64_t mask = __ballot(ok);
+  if (!mask) return false;
+  const int t0 = __builtin_ctzll(mask), n = __popcll(mask);
+  T.y0 = y + t0;
+  T.slot0 += t0 * T.slot_step;
+  T.ncols = n * No;
+  return T.nt * ntile_cols < T.ncols;
+}
+
+// Fragments of `width` that wave w of two holds of `left` rows or columns,
+// fragments taken in turn (w, w + 2, ...), at most f.
+__device__ __forceinline__ int occupied(int64_t left, int w, int width, int f) {
+  const int64_t frags = (left + width - 1) / width;  // of both waves
+  const int mine = (int)((frags - w + 1) / 2);
+  return mine < 0 ? 0 : mine < f ? mine : f;
+}
+
+// Row of segment sg's B operand at column (y, rr) of class cl with A-pair
+// (x1, x2), and its array (0: V(xy) slabs, 1: -T(xy)[L,n], 2: -T(xy)[n,L];
+// the pairs of b_pair, written by the pair and the third index).
+__device__ __forceinline__ int64_t b_row(int cl, int sg, int32_t x1,
+                                         int32_t x2, int32_t y, int32_t rr,
+                                         int64_t Nv, int64_t No, int &which) {
+  const int64_t x = sg == 0 || sg == 3 ? x2 : x1;
+  const bool tr = sg >= 2 && (cl == 2 || (cl == 1 && sg == 3));
+  which = sg < 2 ? 0 : tr ? 2 : 1;
+  return (tr ? y + Nv * x : x + Nv * y) * No + rr;
+}
+
+// Grid of a doubles launch: units padded to the eight XCDs times the tiles
+// of a unit; 0 when it holds nothing.
+inline int64_t doubles_grid(WindowArgs &W, int64_t No, int64_t mt_rows,
+                            int64_t nt_cols) {
+  const int64_t emax = std::max(W.ea, std::max(W.eb, W.ec));
+  W.mtiles = (int)((No * No + mt_rows - 1) / mt_rows);
+  W.ntiles = (int)((emax * No + nt_cols - 1) / nt_cols);
+  const int64_t units =
+      (int64_t)W.nw * (W.ea * W.eb + W.ea * W.ec + W.eb * W.ec);
+  return (units + 7) / 8 * 8 * W.mtiles * W.ntiles;
 }
 
 // W position (i,j,k) of GEMM element (row (p,q), column index rr).

@@ -40,86 +40,38 @@ constexpr int TILE = 128;  // doubles per operand tile
 struct DoublesParams {
   // T3s, H3s: row-swapped copies (null: read the swapped rows of T3, H3)
   const double *T3, *T3s, *V3, *H3, *H3s, *T2N, *T2TN;
-  const int32_t *windows;
-  const uint64_t *aprefix;
+  WindowArgs win;
   double *G;
   int64_t No, Nv, Kv, Ko, N2, N2p, W3, NoP, slots;
-  uint64_t first, last;
-  int nb, mtiles, ntiles;
-  int64_t total, per_xcd;
 };
 
-// B operand of segment sg at column (tuple (a, b, c), index rr): its row.
-__device__ inline const double *b_base(const DoublesParams &P, int cl, int sg,
-                                       int64_t a, int64_t b, int64_t c,
-                                       int64_t rr) {
-  int64_t u, v;
-  const int which = b_pair(cl, sg, a, b, c, u, v);
-  const double *Bt = which == 0 ? P.V3 : which == 1 ? P.T2N : P.T2TN;
-  return Bt + f64_row((u + P.Nv * v) * P.No + rr, sg < 2 ? P.Kv : P.Ko);
-}
-
-template <int FM, int FN>
-__global__ __launch_bounds__(256, FM *FN <= 16 ? 2 : 1) void doubles_f64_kernel(DoublesParams P) {
-  constexpr int MT = 32 * FM, NT = 32 * FN;
-  const int64_t bid = blockIdx.x;
-  const int64_t logical = (bid % 8) * P.per_xcd + bid / 8;  // XCD-aware
-  if (logical >= P.total) return;
-  int64_t rem = logical;
-  const int nt = (int)(rem % P.ntiles); rem /= P.ntiles;
-  const int mt = (int)(rem % P.mtiles); rem /= P.mtiles;
-  const int nb = P.nb;
-  const int pair = (int)(rem % (nb * nb)); rem /= (nb * nb);
-  const int cl = (int)(rem % 3); rem /= 3;
-  const int64_t w = rem;
-  const int64_t al = P.windows[3 * w], be = P.windows[3 * w + 1],
-                ga = P.windows[3 * w + 2];
-  const int o1 = pair / nb, o2 = pair % nb;
-
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// The FM x FN occupied fragments of one wave of a tile of 32 TM x 32 TN.  The
+// two waves of each direction take the tile's fragments in turn, so a tile at
+// the edge of the GEMM leaves both about the same number.
+template <int TM, int TN, int FM, int FN>
+__device__ __forceinline__ void f64_wave(const DoublesParams &P,
+                                         const TileWork &T, int No, int lane,
+                                         int wm, int wn) {
+  constexpr int MT = 32 * TM, NT = 32 * TN;
   const int kk = lane >> 4, l16 = lane & 15;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int64_t No = P.No, N2 = P.N2, Nv = P.Nv;
-
-  // columns (t, rr) of this lane's B fragments
-  int32_t ca[FN], cb[FN], cc[FN], cslot[FN], crr[FN];  // 32-bit: live all loop
-  bool cvalid[FN];
-  bool any = false;
+  const int64_t N2 = P.N2, Nv = P.Nv, N2p = P.N2p;
+  int32_t cy[FN], crr[FN];  // third index and column index of the columns
 #pragma unroll
   for (int g = 0; g < FN; g++) {
-    const int64_t n = (int64_t)nt * NT + wn * (NT / 2) + g * 16 + l16;
-    const int t = (int)(n / No);
-    crr[g] = (int32_t)(n % No);
-    int64_t a, b, c, slot;
-    class_tuple(cl, al, be, ga, nb, o1, o2, t, a, b, c, slot);
-    bool ok = t < nb && tuple_ok(Nv, a, b, c);
-    if (ok && (P.first > 0 || P.last != ~0ULL)) {
-      const uint64_t idx = tuple_index(P.aprefix, Nv, a, b, c);
-      ok = idx >= P.first && idx < P.last;
-    }
-    cvalid[g] = ok;
-    any |= ok;
-    if (!ok) { a = 0; b = 0; c = 0; crr[g] = 0; }  // safe load address
-    ca[g] = (int32_t)a; cb[g] = (int32_t)b; cc[g] = (int32_t)c;
-    cslot[g] = (int32_t)slot;
+    int n = T.nt * NT + (2 * g + wn) * 16 + l16;
+    if (n >= T.ncols) n = T.ncols - 1;  // safe load address, not stored
+    cy[g] = T.y0 + n / No;
+    crr[g] = n % No;
   }
-  if (!__syncthreads_or(any)) return;
-
-  // A-pair of this class: w (a,b), v (a,c), u (b,c)
-  int64_t x1, x2;
-  class_pair(cl, al, be, ga, nb, o1, o2, x1, x2);
-  if (x1 >= Nv) x1 = Nv - 1;
-  if (x2 >= Nv) x2 = Nv - 1;
-
   // rows: straight (p + No q) and swapped (q + No p) row of the A slab
-  int32_t rowS[FM], rowW[FM];  // 32-bit: live all loop
+  // (rows past the last occupied tile read its last row, not stored)
+  int32_t rowS[FM], rowW[FM];
 #pragma unroll
   for (int f = 0; f < FM; f++) {
-    int64_t m = (int64_t)mt * MT + wm * (MT / 2) + f * 16 + l16;
-    if (m >= N2) m = N2 - 1;
-    const int64_t p = m % No, q = m / No;
-    rowS[f] = (int32_t)m;
-    rowW[f] = (int32_t)(q + No * p);
+    int m = T.mt * MT + (2 * f + wm) * 16 + l16;
+    rowS[f] = m < N2p ? m : (int)N2p - 16 + l16;
+    if (m >= N2) m = (int)N2 - 1;
+    rowW[f] = m / No + No * (m % No);
   }
 
   const int64_t Kv = P.Kv, Ko = P.Ko;
@@ -128,15 +80,20 @@ __global__ __launch_bounds__(256, FM *FN <= 16 ? 2 : 1) void doubles_f64_kernel(
 #define SET_PTRS(SG)                                                        \
   {                                                                         \
     const int64_t K_ = (SG) < 2 ? Kv : Ko;                                  \
-    const int64_t xr_ = ((SG) == 0 || (SG) == 3 ? x1 : x2) * P.N2p;         \
+    const int64_t xr_ = ((SG) == 0 || (SG) == 3 ? T.x1 : T.x2) * N2p;       \
     const double *As_ = (SG) < 2 ? P.T3s : P.H3s;                           \
     const bool sw_ = ((SG)&1) && As_;                                       \
     const double *Ab_ = sw_ ? As_ : (SG) < 2 ? P.T3 : P.H3;                 \
     _Pragma("unroll") for (int f = 0; f < FM; f++) ap[f] =                  \
         Ab_ + f64_row(xr_ + (((SG)&1) && !sw_ ? rowW[f] : rowS[f]), K_) +   \
         32 * kk;                                                            \
-    _Pragma("unroll") for (int g = 0; g < FN; g++) bp[g] =                  \
-        b_base(P, cl, (SG), ca[g], cb[g], cc[g], crr[g]) + 32 * kk;         \
+    _Pragma("unroll") for (int g = 0; g < FN; g++) {                        \
+      int wh_;                                                              \
+      const int64_t R_ =                                                    \
+          b_row(T.cl, (SG), T.x1, T.x2, cy[g], crr[g], Nv, No, wh_);        \
+      const double *B_ = wh_ == 0 ? P.V3 : wh_ == 1 ? P.T2N : P.T2TN;       \
+      bp[g] = B_ + f64_row(R_, K_) + 32 * kk;                               \
+    }                                                                       \
   }
   d4 acc[FM][FN];
 #pragma unroll
@@ -172,31 +129,30 @@ __global__ __launch_bounds__(256, FM *FN <= 16 ? 2 : 1) void doubles_f64_kernel(
   // re-reads it, a load never used) so every path into a COMPUTE has the
   // same loads outstanding.
   int sg = 0;
-  int nch = (int)((P.Nv + KC - 1) / KC), c = 0;
+  int nch = (int)((Nv + KC - 1) / KC), c = 0;
   SET_PTRS(0);
 #define ADVANCE()                                                            \
   {                                                                          \
     if (++c == nch && ++sg < 4) {                                            \
       SET_PTRS(sg);                                                          \
-      nch = (int)(((sg < 2 ? P.Nv : No) + KC - 1) / KC);                     \
+      nch = (int)(((sg < 2 ? Nv : No) + KC - 1) / KC);                     \
       c = 0;                                                                 \
     }                                                                        \
   }
 #define NEXT() ((int64_t)(sg < 4 ? c : nch - 1))
   LOAD(a0, b0, 0);
   ADVANCE();
+  // (each segment length occurs twice, so the number of chunks is even; a
+  // second exit in the middle of the loop made the compiler copy the
+  // accumulators between register files on every turn)
 #pragma unroll 1
-  for (;;) {
-    const bool v1 = sg < 4;
+  for (int left = 2 * (int)((Nv + KC - 1) / KC + (No + KC - 1) / KC); left; left -= 2) {
     LOAD(a1, b1, NEXT());
-    if (v1) ADVANCE();
+    ADVANCE();
     COMPUTE(a0, b0);
-    if (!v1) break;
-    const bool v2 = sg < 4;
     LOAD(a0, b0, NEXT());
-    if (v2) ADVANCE();
+    if (sg < 4) ADVANCE();
     COMPUTE(a1, b1);
-    if (!v2) break;
   }
 #undef ADVANCE
 #undef NEXT
@@ -206,23 +162,61 @@ __global__ __launch_bounds__(256, FM *FN <= 16 ? 2 : 1) void doubles_f64_kernel(
 #undef SET_PTRS
   // store: for v_mfma_f64_16x16x4f64, D[i][j] sits in lane j + 16*(i%4),
   // register i/4 (measured on gfx950)
-  double *Gc = P.G + ((int64_t)cl * P.slots + w * (int64_t)nb * nb * nb) * P.W3;
+  const int64_t per = (int64_t)P.win.ea * P.win.eb * P.win.ec;
+  double *Gc = P.G + (T.cl * P.slots + T.w * per) * P.W3;
 #pragma unroll
   for (int g = 0; g < FN; g++) {
-    if (!cvalid[g]) continue;
-    double *Gs = Gc + cslot[g] * P.W3;
-    const int64_t rr = crr[g];
+    const int n = T.nt * NT + (2 * g + wn) * 16 + l16;
+    if (n >= T.ncols) continue;
+    const int t = n / No;
+    double *Gs = Gc + (int64_t)(T.slot0 + t * T.slot_step) * P.W3 + (n - t * No);
 #pragma unroll
     for (int f = 0; f < FM; f++) {
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const int64_t m =
-            (int64_t)mt * MT + wm * (MT / 2) + f * 16 + 4 * r + kk;
-        if (m >= N2) continue;
-        Gs[m * P.NoP + rr] = acc[f][g][r];  // GEMM order: contiguous rows
+        const int64_t m = T.mt * MT + (2 * f + wm) * 16 + 4 * r + kk;
+        if (m < N2) Gs[m * P.NoP] = acc[f][g][r];  // contiguous along n
       }
     }
   }
+}
+
+// Dispatch on the wave's occupied column fragments, n <= FN of them.
+template <int TM, int TN, int FM, int FN>
+__device__ __forceinline__ void f64_columns(const DoublesParams &P,
+                                            const TileWork &T, int No,
+                                            int lane, int wm, int wn, int n) {
+  if constexpr (FN > 1) {
+    if (n < FN) {
+      f64_columns<TM, TN, FM, FN - 1>(P, T, No, lane, wm, wn, n);
+      return;
+    }
+  }
+  f64_wave<TM, TN, FM, FN>(P, T, No, lane, wm, wn);
+}
+
+template <int FM, int FN>
+__global__ __launch_bounds__(256, FM *FN <= 16 ? 2 : 1) void doubles_f64_kernel(
+    DoublesParams P) {
+  const int No = (int)P.No;
+  TileWork T;
+  if (!tile_work(P.win, (uint64_t)P.Nv, No, 32 * FN, T)) return;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  // Fragments of this wave that hold rows and columns.  Tiles at the edges
+  // of the GEMM run the instance of their size instead of the whole tile on
+  // padding: every column count, the row count rounded up to half the tile
+  // (rows have one edge per A-pair, columns one per pair and valid third
+  // index; one instance with per-fragment branches doubled the accumulators).
+  const int m = occupied(P.N2 - (int64_t)T.mt * 32 * FM, wm, 16, FM);
+  const int n = occupied(T.ncols - (int64_t)T.nt * 32 * FN, wn, 16, FN);
+  if (!m || !n) return;
+  constexpr int H = (FM + 1) / 2;
+  if (m > H)
+    f64_columns<FM, FN, FM, FN>(P, T, No, lane, wm, wn, n);
+  else
+    f64_columns<FM, FN, H, FN>(P, T, No, lane, wm, wn, n);
 }
 
 }  // namespace
@@ -238,8 +232,7 @@ hipError_t launch_doubles_f64(const DevSystem &s, const BatchArgs &b,
   P.H3s = use_j ? s.H3Js : s.H3s;
   P.T2N = s.T2N;
   P.T2TN = s.T2TN;
-  P.windows = b.windows;
-  P.aprefix = s.aprefix;
+  P.win = b;
   P.G = G;
   P.No = s.No;
   P.Nv = s.Nv;
@@ -250,17 +243,9 @@ hipError_t launch_doubles_f64(const DevSystem &s, const BatchArgs &b,
   P.NoP = g_pitch(s.No, false);
   P.W3 = g_elems(s.No, false);
   P.slots = b.slots;
-  P.first = b.first;
-  P.last = b.last;
-  P.nb = b.nb;
-  tile = pick_tile(tile, s.No, b.nb);
+  tile = pick_tile(tile, s.No, std::max(b.ea, std::max(b.eb, b.ec)));
   const int FM = tile_fm(tile), FN = tile_fn(tile);
-  const int64_t MT = 32 * FM, NT = 32 * FN;
-  P.mtiles = (int)((P.N2 + MT - 1) / MT);
-  P.ntiles = (int)(((int64_t)b.nb * s.No + NT - 1) / NT);
-  P.total = (int64_t)b.nw * 3 * b.nb * b.nb * P.mtiles * P.ntiles;
-  P.per_xcd = (P.total + 7) / 8;
-  const int64_t grid = P.per_xcd * 8;
+  const int64_t grid = doubles_grid(P.win, s.No, 32 * FM, 32 * FN);
   if (grid <= 0) return hipSuccess;
   if (grid > MAX_GRID) return hipErrorInvalidConfiguration;
 #define LAUNCH(A, B)                                                       \

@@ -36,72 +36,35 @@ struct SplitParams {
   // per operand family: hi (float) and lo (bf16), row-major [row][K]
   const float *T3h, *H3h, *V3h, *T2Nh, *T2TNh;
   const __bf16 *T3l, *H3l, *V3l, *T2Nl, *T2TNl;
-  const int32_t *windows;
-  const uint64_t *aprefix;
+  WindowArgs win;
   float *G;
   int64_t No, Nv, Kv, Ko, N2, W3, NoP, slots;
-  uint64_t first, last;
-  int nb, mtiles, ntiles;
-  int64_t total, per_xcd;
 };
 
-template <int FM, int FN, bool CORR>
-__global__ __launch_bounds__(256) void doubles_split_kernel(SplitParams P) {
-  constexpr int MT = 64 * FM, NT = 64 * FN;
-  const int64_t bid = blockIdx.x;
-  const int64_t logical = (bid % 8) * P.per_xcd + bid / 8;  // XCD-aware
-  if (logical >= P.total) return;
-  int64_t rem = logical;
-  const int nt = (int)(rem % P.ntiles); rem /= P.ntiles;
-  const int mt = (int)(rem % P.mtiles); rem /= P.mtiles;
-  const int nb = P.nb;
-  const int pair = (int)(rem % (nb * nb)); rem /= (nb * nb);
-  const int cl = (int)(rem % 3); rem /= 3;
-  const int64_t w = rem;
-  const int64_t al = P.windows[3 * w], be = P.windows[3 * w + 1],
-                ga = P.windows[3 * w + 2];
-  const int o1 = pair / nb, o2 = pair % nb;
-
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// The FM x FN occupied fragments of one wave of a tile of 64 TM x 64 TN (the
+// waves of each direction take the fragments in turn, as the FP64 kernel).
+template <int TM, int TN, int FM, int FN, bool CORR>
+__device__ __forceinline__ void split_wave(const SplitParams &P, const TileWork &T, int No,
+                                         int lane, int wm, int wn) {
+  constexpr int MT = 64 * TM, NT = 64 * TN;
   const int kh = lane >> 5, l32 = lane & 31;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int64_t No = P.No, N2 = P.N2, Nv = P.Nv;
-
-  int32_t ca[FN], cb[FN], cc[FN], cslot[FN], crr[FN];  // 32-bit: live all loop
-  bool cvalid[FN];
-  bool any = false;
+  const int64_t N2 = P.N2, Nv = P.Nv;
+  int32_t cy[FN], crr[FN];  // third index and column index of the columns
 #pragma unroll
   for (int g = 0; g < FN; g++) {
-    const int64_t n = (int64_t)nt * NT + wn * (NT / 2) + g * 32 + l32;
-    const int t = (int)(n / No);
-    crr[g] = (int32_t)(n % No);
-    int64_t a, b, c, slot;
-    class_tuple(cl, al, be, ga, nb, o1, o2, t, a, b, c, slot);
-    bool ok = t < nb && tuple_ok(Nv, a, b, c);
-    if (ok && (P.first > 0 || P.last != ~0ULL)) {
-      const uint64_t idx = tuple_index(P.aprefix, Nv, a, b, c);
-      ok = idx >= P.first && idx < P.last;
-    }
-    cvalid[g] = ok;
-    any |= ok;
-    if (!ok) { a = 0; b = 0; c = 0; crr[g] = 0; }
-    ca[g] = (int32_t)a; cb[g] = (int32_t)b; cc[g] = (int32_t)c;
-    cslot[g] = (int32_t)slot;
+    int n = T.nt * NT + (2 * g + wn) * 32 + l32;
+    if (n >= T.ncols) n = T.ncols - 1;  // safe load address, not stored
+    cy[g] = T.y0 + n / No;
+    crr[g] = n % No;
   }
-  if (!__syncthreads_or(any)) return;
-
-  int64_t x1, x2;
-  class_pair(cl, al, be, ga, nb, o1, o2, x1, x2);
-  if (x1 >= Nv) x1 = Nv - 1;
-  if (x2 >= Nv) x2 = Nv - 1;
-  int32_t rowS[FM], rowW[FM];  // 32-bit: live all loop
+  // A rows: straight (p + No q) and swapped (q + No p)
+  int32_t rowS[FM], rowW[FM];
 #pragma unroll
   for (int f = 0; f < FM; f++) {
-    int64_t m = (int64_t)mt * MT + wm * (MT / 2) + f * 32 + l32;
-    if (m >= N2) m = N2 - 1;
-    const int64_t p = m % No, q = m / No;
-    rowS[f] = (int32_t)m;
-    rowW[f] = (int32_t)(q + No * p);
+    int m = T.mt * MT + (2 * f + wm) * 32 + l32;
+    if (m >= N2) m = (int)N2 - 1;
+    rowS[f] = m;
+    rowW[f] = m / No + No * (m % No);
   }
 
   const int64_t Kv = P.Kv, Ko = P.Ko;
@@ -110,7 +73,7 @@ __global__ __launch_bounds__(256) void doubles_split_kernel(SplitParams P) {
 #define SET_PTRS(SG)                                                          \
   {                                                                           \
     const int64_t K_ = (SG) < 2 ? Kv : Ko;                                    \
-    const int64_t xa_ = ((SG) == 0 || (SG) == 3) ? x1 : x2;                   \
+    const int64_t xa_ = ((SG) == 0 || (SG) == 3) ? T.x1 : T.x2;                   \
     const int64_t abase_ = xa_ * N2 * K_;                                     \
     const float *Ah_ = ((SG) < 2 ? P.T3h : P.H3h) + abase_;                   \
     const __bf16 *Al_ = ((SG) < 2 ? P.T3l : P.H3l) + abase_;                  \
@@ -120,9 +83,9 @@ __global__ __launch_bounds__(256) void doubles_split_kernel(SplitParams P) {
       apc[f] = Al_ + r_ + 8 * kh;                                             \
     }                                                                         \
     _Pragma("unroll") for (int g = 0; g < FN; g++) {                          \
-      int64_t u_, v_;                                                         \
-      const int wh_ = b_pair(cl, (SG), ca[g], cb[g], cc[g], u_, v_);          \
-      const int64_t c_ = ((u_ + Nv * v_) * No + crr[g]) * K_;                 \
+      int wh_;                                                                \
+      const int64_t c_ =                                                      \
+          b_row(T.cl, (SG), T.x1, T.x2, cy[g], crr[g], Nv, No, wh_) * K_;     \
       const float *Bh_ = wh_ == 0 ? P.V3h : wh_ == 1 ? P.T2Nh : P.T2TNh;      \
       const __bf16 *Bl_ = wh_ == 0 ? P.V3l : wh_ == 1 ? P.T2Nl : P.T2TNl;     \
       bph[g] = Bh_ + c_ + 8 * kh;                                             \
@@ -197,18 +160,17 @@ __global__ __launch_bounds__(256) void doubles_split_kernel(SplitParams P) {
 #define NEXT_OFF() (KCHUNK * (sg < 4 ? c : nch - 1))
   LOAD(a0, b0, 0);
   ADVANCE();
+  // (each segment length occurs twice, so the number of chunks is even; a
+  // second exit in the middle of the loop made the compiler copy the
+  // accumulators between register files on every turn)
 #pragma unroll 1
-  for (;;) {
-    const bool v1 = sg < 4;
+  for (int left = 2 * (int)((Kv + Ko) / KCHUNK); left; left -= 2) {
     LOAD(a1, b1, NEXT_OFF());
-    if (v1) ADVANCE();
+    ADVANCE();
     COMPUTE(a0, b0);
-    if (!v1) break;
-    const bool v2 = sg < 4;
     LOAD(a0, b0, NEXT_OFF());
-    if (v2) ADVANCE();
+    if (sg < 4) ADVANCE();
     COMPUTE(a1, b1);
-    if (!v2) break;
   }
 #undef ADVANCE
 #undef NEXT_OFF
@@ -218,23 +180,57 @@ __global__ __launch_bounds__(256) void doubles_split_kernel(SplitParams P) {
 
   // 32x32 FP32-output MFMAs: D[i][j] in lane j + 32 ((i / 4) % 2), register
   // 4 (i / 8) + i % 4
-  float *Gc = P.G + ((int64_t)cl * P.slots + w * (int64_t)nb * nb * nb) * P.W3;
+  const int64_t per = (int64_t)P.win.ea * P.win.eb * P.win.ec;
+  float *Gc = P.G + (T.cl * P.slots + T.w * per) * P.W3;
 #pragma unroll
   for (int g = 0; g < FN; g++) {
-    if (!cvalid[g]) continue;
-    float *Gs = Gc + cslot[g] * P.W3;
-    const int64_t rr = crr[g];
+    const int n = T.nt * NT + (2 * g + wn) * 32 + l32;
+    if (n >= T.ncols) continue;
+    const int t = n / No;
+    float *Gs = Gc + (int64_t)(T.slot0 + t * T.slot_step) * P.W3 + (n - t * No);
 #pragma unroll
     for (int f = 0; f < FM; f++) {
 #pragma unroll
       for (int r = 0; r < 16; r++) {
-        const int64_t m = (int64_t)mt * MT + wm * (MT / 2) + f * 32 +
-                          8 * (r >> 2) + 4 * kh + (r & 3);
-        if (m >= N2) continue;
-        Gs[m * P.NoP + rr] = acc[f][g][r];  // GEMM order: contiguous rows
+        const int64_t m = T.mt * MT + (2 * f + wm) * 32 + 8 * (r >> 2) + 4 * kh +
+                          (r & 3);
+        if (m < N2) Gs[m * P.NoP] = acc[f][g][r];  // contiguous along n
       }
     }
   }
+}
+
+// Dispatch on the wave's occupied column fragments, n <= FN of them.
+template <int TM, int TN, int FM, int FN, bool CORR>
+__device__ __forceinline__ void split_columns(const SplitParams &P, const TileWork &T,
+                                            int No, int lane, int wm, int wn,
+                                            int n) {
+  if constexpr (FN > 1) {
+    if (n < FN) {
+      split_columns<TM, TN, FM, FN - 1, CORR>(P, T, No, lane, wm, wn, n);
+      return;
+    }
+  }
+  split_wave<TM, TN, FM, FN, CORR>(P, T, No, lane, wm, wn);
+}
+
+template <int FM, int FN, bool CORR>
+__global__ __launch_bounds__(256) void doubles_split_kernel(SplitParams P) {
+  const int No = (int)P.No;
+  TileWork T;
+  if (!tile_work(P.win, (uint64_t)P.Nv, No, 64 * FN, T)) return;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  // edge tiles run the instance of their occupied fragments (FP64 kernel)
+  const int m = occupied(P.N2 - (int64_t)T.mt * 64 * FM, wm, 32, FM);
+  const int n = occupied(T.ncols - (int64_t)T.nt * 64 * FN, wn, 32, FN);
+  if (!m || !n) return;
+  constexpr int H = (FM + 1) / 2;
+  if (m > H)
+    split_columns<FM, FN, FM, FN, CORR>(P, T, No, lane, wm, wn, n);
+  else
+    split_columns<FM, FN, H, FN, CORR>(P, T, No, lane, wm, wn, n);
 }
 
 }  // namespace
@@ -250,8 +246,7 @@ hipError_t launch_doubles_split(const DevSystem &s, const BatchArgs &b,
   P.T3l = (const __bf16 *)s.sT3.l; P.H3l = (const __bf16 *)H.l;
   P.V3l = (const __bf16 *)V.l; P.T2Nl = (const __bf16 *)s.sT2N.l;
   P.T2TNl = (const __bf16 *)s.sT2TN.l;
-  P.windows = b.windows;
-  P.aprefix = s.aprefix;
+  P.win = b;
   P.G = G;
   P.No = s.No;
   P.Nv = s.Nv;
@@ -261,17 +256,9 @@ hipError_t launch_doubles_split(const DevSystem &s, const BatchArgs &b,
   P.NoP = g_pitch(s.No, true);
   P.W3 = g_elems(s.No, true);
   P.slots = b.slots;
-  P.first = b.first;
-  P.last = b.last;
-  P.nb = b.nb;
-  tile = pick_t32_tile(tile, s.No, b.nb);
+  tile = pick_t32_tile(tile, s.No, std::max(b.ea, std::max(b.eb, b.ec)));
   const int FM = t32_fm(tile), FN = t32_fn(tile);
-  const int64_t MT = 64 * FM, NT = 64 * FN;
-  P.mtiles = (int)((P.N2 + MT - 1) / MT);
-  P.ntiles = (int)(((int64_t)b.nb * s.No + NT - 1) / NT);
-  P.total = (int64_t)b.nw * 3 * b.nb * b.nb * P.mtiles * P.ntiles;
-  P.per_xcd = (P.total + 7) / 8;
-  const int64_t grid = P.per_xcd * 8;
+  const int64_t grid = doubles_grid(P.win, s.No, 64 * FM, 64 * FN);
   if (grid <= 0) return hipSuccess;
   if (grid > MAX_GRID) return hipErrorInvalidConfiguration;
 #define LAUNCH(A, B)                                                         \

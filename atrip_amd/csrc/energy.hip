@@ -25,12 +25,9 @@ namespace {
 struct EnergyParams {
   const double *W, *WJ;  // W (and the (cT) pass's W) as cubes, [slot][W3]
   const double *Tai, *VHH, *ei, *ea;
-  const int32_t *windows;
-  const uint64_t *aprefix;
+  WindowArgs win;
   double *e_slot;
   int64_t No, Nv, N2, W3, nbk, slots;  // nbk: cubes per index, W3 = (8 nbk)^3
-  uint64_t first, last;
-  int nb;
   double tai_sign;
 };
 
@@ -258,20 +255,9 @@ template <bool HJ>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8)))
 void energy_kernel(EnergyParams P) {
   const int64_t gslot = blockIdx.x;
-  const int nb = P.nb;
-  const int64_t nb3 = (int64_t)nb * nb * nb;
-  const int64_t w = gslot / nb3, s = gslot % nb3;
-  const int64_t ta = s / (nb * nb), tb = (s / nb) % nb, tc = s % nb;
-  const int64_t a = P.windows[3 * w] * (int64_t)nb + ta;
-  const int64_t b = P.windows[3 * w + 1] * (int64_t)nb + tb;
-  const int64_t c = P.windows[3 * w + 2] * (int64_t)nb + tc;
   const int64_t No = P.No, Nv = P.Nv, N2 = P.N2;
-  bool ok = tuple_ok(Nv, a, b, c);
-  if (ok && (P.first > 0 || P.last != ~0ULL)) {
-    const uint64_t idx = tuple_index(P.aprefix, Nv, a, b, c);
-    ok = idx >= P.first && idx < P.last;
-  }
-  if (!ok) {
+  int64_t a, b, c;
+  if (!slot_tuple(P.win, (uint64_t)Nv, blockIdx.x, a, b, c)) {
     if (threadIdx.x == 0) {
       P.e_slot[2 * gslot] = 0.0;
       P.e_slot[2 * gslot + 1] = 0.0;
@@ -452,12 +438,10 @@ void energy_kernel(EnergyParams P) {
 struct FusedParams {
   const void *G, *GJ;  // class buffers [3][slots][No^2 rows][NoP] (FP64 or FP32)
   const double *Tai, *VHH, *ei, *ea;
-  const int32_t *windows;
-  const uint64_t *aprefix;
+  WindowArgs win;
   double *e_part;  // [slot][triple][2]
   int64_t No, Nv, N2, NoP, W3g, slots, ntri;
-  uint64_t first, last;
-  int nb, nbk;
+  int nbk;
   double tai_sign;
 };
 
@@ -646,23 +630,10 @@ __global__ __launch_bounds__(256) void energy_fused_kernel(FusedParams P) {
   if ((int64_t)gs >= P.slots) return;
   const int64_t gslot = gs;
   const int64_t gid = gslot * P.ntri + tri;
-  const int nb = P.nb;
-  const uint32_t nb2 = (uint32_t)(nb * nb), nb3 = nb2 * (uint32_t)nb;
-  const uint32_t w32 = gs / nb3, s32 = gs - w32 * nb3;
-  const uint32_t ta32 = s32 / nb2, r2 = s32 - ta32 * nb2;
-  const uint32_t tb32 = r2 / (uint32_t)nb, tc32 = r2 - tb32 * (uint32_t)nb;
-  const int64_t w = w32, ta = ta32, tb = tb32, tc = tc32;
-  const int64_t a = P.windows[3 * w] * (int64_t)nb + ta;
-  const int64_t b = P.windows[3 * w + 1] * (int64_t)nb + tb;
-  const int64_t c = P.windows[3 * w + 2] * (int64_t)nb + tc;
   const int64_t No = P.No, Nv = P.Nv;
   const int tid = threadIdx.x;
-  bool ok = tuple_ok(Nv, a, b, c);
-  if (ok && (P.first > 0 || P.last != ~0ULL)) {
-    const uint64_t idx = tuple_index(P.aprefix, Nv, a, b, c);
-    ok = idx >= P.first && idx < P.last;
-  }
-  if (!ok) {
+  int64_t a, b, c;
+  if (!slot_tuple(P.win, (uint64_t)Nv, gs, a, b, c)) {
     if (tid == 0) {
       P.e_part[2 * gid] = 0.0;
       P.e_part[2 * gid + 1] = 0.0;
@@ -841,8 +812,7 @@ hipError_t launch_energy(const DevSystem &s, const BatchArgs &b,
     P.VHH = s.VHH;
     P.ei = s.ei;
     P.ea = s.ea;
-    P.windows = b.windows;
-    P.aprefix = s.aprefix;
+    P.win = b;
     P.e_part = scratch;
     P.No = s.No;
     P.Nv = s.Nv;
@@ -851,9 +821,6 @@ hipError_t launch_energy(const DevSystem &s, const BatchArgs &b,
     P.W3g = g_elems(s.No, g32);
     P.slots = b.slots;
     P.ntri = ntri;
-    P.first = b.first;
-    P.last = b.last;
-    P.nb = b.nb;
     P.nbk = (int)nbk;
     P.tai_sign = tai_sign;
     const int64_t grid = (b.slots + 7) / 8 * 8 * ntri;
@@ -893,8 +860,7 @@ hipError_t launch_energy(const DevSystem &s, const BatchArgs &b,
   P.VHH = s.VHH;
   P.ei = s.ei;
   P.ea = s.ea;
-  P.windows = b.windows;
-  P.aprefix = s.aprefix;
+  P.win = b;
   P.e_slot = e_slot;
   P.No = s.No;
   P.Nv = s.Nv;
@@ -902,9 +868,6 @@ hipError_t launch_energy(const DevSystem &s, const BatchArgs &b,
   P.nbk = w_blocks(s.No);
   P.W3 = W3c;
   P.slots = b.slots;
-  P.first = b.first;
-  P.last = b.last;
-  P.nb = b.nb;
   P.tai_sign = tai_sign;
   const dim3 grid((unsigned)b.slots), block(256);
   if (GJ)

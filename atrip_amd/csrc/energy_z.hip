@@ -40,12 +40,9 @@ __device__ inline double re_div(cplx a, cplx b) {
 struct EnergyZParams {
   const double *Wr, *Wi, *WJr, *WJi;  // cubes, [slot][W3]
   const double *Tair, *Taii, *VHHr, *VHHi, *eir, *eii, *ear;
-  const int32_t *windows;
-  const uint64_t *aprefix;
+  WindowArgs win;
   double *e_slot;
   int64_t No, Nv, N2, W3, nbk, slots;  // nbk: cubes per index, W3 = (8 nbk)^3
-  uint64_t first, last;
-  int nb;
   double tai_sign;
 };
 
@@ -58,19 +55,9 @@ __device__ inline double wave_sum(double v) {
 template <bool HJ>
 __global__ __launch_bounds__(256) void energy_z_kernel(EnergyZParams P) {
   const int64_t gslot = blockIdx.x;
-  const int nb = P.nb;
-  const int64_t nb3 = (int64_t)nb * nb * nb;
-  const int64_t w = gslot / nb3, s = gslot % nb3;
-  const int64_t a = P.windows[3 * w] * (int64_t)nb + s / (nb * nb);
-  const int64_t b = P.windows[3 * w + 1] * (int64_t)nb + (s / nb) % nb;
-  const int64_t c = P.windows[3 * w + 2] * (int64_t)nb + s % nb;
   const int64_t No = P.No, Nv = P.Nv, N2 = P.N2;
-  bool ok = tuple_ok(Nv, a, b, c);
-  if (ok && (P.first > 0 || P.last != ~0ULL)) {
-    const uint64_t idx = tuple_index(P.aprefix, Nv, a, b, c);
-    ok = idx >= P.first && idx < P.last;
-  }
-  if (!ok) {
+  int64_t a, b, c;
+  if (!slot_tuple(P.win, (uint64_t)Nv, blockIdx.x, a, b, c)) {
     if (threadIdx.x == 0) {
       P.e_slot[2 * gslot] = 0.0;
       P.e_slot[2 * gslot + 1] = 0.0;
@@ -216,8 +203,7 @@ hipError_t launch_energy_z(const DevSystem &s, const BatchArgs &b,
   P.eir = s.ei;
   P.eii = s.eii;
   P.ear = s.ea;
-  P.windows = b.windows;
-  P.aprefix = s.aprefix;
+  P.win = b;
   P.e_slot = e_slot;
   P.No = s.No;
   P.Nv = s.Nv;
@@ -225,9 +211,6 @@ hipError_t launch_energy_z(const DevSystem &s, const BatchArgs &b,
   P.nbk = w_blocks(s.No);
   P.W3 = W3c;
   P.slots = b.slots;
-  P.first = b.first;
-  P.last = b.last;
-  P.nb = b.nb;
   P.tai_sign = tai_sign;
   const dim3 grid((unsigned)b.slots), block(256);
   if (GJ)

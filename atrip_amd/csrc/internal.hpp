@@ -314,14 +314,25 @@ namespace atrip_amd {
 
 // ---- launch wrappers (one translation unit each) -----------------------
 
-// Batch of consecutive windows handed to the hot kernels.
-struct BatchArgs {
-  const int32_t *windows;  // device, 3 per window of this batch
-  int nw;                  // windows in the batch
-  int nb;                  // window edge
-  uint64_t first, last;    // canonical tuple range [first, last)
-  int64_t slots;           // nw * nb^3
+// Batch of consecutive windows handed to the hot kernels: window w holds the
+// tuples (a0 + ta, b0 + tb, c0 + tc), ta < ea, tb < eb, tc < ec, from its
+// origin (a0, b0, c0) at windows[3 w]; slot (ta eb + tb) ec + tc of window w
+// is slot w ea eb ec + that of the batch.
+struct WindowArgs {
+  const int32_t *windows;   // device, 3 per window of this batch
+  const uint64_t *aprefix;  // of the system (tuple_index)
+  uint64_t first, last;     // canonical tuple range [first, last)
+  int nw;                   // windows in the batch
+  int ea, eb, ec;           // window edges, at most 32
+  int mtiles, ntiles;       // tiles of a pair's GEMM (set by the launchers)
 };
+struct BatchArgs : WindowArgs {
+  int64_t slots;  // nw * ea * eb * ec
+};
+// Tuple of batch slot gs, false outside the range or the ordered tuples.
+__device__ __forceinline__ bool slot_tuple(const WindowArgs &W, uint64_t Nv,
+                                           uint32_t gs, int64_t &a, int64_t &b,
+                                           int64_t &c);
 
 // Doubles contractions in FP64 MFMA: class buffers G[3][slots][g_elems(No)].
 hipError_t launch_doubles_f64(const DevSystem &s, const BatchArgs &b,
@@ -504,6 +515,23 @@ __host__ __device__ inline uint64_t tuple_index(const uint64_t *aprefix,
 __host__ __device__ inline bool tuple_ok(uint64_t Nv, uint64_t a, uint64_t b,
                                          uint64_t c) {
   return a <= b && b <= c && c < Nv && !(a == b && b == c);
+}
+
+// (32-bit arithmetic: a 64-bit division is ~130 scalar instructions)
+__device__ __forceinline__ bool slot_tuple(const WindowArgs &W, uint64_t Nv,
+                                           uint32_t gs, int64_t &a, int64_t &b,
+                                           int64_t &c) {
+  const uint32_t ebc = (uint32_t)(W.eb * W.ec), per = ebc * (uint32_t)W.ea;
+  const uint32_t w = gs / per, s = gs - w * per;
+  const uint32_t ta = s / ebc, r = s - ta * ebc;
+  const uint32_t tb = r / (uint32_t)W.ec, tc = r - tb * (uint32_t)W.ec;
+  a = W.windows[3 * w] + (int64_t)ta;
+  b = W.windows[3 * w + 1] + (int64_t)tb;
+  c = W.windows[3 * w + 2] + (int64_t)tc;
+  if (!tuple_ok(Nv, a, b, c)) return false;
+  if (W.first == 0 && W.last == ~0ULL) return true;
+  const uint64_t idx = tuple_index(W.aprefix, Nv, a, b, c);
+  return idx >= W.first && idx < W.last;
 }
 
 }  // namespace atrip_amd
