@@ -749,8 +749,33 @@ struct HostIndex {
   }
 };
 
+// Windows of a run: origins (a0, b0, c0), tuples each holds, edges.
+struct Windows {
+  std::vector<int32_t> origin;
+  std::vector<uint64_t> count;
+  int ea = 0, eb = 0, ec = 0;
+  // Adds the window at an origin if it holds a tuple of [first, last): the
+  // tuples of a row (a, b) are consecutive in c.
+  void add(const HostIndex &h, uint64_t first, uint64_t last, uint64_t a0,
+           uint64_t b0, uint64_t c0) {
+    uint64_t n = 0;
+    for (uint64_t a = a0; a < std::min<uint64_t>(a0 + ea, h.Nv); a++)
+      for (uint64_t b = std::max(a, b0); b < std::min<uint64_t>(b0 + eb, h.Nv); b++) {
+        const uint64_t c = std::max(c0, b + (a == b)),
+                       e = std::min<uint64_t>(c0 + ec, h.Nv);
+        if (c >= e) continue;
+        const uint64_t q = std::max(first, h(a, b, c)),
+                       z = std::min(last, h(a, b, e - 1) + 1);
+        if (z > q) n += z - q;
+      }
+    if (!n) return;
+    origin.insert(origin.end(), {(int32_t)a0, (int32_t)b0, (int32_t)c0});
+    count.push_back(n);
+  }
+};
+
 // Window plan for a system at the context's window edge: the block triples
-// in lexicographic order with their canonical index span and tuple count.
+// in lexicographic order holding a tuple, with their tuple counts.
 WindowPlan &get_plan(atrip_hip_ctx *ctx, int sys, const DevSystem &s,
                      int nb_want = 0) {
   if (nb_want <= 0) nb_want = window_edge(ctx, s);
@@ -759,31 +784,14 @@ WindowPlan &get_plan(atrip_hip_ctx *ctx, int sys, const DevSystem &s,
   if (it != ctx->plans.end()) ctx->plans.erase(it);
   WindowPlan p;
   p.nb = nb_want;
-  p.nblk = (int)((s.Nv + p.nb - 1) / p.nb);
-  const HostIndex hidx((uint64_t)s.Nv);
-  const int nb = p.nb;
-  for (int al = 0; al < p.nblk; al++)
-    for (int be = al; be < p.nblk; be++)
-      for (int ga = be; ga < p.nblk; ga++) {
-        uint64_t lo = ~0ULL, hi = 0, cnt = 0;
-        for (int ta = 0; ta < nb; ta++)
-          for (int tb = 0; tb < nb; tb++)
-            for (int tc = 0; tc < nb; tc++) {
-              const uint64_t a = (uint64_t)al * nb + ta,
-                             b = (uint64_t)be * nb + tb,
-                             c = (uint64_t)ga * nb + tc;
-              if (!tuple_ok(s.Nv, a, b, c)) continue;
-              const uint64_t q = hidx(a, b, c);
-              lo = std::min(lo, q);
-              hi = std::max(hi, q);
-              cnt++;
-            }
-        if (!cnt) continue;
-        p.windows.insert(p.windows.end(), {al, be, ga});
-        p.wmin.push_back(lo);
-        p.wmax.push_back(hi);
-        p.wcount.push_back(cnt);
-      }
+  const HostIndex h((uint64_t)s.Nv);
+  Windows w;
+  w.ea = w.eb = w.ec = p.nb;
+  for (int64_t a = 0; a < s.Nv; a += p.nb)
+    for (int64_t b = a; b < s.Nv; b += p.nb)
+      for (int64_t c = b; c < s.Nv; c += p.nb) w.add(h, 0, ~0ULL, a, b, c);
+  p.origin = std::move(w.origin);
+  p.wcount = std::move(w.count);
   return ctx->plans.emplace(sys, std::move(p)).first->second;
 }
 
@@ -868,45 +876,34 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
   if (first >= last) return res;
   const int nb = plan.nb;
   const bool full = first == 0 && last == n;
-  HostIndex hidx((uint64_t)s.Nv);
   // select windows and count their tuples in range
-  std::vector<int32_t> sel;
-  std::vector<uint64_t> counts;
-  const size_t nwin = plan.windows.size() / 3;
-  int64_t pair = -1, prev_al = -1, prev_be = -1;  // (alpha, beta) row index
-  for (size_t w = 0; w < nwin; w++) {
-    const int64_t al = plan.windows[3 * w], be = plan.windows[3 * w + 1],
-                  ga = plan.windows[3 * w + 2];
-    if (al != prev_al || be != prev_be) {
-      pair++;
-      prev_al = al;
-      prev_be = be;
+  Windows win;
+  win.ea = win.eb = win.ec = nb;
+  if (full) {
+    const size_t nwin = plan.wcount.size();
+    int64_t pair = -1, prev_a = -1, prev_b = -1;  // (alpha, beta) row index
+    for (size_t w = 0; w < nwin; w++) {
+      const int32_t *o = &plan.origin[3 * w];
+      if (o[0] != prev_a || o[1] != prev_b) {
+        pair++;
+        prev_a = o[0];
+        prev_b = o[1];
+      }
+      if (w < wsel.wbegin || w >= wsel.wend) continue;
+      if (wsel.stride > 1 && (uint64_t)pair % wsel.stride != wsel.offset % wsel.stride)
+        continue;
+      win.origin.insert(win.origin.end(), o, o + 3);
+      win.count.push_back(plan.wcount[w]);
     }
-    if (w < wsel.wbegin || w >= wsel.wend) continue;
-    if (wsel.stride > 1 && (uint64_t)pair % wsel.stride != wsel.offset % wsel.stride)
-      continue;
-    uint64_t cnt = 0;
-    if (full || (plan.wmin[w] >= first && plan.wmax[w] < last)) {
-      cnt = plan.wcount[w];
-    } else if (plan.wmax[w] < first || plan.wmin[w] >= last) {
-      continue;
-    } else {
-      for (int ta = 0; ta < nb; ta++)
-        for (int tb = 0; tb < nb; tb++)
-          for (int tc = 0; tc < nb; tc++) {
-            const uint64_t a = al * nb + ta, b = be * nb + tb,
-                           c = ga * nb + tc;
-            if (!tuple_ok(s.Nv, a, b, c)) continue;
-            const uint64_t q = hidx(a, b, c);
-            if (q >= first && q < last) cnt++;
-          }
-    }
-    if (!cnt) continue;
-    sel.insert(sel.end(), {(int32_t)al * nb, (int32_t)be * nb, (int32_t)ga * nb});
-    counts.push_back(cnt);
-    res.tuples += cnt;
+  } else {
+    const HostIndex h((uint64_t)s.Nv);
+    for (int64_t a = 0; a < s.Nv; a += nb)
+      for (int64_t b = a; b < s.Nv; b += nb)
+        for (int64_t c = b; c < s.Nv; c += nb) win.add(h, first, last, a, b, c);
   }
-  const int nsel = (int)counts.size();
+  const std::vector<int32_t> &sel = win.origin;
+  for (uint64_t c : win.count) res.tuples += c;
+  const int nsel = (int)win.count.size();
   if (!nsel) return res;
   // Device scratch of the run: class buffers G (and those of the (cT)
   // pass; four sets for complex systems), per-slot energies, the energy
@@ -914,7 +911,7 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
   // and the cube epilogue), batch partials and the window list.  Taken from the context's buffers (grown
   // on demand), or carved out of a fixed region without any allocation
   // (then the windows per launch shrink until the run fits).
-  const int64_t nb3 = (int64_t)nb * nb * nb;
+  const int64_t per = (int64_t)win.ea * win.eb * win.ec;  // slots of a window
   const int64_t W3 = g_elems(s.No, g32);  // one tuple's class buffer
   const bool use_j = s.has_j;
   const int nsets = s.cplx ? 4 : 1;
@@ -927,7 +924,7 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
   };
   auto sizes = [&](int bw_) {
     Sizes z;
-    z.slots_max = (int64_t)std::min(bw_, nsel) * nb3;
+    z.slots_max = (int64_t)std::min(bw_, nsel) * per;
     z.gsz = (size_t)(3 * z.slots_max * W3) * gelem;
     z.g = (size_t)((use_j ? 2 : 1) * nsets) * z.gsz;
     z.e_slot = (size_t)(2 * z.slots_max) * sizeof(double);
@@ -935,7 +932,8 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
                                          s.No, use_j, s.cplx, fused)) *
               sizeof(double);
     z.nbatch = (nsel + bw_ - 1) / bw_;
-    z.partials = (size_t)(4 * z.nbatch) * sizeof(double);
+    z.partials = (size_t)(4 * z.nbatch * slot_partials(z.slots_max)) *
+                 sizeof(double);
     z.windows = sel.size() * sizeof(int32_t);
     return z;
   };
@@ -946,6 +944,9 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
   };
 
   int bw = std::max(1, ctx->batch);
+  if (!ctx->batch_set)
+    bw = std::max(bw, auto_batch((use_j ? 2 : 1) * nsets * 3 * W3 *
+                                     (int64_t)gelem, per));
   void *Gbuf = nullptr, *e_slot = nullptr, *wcube = nullptr,
        *partials = nullptr, *d_sel = nullptr;
   Sizes z;
@@ -961,7 +962,7 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
     if (total(z) > fixed->bytes) {
       // largest window edge whose single window fits (class buffers, cubes
       // and slot energies scale with edge^3)
-      const size_t per_slot = (z.g + z.wcube + z.e_slot) / (size_t)nb3;
+      const size_t per_slot = (z.g + z.wcube + z.e_slot) / (size_t)per;
       const size_t rest = a256(z.partials) + a256(z.windows) + 3 * 256;
       int fit = 0;
       for (int e = nb - 1; e >= 1 && !fit; e--)
@@ -999,12 +1000,23 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
     check(hipMemcpyAsync(d_sel, sel.data(), z.windows, hipMemcpyHostToDevice,
                          ctx->stream),
           "upload windows");
-    ensure((void *&)ctx->G, ctx->G_bytes, z.g, "alloc G");
-    ensure((void *&)ctx->e_slot, ctx->e_slot_bytes, z.e_slot, "alloc e_slot");
-    ensure((void *&)ctx->wcube, ctx->wcube_bytes, z.wcube,
-           "alloc energy scratch");
-    ensure((void *&)ctx->partials, ctx->partials_bytes, z.partials,
-           "alloc partials");
+    for (;;) {
+      try {
+        ensure((void *&)ctx->G, ctx->G_bytes, z.g, "alloc G");
+        ensure((void *&)ctx->e_slot, ctx->e_slot_bytes, z.e_slot, "alloc e_slot");
+        ensure((void *&)ctx->wcube, ctx->wcube_bytes, z.wcube,
+               "alloc energy scratch");
+        ensure((void *&)ctx->partials, ctx->partials_bytes, z.partials,
+               "alloc partials");
+        break;
+      } catch (const Fail &) {
+        // a device with little memory left: launches of the option's size
+        if (bw <= std::max(1, ctx->batch)) throw;
+        (void)hipGetLastError();
+        bw = std::max(1, ctx->batch);
+        z = sizes(bw);
+      }
+    }
     Gbuf = ctx->G;
     e_slot = ctx->e_slot;
     wcube = ctx->wcube;
@@ -1012,6 +1024,7 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
   }
   const size_t gsz = z.gsz;
   const int nbatch = z.nbatch;
+  int64_t nparts = 0;  // partials written
   DevSystem zpass[4];
   if (s.cplx) complex_passes(s, zpass);
   // timing events are objects the runtime creates: none without allocation
@@ -1032,19 +1045,20 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
   void *G = Gbuf;
   void *GJ = use_j ? (void *)((char *)Gbuf + gsz) : nullptr;
   std::vector<double> host_slots;
-
   for (int bi = 0; bi < nbatch; bi++) {
     BatchArgs b;
     const int w0 = bi * bw;
     b.nw = std::min(bw, nsel - w0);
     b.windows = (const int32_t *)d_sel + 3 * w0;
     b.aprefix = s.aprefix;
-    b.ea = b.eb = b.ec = nb;
+    b.ea = win.ea;
+    b.eb = win.eb;
+    b.ec = win.ec;
     b.first = full ? 0 : first;
     b.last = full ? ~0ULL : last;
-    b.slots = (int64_t)b.nw * nb3;
+    b.slots = (int64_t)b.nw * per;
     uint64_t cnt = 0;
-    for (int w = 0; w < b.nw; w++) cnt += counts[w0 + w];
+    for (int w = 0; w < b.nw; w++) cnt += win.count[w0 + w];
     // the batch's timing events; destroyed here unless handed to the
     // context's pending list (a launch that throws leaves none behind)
     struct BatchEvents {
@@ -1099,11 +1113,14 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
       ctx->pending_flop.push_back(0.0);
       ev.handed = true;
     }
-    check(launch_batch_reduce(s, b, (double *)e_slot, (double *)partials, bi,
-                              st),
-          "reduce kernel");
+    check(launch_slot_sums(fused && !s.cplx ? (const double *)wcube : nullptr,
+                           b.slots, n_triples(w_blocks(s.No)),
+                           (double *)e_slot, (double *)partials + 4 * nparts,
+                           st),
+          "slot sums kernel");
+    nparts += slot_partials(b.slots);
     if constexpr (kWinSums) {
-      check(launch_window_sums((const double *)e_slot, b.nw, nb3,
+      check(launch_window_sums((const double *)e_slot, b.nw, per,
                                wsum_dev + 2 * w0, st),
             "window sums kernel");
     } else if (sink.active()) {
@@ -1113,10 +1130,10 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
                            hipMemcpyDeviceToHost, st),
             "download slots");
       check(hipStreamSynchronize(st), "slots");
-      sink(sel.data() + 3 * w0, b.nw, nb, host_slots);
+      sink(sel.data() + 3 * w0, b, host_slots);
     }
   }
-  std::vector<double> part(4 * nbatch);
+  std::vector<double> part(4 * nparts);
   check(hipMemcpyAsync(part.data(), (double *)partials, part.size() * sizeof(double),
                        hipMemcpyDeviceToHost, st),
         "download partials");
@@ -1127,14 +1144,14 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
           "download window sums");
   check(hipStreamSynchronize(st), "run");
   if constexpr (kWinSums) sink.windows(wsums);
-  // Neumaier over the batch partials in batch order
+  // Neumaier over the partials in slot order
   double s0 = 0, c0 = 0, s1 = 0, c1 = 0;
   auto add = [](double &sum, double &comp, double x) {
     const double t = sum + x;
     comp += (std::fabs(sum) >= std::fabs(x)) ? (sum - t) + x : (x - t) + sum;
     sum = t;
   };
-  for (int bi = 0; bi < nbatch; bi++) {
+  for (int64_t bi = 0; bi < nparts; bi++) {
     add(s0, c0, part[4 * bi]);
     add(s0, c0, part[4 * bi + 1]);
     add(s1, c1, part[4 * bi + 2]);
@@ -1160,7 +1177,7 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
 struct NoSink {
   static constexpr bool window_sums() { return false; }
   bool active() const { return false; }
-  void operator()(const int32_t *, int, int, const std::vector<double> &) {}
+  void operator()(const int32_t *, const BatchArgs &, const std::vector<double> &) {}
 };
 
 }  // namespace
@@ -1171,7 +1188,7 @@ int atrip_amd::window_edge(const atrip_hip_ctx *ctx, const DevSystem &s) {
 
 uint64_t atrip_amd::plan_windows(atrip_hip_ctx *ctx, int sys, int nb) {
   DevSystem &s = get_sys(ctx, sys);
-  return get_plan(ctx, sys, s, nb).windows.size() / 3;
+  return get_plan(ctx, sys, s, nb).wcount.size();
 }
 
 void atrip_amd::run_plan_windows(atrip_hip_ctx *ctx, int sys, int precision,
@@ -1482,20 +1499,22 @@ int atrip_hip_tuple_energies(atrip_hip_ctx *ctx, int sys, int precision,
       const HostIndex *h;
       uint64_t first, last, Nv;
       double *e, *ect;
-      void operator()(const int32_t *win, int nw, int nb,
+      void operator()(const int32_t *win, const BatchArgs &b,
                       const std::vector<double> &slots) {
-        const int64_t nb3 = (int64_t)nb * nb * nb;
-        for (int w = 0; w < nw; w++)
-          for (int64_t q = 0; q < nb3; q++) {
-            const uint64_t a = (uint64_t)win[3 * w] + q / (nb * nb);
-            const uint64_t b = (uint64_t)win[3 * w + 1] + (q / nb) % nb;
-            const uint64_t c = (uint64_t)win[3 * w + 2] + q % nb;
-            if (!tuple_ok(Nv, a, b, c)) continue;
-            const uint64_t idx = (*h)(a, b, c);
-            if (idx < first || idx >= last) continue;
-            e[idx - first] = slots[2 * (w * nb3 + q)];
-            if (ect) ect[idx - first] = slots[2 * (w * nb3 + q) + 1];
-          }
+        size_t q = 0;
+        for (int w = 0; w < b.nw; w++)
+          for (int ta = 0; ta < b.ea; ta++)
+            for (int tb = 0; tb < b.eb; tb++)
+              for (int tc = 0; tc < b.ec; tc++, q++) {
+                const uint64_t x = (uint64_t)win[3 * w] + ta,
+                               y = (uint64_t)win[3 * w + 1] + tb,
+                               z = (uint64_t)win[3 * w + 2] + tc;
+                if (!tuple_ok(Nv, x, y, z)) continue;
+                const uint64_t idx = (*h)(x, y, z);
+                if (idx < first || idx >= last) continue;
+                e[idx - first] = slots[2 * q];
+                if (ect) ect[idx - first] = slots[2 * q + 1];
+              }
       }
     } sink{&hidx, first, last, (uint64_t)s.Nv, e, e_ct};
     run_range(ctx, sys, precision, ijkabc, first, last, sink);
@@ -1512,6 +1531,7 @@ int atrip_hip_set_option(atrip_hip_ctx *ctx, const char *key, int64_t value) {
     } else if (k == "batch") {
       if (value < 1 || value > 4096) throw Fail{"batch must be in 1..4096"};
       ctx->batch = (int)value;
+      ctx->batch_set = true;
     } else if (k == "timing") {
       ctx->timing = value != 0;
     } else if (k == "tile") {

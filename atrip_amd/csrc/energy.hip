@@ -433,13 +433,13 @@ void energy_kernel(EnergyParams P) {
 // (w + v) + u, the order of wsum_kernel, so W is the same bits as in the
 // cube path; then the triple's points follow triple_points, and the
 // workgroup's energy (a fixed shuffle/LDS tree) goes to its own entry of
-// e_part.  triple_sum_kernel adds a tuple's triples in order.  Nothing
+// e_part.  slot_sum_kernel adds a tuple's triples in order.  Nothing
 // about W leaves the chip: no cube is written to memory and read back.
 struct FusedParams {
   const void *G, *GJ;  // class buffers [3][slots][No^2 rows][NoP] (FP64 or FP32)
   const double *Tai, *VHH, *ei, *ea;
   WindowArgs win;
-  double *e_part;  // [slot][triple][2]
+  double *e_part;  // [triple][slot][2]
   int64_t No, Nv, N2, NoP, W3g, slots, ntri;
   int nbk;
   double tai_sign;
@@ -629,7 +629,7 @@ __global__ __launch_bounds__(256) void energy_fused_kernel(FusedParams P) {
   const int tri = (int)(r - rq * ntri);
   if ((int64_t)gs >= P.slots) return;
   const int64_t gslot = gs;
-  const int64_t gid = gslot * P.ntri + tri;
+  const int64_t gid = tri * P.slots + gslot;
   const int64_t No = P.No, Nv = P.Nv;
   const int tid = threadIdx.x;
   int64_t a, b, c;
@@ -702,81 +702,81 @@ __global__ __launch_bounds__(256) void energy_fused_kernel(FusedParams P) {
                                     cubeJ, tA, tB, tC, sE, sV, red);
 }
 
-// Energy of each tuple slot: its triples' partials added in triple order.
-__global__ __launch_bounds__(256) void triple_sum_kernel(const double *e_part,
-                                                         int64_t slots,
-                                                         int64_t ntri,
-                                                         double *e_slot) {
-  const int64_t slot = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (slot >= slots) return;
-  const double *p = e_part + 2 * slot * ntri;
-  double e = 0.0, ect = 0.0;
-  for (int64_t t = 0; t < ntri; t++) {
-    e += p[2 * t];
-    ect += p[2 * t + 1];
-  }
-  e_slot[2 * slot] = e;
-  e_slot[2 * slot + 1] = ect;
+// Neumaier step on a (sum, compensation) pair.
+__device__ inline void nadd(double &s, double &c, double x) {
+  const double t = s + x;
+  c += (fabs(s) >= fabs(x)) ? (s - t) + x : (x - t) + s;
+  s = t;
 }
 
-// Per window of a batch, a compensated (Neumaier) sum of its slots' energies
-// in slot order: (sum, comp) to out[2 w], out[2 w + 1].
-__global__ __launch_bounds__(256) void window_sum_kernel(const double *e_slot,
-                                                         int nw, int64_t nb3,
-                                                         double *out) {
-  const int w = blockIdx.x * 256 + threadIdx.x;
-  if (w >= nw) return;
-  double sum = 0.0, comp = 0.0;
-  for (int64_t q = 0; q < nb3; q++) {
-    const double x = e_slot[2 * (w * nb3 + q)];
-    const double t = sum + x;
-    comp += (fabs(sum) >= fabs(x)) ? (sum - t) + x : (x - t) + sum;
-    sum = t;
-  }
-  out[2 * w] = sum;
-  out[2 * w + 1] = comp;
-}
-
-// Compensated sum of the slot energies of one batch: 256 threads each sum a
-// fixed strided subset (Neumaier), then a fixed pairwise tree of (sum, comp).
-__global__ __launch_bounds__(256) void batch_reduce_kernel(
-    const double *e_slot, int64_t slots, double *partials, int index) {
-  __shared__ double sh[4][256];
-  double s0 = 0.0, c0 = 0.0, s1 = 0.0, c1 = 0.0;
-  auto add = [](double &s, double &c, double x) {
-    const double t = s + x;
-    c += (fabs(s) >= fabs(x)) ? (s - t) + x : (x - t) + s;
-    s = t;
-  };
-  for (int64_t q = threadIdx.x; q < slots; q += 256) {
-    add(s0, c0, e_slot[2 * q]);
-    add(s1, c1, e_slot[2 * q + 1]);
-  }
-  sh[0][threadIdx.x] = s0;
-  sh[1][threadIdx.x] = c0;
-  sh[2][threadIdx.x] = s1;
-  sh[3][threadIdx.x] = c1;
+// Compensated sum of the workgroup's 256 (sum, compensation) pairs of e and
+// e_ct by a fixed pairwise tree; thread 0 writes out[0 .. 3].
+__device__ inline void pair_tree(double s0, double c0, double s1, double c1,
+                                 double (*sh)[256], double *out) {
+  const int tid = threadIdx.x;
+  sh[0][tid] = s0; sh[1][tid] = c0; sh[2][tid] = s1; sh[3][tid] = c1;
   __syncthreads();
   for (int h = 128; h > 0; h >>= 1) {
-    if ((int)threadIdx.x < h) {
-      double s = sh[0][threadIdx.x], c = sh[1][threadIdx.x] + sh[1][threadIdx.x + h];
-      add(s, c, sh[0][threadIdx.x + h]);
-      sh[0][threadIdx.x] = s;
-      sh[1][threadIdx.x] = c;
-      s = sh[2][threadIdx.x];
-      c = sh[3][threadIdx.x] + sh[3][threadIdx.x + h];
-      add(s, c, sh[2][threadIdx.x + h]);
-      sh[2][threadIdx.x] = s;
-      sh[3][threadIdx.x] = c;
+    if (tid < h) {
+      for (int k = 0; k < 4; k += 2) {
+        double s = sh[k][tid], c = sh[k + 1][tid] + sh[k + 1][tid + h];
+        nadd(s, c, sh[k][tid + h]);
+        sh[k][tid] = s;
+        sh[k + 1][tid] = c;
+      }
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    partials[4 * index + 0] = sh[0][0];
-    partials[4 * index + 1] = sh[1][0];
-    partials[4 * index + 2] = sh[2][0];
-    partials[4 * index + 3] = sh[3][0];
+  if (tid < 4) out[tid] = sh[tid][0];
+}
+
+// Energy of each tuple slot (with e_part: its triples' partials added in
+// triple order, read across the slots), and per 256 slots a compensated sum
+// of them to partials[4 * workgroup + {sum, comp, sum_ct, comp_ct}], which
+// the host adds in order.  (One workgroup summing a launch's slots by itself
+// was a chain of slots / 256 dependent loads: 4.7-8.6 us per launch of 2048
+// slots behind a 4.7 us kernel for the triples; both together now 5 us, and
+// longer launches cost no more per slot.)
+__global__ __launch_bounds__(256) void slot_sum_kernel(const double *e_part,
+                                                       int64_t slots,
+                                                       int64_t ntri,
+                                                       double *e_slot,
+                                                       double *partials) {
+  __shared__ double sh[4][256];
+  const int64_t slot = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  double e = 0.0, ect = 0.0;
+  if (slot < slots) {
+    if (e_part) {
+      for (int64_t t = 0; t < ntri; t++) {
+        const double *p = e_part + 2 * (t * slots + slot);
+        e += p[0];
+        ect += p[1];
+      }
+      e_slot[2 * slot] = e;
+      e_slot[2 * slot + 1] = ect;
+    } else {
+      e = e_slot[2 * slot];
+      ect = e_slot[2 * slot + 1];
+    }
   }
+  pair_tree(e, 0.0, ect, 0.0, sh, partials + 4 * (int64_t)blockIdx.x);
+}
+
+// Per window of a batch, a compensated sum of its `per` slot energies: each
+// thread over a fixed strided subset, then the fixed tree; (sum, comp) to
+// out[2 w], out[2 w + 1].  One workgroup per window (one thread per window
+// walked its slots alone: 42 us per launch, 17 % of a served step).
+__global__ __launch_bounds__(256) void window_sum_kernel(const double *e_slot,
+                                                         int64_t per,
+                                                         double *out) {
+  __shared__ double sh[4][256];
+  __shared__ double res[4];
+  const double *e = e_slot + 2 * blockIdx.x * per;
+  double sum = 0.0, comp = 0.0;
+  for (int64_t q = threadIdx.x; q < per; q += 256) nadd(sum, comp, e[2 * q]);
+  pair_tree(sum, comp, 0.0, 0.0, sh, res);
+  __syncthreads();
+  if (threadIdx.x < 2) out[2 * (int64_t)blockIdx.x + threadIdx.x] = res[threadIdx.x];
 }
 
 }  // namespace
@@ -840,11 +840,6 @@ hipError_t launch_energy(const DevSystem &s, const BatchArgs &b,
     else
       hipLaunchKernelGGL((energy_fused_kernel<double, false>), dim3((unsigned)grid),
                          dim3(256), 0, st, P);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(triple_sum_kernel, dim3((unsigned)((b.slots + 255) / 256)),
-                       dim3(256), 0, st, (const double *)scratch, b.slots, ntri,
-                       e_slot);
     return hipGetLastError();
   }
   const int64_t W3c = w_cube(s.No);
@@ -877,19 +872,19 @@ hipError_t launch_energy(const DevSystem &s, const BatchArgs &b,
   return hipGetLastError();
 }
 
-hipError_t launch_window_sums(const double *e_slot, int nw, int64_t nb3,
+hipError_t launch_window_sums(const double *e_slot, int nw, int64_t per,
                               double *out, hipStream_t st) {
   if (nw <= 0) return hipSuccess;
-  hipLaunchKernelGGL(window_sum_kernel, dim3((unsigned)((nw + 255) / 256)),
-                     dim3(256), 0, st, e_slot, nw, nb3, out);
+  hipLaunchKernelGGL(window_sum_kernel, dim3((unsigned)nw), dim3(256), 0, st,
+                     e_slot, per, out);
   return hipGetLastError();
 }
 
-hipError_t launch_batch_reduce(const DevSystem &, const BatchArgs &b,
-                               const double *e_slot, double *partials,
-                               int index, hipStream_t st) {
-  hipLaunchKernelGGL(batch_reduce_kernel, dim3(1), dim3(256), 0, st, e_slot,
-                     b.slots, partials, index);
+hipError_t launch_slot_sums(const double *e_part, int64_t slots, int64_t ntri,
+                            double *e_slot, double *partials, hipStream_t st) {
+  if (slots <= 0) return hipSuccess;
+  hipLaunchKernelGGL(slot_sum_kernel, dim3((unsigned)slot_partials(slots)),
+                     dim3(256), 0, st, e_part, slots, ntri, e_slot, partials);
   return hipGetLastError();
 }
 

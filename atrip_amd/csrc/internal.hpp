@@ -240,13 +240,12 @@ __device__ inline void sink_put8(const double (&v)[8], const OpSink &s,
   if (s.t) tri_put8(v, s.t, R, k8, g.K);
 }
 
-// Tuple windows: block triples (alpha <= beta <= gamma) of edge nb.
+// Tuple windows of a system: block triples (alpha <= beta <= gamma) of edge
+// nb in lexicographic order.
 struct WindowPlan {
   int nb = 0;
-  int nblk = 0;
-  std::vector<int32_t> windows;  // 3 per window, lexicographic
-  // per window: smallest and largest canonical index and number of tuples
-  std::vector<uint64_t> wmin, wmax, wcount;
+  std::vector<int32_t> origin;   // (a0, b0, c0) per window
+  std::vector<uint64_t> wcount;  // tuples per window
 };
 
 struct KernelStat {
@@ -276,6 +275,7 @@ struct atrip_hip_ctx {
   // options
   int window = 0;  // window edge; 0: automatic per system (auto_window)
   int batch = 4;
+  bool batch_set = false;  // the caller chose `batch`
   int timing = 0;
   int tile = -1;  // -1: chosen per system shape
   int operand_store = 0;  // store mode of the next uploads (DevSystem::store)
@@ -290,7 +290,7 @@ struct atrip_hip_ctx {
   size_t wcube_bytes = 0;
   double *e_slot = nullptr;  // per-slot energies (2 per slot: e, e_ct)
   size_t e_slot_bytes = 0;
-  double *partials = nullptr;  // per-batch (sum, comp) x 2
+  double *partials = nullptr;  // (sum, comp) x 2 per 256 slots of a run
   size_t partials_bytes = 0;
   void *sel = nullptr;  // a run's window list (and per-window sums)
   size_t sel_bytes = 0;
@@ -356,11 +356,12 @@ hipError_t launch_doubles_tri(const DevSystem &s, const BatchArgs &b,
 hipError_t launch_wsum(const DevSystem &s, const BatchArgs &b, const void *A,
                        const void *B, bool g32, double *out, hipStream_t st);
 
-// Class sums and singles + energy epilogue; writes e_slot[2*slot + {0,1}].
-// fused: one kernel gathers each block triple's W straight from the class
-// buffers (scratch: slots * n_triples * 2 doubles of per-triple partials);
-// otherwise the class-sum kernel writes W as cubes first (scratch: (GJ ? 2
-// : 1) * slots * w_cube(No) doubles).  Same W bits either way.
+// Class sums and singles + energy epilogue.  fused: one kernel gathers each
+// block triple's W straight from the class buffers and writes the triple's
+// energies to scratch ([triple][slot][2], slots * n_triples * 2 doubles),
+// which launch_slot_sums adds up; otherwise the class-sum kernel writes W as
+// cubes first (scratch: (GJ ? 2 : 1) * slots * w_cube(No) doubles) and
+// e_slot[2*slot + {0,1}] is written here.  Same W bits either way.
 hipError_t launch_energy(const DevSystem &s, const BatchArgs &b,
                          const void *G, const void *GJ, bool g32,
                          double tai_sign, double *e_slot, double *scratch,
@@ -380,16 +381,18 @@ hipError_t launch_energy_z(const DevSystem &s, const BatchArgs &b,
                            double tai_sign, double *e_slot, double *wcube,
                            hipStream_t st);
 
-// Per window of a batch (nw windows of nb3 slots), the Neumaier sum of its
-// slot energies in slot order: out[2 w] = sum, out[2 w + 1] = compensation.
-hipError_t launch_window_sums(const double *e_slot, int nw, int64_t nb3,
+// Per window of a batch (nw windows of `per` slots), a compensated sum of
+// its slot energies in a fixed order: out[2 w] = sum, out[2 w + 1] =
+// compensation.
+hipError_t launch_window_sums(const double *e_slot, int nw, int64_t per,
                               double *out, hipStream_t st);
 
-// Deterministic compensated sum of the valid slot energies of a batch into
-// partials[4*index + {sum, comp, sum_ct, comp_ct}].
-hipError_t launch_batch_reduce(const DevSystem &s, const BatchArgs &b,
-                               const double *e_slot, double *partials,
-                               int index, hipStream_t st);
+// Slot energies from the triples' partials (e_part null: e_slot holds them)
+// and their compensated sums, one quadruple {sum, comp, sum_ct, comp_ct} of
+// partials per 256 slots.
+hipError_t launch_slot_sums(const double *e_part, int64_t slots, int64_t ntri,
+                            double *e_slot, double *partials, hipStream_t st);
+inline int64_t slot_partials(int64_t slots) { return (slots + 255) / 256; }
 
 // Upload helpers.
 hipError_t launch_transpose(const double *src, double *dst, int64_t n_outer,
