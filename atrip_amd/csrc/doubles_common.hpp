@@ -76,26 +76,40 @@ struct TileWork {
   int slot0, slot_step;
 };
 
-// Work of this workgroup; false when its tile holds no column.  Units
-// (window, class, pair) go round the eight XCDs (workgroup b runs on XCD
-// b % 8) and a unit's tiles stay on one, so they share the pair's A rows and
-// columns in its L2, and the units that hold few columns (windows on the
-// diagonal, ends of a range) spread evenly: with one contiguous eighth of the
-// launch per XCD the XCDs that got the diagonal windows ran out of work.
+// Work of this workgroup; false when its tile holds no column.  Workgroup b
+// runs on XCD b % 8, and an XCD hands its workgroups to its shader engines in
+// turn, whatever they cost.  So
+//  - the units (class, pair) of a window go round the XCDs and a unit's tiles
+//    stay on one, where they share the pair's A rows and columns in its L2
+//    (one contiguous eighth of the launch per XCD left the XCDs without
+//    diagonal windows to work longer), and
+//  - each unit starts its tiles, and each window its units, one place further
+//    on, and the column tiles of a row of tiles are turned by a mix of the
+//    row's bits: with a fixed order the tiles at the GEMM's edges, or those
+//    without a valid column, came to the same shader engines in every unit
+//    (No=20, Nv=183 with 4x4 tiles, columns 128 + 32: half the chip idle,
+//    29.7 TFLOP/s against 50.7; No=38, Nv=204 with 3x3: 37.7 against 50.6).
+//    Column tiles stay next to each other (row tiles first costs 4x4 at No=40
+//    5 %: neighbours then share no A rows).
 __device__ __forceinline__ bool tile_work(const WindowArgs &W, uint64_t Nv,
                                           int No, int ntile_cols,
                                           TileWork &T) {
   const uint32_t bid = blockIdx.x, j = bid >> 3;
   const uint32_t tiles = (uint32_t)(W.mtiles * W.ntiles);
-  const uint32_t uq = j / tiles, tile = j - uq * tiles;
-  const uint32_t unit = 8 * uq + (bid & 7);
   const uint32_t units =
       (uint32_t)(W.ea * W.eb + W.ea * W.ec + W.eb * W.ec);
-  if (unit >= units * (uint32_t)W.nw) return false;
-  T.mt = (int)(tile / (uint32_t)W.ntiles);
-  T.nt = (int)(tile - (uint32_t)T.mt * (uint32_t)W.ntiles);
-  T.w = (int)(unit / units);
-  int u = (int)(unit - (uint32_t)T.w * units);
+  const uint32_t per = (units + 7) / 8 * tiles;  // of a window, per XCD
+  T.w = (int)(j / per);
+  uint32_t q = j - (uint32_t)T.w * per + (uint32_t)T.w % per;
+  if (q >= per) q -= per;
+  const uint32_t uq = q / tiles;
+  uint32_t tile = q - uq * tiles + uq % tiles;
+  if (tile >= tiles) tile -= tiles;
+  int u = (int)(8 * uq + (bid & 7));
+  if (u >= (int)units) return false;
+  const uint32_t mt = tile / (uint32_t)W.ntiles;
+  T.mt = (int)mt;
+  T.nt = (int)((tile + mt + (mt >> 1) + (mt >> 2)) % (uint32_t)W.ntiles);
   const int32_t a0 = W.windows[3 * T.w], b0 = W.windows[3 * T.w + 1],
                 c0 = W.windows[3 * T.w + 2];
   int edge;
@@ -136,12 +150,13 @@ __device__ __forceinline__ bool tile_work(const WindowArgs &W, uint64_t Nv,
   return T.nt * ntile_cols < T.ncols;
 }
 
-// Fragments of `width` that wave w of two holds of `left` rows or columns,
-// fragments taken in turn (w, w + 2, ...), at most f.
-__device__ __forceinline__ int occupied(int64_t left, int w, int width, int f) {
-  const int64_t frags = (left + width - 1) / width;  // of both waves
-  const int mine = (int)((frags - w + 1) / 2);
-  return mine < 0 ? 0 : mine < f ? mine : f;
+// Fragments of `width` that wave w of nw holds of `left` rows or columns of a
+// tile of at most `most` fragments, taken in turn (w, w + nw, ...).
+__device__ __forceinline__ int occupied(int64_t left, int w, int nw, int width,
+                                        int most) {
+  const int64_t all = (left + width - 1) / width;
+  const int frags = all < most ? (int)all : most;
+  return frags > w ? (frags - w + nw - 1) / nw : 0;
 }
 
 // Row of segment sg's B operand at column (y, rr) of class cl with A-pair
@@ -163,9 +178,8 @@ inline int64_t doubles_grid(WindowArgs &W, int64_t No, int64_t mt_rows,
   const int64_t emax = std::max(W.ea, std::max(W.eb, W.ec));
   W.mtiles = (int)((No * No + mt_rows - 1) / mt_rows);
   W.ntiles = (int)((emax * No + nt_cols - 1) / nt_cols);
-  const int64_t units =
-      (int64_t)W.nw * (W.ea * W.eb + W.ea * W.ec + W.eb * W.ec);
-  return (units + 7) / 8 * 8 * W.mtiles * W.ntiles;
+  const int64_t units = W.ea * W.eb + W.ea * W.ec + W.eb * W.ec;
+  return (units + 7) / 8 * 8 * W.nw * W.mtiles * W.ntiles;
 }
 
 // W position (i,j,k) of GEMM element (row (p,q), column index rr).

@@ -45,10 +45,17 @@ struct DoublesParams {
   int64_t No, Nv, Kv, Ko, N2, N2p, W3, NoP, slots;
 };
 
+// Operand sets of a wave of FM x FN fragments: two, four where a chunk is
+// shorter than 1000 cycles (2x2 at No=40: 52.1 -> 55.4 TFLOP/s; deeper sets
+// from 4x2 on cost more registers than they hide: 59.7 -> 57.0 at No=16).
+constexpr int depth(int FM, int FN) {
+  return FM * FN >= 8 ? 2 : 4;
+}
+
 // The FM x FN occupied fragments of one wave of a tile of 32 TM x 32 TN.  The
 // two waves of each direction take the tile's fragments in turn, so a tile at
 // the edge of the GEMM leaves both about the same number.
-template <int TM, int TN, int FM, int FN>
+template <int TM, int TN, int WR, int FM, int FN>
 __device__ __forceinline__ void f64_wave(const DoublesParams &P,
                                          const TileWork &T, int No, int lane,
                                          int wm, int wn) {
@@ -68,7 +75,7 @@ __device__ __forceinline__ void f64_wave(const DoublesParams &P,
   int32_t rowS[FM], rowW[FM];
 #pragma unroll
   for (int f = 0; f < FM; f++) {
-    int m = T.mt * MT + (2 * f + wm) * 16 + l16;
+    int m = T.mt * MT + (WR * f + wm) * 16 + l16;
     rowS[f] = m < N2p ? m : (int)N2p - 16 + l16;
     if (m >= N2) m = (int)N2 - 1;
     rowW[f] = m / No + No * (m % No);
@@ -101,29 +108,33 @@ __device__ __forceinline__ void f64_wave(const DoublesParams &P,
 #pragma unroll
     for (int g = 0; g < FN; g++) acc[f][g] = d4{0.0, 0.0, 0.0, 0.0};
 
-  // Software pipeline: two operand sets in ping-pong, so the loads of one
-  // chunk are in flight while the MFMAs of the other run (no register
-  // copies between the sets, hence no wait on the in-flight loads).
+  // Software pipeline of D operand sets used in turn: the loads of D - 1
+  // chunks are in flight behind the MFMAs of one (no register copies between
+  // the sets, hence no wait on the in-flight loads).  A chunk is 128 FM FN
+  // cycles of MFMA against a load latency of 1000 (L2) to 2500 cycles, so
+  // small fragments need more sets: see depth().
+  constexpr int D = depth(FM, FN);
   const double *ap[FM], *bp[FN];
-#define LOAD(AV, BV, C)                                                 \
-  {                                                                     \
-    _Pragma("unroll") for (int f = 0; f < FM; f++) AV[f] =              \
-        *(const d2 *)(ap[f] + TILE * (C));                              \
-    _Pragma("unroll") for (int g = 0; g < FN; g++) BV[g] =              \
-        *(const d2 *)(bp[g] + TILE * (C));                              \
-    __builtin_amdgcn_sched_barrier(0);                                  \
+  d2 a[D][FM], b[D][FN];
+#define LOAD(J)                                                             \
+  {                                                                         \
+    const int64_t at_ = TILE * (int64_t)(sg < 4 ? c : nch - 1);             \
+    _Pragma("unroll") for (int f = 0; f < FM; f++) a[J][f] =                \
+        *(const d2 *)(ap[f] + at_);                                         \
+    _Pragma("unroll") for (int g = 0; g < FN; g++) b[J][g] =                \
+        *(const d2 *)(bp[g] + at_);                                         \
+    __builtin_amdgcn_sched_barrier(0);                                      \
   }
-#define COMPUTE(AV, BV)                                                 \
-  _Pragma("unroll") for (int s = 0; s < 2; s++)                         \
-      _Pragma("unroll") for (int f = 0; f < FM; f++)                    \
-          _Pragma("unroll") for (int g = 0; g < FN; g++) acc[f][g] =    \
-              __builtin_amdgcn_mfma_f64_16x16x4f64(AV[f][s], BV[g][s],  \
+#define COMPUTE(J)                                                          \
+  _Pragma("unroll") for (int s = 0; s < 2; s++)                             \
+      _Pragma("unroll") for (int f = 0; f < FM; f++)                        \
+          _Pragma("unroll") for (int g = 0; g < FN; g++) acc[f][g] =        \
+              __builtin_amdgcn_mfma_f64_16x16x4f64(a[J][f][s], b[J][g][s],  \
                                                    acc[f][g], 0, 0, 0);
-  d2 a0[FM], b0[FN], a1[FM], b1[FN];
   // One pipeline through the four segments: (sg, c) is the next chunk to
   // load, and past a segment's end the pointers move to the next segment's
   // chunk 0 in place, so every segment but the first starts with its first
-  // chunk in flight (3 % faster at No=40 than a pipeline restarted per
+  // chunks in flight (3 % faster at No=40 than a pipeline restarted per
   // segment).  A segment ends at the last chunk that holds an occupied
   // kappa.  The prefetch is issued unconditionally (after the last chunk it
   // re-reads it, a load never used) so every path into a COMPUTE has the
@@ -132,30 +143,33 @@ __device__ __forceinline__ void f64_wave(const DoublesParams &P,
   int nch = (int)((Nv + KC - 1) / KC), c = 0;
   SET_PTRS(0);
 #define ADVANCE()                                                            \
-  {                                                                          \
-    if (++c == nch && ++sg < 4) {                                            \
-      SET_PTRS(sg);                                                          \
-      nch = (int)(((sg < 2 ? Nv : No) + KC - 1) / KC);                     \
-      c = 0;                                                                 \
-    }                                                                        \
+  if (sg < 4 && ++c == nch && ++sg < 4) {                                    \
+    SET_PTRS(sg);                                                            \
+    nch = (int)(((sg < 2 ? Nv : No) + KC - 1) / KC);                         \
+    c = 0;                                                                   \
   }
-#define NEXT() ((int64_t)(sg < 4 ? c : nch - 1))
-  LOAD(a0, b0, 0);
-  ADVANCE();
-  // (each segment length occurs twice, so the number of chunks is even; a
-  // second exit in the middle of the loop made the compiler copy the
-  // accumulators between register files on every turn)
-#pragma unroll 1
-  for (int left = 2 * (int)((Nv + KC - 1) / KC + (No + KC - 1) / KC); left; left -= 2) {
-    LOAD(a1, b1, NEXT());
+#pragma unroll
+  for (int j = 0; j < D - 1; j++) {
+    LOAD(j);
     ADVANCE();
-    COMPUTE(a0, b0);
-    LOAD(a0, b0, NEXT());
-    if (sg < 4) ADVANCE();
-    COMPUTE(a1, b1);
   }
+  // (one exit: leaving the loop between two sets made the compiler copy the
+  // accumulators between register files on every turn; the chunks of a last
+  // part turn follow it)
+  int left = 2 * (int)((Nv + KC - 1) / KC + (No + KC - 1) / KC);
+#pragma unroll 1
+  for (; left >= D; left -= D) {
+#pragma unroll
+    for (int j = 0; j < D; j++) {
+      LOAD((j + D - 1) % D);
+      ADVANCE();
+      COMPUTE(j);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < D - 1; j++)
+    if (j < left) COMPUTE(j);
 #undef ADVANCE
-#undef NEXT
 #undef LOAD
 #undef COMPUTE
 
@@ -174,7 +188,7 @@ __device__ __forceinline__ void f64_wave(const DoublesParams &P,
     for (int f = 0; f < FM; f++) {
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const int64_t m = T.mt * MT + (2 * f + wm) * 16 + 4 * r + kk;
+        const int64_t m = T.mt * MT + (WR * f + wm) * 16 + 4 * r + kk;
         if (m < N2) Gs[m * P.NoP] = acc[f][g][r];  // contiguous along n
       }
     }
@@ -182,41 +196,49 @@ __device__ __forceinline__ void f64_wave(const DoublesParams &P,
 }
 
 // Dispatch on the wave's occupied column fragments, n <= FN of them.
-template <int TM, int TN, int FM, int FN>
+template <int TM, int TN, int WR, int FM, int FN>
 __device__ __forceinline__ void f64_columns(const DoublesParams &P,
                                             const TileWork &T, int No,
                                             int lane, int wm, int wn, int n) {
   if constexpr (FN > 1) {
     if (n < FN) {
-      f64_columns<TM, TN, FM, FN - 1>(P, T, No, lane, wm, wn, n);
+      f64_columns<TM, TN, WR, FM, FN - 1>(P, T, No, lane, wm, wn, n);
       return;
     }
   }
-  f64_wave<TM, TN, FM, FN>(P, T, No, lane, wm, wn);
+  f64_wave<TM, TN, WR, FM, FN>(P, T, No, lane, wm, wn);
 }
 
-template <int FM, int FN>
-__global__ __launch_bounds__(256, FM *FN <= 16 ? 2 : 1) void doubles_f64_kernel(
+template <int FM, int FN, int WR>
+__global__ __launch_bounds__(128 * WR, 2) void doubles_f64_kernel(
     DoublesParams P) {
   const int No = (int)P.No;
   TileWork T;
   if (!tile_work(P.win, (uint64_t)P.Nv, No, 32 * FN, T)) return;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wm = wave >> 1, wn = wave & 1;
+  // wave -> (row, column) of the WR x 2 waves.  The tiles beyond 4x4 run
+  // eight waves (four rows), two per SIMD, instead of four of twice the
+  // registers: the second wave covers the other's loads (5x5 at No=40,
+  // Nv=400 61.4 -> 66.3 TFLOP/s with the valid columns, 4x5 at No=26 44.7 ->
+  // 50.7, 5x4 at No=31 48.5 -> 50.7).  The two waves of a SIMD (w, w + 4) are
+  // two rows apart, so that they hold five of ten row fragments between them.
+  const int wn = WR == 2 ? wave & 1 : wave >> 2;
+  const int wm = WR == 2 ? wave >> 1 : (wave + 2 * wn) & 3;
   // Fragments of this wave that hold rows and columns.  Tiles at the edges
   // of the GEMM run the instance of their size instead of the whole tile on
   // padding: every column count, the row count rounded up to half the tile
   // (rows have one edge per A-pair, columns one per pair and valid third
   // index; one instance with per-fragment branches doubled the accumulators).
-  const int m = occupied(P.N2 - (int64_t)T.mt * 32 * FM, wm, 16, FM);
-  const int n = occupied(T.ncols - (int64_t)T.nt * 32 * FN, wn, 16, FN);
+  constexpr int RF = (2 * FM + WR - 1) / WR;  // row fragments of a wave
+  const int m = occupied(P.N2 - (int64_t)T.mt * 32 * FM, wm, WR, 16, 2 * FM);
+  const int n = occupied(T.ncols - (int64_t)T.nt * 32 * FN, wn, 2, 16, 2 * FN);
   if (!m || !n) return;
-  constexpr int H = (FM + 1) / 2;
+  constexpr int H = (RF + 1) / 2;
   if (m > H)
-    f64_columns<FM, FN, FM, FN>(P, T, No, lane, wm, wn, n);
+    f64_columns<FM, FN, WR, RF, FN>(P, T, No, lane, wm, wn, n);
   else
-    f64_columns<FM, FN, H, FN>(P, T, No, lane, wm, wn, n);
+    f64_columns<FM, FN, WR, H, FN>(P, T, No, lane, wm, wn, n);
 }
 
 }  // namespace
@@ -248,12 +270,12 @@ hipError_t launch_doubles_f64(const DevSystem &s, const BatchArgs &b,
   const int64_t grid = doubles_grid(P.win, s.No, 32 * FM, 32 * FN);
   if (grid <= 0) return hipSuccess;
   if (grid > MAX_GRID) return hipErrorInvalidConfiguration;
-#define LAUNCH(A, B)                                                       \
-  if (FM == A && FN == B)                                                  \
-    hipLaunchKernelGGL((doubles_f64_kernel<A, B>), dim3((unsigned)grid),   \
-                       dim3(256), 0, st, P);
-  LAUNCH(2, 2) LAUNCH(4, 2) LAUNCH(2, 4) LAUNCH(4, 4) LAUNCH(3, 3)
-  LAUNCH(5, 5) LAUNCH(4, 5) LAUNCH(5, 4)
+#define LAUNCH(A, B, WR)                                                     \
+  if (FM == A && FN == B)                                                    \
+    hipLaunchKernelGGL((doubles_f64_kernel<A, B, WR>), dim3((unsigned)grid), \
+                       dim3(128 * WR), 0, st, P);
+  LAUNCH(2, 2, 2) LAUNCH(4, 2, 2) LAUNCH(2, 4, 2) LAUNCH(4, 4, 2)
+  LAUNCH(3, 3, 2) LAUNCH(5, 5, 4) LAUNCH(4, 5, 4) LAUNCH(5, 4, 4)
 #undef LAUNCH
   return hipGetLastError();
 }

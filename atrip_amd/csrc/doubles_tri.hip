@@ -216,8 +216,8 @@ __global__ __launch_bounds__(256) void doubles_tri_kernel(TriParams P) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave >> 1, wn = wave & 1;
   // edge tiles run the instance of their occupied fragments (FP64 kernel)
-  const int m = occupied(P.N2 - (int64_t)T.mt * 64 * FM, wm, 32, FM);
-  const int n = occupied(T.ncols - (int64_t)T.nt * 64 * FN, wn, 32, FN);
+  const int m = occupied(P.N2 - (int64_t)T.mt * 64 * FM, wm, 2, 32, 2 * FM);
+  const int n = occupied(T.ncols - (int64_t)T.nt * 64 * FN, wn, 2, 32, 2 * FN);
   if (!m || !n) return;
   constexpr int H = (FM + 1) / 2;
   if (m > H)
