@@ -747,6 +747,10 @@ struct HostIndex {
   uint64_t operator()(uint64_t a, uint64_t b, uint64_t c) const {
     return tuple_index(pre.data(), Nv, a, b, c);
   }
+  // First index of tuple q.
+  int64_t first_of(uint64_t q) const {
+    return std::upper_bound(pre.begin(), pre.end(), q) - pre.begin() - 1;
+  }
 };
 
 // Windows of a run: origins (a0, b0, c0), tuples each holds, edges.
@@ -896,10 +900,17 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
       win.count.push_back(plan.wcount[w]);
     }
   } else {
+    // A range holds few first indices (1 % of No=40, Nv=400 about two), so it
+    // takes windows of its own: the first index of the range's tuples cut
+    // evenly into blocks of at most the edge.  Blocks aligned as the plan's
+    // left the window columns of the other first indices empty.
     const HostIndex h((uint64_t)s.Nv);
-    for (int64_t a = 0; a < s.Nv; a += nb)
-      for (int64_t b = a; b < s.Nv; b += nb)
-        for (int64_t c = b; c < s.Nv; c += nb) win.add(h, first, last, a, b, c);
+    const int64_t a0 = h.first_of(first), a1 = h.first_of(last - 1);
+    const int64_t na = a1 - a0 + 1, blocks = (na + nb - 1) / nb;
+    win.ea = (int)((na + blocks - 1) / blocks);
+    for (int64_t a = a0; a <= a1; a += win.ea)
+      for (int64_t b = a0 + (a - a0) / win.eb * win.eb; b < s.Nv; b += win.eb)
+        for (int64_t c = b; c < s.Nv; c += win.ec) win.add(h, first, last, a, b, c);
   }
   const std::vector<int32_t> &sel = win.origin;
   for (uint64_t c : win.count) res.tuples += c;
@@ -943,7 +954,10 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
            a256(z.windows);
   };
 
-  int bw = std::max(1, ctx->batch);
+  // (a window of a range counts by its slots)
+  int bw = (int)std::min<int64_t>(
+      4096, std::max<int64_t>(1, ctx->batch * (int64_t)nb * nb * nb / per));
+  const int bw_least = bw;
   if (!ctx->batch_set)
     bw = std::max(bw, auto_batch((use_j ? 2 : 1) * nsets * 3 * W3 *
                                      (int64_t)gelem, per));
@@ -1011,9 +1025,9 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
         break;
       } catch (const Fail &) {
         // a device with little memory left: launches of the option's size
-        if (bw <= std::max(1, ctx->batch)) throw;
+        if (bw <= bw_least) throw;
         (void)hipGetLastError();
-        bw = std::max(1, ctx->batch);
+        bw = bw_least;
         z = sizes(bw);
       }
     }
