@@ -923,7 +923,7 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
   // on demand), or carved out of a fixed region without any allocation
   // (then the windows per launch shrink until the run fits).
   const int64_t per = (int64_t)win.ea * win.eb * win.ec;  // slots of a window
-  const int64_t W3 = g_elems(s.No, g32);  // one tuple's class buffer
+  const int64_t W3 = g_elems(s.No);  // one tuple's class buffer
   const bool use_j = s.has_j;
   const int nsets = s.cplx ? 4 : 1;
   const size_t gelem = g32 ? sizeof(float) : sizeof(double);

@@ -42,7 +42,8 @@ struct DoublesParams {
   const double *T3, *T3s, *V3, *H3, *H3s, *T2N, *T2TN;
   WindowArgs win;
   double *G;
-  int64_t No, Nv, Kv, Ko, N2, N2p, W3, NoP, slots;
+  int64_t No, Nv, Kv, Ko, N2, N2p, W3, slots;
+  GLayout lay;
 };
 
 // Operand sets of a wave of FM x FN fragments: two, four where a chunk is
@@ -178,21 +179,26 @@ __device__ __forceinline__ void f64_wave(const DoublesParams &P,
   // register i/4 (measured on gfx950)
   const int64_t per = (int64_t)P.win.ea * P.win.eb * P.win.ec;
   double *Gc = P.G + (T.cl * P.slots + T.w * per) * P.W3;
+  double *Gs[FN];  // column bases; null past the last column
 #pragma unroll
   for (int g = 0; g < FN; g++) {
     const int n = T.nt * NT + (2 * g + wn) * 16 + l16;
-    if (n >= T.ncols) continue;
     const int t = n / No;
-    double *Gs = Gc + (int64_t)(T.slot0 + t * T.slot_step) * P.W3 + (n - t * No);
-#pragma unroll
-    for (int f = 0; f < FM; f++) {
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int64_t m = T.mt * MT + (WR * f + wm) * 16 + 4 * r + kk;
-        if (m < N2) Gs[m * P.NoP] = acc[f][g][r];  // contiguous along n
-      }
-    }
+    Gs[g] = n < T.ncols ? Gc + (int64_t)(T.slot0 + t * T.slot_step) * P.W3 +
+                              g_col(n - t * No)
+                        : nullptr;
   }
+#pragma unroll
+  for (int f = 0; f < FM; f++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int m = T.mt * MT + (WR * f + wm) * 16 + 4 * r + kk;
+      if (m >= N2) continue;
+      const uint32_t o = g_row(P.lay, m);
+#pragma unroll
+      for (int g = 0; g < FN; g++)
+        if (Gs[g]) Gs[g][o] = acc[f][g][r];
+    }
 }
 
 // Dispatch on the wave's occupied column fragments, n <= FN of them.
@@ -262,8 +268,8 @@ hipError_t launch_doubles_f64(const DevSystem &s, const BatchArgs &b,
   P.Ko = s.Ko;
   P.N2 = s.No * s.No;
   P.N2p = pad16(P.N2);
-  P.NoP = g_pitch(s.No, false);
-  P.W3 = g_elems(s.No, false);
+  P.lay = g_layout(s.No);
+  P.W3 = g_elems(s.No);
   P.slots = b.slots;
   tile = pick_tile(tile, s.No, std::max(b.ea, std::max(b.eb, b.ec)));
   const int FM = tile_fm(tile), FN = tile_fn(tile);

@@ -38,7 +38,8 @@ struct SplitParams {
   const __bf16 *T3l, *H3l, *V3l, *T2Nl, *T2TNl;
   WindowArgs win;
   float *G;
-  int64_t No, Nv, Kv, Ko, N2, W3, NoP, slots;
+  int64_t No, Nv, Kv, Ko, N2, W3, slots;
+  GLayout lay;
 };
 
 // The FM x FN occupied fragments of one wave of a tile of 64 TM x 64 TN (the
@@ -182,22 +183,26 @@ __device__ __forceinline__ void split_wave(const SplitParams &P, const TileWork 
   // 4 (i / 8) + i % 4
   const int64_t per = (int64_t)P.win.ea * P.win.eb * P.win.ec;
   float *Gc = P.G + (T.cl * P.slots + T.w * per) * P.W3;
+  float *Gs[FN];  // column bases; null past the last column
 #pragma unroll
   for (int g = 0; g < FN; g++) {
     const int n = T.nt * NT + (2 * g + wn) * 32 + l32;
-    if (n >= T.ncols) continue;
     const int t = n / No;
-    float *Gs = Gc + (int64_t)(T.slot0 + t * T.slot_step) * P.W3 + (n - t * No);
-#pragma unroll
-    for (int f = 0; f < FM; f++) {
-#pragma unroll
-      for (int r = 0; r < 16; r++) {
-        const int64_t m = T.mt * MT + (2 * f + wm) * 32 + 8 * (r >> 2) + 4 * kh +
-                          (r & 3);
-        if (m < N2) Gs[m * P.NoP] = acc[f][g][r];  // contiguous along n
-      }
-    }
+    Gs[g] = n < T.ncols ? Gc + (int64_t)(T.slot0 + t * T.slot_step) * P.W3 +
+                              g_col(n - t * No)
+                        : nullptr;
   }
+#pragma unroll
+  for (int f = 0; f < FM; f++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const int m = T.mt * MT + (2 * f + wm) * 32 + 8 * (r >> 2) + 4 * kh + (r & 3);
+      if (m >= N2) continue;
+      const uint32_t o = g_row(P.lay, m);
+#pragma unroll
+      for (int g = 0; g < FN; g++)
+        if (Gs[g]) Gs[g][o] = acc[f][g][r];
+    }
 }
 
 // Dispatch on the wave's occupied column fragments, n <= FN of them.
@@ -253,8 +258,8 @@ hipError_t launch_doubles_split(const DevSystem &s, const BatchArgs &b,
   P.Kv = s.Kv;
   P.Ko = s.Ko;
   P.N2 = s.No * s.No;
-  P.NoP = g_pitch(s.No, true);
-  P.W3 = g_elems(s.No, true);
+  P.lay = g_layout(s.No);
+  P.W3 = g_elems(s.No);
   P.slots = b.slots;
   tile = pick_t32_tile(tile, s.No, std::max(b.ea, std::max(b.eb, b.ec)));
   const int FM = t32_fm(tile), FN = t32_fn(tile);

@@ -38,89 +38,89 @@ __device__ inline double wave_sum(double v) {
   return v;
 }
 
-// Class sums of one 16x16x16 brick of W for every slot of the batch:
-// out = sum(A) [+ sum(B)], sum(X) = (Xw + Xv) + Xu, written as cubes.
+// Thread's pair of elements e = 2 tid, 2 tid + 1 of an 8^3 block in class
+// order: class cls of W block (bx, by, bz); the pair runs along the class's
+// own fastest index.  `at` is its offset in the slot's class buffer, pos the
+// place of its first element in an LDS block x + CY y + CZ z and step that of
+// the second after it, in0, in1 whether the elements exist (No: W edge).
+struct PairAt {
+  uint32_t at;
+  int pos, step;
+  bool in0, in1;
+};
+// (FULL: every block the caller reads lies inside the occupied range.)
+template <int CY, int CZ, bool FULL>
+__device__ __forceinline__ PairAt pair_at(int cls, int bx, int by, int bz,
+                                          int nbk, int no, int tid) {
+  const int e = 2 * tid, r = e & 7, p = (e >> 3) & 7, q = e >> 6;
+  // (p, q, r) in W indices: w (x,y,z), v (x,z,y), u (y,z,x)
+  const int bp = cls == 2 ? by : bx, bq = cls == 0 ? by : bz,
+            br = cls == 0 ? bz : cls == 1 ? by : bx;
+  const int x = cls == 2 ? r : p, y = cls == 0 ? q : cls == 1 ? r : p,
+            z = cls == 0 ? r : q;
+  PairAt a;
+  const bool in = FULL || ((8 * bp + p < no) & (8 * bq + q < no));
+  a.in0 = FULL || (in & (8 * br + r < no));
+  a.in1 = FULL || (in & (8 * br + r + 1 < no));
+  const uint32_t blk = (uint32_t)((bq * nbk + bp) * nbk + br) << 9;
+  a.at = blk + (a.in0 ? (uint32_t)e : 0u);  // always inside the buffer
+  a.pos = x + CY * y + CZ * z;
+  a.step = cls == 0 ? CZ : cls == 1 ? CY : 1;
+  return a;
+}
+
+// Class sums of one 8^3 block of W for every slot of the batch: out = sum(A)
+// [+ sum(B)], sum(X) = (Xw + Xv) + Xu, written as cubes.
 template <typename GT>
 __global__ __launch_bounds__(256) void wsum_kernel(const GT *A, const GT *B,
-                                                   double *out, int64_t No,
-                                                   int64_t NoP, int64_t W3g,
-                                                   int64_t slots, int nbk,
-                                                   int nbr) {
-  // LDS brick [z][y][x] with pitch 17 (conflict-free transposed writes)
-  __shared__ double br[16 * 17 * 17];
-  const int64_t bid = blockIdx.x;
-  const int64_t slot = bid / ((int64_t)nbr * nbr * nbr);
-  const int brick = (int)(bid % ((int64_t)nbr * nbr * nbr));
-  const int bx = brick % nbr, by = (brick / nbr) % nbr, bz = brick / (nbr * nbr);
-  const int tid = threadIdx.x, no = (int)No;
-  const int x0 = 16 * bx, y0 = 16 * by, z0 = 16 * bz;
-  auto at = [](int x, int y, int z) { return x + 17 * (y + 17 * z); };
-  double *o = out + slot * (int64_t)(512 * nbk * nbk * nbk);
+                                                   double *out, int no,
+                                                   int64_t W3g, int64_t slots,
+                                                   int nbk) {
+  typedef GT g2 __attribute__((ext_vector_type(2)));
+  constexpr int CZ = 69;
+  __shared__ double br[7 * CZ + 64];
+  const uint32_t n3 = (uint32_t)(nbk * nbk * nbk), bid = blockIdx.x;
+  const int64_t slot = bid / n3;
+  const int blk = (int)(bid - (uint32_t)slot * n3);
+  const int bx = blk % nbk, by = (blk / nbk) % nbk, bz = blk / (nbk * nbk);
+  const int tid = threadIdx.x;
+  double sum[2] = {0.0, 0.0};
   for (int set = 0; set < (B ? 2 : 1); set++) {
     const GT *S = set == 0 ? A : B;
-    const GT *Sw = S + slot * W3g, *Sv = S + (slots + slot) * W3g,
-             *Su = S + (2 * slots + slot) * W3g;
-    GT v[16], t[16];  // widened to FP64 only when added into the brick
-    // class w: (x + No y) No + z, z fastest
+    PairAt a[3];
+    g2 v[3];
 #pragma unroll
-    for (int it = 0; it < 16; it++) {
-      const int e = tid + 256 * it;
-      const int z = z0 + (e & 15), y = y0 + ((e >> 4) & 15), x = x0 + (e >> 8);
-      const bool in = x < no && y < no && z < no;
-      v[it] = Sw[in ? (x + no * y) * NoP + z : 0];  // always a valid address
-      if (!in) v[it] = (GT)0;
+    for (int cls = 0; cls < 3; cls++) {
+      a[cls] = pair_at<8, CZ, false>(cls, bx, by, bz, nbk, no, tid);
+      v[cls] = *(const g2 *)(S + (cls * slots + slot) * W3g + a[cls].at);
     }
-    // class v: (x + No z) No + y, y fastest
 #pragma unroll
-    for (int it = 0; it < 16; it++) {
-      const int e = tid + 256 * it;
-      const int y = y0 + (e & 15), x = x0 + ((e >> 4) & 15), z = z0 + (e >> 8);
-      const bool in = x < no && y < no && z < no;
-      t[it] = Sv[in ? (x + no * z) * NoP + y : 0];
-      if (!in) t[it] = (GT)0;
+    for (int cls = 0; cls < 3; cls++) {
+      const double v0 = a[cls].in0 ? (double)v[cls][0] : 0.0,
+                   v1 = a[cls].in1 ? (double)v[cls][1] : 0.0;
+      double *b0 = br + a[cls].pos, *b1 = b0 + a[cls].step;
+      if (cls == 0) {
+        *b0 = v0;
+        *b1 = v1;
+      } else {
+        *b0 += v0;
+        *b1 += v1;
+      }
+      __syncthreads();
     }
-    __syncthreads();  // the previous set's cube writes are done with br
+    // the two elements of the cube this thread writes
 #pragma unroll
-    for (int it = 0; it < 16; it++) {
-      const int e = tid + 256 * it;
-      br[at(e >> 8, (e >> 4) & 15, e & 15)] = (double)v[it];
-    }
-    // class u: (y + No z) No + x, x fastest
-#pragma unroll
-    for (int it = 0; it < 16; it++) {
-      const int e = tid + 256 * it;
-      const int x = x0 + (e & 15), y = y0 + ((e >> 4) & 15), z = z0 + (e >> 8);
-      const bool in = x < no && y < no && z < no;
-      v[it] = Su[in ? (y + no * z) * NoP + x : 0];
-      if (!in) v[it] = (GT)0;
+    for (int h = 0; h < 2; h++) {
+      const int e = tid + 256 * h;
+      sum[h] = set == 0 ? br[(e & 63) + CZ * (e >> 6)]
+                        : sum[h] + br[(e & 63) + CZ * (e >> 6)];
     }
     __syncthreads();
-#pragma unroll
-    for (int it = 0; it < 16; it++) {
-      const int e = tid + 256 * it;
-      br[at((e >> 4) & 15, e & 15, e >> 8)] += (double)t[it];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int it = 0; it < 16; it++) {
-      const int e = tid + 256 * it;
-      br[at(e & 15, (e >> 4) & 15, e >> 8)] += (double)v[it];
-    }
-    __syncthreads();
-    // the brick's cubes, 512 contiguous doubles each; the second set adds
-    // to what the same thread wrote for the first
-#pragma unroll
-    for (int it = 0; it < 16; it++) {
-      const int e = tid + 256 * it;
-      const int cube = e >> 9, q = e & 511;
-      const int cx = cube & 1, cy = (cube >> 1) & 1, cz = cube >> 2;
-      const int gx = 2 * bx + cx, gy = 2 * by + cy, gz = 2 * bz + cz;
-      if (gx >= nbk || gy >= nbk || gz >= nbk) continue;
-      const double val = br[at(8 * cx + (q & 7), 8 * cy + ((q >> 3) & 7), 8 * cz + (q >> 6))];
-      double *dst = o + ((int64_t)((gz * nbk + gy) * nbk + gx) << 9) + q;
-      *dst = set == 0 ? val : *dst + val;
-    }
   }
+  double *o = out + slot * (int64_t)(512 * n3) +
+              ((int64_t)((bz * nbk + by) * nbk + bx) << 9);
+  o[tid] = sum[0];
+  o[tid + 256] = sum[1];
 }
 
 // Energy of one tuple per workgroup.  The i>=j>=k points are visited per
@@ -156,7 +156,7 @@ __device__ __forceinline__ void orbit(int B1, int B2, int B3, int nbk,
 // Energy terms of the i>=j>=k points of block triple (B1, B2, B3) (edge 8)
 // of one tuple, two points per thread, added to e_acc (and, with the (cT)
 // W, to ect_acc).  The six permuted W cubes of the triple's orbit sit in
-// LDS (cube[alias[p]] holds W at permutation p, element x + 8 y + CZ z), as
+// LDS (cube[alias[p]] holds W at permutation p, element x + CY y + CZ z), as
 // do the singles tables tA/tB/tC (Tai at (a,x), (b,x), (c,x), slot 8 * position
 // + local index), the eps_i table sE and the V^bc, V^ac, V^ab 8x8 block pairs
 // sV.  Z = W + singles (reference src/atrip/Equations.cxx:387-426) and the
@@ -164,16 +164,20 @@ __device__ __forceinline__ void orbit(int B1, int B2, int B3, int nbk,
 // reference's expression order.
 // sV holds the 8x8 V blocks of the triple, [slice][block pair][ly + 8 lz]:
 // all nine ordered position pairs (V6 false) or only the six with two
-// different positions (V6 true), the only ones a point reads.
-template <bool HJ, int CZ, int CSZ, bool V6>
+// different positions (V6 true), the only ones a point reads, then with
+// rows 9 apart (a point reads V at (j, i) and (k, i) too, lanes along i: rows
+// 8 apart met in two banks).  ALL: every point of the triple is an ordered
+// triple i > j > k inside the range.
+constexpr int V6_BLOCK = 72;  // doubles of an 8 x 8 V block with rows 9 apart
+template <bool HJ, int CY, int CZ, int CSZ, bool V6, bool ALL>
 __device__ __forceinline__ void triple_points(
     int B1, int B2, int B3, int no, int distinct, double epsabc,
     const int (&alias)[6], const double (*cube)[CSZ], const double *cubeJ,
     const double *tA, const double *tB, const double *tC, const double *sE,
     const double *sV, int tid, double &e_acc, double &ect_acc) {
-  auto vb = [](int v, int r, int s2, int q) {
-    return V6 ? (v * 6 + 2 * r + s2 - (s2 > r ? 1 : 0)) * 64 + q
-              : ((v * 3 + r) * 3 + s2) * 64 + q;
+  auto vb = [](int v, int r, int s2, int ly, int lz) {
+    return V6 ? (v * 6 + 2 * r + s2 - (s2 > r ? 1 : 0)) * V6_BLOCK + ly + 9 * lz
+              : ((v * 3 + r) * 3 + s2) * 64 + ly + 8 * lz;
   };
   // both points of a thread in one body, so their LDS reads and FP64
   // chains interleave
@@ -181,25 +185,25 @@ __device__ __forceinline__ void triple_points(
   for (int pt = tid; pt < 512; pt += 256) {
     const int li = pt & 7, lj = (pt >> 3) & 7, lk = pt >> 6;
     const int i = B1 * 8 + li, j = B2 * 8 + lj, k = B3 * 8 + lk;
-    if (i >= no || j >= no || k >= no || i < j || j < k) continue;
+    if (!ALL && (i >= no || j >= no || k >= no || i < j || j < k)) continue;
     const double ei = sE[li], ej = sE[8 + lj], ek = sE[16 + lk];
-    const double facjk = j == k ? 0.5 : 1.0;
-    const double facij = i == j ? 0.5 : 1.0;
+    const double facjk = !ALL && j == k ? 0.5 : 1.0;
+    const double facij = !ALL && i == j ? 0.5 : 1.0;
     const double eijk = (ei + ej) + ek;
     const double denominator = epsabc - eijk;
     // local offsets of the permutations inside their cubes
-    const int o_ijk = li + 8 * lj + CZ * lk, o_ikj = li + 8 * lk + CZ * lj,
-              o_jik = lj + 8 * li + CZ * lk, o_jki = lj + 8 * lk + CZ * li,
-              o_kij = lk + 8 * li + CZ * lj, o_kji = lk + 8 * lj + CZ * li;
+    const int o_ijk = li + CY * lj + CZ * lk, o_ikj = li + CY * lk + CZ * lj,
+              o_jik = lj + CY * li + CZ * lk, o_jki = lj + CY * lk + CZ * li,
+              o_kij = lk + CY * li + CZ * lj, o_kji = lk + CY * lj + CZ * li;
     // singles at a permutation (x,y,z): t_a[x] V^bc_yz + t_b[y] V^ac_xz
     // + t_c[z] V^ab_xy; slot s = 8 * position + local index (position 0:
     // i, 1: j, 2: k)
     auto Z = [&](double wv, int sx, int sy, int sz) {
       const int px = sx >> 3, py = sy >> 3, pz = sz >> 3;
       const int lx = sx & 7, ly = sy & 7, lz = sz & 7;
-      double zz = wv + tA[sx] * sV[vb(0, py, pz, ly + 8 * lz)];
-      zz = zz + tB[sy] * sV[vb(1, px, pz, lx + 8 * lz)];
-      zz = zz + tC[sz] * sV[vb(2, px, py, lx + 8 * ly)];
+      double zz = wv + tA[sx] * sV[vb(0, py, pz, ly, lz)];
+      zz = zz + tB[sy] * sV[vb(1, px, pz, lx, lz)];
+      zz = zz + tC[sz] * sV[vb(2, px, py, lx, ly)];
       return zz;
     };
     auto J = [&](int p, int o) { return cubeJ[alias[p] * CSZ + o]; };
@@ -396,7 +400,7 @@ void energy_kernel(EnergyParams P) {
       int cb_[6], nc_;
       orbit(B1, B2, B3, nbk, cb_, nc_, alias);
     }
-    triple_points<HJ, CZ, CSZ, false>(B1, B2, B3, no, distinct, epsabc,
+    triple_points<HJ, 8, CZ, CSZ, false, false>(B1, B2, B3, no, distinct, epsabc,
                                       alias, cube, &cubeJ[0][0], tA, tB, tC,
                                       sE, &sV[0][0][0][0], tid, e_acc,
                                       ect_acc);
@@ -426,21 +430,26 @@ void energy_kernel(EnergyParams P) {
 }
 
 // Fused class sums + singles + energy: one workgroup per (tuple slot, block
-// triple B1 >= B2 >= B3 of edge 8).  The workgroup gathers the (up to) six
+// triple B1 >= B2 >= B3 of edge 8).  The workgroup reads the (up to) six
 // permuted W cubes of the triple's orbit straight from the three class
-// buffers the doubles kernel wrote (each read along its own fastest index
-// in 64-byte row pieces) and sums them in LDS in the fixed order
-// (w + v) + u, the order of wsum_kernel, so W is the same bits as in the
-// cube path; then the triple's points follow triple_points, and the
-// workgroup's energy (a fixed shuffle/LDS tree) goes to its own entry of
-// e_part.  slot_sum_kernel adds a tuple's triples in order.  Nothing
-// about W leaves the chip: no cube is written to memory and read back.
+// buffers the doubles kernel wrote (4 KiB runs, two elements per lane) and
+// sums them in LDS in the fixed order (w + v) + u, the order of wsum_kernel,
+// so W is the same bits as in the cube path; then the triple's points follow
+// triple_points, and the workgroup's energy (a fixed shuffle/LDS tree) goes
+// to its own entry of e_part.  slot_sum_kernel adds a tuple's triples in
+// order.  Nothing about W leaves the chip: no cube is written to memory and
+// read back.
+// Bound by HBM with FP64 buffers (5.8 TB/s read at No=40), by LDS and VALU
+// with FP32 ones.  For 155,248 tuples at No=40, Nv=400, FP64 / bf16x3 in ms:
+// 57.1 / 55.7 from GEMM-ordered buffers, 53.7 / 47.4 from 8^3 blocks, 41.5 /
+// 39.8 with one instance per orbit type and for triples inside the range,
+// 40.8 / 36.8 with the LDS strides below; No=60, Nv=240 131 / 119 -> 95 / 83.
 struct FusedParams {
   const void *G, *GJ;  // class buffers [3][slots][No^2 rows][NoP] (FP64 or FP32)
   const double *Tai, *VHH, *ei, *ea;
   WindowArgs win;
   double *e_part;  // [triple][slot][2]
-  int64_t No, Nv, N2, NoP, W3g, slots, ntri;
+  int64_t No, Nv, N2, W3g, slots, ntri;
   int nbk;
   double tai_sign;
 };
@@ -467,74 +476,70 @@ __device__ __forceinline__ void triple_of(int t, int nbk, int &B1, int &B2,
   B1 = B2 + r;
 }
 
-// The loads, class phases and points of one block triple's orbit, whose
-// NC distinct cubes (6, 3 or 1) are qc[0 .. NC - 1]: one compile-time
-// instance per NC, so every load of an instance is issued before any is
-// waited on and none is spent on a repeated cube.
-template <typename GT, bool HJ, int NC, int CZ, int CSZ>
+// The orbit of a block triple B1 >= B2 >= B3 under the six index
+// permutations (ijk ikj jik jki kij kji), by type: 0 all different, 1 B1 =
+// B2, 2 B2 = B3, 3 all equal.  NC: its distinct cubes; CUBE: their block
+// coordinates as positions in (B1, B2, B3); ALIAS: cube of each permutation.
+template <int TYPE> struct Orbit;
+template <> struct Orbit<0> {
+  static constexpr int NC = 6, ALIAS[6] = {0, 1, 2, 3, 4, 5};
+  static constexpr int CUBE[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2},
+                                     {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
+};
+template <> struct Orbit<1> {
+  static constexpr int NC = 3, ALIAS[6] = {0, 1, 0, 1, 2, 2};
+  static constexpr int CUBE[3][3] = {{0, 0, 2}, {0, 2, 0}, {2, 0, 0}};
+};
+template <> struct Orbit<2> {
+  static constexpr int NC = 3, ALIAS[6] = {0, 0, 1, 2, 1, 2};
+  static constexpr int CUBE[3][3] = {{0, 1, 1}, {1, 0, 1}, {1, 1, 0}};
+};
+template <> struct Orbit<3> {
+  static constexpr int NC = 1, ALIAS[6] = {0, 0, 0, 0, 0, 0};
+  static constexpr int CUBE[1][3] = {{0, 0, 0}};
+};
+
+// The loads, class phases and points of one block triple of orbit TYPE: one
+// compile-time instance per type, and per triple whose blocks lie inside the
+// occupied range (FULL), so every load of an instance is issued before any is
+// waited on, none is spent on a repeated cube, and its addresses and LDS
+// places are constants next to one per-thread offset (with run-time cube
+// codes and range checks 692 VALU instructions per wave, of which about 150
+// were the points' arithmetic).
+template <typename GT, bool HJ, int TYPE, bool FULL, int CY, int CZ, int CSZ>
 __device__ __forceinline__ void fused_orbit(
     const FusedParams &P, int64_t gid, int64_t gslot, int tid, int no,
     int64_t a, int64_t b, int64_t c, int B1, int B2, int B3, int distinct,
-    double epsabc, const int (&qc)[6], const int (&alias)[6],
-    double (*cube)[CSZ], double (*cubeJ)[HJ ? CSZ : 1], double *tA,
+    double epsabc, double (*cube)[CSZ], double (*cubeJ)[HJ ? CSZ : 1], double *tA,
     double *tB, double *tC, double *sE, double *sV, double (*red)[4]) {
   const int64_t No = P.No, Nv = P.Nv, N2 = P.N2;
-  // element e = tid + 256 h of a cube, per class: row e >> 3 of the class's
-  // two slower indices, f = e & 7 along its fastest index
-  const GT *G = (const GT *)P.G;
-  const GT *GJ = (const GT *)P.GJ;
   const int64_t W3g = P.W3g, slots = P.slots;
-  const int nop = (int)P.NoP;  // 32-bit: offsets use the 32x32->64 multiply-add
-  const int64_t bw = gslot * W3g, bv = (slots + gslot) * W3g,
-                bu = (2 * slots + gslot) * W3g;
-  // element (q, h) of class cls for this thread: its offset inside the
-  // slot's class buffer (0 outside the occupied range, with in false) and
-  // its LDS position.  Branch-free, and 32-bit: the class base is
-  // wave-uniform, so a load is a scalar base plus a 32-bit lane offset
-  // (No^2 times the row pitch stays far below 2^32).
-  auto elem = [&](int q, int h, int cls, int &pos, bool &in) -> uint32_t {
-    const int e = tid + 256 * h, r = e >> 3, f = e & 7;
-    const int r0 = r & 7, r1 = r >> 3;
-    const int x = cls == 2 ? f : r0;
-    const int y = cls == 0 ? r1 : cls == 1 ? f : r0;
-    const int z = cls == 0 ? f : r1;
-    pos = x + 8 * y + CZ * z;
-    const int i = 8 * (qc[q] & 255) + x, j = 8 * ((qc[q] >> 8) & 255) + y,
-              k = 8 * (qc[q] >> 16) + z;
-    in = (i < no) & (j < no) & (k < no);
-    const uint32_t o =
-        cls == 0 ? (uint32_t)((i + no * j) * nop + k)      // w: k fastest
-      : cls == 1 ? (uint32_t)((i + no * k) * nop + j)      // v: j fastest
-                 : (uint32_t)((j + no * k) * nop + i);     // u: i fastest
-    return in ? o : 0u;  // always a valid address
+  const GT *Gs = (const GT *)P.G + gslot * W3g;
+  const GT *GJs = (const GT *)P.GJ + gslot * W3g;
+  typedef GT g2 __attribute__((ext_vector_type(2)));
+  constexpr int NC = Orbit<TYPE>::NC;
+  const int alias[6] = {Orbit<TYPE>::ALIAS[0], Orbit<TYPE>::ALIAS[1],
+                        Orbit<TYPE>::ALIAS[2], Orbit<TYPE>::ALIAS[3],
+                        Orbit<TYPE>::ALIAS[4], Orbit<TYPE>::ALIAS[5]};
+  auto pair = [&](int q, int cls) {
+    const int *c = Orbit<TYPE>::CUBE[q];
+    auto B = [&](int x) { return x == 0 ? B1 : x == 1 ? B2 : B3; };
+    return pair_at<CY, CZ, FULL>(cls, B(c[0]), B(c[1]), B(c[2]), P.nbk, no, tid);
   };
-  auto gather = [&](const GT *S, int q, int h, int cls) -> double {
-    int pos;
-    bool in;
-    const uint32_t o = elem(q, h, cls, pos, in);
-    const GT *Sc = S + (cls == 0 ? bw : cls == 1 ? bv : bu);
-    const GT v = Sc[o];
-    return in ? (double)v : 0.0;
-  };
-  // The loads, class phases and points for the orbit's nc distinct cubes
-  // (6, 3 or 1), one compile-time instance each, selected by a uniform
-  // branch: every load of an instance is issued before any is waited on
-  // and none is spent on a repeated cube.
   // Every global load of the workgroup is issued before any is waited on
   // (a load behind a branch is waited on before the branch joins, which
   // serialised the first version's loads): W and the (cT) W of the orbit's
   // cubes, the V^bc, V^ac, V^ab blocks of the triple, and (wave 0) t at
   // (a,x), (b,x), (c,x) and eps_i for x in the blocks B1, B2, B3.
-  double vals[HJ ? 2 : 1][3][NC][2];
+  g2 vals[HJ ? 2 : 1][3][NC];
 #pragma unroll
   for (int set = 0; set < (HJ ? 2 : 1); set++)
 #pragma unroll
     for (int cls = 0; cls < 3; cls++)
 #pragma unroll
       for (int q = 0; q < NC; q++)
-#pragma unroll
-        for (int h = 0; h < 2; h++)
-          vals[set][cls][q][h] = gather(set ? GJ : G, q, h, cls);
+        vals[set][cls][q] =
+            *(const g2 *)((set ? GJs : Gs) + cls * slots * W3g + pair(q, cls).at);
   double vv[5];
   {
     const double *Vbc = P.VHH + (b + Nv * c) * N2;
@@ -553,7 +558,7 @@ __device__ __forceinline__ void fused_orbit(
       const int Bs = s2 == 0 ? B1 : s2 == 1 ? B2 : B3;
       const int y = Br * 8 + (l & 7), z = Bs * 8 + (l >> 3);
       const double *V = v == 0 ? Vbc : v == 1 ? Vac : Vab;
-      const bool ok_ = (e < 3 * 6 * 64) & (y < No) & (z < No);
+      const bool ok_ = (it < 4 || e < 3 * 6 * 64) & (FULL || ((y < No) & (z < No)));
       const double val = V[ok_ ? y + No * z : 0];
       vv[it] = ok_ ? val : 0.0;
     }
@@ -572,30 +577,37 @@ __device__ __forceinline__ void fused_orbit(
     sE[tid] = ex;
   }
 #pragma unroll
-  for (int it = 0; it < 5; it++) sV[tid + 256 * it] = vv[it];
+  for (int it = 0; it < 5; it++) {
+    const int e = tid + 256 * it;
+    if (it < 4 || e < 3 * 6 * 64)
+      sV[(e >> 6) * V6_BLOCK + (e & 7) + 9 * ((e >> 3) & 7)] = vv[it];
+  }
   // the three class phases into LDS in the order w, v, u
 #pragma unroll
   for (int cls = 0; cls < 3; cls++) {
 #pragma unroll
-    for (int q = 0; q < NC; q++)
+    for (int q = 0; q < NC; q++) {
+      const PairAt a = pair(q, cls);
 #pragma unroll
-      for (int h = 0; h < 2; h++) {
-        int at;
-        bool in_;
-        (void)elem(q, h, cls, at, in_);
+      for (int set = 0; set < (HJ ? 2 : 1); set++) {
+        const g2 v = vals[set][cls][q];
+        const double v0 = a.in0 ? (double)v[0] : 0.0,
+                     v1 = a.in1 ? (double)v[1] : 0.0;
+        double *b0 = set ? &cubeJ[q][a.pos] : &cube[q][a.pos], *b1 = b0 + a.step;
         if (cls == 0) {
-          cube[q][at] = vals[0][0][q][h];
-          if constexpr (HJ) cubeJ[q][at] = vals[HJ ? 1 : 0][0][q][h];
+          *b0 = v0;
+          *b1 = v1;
         } else {
-          cube[q][at] += vals[0][cls][q][h];
-          if constexpr (HJ) cubeJ[q][at] += vals[HJ ? 1 : 0][cls][q][h];
+          *b0 += v0;
+          *b1 += v1;
         }
       }
+    }
     __syncthreads();
   }
 
   double e_acc = 0.0, ect_acc = 0.0;
-  triple_points<HJ, CZ, CSZ, true>(B1, B2, B3, no, distinct, epsabc, alias,
+  triple_points<HJ, CY, CZ, CSZ, true, TYPE == 0 && FULL>(B1, B2, B3, no, distinct, epsabc, alias,
                                    cube, &cubeJ[0][0], tA, tB, tC, sE, sV,
                                    tid, e_acc, ect_acc);
   e_acc = wave_sum(e_acc);
@@ -615,7 +627,8 @@ __device__ __forceinline__ void fused_orbit(
 }
 
 template <typename GT, bool HJ>
-__global__ __launch_bounds__(256) void energy_fused_kernel(FusedParams P) {
+__global__ __launch_bounds__(256, HJ ? 2 : 4) void energy_fused_kernel(
+    FusedParams P) {
   // workgroups go to the 8 XCDs round-robin: XCD x runs the triples of
   // slots x, x + 8, x + 16, ... one slot after the other, so the triples of
   // a slot (whose row pieces share 128-byte lines) meet in one L2, and the
@@ -626,7 +639,11 @@ __global__ __launch_bounds__(256) void energy_fused_kernel(FusedParams P) {
   const uint32_t bid = blockIdx.x, r = bid >> 3, ntri = (uint32_t)P.ntri;
   const uint32_t rq = r / ntri;
   const uint32_t gs = 8 * rq + (bid & 7);
-  const int tri = (int)(r - rq * ntri);
+  // each slot starts one triple further on: with 4, 20 or 120 triples a fixed
+  // order brings the triples of one cube to the same shader engine every time
+  uint32_t tr = r - rq * ntri + rq % ntri;
+  if (tr >= ntri) tr -= ntri;
+  const int tri = (int)tr;
   if ((int64_t)gs >= P.slots) return;
   const int64_t gslot = gs;
   const int64_t gid = tri * P.slots + gslot;
@@ -640,14 +657,17 @@ __global__ __launch_bounds__(256) void energy_fused_kernel(FusedParams P) {
     }
     return;
   }
-  constexpr int CZ = 69, CSZ = 7 * CZ + 64;
+  // element x + 9 y + 74 z of a cube: of the 16 lanes that share an LDS cycle
+  // at most two meet in a bank, in the class phases (lanes along a pair of
+  // x, y or z and the class's second index) and in the points' six reads
+  // (lanes along i and j); with x + 8 y + 69 z four did in half of them
+  constexpr int CY = 9, CZ = 74, CSZ = 7 * (CY + CZ) + 8;
   __shared__ double cube[6][CSZ];
   __shared__ double cubeJ[HJ ? 6 : 1][HJ ? CSZ : 1];
   // singles tables (entries 0..23 used; wave 0 writes all 64) and the V
-  // blocks of the six block pairs of different positions (1152 used; every
-  // thread writes its five, 1280)
+  // blocks of the six block pairs of different positions
   __shared__ double tA[64], tB[64], tC[64], sE[64];
-  __shared__ double sV[5 * 256];
+  __shared__ double sV[3 * 6 * V6_BLOCK];
   __shared__ double red[2][4];
 
   int distinct = 0;
@@ -657,49 +677,23 @@ __global__ __launch_bounds__(256) void energy_fused_kernel(FusedParams P) {
   const int no = (int)No;
   int B1, B2, B3;
   triple_of(tri, P.nbk, B1, B2, B3);
-  // The orbit's distinct cubes.  Permutation p (ijk ikj jik jki kij kji)
-  // holds its W in the cube of block coordinates code[p] (i | j << 8 |
-  // k << 16); the distinct codes, in order of first appearance, are cubes
-  // 0 .. nc - 1 (qc), and alias[p] is the cube of permutation p.  Every
-  // array index below is a compile-time constant, so all of it stays in
-  // registers.
-  const int code[6] = {B1 | B2 << 8 | B3 << 16, B1 | B3 << 8 | B2 << 16,
-                       B2 | B1 << 8 | B3 << 16, B2 | B3 << 8 | B1 << 16,
-                       B3 | B1 << 8 | B2 << 16, B3 | B2 << 8 | B1 << 16};
-  int alias[6], qc[6], nc = 0;
-#pragma unroll
-  for (int q = 0; q < 6; q++) qc[q] = 0;
-#pragma unroll
-  for (int p = 0; p < 6; p++) {
-    int first = p;  // earliest permutation with the same cube
-#pragma unroll
-    for (int q = p - 1; q >= 0; q--)
-      if (code[q] == code[p]) first = q;
-    int al = nc;
-#pragma unroll
-    for (int q = 0; q < p; q++)
-      if (q == first) al = alias[q];
-    alias[p] = al;
-    if (first == p) {
-#pragma unroll
-      for (int q = 0; q < 6; q++)
-        if (q == nc) qc[q] = code[p];
-      nc++;
-    }
+  // wave-uniform choice of the instance: only the last block of the range can
+  // be partly empty, and B1 is the largest
+  const bool full = 8 * (B1 + 1) <= no;
+#define ORBIT(T, F)                                                           \
+  fused_orbit<GT, HJ, T, F, CY, CZ, CSZ>(P, gid, gslot, tid, no, a, b, c, B1, B2, \
+                                     B3, distinct, epsabc, cube, cubeJ, tA,   \
+                                     tB, tC, sE, sV, red)
+  if (B1 > B2 && B2 > B3) {
+    if (full) ORBIT(0, true); else ORBIT(0, false);
+  } else if (B1 > B2) {
+    if (full) ORBIT(2, true); else ORBIT(2, false);
+  } else if (B2 > B3) {
+    if (full) ORBIT(1, true); else ORBIT(1, false);
+  } else {
+    ORBIT(3, false);
   }
-
-  if (nc == 6)
-    fused_orbit<GT, HJ, 6, CZ, CSZ>(P, gid, gslot, tid, no, a, b, c, B1, B2,
-                                    B3, distinct, epsabc, qc, alias, cube,
-                                    cubeJ, tA, tB, tC, sE, sV, red);
-  else if (nc == 3)
-    fused_orbit<GT, HJ, 3, CZ, CSZ>(P, gid, gslot, tid, no, a, b, c, B1, B2,
-                                    B3, distinct, epsabc, qc, alias, cube,
-                                    cubeJ, tA, tB, tC, sE, sV, red);
-  else
-    fused_orbit<GT, HJ, 1, CZ, CSZ>(P, gid, gslot, tid, no, a, b, c, B1, B2,
-                                    B3, distinct, epsabc, qc, alias, cube,
-                                    cubeJ, tA, tB, tC, sE, sV, red);
+#undef ORBIT
 }
 
 // Neumaier step on a (sum, compensation) pair.
@@ -783,19 +777,19 @@ __global__ __launch_bounds__(256) void window_sum_kernel(const double *e_slot,
 
 hipError_t launch_wsum(const DevSystem &s, const BatchArgs &b, const void *A,
                        const void *B, bool g32, double *out, hipStream_t st) {
-  const int nbk = (int)w_blocks(s.No), nbr = (nbk + 1) / 2;
-  const int64_t grid = b.slots * (int64_t)nbr * nbr * nbr;
+  const int nbk = (int)w_blocks(s.No);
+  const int64_t grid = b.slots * (int64_t)nbk * nbk * nbk;
   if (grid <= 0) return hipSuccess;
   if (grid > MAX_GRID) return hipErrorInvalidConfiguration;
-  const int64_t NoP = g_pitch(s.No, g32), W3g = g_elems(s.No, g32);
+  const int64_t W3g = g_elems(s.No);
   if (g32)
     hipLaunchKernelGGL(wsum_kernel<float>, dim3((unsigned)grid), dim3(256), 0,
-                       st, (const float *)A, (const float *)B, out, s.No, NoP, W3g,
-                       b.slots, nbk, nbr);
+                       st, (const float *)A, (const float *)B, out, (int)s.No,
+                       W3g, b.slots, nbk);
   else
     hipLaunchKernelGGL(wsum_kernel<double>, dim3((unsigned)grid), dim3(256),
-                       0, st, (const double *)A, (const double *)B, out, s.No,
-                       NoP, W3g, b.slots, nbk, nbr);
+                       0, st, (const double *)A, (const double *)B, out,
+                       (int)s.No, W3g, b.slots, nbk);
   return hipGetLastError();
 }
 
@@ -817,8 +811,7 @@ hipError_t launch_energy(const DevSystem &s, const BatchArgs &b,
     P.No = s.No;
     P.Nv = s.Nv;
     P.N2 = s.No * s.No;
-    P.NoP = g_pitch(s.No, g32);
-    P.W3g = g_elems(s.No, g32);
+    P.W3g = g_elems(s.No);
     P.slots = b.slots;
     P.ntri = ntri;
     P.nbk = (int)nbk;
@@ -826,7 +819,7 @@ hipError_t launch_energy(const DevSystem &s, const BatchArgs &b,
     const int64_t grid = (b.slots + 7) / 8 * 8 * ntri;
     if (grid <= 0) return hipSuccess;
     // (the kernel decodes its block id and class-buffer offsets in 32 bits)
-    if (grid > MAX_GRID || g_elems(s.No, g32) >= (int64_t(1) << 31))
+    if (grid > MAX_GRID || g_elems(s.No) >= (int64_t(1) << 31))
       return hipErrorInvalidConfiguration;
     if (g32 && GJ)
       hipLaunchKernelGGL((energy_fused_kernel<float, true>), dim3((unsigned)grid),

@@ -70,32 +70,46 @@ __host__ __device__ inline int64_t f64_elems(const TriGeom &g) {
 }
 
 // Layout of the per-tuple class buffers written by the doubles kernels and
-// read by the energy kernels: each class keeps its GEMM output order,
-// element (row m, column index r) at m * P + r with the row pitch
-// P = g_pitch(No), so a 16-column MFMA output fragment row is one contiguous
-// store and every row starts on a 64-byte boundary.  In W indices:
-//   class w: m = i + No j, r = k   ->  (i + No j) P + k
-//   class v: m = i + No k, r = j   ->  (i + No k) P + j
-//   class u: m = j + No k, r = i   ->  (j + No k) P + i
-// Row pitch: No rounded up to 8 elements for FP64 buffers, 16 for FP32 (the
-// FP32-product forms), so the 64-byte row pieces the epilogue gathers never
-// straddle a line; the pad columns are never written or read.
-__host__ __device__ inline int64_t g_pitch(int64_t No, bool g32) {
-  const int64_t q = g32 ? 16 : 8;
-  return (No + q - 1) / q * q;
-}
-// Largest one-dimensional grid a launch takes (workgroups); launchers
-// refuse larger ones instead of truncating the count.
-constexpr int64_t MAX_GRID = 0xFFFFFFFFLL;
-// Elements of one tuple's class buffer.
-__host__ __device__ inline int64_t g_elems(int64_t No, bool g32) {
-  return No * No * g_pitch(No, g32);
-}
-// The energy kernels stage 8x8x8 blocks of W in LDS (edge WCUBE).
+// read by the energy kernels: blocks of 8 x 8 x 8 elements of the GEMM output
+// (row m = p + No q, column r), element (p, q, r) at block
+// ((q / 8) nbk + p / 8) nbk + r / 8, inside it 64 (q % 8) + 8 (p % 8) + r % 8;
+// in W indices
+//   class w: (p, q, r) = (i, j, k)
+//   class v: (p, q, r) = (i, k, j)
+//   class u: (p, q, r) = (j, k, i)
+// so the 8^3 block of W an epilogue workgroup needs is one run of 4 KiB (FP64;
+// 2 KiB FP32) in each class, where a GEMM-ordered buffer held it in 64 pieces
+// of 64 bytes, one request each.  Elements past No are neither written nor
+// read.
+// Edge of the blocks (of the class buffers, and of W in LDS).
 constexpr int WCUBE = 8;
 __host__ __device__ inline int64_t w_blocks(int64_t No) {
   return (No + WCUBE - 1) / WCUBE;
 }
+// Elements of one tuple's class buffer.
+__host__ __device__ inline int64_t g_elems(int64_t No) {
+  const int64_t n = w_blocks(No) * WCUBE;
+  return n * n * n;
+}
+// Offset of a GEMM row and of a GEMM column in it.
+struct GLayout {
+  uint32_t No, nbk, magic;  // magic: ceil(2^32 / No), exact for rows < No^2
+};
+inline GLayout g_layout(int64_t No) {
+  return {(uint32_t)No, (uint32_t)w_blocks(No),
+          No == 1 ? 0u : (uint32_t)((((uint64_t)1 << 32) + No - 1) / No)};
+}
+__device__ __forceinline__ uint32_t g_row(const GLayout &L, uint32_t m) {
+  const uint32_t q = L.No == 1 ? m : __umulhi(m, L.magic), p = m - q * L.No;
+  return (((q >> 3) * L.nbk + (p >> 3)) * L.nbk << 9) + ((q & 7) << 6) +
+         ((p & 7) << 3);
+}
+__device__ __forceinline__ uint32_t g_col(uint32_t r) {
+  return ((r >> 3) << 9) + (r & 7);
+}
+// Largest one-dimensional grid a launch takes (workgroups); launchers
+// refuse larger ones instead of truncating the count.
+constexpr int64_t MAX_GRID = 0xFFFFFFFFLL;
 // Doubles of one tuple's W in the cube layout the energy kernels read: the
 // occupied range padded to whole cubes, cube (bx, by, bz) at
 // ((bz nbk + by) nbk + bx) * 512, element x + 8 y + 64 z inside.
