@@ -708,7 +708,9 @@ void complex_negations(atrip_hip_ctx *ctx, DevSystem &s) {
   check(hipStreamSynchronize(ctx->stream), "negations");
 }
 
-// The four real class-GEMM passes of a complex system: W = Wr + i Wi with
+// The four real products of a complex system, two per plane of W and class
+// GEMM (one after the other along K: a plane is written once): W = Wr + i Wi
+// with
 //   Wr = [T3r V3r + H3r N_r] + [(-T3i) V3i + H3i N_i]
 //   Wi = [T3r V3i + H3r N_i] + [T3i V3r + (-H3i) N_r]
 // where N = -T2 (the pre-negated hole operands) and the hole terms carry
@@ -917,7 +919,7 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
   const int nsel = (int)win.count.size();
   if (!nsel) return res;
   // Device scratch of the run: class buffers G (and those of the (cT)
-  // pass; four sets for complex systems), per-slot energies, the energy
+  // pass; two planes each for complex systems), per-slot energies, the energy
   // kernels' scratch (per-triple partials, or W cubes for complex systems
   // and the cube epilogue), batch partials and the window list.  Taken from the context's buffers (grown
   // on demand), or carved out of a fixed region without any allocation
@@ -925,7 +927,7 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
   const int64_t per = (int64_t)win.ea * win.eb * win.ec;  // slots of a window
   const int64_t W3 = g_elems(s.No);  // one tuple's class buffer
   const bool use_j = s.has_j;
-  const int nsets = s.cplx ? 4 : 1;
+  const int nsets = s.cplx ? 2 : 1;  // W's planes
   const size_t gelem = g32 ? sizeof(float) : sizeof(double);
   const bool fused = ctx->epilogue == 0;
   struct Sizes {
@@ -1051,10 +1053,10 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
                       : precision == ATRIP_BF16X3     ? "doubles_bf16x3"
                                                       : "doubles_fp32";
   hipStream_t st = ctx->stream;
-  double *Gz[4], *GJz[4];
-  for (int q = 0; q < 4; q++) {
+  double *Gz[2], *GJz[2];
+  for (int q = 0; q < 2; q++) {
     Gz[q] = (double *)((char *)Gbuf + q * gsz);
-    GJz[q] = (double *)((char *)Gbuf + (4 + q) * gsz);
+    GJz[q] = (double *)((char *)Gbuf + (2 + q) * gsz);
   }
   void *G = Gbuf;
   void *GJ = use_j ? (void *)((char *)Gbuf + gsz) : nullptr;
@@ -1089,14 +1091,15 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
       check(hipEventRecord(ev.e[0], st), "event");
     }
     for (int pass = 0; pass < (use_j ? 2 : 1) && s.cplx; pass++)
-      for (int q = 0; q < 4; q++)
-        check(launch_doubles_f64(zpass[q], b, pass == 1,
+      for (int q = 0; q < 2; q++)
+        check(launch_doubles_f64(zpass[2 * q], &zpass[2 * q + 1], b, pass == 1,
                                  pass == 0 ? Gz[q] : GJz[q], ctx->tile, st),
-              "doubles kernel (complex pass)");
+              "doubles kernel (complex plane)");
     for (int pass = 0; pass < (use_j ? 2 : 1) && !s.cplx; pass++) {
       void *Gp = pass == 0 ? G : GJ;
       if (precision == ATRIP_FP64)
-        check(launch_doubles_f64(s, b, pass == 1, (double *)Gp, ctx->tile, st),
+        check(launch_doubles_f64(s, nullptr, b, pass == 1, (double *)Gp,
+                                 ctx->tile, st),
               "doubles kernel");
       else if (precision == ATRIP_BF16X3)
         check(launch_doubles_tri(s, b, pass == 1, (float *)Gp, ctx->tile, st),

@@ -37,9 +37,19 @@ typedef double d2 __attribute__((ext_vector_type(2)));
 constexpr int KC = 8;     // kappa per chunk: one operand tile
 constexpr int TILE = 128;  // doubles per operand tile
 
-struct DoublesParams {
+// Operands of one set of four K segments.
+struct OperandSet {
   // T3s, H3s: row-swapped copies (null: read the swapped rows of T3, H3)
   const double *T3, *T3s, *V3, *H3, *H3s, *T2N, *T2TN;
+};
+struct DoublesParams {
+  OperandSet op;
+  // bytes from each array of the first set to the second's (chosen at run
+  // time by mask: a choice between two pointer members put P in scratch)
+  struct {
+    int64_t T3, T3s, V3, H3, H3s, T2N, T2TN;
+  } to2;
+  int nseg;  // K segments: 4, or 8 over both sets (a complex product's plane)
   WindowArgs win;
   double *G;
   int64_t No, Nv, Kv, Ko, N2, N2p, W3, slots;
@@ -85,21 +95,25 @@ __device__ __forceinline__ void f64_wave(const DoublesParams &P,
   const int64_t Kv = P.Kv, Ko = P.Ko;
   // segments: 0 T3[x1] straight, 1 T3[x2] swapped, 2 H3[x2] straight,
   //           3 H3[x1] swapped
+#define SEL(x) ((const double *)((const char *)P.op.x + (o2_ & P.to2.x)))
 #define SET_PTRS(SG)                                                        \
   {                                                                         \
-    const int64_t K_ = (SG) < 2 ? Kv : Ko;                                  \
-    const int64_t xr_ = ((SG) == 0 || (SG) == 3 ? T.x1 : T.x2) * N2p;       \
-    const double *As_ = (SG) < 2 ? P.T3s : P.H3s;                           \
-    const bool sw_ = ((SG)&1) && As_;                                       \
-    const double *Ab_ = sw_ ? As_ : (SG) < 2 ? P.T3 : P.H3;                 \
+    const int64_t o2_ = (SG) >= 4 ? -1 : 0;                                 \
+    const int s_ = (SG)&3;                                                  \
+    const int64_t K_ = s_ < 2 ? Kv : Ko;                                    \
+    const int64_t xr_ = (s_ == 0 || s_ == 3 ? T.x1 : T.x2) * N2p;           \
+    const bool sw_ = (s_ & 1) && (s_ < 2 ? P.op.T3s : P.op.H3s);            \
+    const double *Ab_ = sw_ ? (s_ < 2 ? SEL(T3s) : SEL(H3s))                \
+                            : (s_ < 2 ? SEL(T3) : SEL(H3));                 \
     _Pragma("unroll") for (int f = 0; f < FM; f++) ap[f] =                  \
-        Ab_ + f64_row(xr_ + (((SG)&1) && !sw_ ? rowW[f] : rowS[f]), K_) +   \
+        Ab_ + f64_row(xr_ + ((s_ & 1) && !sw_ ? rowW[f] : rowS[f]), K_) +   \
         32 * kk;                                                            \
     _Pragma("unroll") for (int g = 0; g < FN; g++) {                        \
       int wh_;                                                              \
       const int64_t R_ =                                                    \
-          b_row(T.cl, (SG), T.x1, T.x2, cy[g], crr[g], Nv, No, wh_);        \
-      const double *B_ = wh_ == 0 ? P.V3 : wh_ == 1 ? P.T2N : P.T2TN;       \
+          b_row(T.cl, s_, T.x1, T.x2, cy[g], crr[g], Nv, No, wh_);          \
+      const double *B_ = wh_ == 0 ? SEL(V3) : wh_ == 1 ? SEL(T2N)           \
+                                                       : SEL(T2TN);         \
       bp[g] = B_ + f64_row(R_, K_) + 32 * kk;                               \
     }                                                                       \
   }
@@ -119,7 +133,7 @@ __device__ __forceinline__ void f64_wave(const DoublesParams &P,
   d2 a[D][FM], b[D][FN];
 #define LOAD(J)                                                             \
   {                                                                         \
-    const int64_t at_ = TILE * (int64_t)(sg < 4 ? c : nch - 1);             \
+    const int64_t at_ = TILE * (int64_t)(sg < nseg ? c : nch - 1);          \
     _Pragma("unroll") for (int f = 0; f < FM; f++) a[J][f] =                \
         *(const d2 *)(ap[f] + at_);                                         \
     _Pragma("unroll") for (int g = 0; g < FN; g++) b[J][g] =                \
@@ -132,7 +146,7 @@ __device__ __forceinline__ void f64_wave(const DoublesParams &P,
           _Pragma("unroll") for (int g = 0; g < FN; g++) acc[f][g] =        \
               __builtin_amdgcn_mfma_f64_16x16x4f64(a[J][f][s], b[J][g][s],  \
                                                    acc[f][g], 0, 0, 0);
-  // One pipeline through the four segments: (sg, c) is the next chunk to
+  // One pipeline through the segments: (sg, c) is the next chunk to
   // load, and past a segment's end the pointers move to the next segment's
   // chunk 0 in place, so every segment but the first starts with its first
   // chunks in flight (3 % faster at No=40 than a pipeline restarted per
@@ -140,13 +154,14 @@ __device__ __forceinline__ void f64_wave(const DoublesParams &P,
   // kappa.  The prefetch is issued unconditionally (after the last chunk it
   // re-reads it, a load never used) so every path into a COMPUTE has the
   // same loads outstanding.
+  const int nseg = P.nseg;
   int sg = 0;
   int nch = (int)((Nv + KC - 1) / KC), c = 0;
   SET_PTRS(0);
 #define ADVANCE()                                                            \
-  if (sg < 4 && ++c == nch && ++sg < 4) {                                    \
+  if (sg < nseg && ++c == nch && ++sg < nseg) {                              \
     SET_PTRS(sg);                                                            \
-    nch = (int)(((sg < 2 ? Nv : No) + KC - 1) / KC);                         \
+    nch = (int)((((sg & 3) < 2 ? Nv : No) + KC - 1) / KC);                   \
     c = 0;                                                                   \
   }
 #pragma unroll
@@ -157,7 +172,7 @@ __device__ __forceinline__ void f64_wave(const DoublesParams &P,
   // (one exit: leaving the loop between two sets made the compiler copy the
   // accumulators between register files on every turn; the chunks of a last
   // part turn follow it)
-  int left = 2 * (int)((Nv + KC - 1) / KC + (No + KC - 1) / KC);
+  int left = nseg / 2 * (int)((Nv + KC - 1) / KC + (No + KC - 1) / KC);
 #pragma unroll 1
   for (; left >= D; left -= D) {
 #pragma unroll
@@ -175,6 +190,7 @@ __device__ __forceinline__ void f64_wave(const DoublesParams &P,
 #undef COMPUTE
 
 #undef SET_PTRS
+#undef SEL
   // store: for v_mfma_f64_16x16x4f64, D[i][j] sits in lane j + 16*(i%4),
   // register i/4 (measured on gfx950)
   const int64_t per = (int64_t)P.win.ea * P.win.eb * P.win.ec;
@@ -249,17 +265,25 @@ __global__ __launch_bounds__(128 * WR, 2) void doubles_f64_kernel(
 
 }  // namespace
 
-hipError_t launch_doubles_f64(const DevSystem &s, const BatchArgs &b,
-                              bool use_j, double *G, int tile,
-                              hipStream_t st) {
+hipError_t launch_doubles_f64(const DevSystem &s, const DevSystem *s2,
+                              const BatchArgs &b, bool use_j, double *G,
+                              int tile, hipStream_t st) {
   DoublesParams P;
-  P.T3 = s.T3;
-  P.T3s = s.T3s;
-  P.V3 = use_j ? s.V3J : s.V3;
-  P.H3 = use_j ? s.H3J : s.H3;
-  P.H3s = use_j ? s.H3Js : s.H3s;
-  P.T2N = s.T2N;
-  P.T2TN = s.T2TN;
+  P.nseg = s2 ? 8 : 4;
+  auto set = [&](const DevSystem &x) {
+    return OperandSet{x.T3, x.T3s, use_j ? x.V3J : x.V3, use_j ? x.H3J : x.H3,
+                      use_j ? x.H3Js : x.H3s, x.T2N, x.T2TN};
+  };
+  const OperandSet a = set(s), z = set(s2 ? *s2 : s);
+  P.op = a;
+  // (swapped copies are used when both sets have them)
+  if (!a.T3s || !z.T3s) P.op.T3s = nullptr;
+  if (!a.H3s || !z.H3s) P.op.H3s = nullptr;
+  auto to = [](const double *x, const double *y) {
+    return (int64_t)((intptr_t)y - (intptr_t)x);
+  };
+  P.to2 = {to(a.T3, z.T3), to(a.T3s, z.T3s), to(a.V3, z.V3), to(a.H3, z.H3),
+           to(a.H3s, z.H3s), to(a.T2N, z.T2N), to(a.T2TN, z.T2TN)};
   P.win = b;
   P.G = G;
   P.No = s.No;

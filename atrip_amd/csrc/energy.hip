@@ -69,13 +69,12 @@ __device__ __forceinline__ PairAt pair_at(int cls, int bx, int by, int bz,
   return a;
 }
 
-// Class sums of one 8^3 block of W for every slot of the batch: out = sum(A)
-// [+ sum(B)], sum(X) = (Xw + Xv) + Xu, written as cubes.
+// Class sums of one 8^3 block of W for every slot of the batch: out = (Aw +
+// Av) + Au, written as cubes.
 template <typename GT>
-__global__ __launch_bounds__(256) void wsum_kernel(const GT *A, const GT *B,
-                                                   double *out, int no,
-                                                   int64_t W3g, int64_t slots,
-                                                   int nbk) {
+__global__ __launch_bounds__(256) void wsum_kernel(const GT *A, double *out,
+                                                   int no, int64_t W3g,
+                                                   int64_t slots, int nbk) {
   typedef GT g2 __attribute__((ext_vector_type(2)));
   constexpr int CZ = 69;
   __shared__ double br[7 * CZ + 64];
@@ -84,43 +83,31 @@ __global__ __launch_bounds__(256) void wsum_kernel(const GT *A, const GT *B,
   const int blk = (int)(bid - (uint32_t)slot * n3);
   const int bx = blk % nbk, by = (blk / nbk) % nbk, bz = blk / (nbk * nbk);
   const int tid = threadIdx.x;
-  double sum[2] = {0.0, 0.0};
-  for (int set = 0; set < (B ? 2 : 1); set++) {
-    const GT *S = set == 0 ? A : B;
-    PairAt a[3];
-    g2 v[3];
+  PairAt a[3];
+  g2 v[3];
 #pragma unroll
-    for (int cls = 0; cls < 3; cls++) {
-      a[cls] = pair_at<8, CZ, false>(cls, bx, by, bz, nbk, no, tid);
-      v[cls] = *(const g2 *)(S + (cls * slots + slot) * W3g + a[cls].at);
-    }
+  for (int cls = 0; cls < 3; cls++) {
+    a[cls] = pair_at<8, CZ, false>(cls, bx, by, bz, nbk, no, tid);
+    v[cls] = *(const g2 *)(A + (cls * slots + slot) * W3g + a[cls].at);
+  }
 #pragma unroll
-    for (int cls = 0; cls < 3; cls++) {
-      const double v0 = a[cls].in0 ? (double)v[cls][0] : 0.0,
-                   v1 = a[cls].in1 ? (double)v[cls][1] : 0.0;
-      double *b0 = br + a[cls].pos, *b1 = b0 + a[cls].step;
-      if (cls == 0) {
-        *b0 = v0;
-        *b1 = v1;
-      } else {
-        *b0 += v0;
-        *b1 += v1;
-      }
-      __syncthreads();
-    }
-    // the two elements of the cube this thread writes
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-      const int e = tid + 256 * h;
-      sum[h] = set == 0 ? br[(e & 63) + CZ * (e >> 6)]
-                        : sum[h] + br[(e & 63) + CZ * (e >> 6)];
+  for (int cls = 0; cls < 3; cls++) {
+    const double v0 = a[cls].in0 ? (double)v[cls][0] : 0.0,
+                 v1 = a[cls].in1 ? (double)v[cls][1] : 0.0;
+    double *b0 = br + a[cls].pos, *b1 = b0 + a[cls].step;
+    if (cls == 0) {
+      *b0 = v0;
+      *b1 = v1;
+    } else {
+      *b0 += v0;
+      *b1 += v1;
     }
     __syncthreads();
   }
   double *o = out + slot * (int64_t)(512 * n3) +
               ((int64_t)((bz * nbk + by) * nbk + bx) << 9);
-  o[tid] = sum[0];
-  o[tid + 256] = sum[1];
+#pragma unroll
+  for (int e = tid; e < 512; e += 256) o[e] = br[(e & 63) + CZ * (e >> 6)];
 }
 
 // Energy of one tuple per workgroup.  The i>=j>=k points are visited per
@@ -776,7 +763,7 @@ __global__ __launch_bounds__(256) void window_sum_kernel(const double *e_slot,
 }  // namespace
 
 hipError_t launch_wsum(const DevSystem &s, const BatchArgs &b, const void *A,
-                       const void *B, bool g32, double *out, hipStream_t st) {
+                       bool g32, double *out, hipStream_t st) {
   const int nbk = (int)w_blocks(s.No);
   const int64_t grid = b.slots * (int64_t)nbk * nbk * nbk;
   if (grid <= 0) return hipSuccess;
@@ -784,12 +771,12 @@ hipError_t launch_wsum(const DevSystem &s, const BatchArgs &b, const void *A,
   const int64_t W3g = g_elems(s.No);
   if (g32)
     hipLaunchKernelGGL(wsum_kernel<float>, dim3((unsigned)grid), dim3(256), 0,
-                       st, (const float *)A, (const float *)B, out, (int)s.No,
-                       W3g, b.slots, nbk);
+                       st, (const float *)A, out, (int)s.No, W3g, b.slots,
+                       nbk);
   else
     hipLaunchKernelGGL(wsum_kernel<double>, dim3((unsigned)grid), dim3(256),
-                       0, st, (const double *)A, (const double *)B, out,
-                       (int)s.No, W3g, b.slots, nbk);
+                       0, st, (const double *)A, out, (int)s.No, W3g, b.slots,
+                       nbk);
   return hipGetLastError();
 }
 
@@ -837,9 +824,9 @@ hipError_t launch_energy(const DevSystem &s, const BatchArgs &b,
   }
   const int64_t W3c = w_cube(s.No);
   double *W = scratch, *WJ = GJ ? scratch + b.slots * W3c : nullptr;
-  hipError_t e = launch_wsum(s, b, G, nullptr, g32, W, st);
+  hipError_t e = launch_wsum(s, b, G, g32, W, st);
   if (e != hipSuccess) return e;
-  if (GJ && (e = launch_wsum(s, b, GJ, nullptr, g32, WJ, st)) != hipSuccess)
+  if (GJ && (e = launch_wsum(s, b, GJ, g32, WJ, st)) != hipSuccess)
     return e;
   EnergyParams P;
   P.W = W;

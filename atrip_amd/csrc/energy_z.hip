@@ -1,9 +1,9 @@
 // Singles + energy epilogue of complex (T) (atrip::Atrip::run<Complex>).
 //
-// The doubles of a complex system run as four real class-GEMM passes on
-// real/imaginary operand planes (see the run loop), so W = Wr + i Wi arrives
-// as four sets of class buffers: Wr = sum(G0) + sum(G1), Wi = sum(G2) +
-// sum(G3), summed into cubes by launch_wsum.  Per tuple (one workgroup), for each block
+// The doubles of a complex system run as real class GEMMs on real/imaginary
+// operand planes (see the run loop), so W = Wr + i Wi arrives as two sets of
+// class buffers, summed into cubes by launch_wsum.
+// Per tuple (one workgroup), for each block
 // triple of edge 8 the cubes holding W at the six index permutations are
 // summed into LDS as (re, im), Z = W + singles is formed with complex
 // products (reference src/atrip/Equations.cxx:387-426), and the energy
@@ -179,7 +179,7 @@ __global__ __launch_bounds__(256) void energy_z_kernel(EnergyZParams P) {
 }  // namespace
 
 hipError_t launch_energy_z(const DevSystem &s, const BatchArgs &b,
-                           double *const G[4], double *const GJ[4],
+                           double *const G[2], double *const GJ[2],
                            double tai_sign, double *e_slot, double *wcube,
                            hipStream_t st) {
   const int64_t W3c = w_cube(s.No), n = b.slots * W3c;
@@ -189,12 +189,12 @@ hipError_t launch_energy_z(const DevSystem &s, const BatchArgs &b,
   P.WJr = GJ ? wcube + 2 * n : nullptr;
   P.WJi = GJ ? wcube + 3 * n : nullptr;
   hipError_t e;
-  if ((e = launch_wsum(s, b, G[0], G[1], false, (double *)P.Wr, st)) != hipSuccess ||
-      (e = launch_wsum(s, b, G[2], G[3], false, (double *)P.Wi, st)) != hipSuccess)
+  if ((e = launch_wsum(s, b, G[0], false, (double *)P.Wr, st)) != hipSuccess ||
+      (e = launch_wsum(s, b, G[1], false, (double *)P.Wi, st)) != hipSuccess)
     return e;
   if (GJ &&
-      ((e = launch_wsum(s, b, GJ[0], GJ[1], false, (double *)P.WJr, st)) != hipSuccess ||
-       (e = launch_wsum(s, b, GJ[2], GJ[3], false, (double *)P.WJi, st)) != hipSuccess))
+      ((e = launch_wsum(s, b, GJ[0], false, (double *)P.WJr, st)) != hipSuccess ||
+       (e = launch_wsum(s, b, GJ[1], false, (double *)P.WJi, st)) != hipSuccess))
     return e;
   P.Tair = s.Tai;
   P.Taii = s.Taii;

@@ -349,9 +349,11 @@ __device__ __forceinline__ bool slot_tuple(const WindowArgs &W, uint64_t Nv,
                                            int64_t &c);
 
 // Doubles contractions in FP64 MFMA: class buffers G[3][slots][g_elems(No)].
-hipError_t launch_doubles_f64(const DevSystem &s, const BatchArgs &b,
-                              bool use_j, double *G, int tile,
-                              hipStream_t st);
+// With s2 its four products are added to those of s (same shape) in the same
+// GEMM: one plane of a complex product.
+hipError_t launch_doubles_f64(const DevSystem &s, const DevSystem *s2,
+                              const BatchArgs &b, bool use_j, double *G,
+                              int tile, hipStream_t st);
 
 // Doubles contractions in split FP32.
 // Doubles contractions with FP32 products (class buffers in FP32):
@@ -365,10 +367,10 @@ hipError_t launch_doubles_split(const DevSystem &s, const BatchArgs &b,
 hipError_t launch_doubles_tri(const DevSystem &s, const BatchArgs &b,
                               bool use_j, float *G, int tile, hipStream_t st);
 
-// Class sums: out[slot] = sum(A) (+ sum(B)) as cubes (w_cube per slot), for
-// class-buffer sets A, B (FP64, or FP32 when g32).
+// Class sums: out[slot] = sum(A) as cubes (w_cube per slot), for class-buffer
+// set A (FP64, or FP32 when g32).
 hipError_t launch_wsum(const DevSystem &s, const BatchArgs &b, const void *A,
-                       const void *B, bool g32, double *out, hipStream_t st);
+                       bool g32, double *out, hipStream_t st);
 
 // Class sums and singles + energy epilogue.  fused: one kernel gathers each
 // block triple's W straight from the class buffers and writes the triple's
@@ -387,11 +389,11 @@ inline int64_t energy_scratch_per_slot(int64_t No, bool use_j, bool cplx,
   return (use_j ? 2 : 1) * (cplx ? 2 : 1) * w_cube(No);
 }
 
-// Singles + energy of complex systems from the four class-buffer sets of
-// the real passes (Wr = G0 + G1, Wi = G2 + G3); GJ null without (cT).
+// Singles + energy of complex systems from the class-buffer sets of W's real
+// and imaginary plane; GJ null without (cT).
 // wcube: scratch of (GJ ? 4 : 2) * slots * w_cube(No) doubles.
 hipError_t launch_energy_z(const DevSystem &s, const BatchArgs &b,
-                           double *const G[4], double *const GJ[4],
+                           double *const G[2], double *const GJ[2],
                            double tai_sign, double *e_slot, double *wcube,
                            hipStream_t st);
 
