@@ -1105,9 +1105,9 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
         check(launch_doubles_tri(s, b, pass == 1, (float *)Gp, ctx->tile, st),
               "doubles (bf16x3) kernel");
       else
-        check(launch_doubles_split(s, b, pass == 1, (float *)Gp,
-                                   precision == ATRIP_SPLIT_FP32, ctx->tile,
-                                   st),
+        check((precision == ATRIP_SPLIT_FP32 ? launch_doubles_split
+                                             : launch_doubles_fp32)(
+                  s, b, pass == 1, (float *)Gp, ctx->tile, st),
               "doubles (FP32 products) kernel");
     }
     if (timing) check(hipEventRecord(ev.e[1], st), "event");

@@ -231,6 +231,20 @@ __device__ __forceinline__ void f64_columns(const DoublesParams &P,
   f64_wave<TM, TN, WR, FM, FN>(P, T, No, lane, wm, wn);
 }
 
+// Dispatch on the wave's occupied row fragments, m <= FM of them.
+template <int TM, int TN, int WR, int FM, int FN>
+__device__ __forceinline__ void f64_rows(const DoublesParams &P,
+                                         const TileWork &T, int No, int lane,
+                                         int wm, int wn, int m, int n) {
+  if constexpr (FM > 1) {
+    if (m < FM) {
+      f64_rows<TM, TN, WR, FM - 1, FN>(P, T, No, lane, wm, wn, m, n);
+      return;
+    }
+  }
+  f64_columns<TM, TN, WR, FM, FN>(P, T, No, lane, wm, wn, n);
+}
+
 template <int FM, int FN, int WR>
 __global__ __launch_bounds__(128 * WR, 2) void doubles_f64_kernel(
     DoublesParams P) {
@@ -249,18 +263,14 @@ __global__ __launch_bounds__(128 * WR, 2) void doubles_f64_kernel(
   const int wm = WR == 2 ? wave >> 1 : (wave + 2 * wn) & 3;
   // Fragments of this wave that hold rows and columns.  Tiles at the edges
   // of the GEMM run the instance of their size instead of the whole tile on
-  // padding: every column count, the row count rounded up to half the tile
-  // (rows have one edge per A-pair, columns one per pair and valid third
-  // index; one instance with per-fragment branches doubled the accumulators).
+  // padding (one instance with per-fragment branches doubled the
+  // accumulators; with only whole and half row counts No=14, 12.25 row
+  // fragments, paid for 16 instead of 14).
   constexpr int RF = (2 * FM + WR - 1) / WR;  // row fragments of a wave
   const int m = occupied(P.N2 - (int64_t)T.mt * 32 * FM, wm, WR, 16, 2 * FM);
   const int n = occupied(T.ncols - (int64_t)T.nt * 32 * FN, wn, 2, 16, 2 * FN);
   if (!m || !n) return;
-  constexpr int H = (RF + 1) / 2;
-  if (m > H)
-    f64_columns<FM, FN, WR, RF, FN>(P, T, No, lane, wm, wn, n);
-  else
-    f64_columns<FM, FN, WR, H, FN>(P, T, No, lane, wm, wn, n);
+  f64_rows<FM, FN, WR, RF, FN>(P, T, No, lane, wm, wn, m, n);
 }
 
 }  // namespace

@@ -19,6 +19,11 @@
 // singles, the energy and all sums stay FP64 (energy.hip).
 #include "doubles_common.hpp"
 
+#ifndef ATRIP_SPLIT_CORR
+#define ATRIP_SPLIT_CORR true
+#define ATRIP_SPLIT_LAUNCH launch_doubles_split
+#endif
+
 namespace atrip_amd {
 namespace {
 
@@ -219,6 +224,20 @@ __device__ __forceinline__ void split_columns(const SplitParams &P, const TileWo
   split_wave<TM, TN, FM, FN, CORR>(P, T, No, lane, wm, wn);
 }
 
+// Dispatch on the wave's occupied row fragments, m <= FM of them.
+template <int TM, int TN, int FM, int FN, bool CORR>
+__device__ __forceinline__ void split_rows(const SplitParams &P, const TileWork &T, int No,
+                                         int lane, int wm, int wn, int m,
+                                         int n) {
+  if constexpr (FM > 1) {
+    if (m < FM) {
+      split_rows<TM, TN, FM - 1, FN, CORR>(P, T, No, lane, wm, wn, m, n);
+      return;
+    }
+  }
+  split_columns<TM, TN, FM, FN, CORR>(P, T, No, lane, wm, wn, n);
+}
+
 template <int FM, int FN, bool CORR>
 __global__ __launch_bounds__(256) void doubles_split_kernel(SplitParams P) {
   const int No = (int)P.No;
@@ -231,18 +250,14 @@ __global__ __launch_bounds__(256) void doubles_split_kernel(SplitParams P) {
   const int m = occupied(P.N2 - (int64_t)T.mt * 64 * FM, wm, 2, 32, 2 * FM);
   const int n = occupied(T.ncols - (int64_t)T.nt * 64 * FN, wn, 2, 32, 2 * FN);
   if (!m || !n) return;
-  constexpr int H = (FM + 1) / 2;
-  if (m > H)
-    split_columns<FM, FN, FM, FN, CORR>(P, T, No, lane, wm, wn, n);
-  else
-    split_columns<FM, FN, H, FN, CORR>(P, T, No, lane, wm, wn, n);
+  split_rows<FM, FN, FM, FN, CORR>(P, T, No, lane, wm, wn, m, n);
 }
 
 }  // namespace
 
-hipError_t launch_doubles_split(const DevSystem &s, const BatchArgs &b,
-                                bool use_j, float *G, bool corrections,
-                                int tile, hipStream_t st) {
+// (compiled once per form, in parallel: doubles_fp32.hip includes this file)
+hipError_t ATRIP_SPLIT_LAUNCH(const DevSystem &s, const BatchArgs &b,
+                              bool use_j, float *G, int tile, hipStream_t st) {
   SplitParams P;
   const DevSystem::Split &V = use_j ? s.sV3J : s.sV3;
   const DevSystem::Split &H = use_j ? s.sH3J : s.sH3;
@@ -267,14 +282,9 @@ hipError_t launch_doubles_split(const DevSystem &s, const BatchArgs &b,
   if (grid <= 0) return hipSuccess;
   if (grid > MAX_GRID) return hipErrorInvalidConfiguration;
 #define LAUNCH(A, B)                                                         \
-  if (FM == A && FN == B) {                                                  \
-    if (corrections)                                                         \
-      hipLaunchKernelGGL((doubles_split_kernel<A, B, true>),                 \
-                         dim3((unsigned)grid), dim3(256), 0, st, P);         \
-    else                                                                     \
-      hipLaunchKernelGGL((doubles_split_kernel<A, B, false>),                \
-                         dim3((unsigned)grid), dim3(256), 0, st, P);         \
-  }
+  if (FM == A && FN == B)                                                    \
+    hipLaunchKernelGGL((doubles_split_kernel<A, B, ATRIP_SPLIT_CORR>),       \
+                       dim3((unsigned)grid), dim3(256), 0, st, P);
   LAUNCH(2, 2) LAUNCH(2, 3) LAUNCH(3, 2) LAUNCH(2, 4) LAUNCH(3, 3)
   LAUNCH(2, 5) LAUNCH(3, 5) LAUNCH(4, 4) LAUNCH(3, 4) LAUNCH(4, 3)
 #undef LAUNCH

@@ -212,6 +212,20 @@ __device__ __forceinline__ void tri_columns(const TriParams &P, const TileWork &
   tri_wave<TM, TN, FM, FN>(P, T, No, lane, wm, wn);
 }
 
+// Dispatch on the wave's occupied row fragments, m <= FM of them.
+template <int TM, int TN, int FM, int FN>
+__device__ __forceinline__ void tri_rows(const TriParams &P, const TileWork &T, int No,
+                                         int lane, int wm, int wn, int m,
+                                         int n) {
+  if constexpr (FM > 1) {
+    if (m < FM) {
+      tri_rows<TM, TN, FM - 1, FN>(P, T, No, lane, wm, wn, m, n);
+      return;
+    }
+  }
+  tri_columns<TM, TN, FM, FN>(P, T, No, lane, wm, wn, n);
+}
+
 template <int FM, int FN>
 __global__ __launch_bounds__(256) void doubles_tri_kernel(TriParams P) {
   const int No = (int)P.No;
@@ -224,11 +238,7 @@ __global__ __launch_bounds__(256) void doubles_tri_kernel(TriParams P) {
   const int m = occupied(P.N2 - (int64_t)T.mt * 64 * FM, wm, 2, 32, 2 * FM);
   const int n = occupied(T.ncols - (int64_t)T.nt * 64 * FN, wn, 2, 32, 2 * FN);
   if (!m || !n) return;
-  constexpr int H = (FM + 1) / 2;
-  if (m > H)
-    tri_columns<FM, FN, FM, FN>(P, T, No, lane, wm, wn, n);
-  else
-    tri_columns<FM, FN, H, FN>(P, T, No, lane, wm, wn, n);
+  tri_rows<FM, FN, FM, FN>(P, T, No, lane, wm, wn, m, n);
 }
 
 }  // namespace

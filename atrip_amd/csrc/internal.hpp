@@ -355,12 +355,12 @@ hipError_t launch_doubles_f64(const DevSystem &s, const DevSystem *s2,
                               const BatchArgs &b, bool use_j, double *G,
                               int tile, hipStream_t st);
 
-// Doubles contractions in split FP32.
-// Doubles contractions with FP32 products (class buffers in FP32):
-// corrections = true adds the hi*lo + lo*hi terms (split FP32).
+// Doubles contractions with FP32 products (class buffers in FP32): split FP32
+// (with the hi*lo + lo*hi corrections), and FP32 only.
 hipError_t launch_doubles_split(const DevSystem &s, const BatchArgs &b,
-                                bool use_j, float *G, bool corrections,
-                                int tile, hipStream_t st);
+                                bool use_j, float *G, int tile, hipStream_t st);
+hipError_t launch_doubles_fp32(const DevSystem &s, const BatchArgs &b,
+                               bool use_j, float *G, int tile, hipStream_t st);
 
 // Doubles contractions in bf16x3 (six part products on bf16 MFMA, FP32
 // accumulation, class buffers in FP32).
