@@ -46,12 +46,16 @@ static double n_windows(int64_t Nv, int nb) {
 }
 
 // Modelled cycles of one full window on one workgroup of four waves: the
-// wave tiles of the three classes (per 16-deep K chunk, 4*fm*fn MFMA of 64
-// cycles or the chunk's fm+fn fragment loads, whichever is longer, plus a
-// memory latency per K segment) and the energies (one wave per tuple).
+// wave tiles of the three classes (per 16-deep K chunk the 4*fm*fn MFMA of 64
+// cycles and a share of the chunk's fm+fn fragment loads that the other wave
+// of the SIMD does not hide, plus a memory latency per K segment; a tile at the
+// edge runs the variant of the fragments it holds), the energies (one wave per
+// tuple) and W's traffic.  The load share is fitted to No=12, Nv=100 (3x3 tiles
+// 38.4, 4x2 31.7 TFLOP/s at edge 4) and No=16, Nv=110 (4x2 43.2, 2x2 38.7 at
+// edge 2); its picks at No 4..20 measure within 6 % of the best of 30 choices,
+// where the larger of the two times, charged before, lost 18 % at No=10, Nv=90.
 double window_cycles(int64_t No, int64_t Nv, int nb, int tile,
                      int precision) {
-  const double fm = bfm(tile), fn = bfn(tile);
   // MFMA cycles per 16-deep chunk and 16x16 output fragment: 4 FP64 16x16x4
   // (64 cycles each); 4 FP32 16x16x4 (32 each), plus one bf16 16x16x32 (16)
   // for the split corrections
@@ -59,17 +63,30 @@ double window_cycles(int64_t No, int64_t Nv, int nb, int tile,
                     : precision == ATRIP_SPLIT_FP32 ? 4 * 32.0 + 16.0
                                                     : 4 * 32.0;
   // fragment loads per chunk: 32 B/lane FP64, 16 B FP32 (+16 B bf16 pairs)
-  const double ld = precision == ATRIP_FP64 ? 180.0
+  const double ld = precision == ATRIP_FP64 ? 200.0
                     : precision == ATRIP_SPLIT_FP32 ? 180.0 : 120.0;
-  const double N2 = (double)No * No;
-  const double mt = std::ceil(N2 / (16 * fm)), nt = std::ceil(nb * No / (16 * fn));
-  const double subs = 3.0 * nb * nb * mt * nt;
   const double chunks = (2.0 * pad16(Nv) + 2.0 * pad16(No)) / 16.0;
-  const double per_chunk = std::max(mf * fm * fn, ld * (fm + fn));
-  const double sub = 4 * 1200.0 + chunks * per_chunk + 300.0 * fm * fn;
+  auto cost = [&](int nr, int nc) {
+    const int v = fitting_tile(tile, nr, nc);
+    const double m = bfm(v), n = bfn(v);
+    return 4 * 1200.0 + chunks * (mf * m * n + ld * (m + n)) + 300.0 * m * n;
+  };
+  const int fm = bfm(tile), fn = bfn(tile);
+  const int64_t R = (No * No + 15) / 16, C = (nb * No + 15) / 16;
+  double pair = 0.0;  // a pair's tiles: full ones, then the edges
+  for (int64_t r = 0; r < R; r += fm)
+    pair += (double)(C / fn) * cost((int)std::min<int64_t>(fm, R - r), fn) +
+            (C % fn ? cost((int)std::min<int64_t>(fm, R - r), (int)(C % fn))
+                    : 0.0);
   const double npts = (double)No * (No + 1) * (No + 2) / 6.0;
   const double energy = nb * nb * nb / 4.0 * (std::ceil(npts / 64.0) * 400.0 + 2000.0);
-  return subs * sub / 4.0 + energy;
+  // W of the window: three passes of stores and atomic adds and one of loads,
+  // from memory where the workgroups' windows (two a CU) exceed the 256 MB
+  // last-level cache.  No=12, Nv=100, 3x3 tiles: edge 4 (0.45 GB in all) 38.4
+  // TFLOP/s, edge 8 (3.6 GB) 33.4; No=14, Nv=120: 33.9 and 23.3.
+  const double welems = (double)nb * nb * nb * No * No * No;
+  const double miss = 1.0 - std::min(1.0, 256e6 / (512.0 * 8.0 * welems));
+  return 3.0 * nb * nb * pair / 4.0 + energy + 2.0 * miss * welems;
 }
 
 bool nb_fits(int64_t No, int nb, int64_t scratch_mb, int grid) {

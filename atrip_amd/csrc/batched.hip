@@ -6,12 +6,13 @@
 // host scheduler chose, and does everything for its window itself:
 //   1. the doubles contractions (reference src/atrip/Equations.cxx:455-728,
 //      regrouped into the three classes w, v, u of the FP64 doubles kernel),
-//      class by class.  Each of the four waves takes wave tiles of
-//      (16*FM) x (16*FN) outputs (FM, FN per system, from the tuner), runs
-//      the FP64 MFMA K loop with operands straight from global memory and
-//      adds the tile into W of the window's tuples in the workgroup's own
-//      scratch (class w stores, v and u add after a barrier, so W sums the
-//      classes in the fixed order (w + v) + u);
+//      class by class, over the columns of valid tuples only.  Each of the four
+//      waves takes wave tiles of (16*FM) x (16*FN) outputs (FM, FN per system,
+//      from the tuner; a tile at the edge takes the variant of the fragments
+//      it holds), runs the FP64 MFMA K loop with operands straight from
+//      global memory and adds the tile into W of the window's tuples in the
+//      workgroup's own scratch (class w stores, v and u add after a barrier,
+//      so W sums the classes in the fixed order (w + v) + u);
 //   2. singles and energy of each tuple of the window (reference
 //      src/atrip/Equations.cxx:101-238 and :387-426, selection as
 //      src/atrip/Atrip.cxx:636-670), one wave per tuple over the i>=j>=k
@@ -21,6 +22,16 @@
 // systems of the launch, so a system's energy is the same alone and in any
 // mix.  No workgroup waits on another; the loop ends when the counter passes
 // the number of work items.
+//
+// Bound by FP64 MFMA issue at the clock the chip holds under it: the matrix
+// units are busy 64 % of the time at No=12, Nv=120 (window edge 4, 3x3 tiles,
+// 43 TFLOP/s), the rest is what two waves a SIMD do not hide of a wave's setup,
+// W updates and energies.  Three waves a SIMD raise it to 68 % at a lower clock
+// and the same rate.  Before operands were swapped for w and v, W added to by
+// atomics, empty columns left out and a tile's place kept in scalar registers
+// it was 54 % and 37 TFLOP/s; 64 systems of No 4..16, Nv 20..120: 329 ms then,
+// 287 ms now.  Task lists per XCD change nothing (L2 hit rates of operands do
+// not bound it).
 #include "doubles_common.hpp"
 
 namespace atrip_amd {
@@ -49,163 +60,161 @@ __device__ inline double wave_sum(double v) {
   return v;
 }
 
-// B operand row of segment sg at index rr of column tuple (a,b,c), class cl.
-__device__ __forceinline__ const double *bbase(const BSys &S, int cl, int sg, int64_t a,
-                                      int64_t b, int64_t c, int64_t rr) {
-  int64_t u, v;
-  const int which = b_pair(cl, sg, a, b, c, u, v);
-  const double *Bt = which == 0 ? S.V3 : which == 1 ? S.T2N : S.T2TN;
-  return Bt + f64_row((u + S.Nv * v) * S.No + rr, sg < 2 ? S.Kv : S.Ko);
+// n / d for 0 <= n < 2^16, 0 < d <= 64, from r = 1 / d: the quotient of n + 1/2
+// is at least 1 / 128 away from a whole number, far beyond the error of the
+// two FP32 operations, so the integer part is exact.
+__device__ __forceinline__ int small_div(int n, float r) {
+  return (int)(((float)n + 0.5f) * r);
 }
 
-// Adds one wave tile into W (order i + No j + No^2 k).  Class u's column
-// index is i, so its fragment rows are stored as they are (16 consecutive
-// i per row, 128 bytes).  For classes w and v the fragment is first
-// transposed through the wave's 16 x 17 LDS area so that a store
-// instruction covers 16 consecutive rows m (consecutive i) of 4 columns.
-// Per column group the element offsets come first and every old value
-// (classes v and u add) is loaded before any store, the next group's
-// before this group's stores, so the adds wait on memory about once per
-// tile instead of once per element (a load after a store to a possibly
-// aliasing address cannot be moved above it).  Every element
-// of W receives one contribution per class, so within a class the tiles'
-// elements are disjoint.
-// OUT = 8: FP64 MFMA layout D[i][j] in lane j + 16 (i % 4), register i / 4;
-// OUT = 4: FP32 MFMA layout D[i][j] in lane j + 16 (i / 4), register i % 4.
-template <int FM, int FN, int OUT, typename V4>
-__device__ __forceinline__ void store_tile(const V4 (&acc)[FM][FN], int cl,
-                                           int mt, int nt, int64_t No,
-                                           const bool *cvalid,
-                                           const int32_t *cslot,
-                                           const int32_t *crr, double *Gwin,
-                                           bool add, int lane, double *xp) {
-  const int kk = lane >> 4, l16 = lane & 15;
-  const int no = (int)No, n2 = no * no, w3 = n2 * no;
-  int off[2][FM][4];     // element offsets in the window's W, -1 if none
-  double old[2][FM][4];  // their old values (classes v and u)
-  // offsets and old values of column group g into set h
-#define GROUP_LOAD(g, h)                                                       \
-  {                                                                            \
-    if (cl == 2) {                                                             \
-      _Pragma("unroll") for (int f = 0; f < FM; f++)                           \
-          _Pragma("unroll") for (int r = 0; r < 4; r++) {                      \
-        const int row = OUT == 8 ? 4 * r + kk : 4 * kk + r;                    \
-        const int m = mt * 16 * FM + f * 16 + row;                             \
-        const int p = m % no, q = m / no;                                      \
-        off[h][f][r] = cvalid[g] && m < n2                                     \
-                           ? cslot[g] * w3 + crr[g] + no * (p + no * q)        \
-                           : -1;                                               \
-      }                                                                        \
-    } else {                                                                   \
-      _Pragma("unroll") for (int r = 0; r < 4; r++) {                          \
-        const int col = 4 * r + kk;                                            \
-        const int slot = __shfl(cslot[g], col, 64);                            \
-        const int rr = __shfl(crr[g], col, 64);                                \
-        const bool ok = __shfl((int)cvalid[g], col, 64) != 0;                  \
-        _Pragma("unroll") for (int f = 0; f < FM; f++) {                       \
-          const int m = mt * 16 * FM + f * 16 + l16;                           \
-          const int p = m % no, q = m / no;                                    \
-          const int o =                                                        \
-              cl == 0 ? p + no * (q + no * rr) : p + no * (rr + no * q);       \
-          off[h][f][r] = ok && m < n2 ? slot * w3 + o : -1;                    \
-        }                                                                      \
-      }                                                                        \
-    }                                                                          \
-    if (add)                                                                   \
-      _Pragma("unroll") for (int f = 0; f < FM; f++)                           \
-          _Pragma("unroll") for (int r = 0; r < 4; r++) old[h][f][r] =         \
-              Gwin[off[h][f][r] >= 0 ? off[h][f][r] : 0];                      \
+// One A-pair of a class in a window.  The valid third indices of a pair are
+// consecutive, y0 .. y0 + ncols / No - 1, and only their columns exist:
+// column n is index n % No of third index y0 + n / No, of the window slot
+// slot0 + (n / No) step.
+struct Sub {
+  int32_t x1, x2, y0;  // w (a,b), v (a,c), u (b,c); first valid third index
+  int ncols, slot0, step;
+};
+__device__ __forceinline__ Sub sub_work(const BSys &S, const BTask &T, int cl,
+                                        int o1, int o2) {
+  const int nb = S.nb, Nv = (int)S.Nv;
+  const int a0 = T.al * nb, b0 = T.be * nb, c0 = T.ga * nb;
+  Sub u;
+  int hi;
+  bool ok;
+  if (cl == 0) {
+    u.x1 = a0 + o1; u.x2 = b0 + o2;
+    u.y0 = max(c0, u.x2 + (u.x1 == u.x2));
+    hi = min(c0 + nb, Nv);
+    ok = u.x1 <= u.x2 && u.x2 < Nv;
+    u.step = 1;
+    u.slot0 = (o1 * nb + o2) * nb + (u.y0 - c0);
+  } else if (cl == 1) {
+    u.x1 = a0 + o1; u.x2 = c0 + o2;
+    u.y0 = max(b0, u.x1);
+    hi = min(b0 + nb, u.x2 + 1);
+    ok = u.x1 < u.x2 && u.x2 < Nv;
+    u.step = nb;
+    u.slot0 = (o1 * nb + (u.y0 - b0)) * nb + o2;
+  } else {
+    u.x1 = b0 + o1; u.x2 = c0 + o2;
+    u.y0 = a0;
+    hi = min(a0 + nb, u.x1 + (u.x1 != u.x2));
+    ok = u.x1 <= u.x2 && u.x2 < Nv;
+    u.step = nb * nb;
+    u.slot0 = o1 * nb + o2;
   }
-  GROUP_LOAD(0, 0)
+  u.ncols = ok && hi > u.y0 ? (hi - u.y0) * (int)S.No : 0;
+  return u;
+}
+
+// A lane's columns and rows of a wave tile (fragment f / g: row or column
+// 16 f + lane % 16 behind the tile's first), clamped into the GEMM.
+template <int FM, int FN>
+struct TileAt {
+  // column: index of the third index behind y0 in the upper, column index in
+  // the lower half; row: p in the upper, q in the lower half
+  uint32_t col[FN], row[FM];
+  __device__ __forceinline__ void set(int no, const Sub &u, int r0, int c0,
+                                      int l16) {
+    const float r = 1.0f / (float)no;
 #pragma unroll
-  for (int g = 0; g < FN; g++) {
-    const int h = g & 1;
-    // the next group's old values are requested before this group's stores
-    if (g + 1 < FN) GROUP_LOAD(g + 1, h ^ 1)
+    for (int g = 0; g < FN; g++) {
+      const int n = min((c0 + g) * 16 + l16, u.ncols - 1), t = small_div(n, r);
+      col[g] = (uint32_t)t << 16 | (uint32_t)(n - t * no);
+    }
 #pragma unroll
     for (int f = 0; f < FM; f++) {
-      double v[4];
-      if (cl == 2) {
-#pragma unroll
-        for (int r = 0; r < 4; r++) v[r] = (double)acc[f][g][r];
-      } else {
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const int row = OUT == 8 ? 4 * r + kk : 4 * kk + r;
-          xp[row * 17 + l16] = (double)acc[f][g][r];
-        }
-        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): LDS writes done
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int r = 0; r < 4; r++) v[r] = xp[l16 * 17 + 4 * r + kk];
-        __builtin_amdgcn_s_waitcnt(0xC07F);  // reads done before the next tile
-        __builtin_amdgcn_wave_barrier();
-      }
-#pragma unroll
-      for (int r = 0; r < 4; r++)
-        if (off[h][f][r] >= 0)
-          Gwin[off[h][f][r]] = add ? old[h][f][r] + v[r] : v[r];
+      const int m = min((r0 + f) * 16 + l16, no * no - 1), q = small_div(m, r);
+      row[f] = (uint32_t)(m - q * no) << 16 | (uint32_t)q;
     }
   }
-#undef GROUP_LOAD
-}
+};
 
-// One wave tile: rows mt*16*FM .. of the No^2 (p,q) rows, columns
-// nt*16*FN .. of the nb*No (t, r) columns of class cl at A-pair (o1,o2).
-// W of window slot s sits at Gwin + s*No^3 in the order i + No j + No^2 k.
-template <int FM, int FN>
-__device__ __forceinline__ void wave_tile(const BSys &S, int cl, int al,
-                                          int be, int ga, int o1, int o2,
-                                          int mt, int nt, double *Gwin,
-                                          bool add, int lane, double *xp) {
-  const int nb = S.nb;
-  const int64_t No = S.No, Nv = S.Nv, N2 = No * No, Kv = S.Kv, Ko = S.Ko;
-  const int kk = lane >> 4, l16 = lane & 15;
-  int32_t ca[FN], cb[FN], cc[FN], cslot[FN], crr[FN];
-  bool cvalid[FN];
-  bool any = false;
+// Adds one wave tile into W (order i + No j + No^2 k).  W's offset is a row
+// part plus a column part: class w m + No^2 r, class v p + No^2 q + No r, class
+// u No m + r.  The lanes of a fragment run along the index that is consecutive
+// in W: the rows for w and v (SW, the MFMA's operands swapped: the fragment
+// then comes out transposed and nothing passes through LDS), the column
+// index for u.  Class w stores; v and u add with atomics that return nothing
+// and are carried out in L2, so a wave never waits for old values: with loads
+// and stores instead a 3x3 tile at No=12, Nv=120 spent 22 of its 101 k cycles
+// here.  Every element receives one contribution per class and the
+// classes are separated by barriers, so the sum is (w + v) + u whatever the
+// order of the tiles.
+// OUT = 8: FP64 MFMA layout D[i][j] in lane j + 16 (i % 4), register i / 4;
+// OUT = 4: FP32 MFMA layout D[i][j] in lane j + 16 (i / 4), register i % 4.
+template <bool SW, int OUT, int FM, int FN, typename V4>
+__device__ __forceinline__ void store_tile(const V4 (&acc)[FM][FN],
+                                           const TileAt<FM, FN> &at,
+                                           const Sub &u, int cl, int r0, int c0,
+                                           int no, double *Gwin, int lane) {
+  const int kk = lane >> 4, l16 = lane & 15, n2 = no * no;
+  int wcol[FN], wrow[FM];
 #pragma unroll
   for (int g = 0; g < FN; g++) {
-    const int64_t n = (int64_t)nt * 16 * FN + g * 16 + l16;
-    const int t = (int)(n / No);
-    crr[g] = (int32_t)(n % No);
-    int64_t a, b, c, slot;
-    class_tuple(cl, al, be, ga, nb, o1, o2, t, a, b, c, slot);
-    const bool ok = t < nb && tuple_ok(Nv, a, b, c);
-    cvalid[g] = ok;
-    any |= ok;
-    if (!ok) { a = 0; b = 0; c = 0; crr[g] = 0; slot = 0; }
-    ca[g] = (int32_t)a; cb[g] = (int32_t)b; cc[g] = (int32_t)c;
-    cslot[g] = (int32_t)slot;
+    const int t = at.col[g] >> 16, rr = at.col[g] & 0xffff;
+    wcol[g] = (c0 + g) * 16 + l16 < u.ncols
+                  ? (u.slot0 + t * u.step) * n2 * no +
+                        rr * (cl == 0 ? n2 : cl == 1 ? no : 1)
+                  : -1;
   }
-  if (!__any(any)) return;
-
-  int64_t x1, x2;
-  class_pair(cl, al, be, ga, nb, o1, o2, x1, x2);
-  if (x1 >= Nv) x1 = Nv - 1;
-  if (x2 >= Nv) x2 = Nv - 1;
-  int32_t rowS[FM], rowW[FM];
+  if (SW) {
 #pragma unroll
-  for (int f = 0; f < FM; f++) {
-    int64_t m = (int64_t)mt * 16 * FM + f * 16 + l16;
-    if (m >= N2) m = N2 - 1;
-    rowS[f] = (int32_t)m;
-    rowW[f] = (int32_t)(m / No + No * (m % No));
+    for (int f = 0; f < FM; f++) {
+      const int p = at.row[f] >> 16, q = at.row[f] & 0xffff;
+      wrow[f] = (r0 + f) * 16 + l16 < n2 ? p + (cl == 0 ? no : n2) * q : -1;
+    }
   }
+#pragma unroll
+  for (int g = 0; g < FN; g++) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int i = OUT == 8 ? 4 * r + kk : 4 * kk + r;
+      const int col = SW ? __shfl(wcol[g], i, 64) : wcol[g];
+#pragma unroll
+      for (int f = 0; f < FM; f++) {
+        const int m = (r0 + f) * 16 + i;
+        const int row = SW ? wrow[f] : m < n2 ? no * m : -1;
+        if (row >= 0 && col >= 0) {
+          const double v = (double)acc[f][g][r];
+          if (cl > 0)
+            unsafeAtomicAdd(Gwin + row + col, v);
+          else
+            Gwin[row + col] = v;
+        }
+      }
+    }
+  }
+}
+
+// One wave tile: row fragments r0 .. of the No^2 (p,q) rows, column fragments
+// c0 .. of an A-pair's columns.  W of window slot s sits at Gwin + s*No^3 in the
+// order i + No j + No^2 k.
+template <bool SW, int FM, int FN>
+__device__ __forceinline__ void wave_tile(const BSys &S, const Sub &u, int cl,
+                                          int r0, int c0, double *Gwin,
+                                          int lane) {
+  const int64_t No = S.No, Nv = S.Nv, N2 = No * No, Kv = S.Kv, Ko = S.Ko;
+  const int kk = lane >> 4, l16 = lane & 15;
+  TileAt<FM, FN> at;
+  at.set((int)No, u, r0, c0, l16);
 
   d4 acc[FM][FN];
 #pragma unroll
   for (int f = 0; f < FM; f++)
 #pragma unroll
     for (int g = 0; g < FN; g++) acc[f][g] = d4{0.0, 0.0, 0.0, 0.0};
-  const double *ap[FM], *bp[FN];
+  uint32_t ao[FM], bo[FN];  // byte offsets from the uniform bases ap, bp
   d2 a0[FM], b0[FN], a1[FM], b1[FN];
 #define LOAD(AV, BV, C)                                                 \
   {                                                                     \
+    const char *ac_ = ap + (int64_t)1024 * (C);                         \
+    const char *bc_ = bp + (int64_t)1024 * (C);                         \
     _Pragma("unroll") for (int f = 0; f < FM; f++) AV[f] =              \
-        *(const d2 *)(ap[f] + 128 * (C));                               \
+        *(const d2 *)(ac_ + ao[f]);                                     \
     _Pragma("unroll") for (int g = 0; g < FN; g++) BV[g] =              \
-        *(const d2 *)(bp[g] + 128 * (C));                               \
+        *(const d2 *)(bc_ + bo[g]);                                     \
     __builtin_amdgcn_sched_barrier(0);                                  \
   }
 #define COMPUTE(AV, BV)                                                   \
@@ -213,8 +222,9 @@ __device__ __forceinline__ void wave_tile(const BSys &S, int cl, int al,
     _Pragma("unroll") for (int s = 0; s < 2; s++)                         \
         _Pragma("unroll") for (int f = 0; f < FM; f++)                    \
             _Pragma("unroll") for (int g = 0; g < FN; g++) acc[f][g] =    \
-                __builtin_amdgcn_mfma_f64_16x16x4f64(AV[f][s], BV[g][s],  \
-                                                     acc[f][g], 0, 0, 0); \
+                __builtin_amdgcn_mfma_f64_16x16x4f64(                     \
+                    SW ? BV[g][s] : AV[f][s], SW ? AV[f][s] : BV[g][s],   \
+                    acc[f][g], 0, 0, 0);                                  \
   }
   // segments: 0 T3[x1] straight, 1 T3[x2] swapped, 2 H3[x2] straight,
   //           3 H3[x1] swapped, in 8-deep chunks (one operand tile each).
@@ -228,13 +238,30 @@ __device__ __forceinline__ void wave_tile(const BSys &S, int cl, int al,
     const double *As = sg < 2 ? S.T3s : S.H3s;  // null: the straight array
     const bool sw = (sg & 1) && As;
     const double *Ab = sw ? As : sg < 2 ? S.T3 : S.H3;
-    const int64_t xr = (sg == 0 || sg == 3 ? x1 : x2) * N2p;
+    const int64_t xr = (sg == 0 || sg == 3 ? u.x1 : u.x2) * N2p;
+    const char *ap = (const char *)(Ab + f64_row(xr, K_));
 #pragma unroll
-    for (int f = 0; f < FM; f++)
-      ap[f] = Ab + f64_row(xr + ((sg & 1) && !sw ? rowW[f] : rowS[f]), K_) + 32 * kk;
+    for (int f = 0; f < FM; f++) {
+      const uint32_t p = at.row[f] >> 16, q = at.row[f] & 0xffff;
+      const uint32_t m = (sg & 1) && !sw ? q + (uint32_t)No * p : p + (uint32_t)No * q;
+      ao[f] = 8 * (uint32_t)f64_row(m, K_) + 256 * kk;
+    }
+    // the columns' rows lie within seven third indices of the first one's, so
+    // 32 bits hold the offsets for any system that fits the device
+    int which;
+    const int64_t row0 = b_row(cl, sg, u.x1, u.x2, u.y0, 0, Nv, No, which);
+    const int64_t rstep =
+        b_row(cl, sg, u.x1, u.x2, u.y0 + 1, 0, Nv, No, which) - row0;
+    const char *bp =
+        (const char *)((which == 0 ? S.V3 : which == 1 ? S.T2N : S.T2TN) +
+                       f64_row(row0 & ~15LL, K_));
 #pragma unroll
-    for (int g = 0; g < FN; g++)
-      bp[g] = bbase(S, cl, sg, ca[g], cb[g], cc[g], crr[g]) + 32 * kk;
+    for (int g = 0; g < FN; g++) {
+      const uint32_t r = (uint32_t)(row0 & 15) +
+                         (at.col[g] >> 16) * (uint32_t)rstep +
+                         (at.col[g] & 0xffff);
+      bo[g] = (r >> 4) * (128 * (uint32_t)K_) + 16 * (r & 15) + 256 * kk;
+    }
     const int last = (int)(((sg < 2 ? Nv : No) + 7) / 8) - 1;
     LOAD(a0, b0, 0);
     for (int c = 0;; c += 2) {
@@ -248,8 +275,7 @@ __device__ __forceinline__ void wave_tile(const BSys &S, int cl, int al,
   }
 #undef LOAD
 #undef COMPUTE
-  store_tile<FM, FN, 8>(acc, cl, mt, nt, No, cvalid, cslot, crr, Gwin, add,
-                        lane, xp);
+  store_tile<SW, 8>(acc, at, u, cl, r0, c0, (int)No, Gwin, lane);
 }
 
 // The same wave tile with FP32 products (mixed forms): hi*hi on
@@ -257,64 +283,31 @@ __device__ __forceinline__ void wave_tile(const BSys &S, int cl, int al,
 // v_mfma_f32_16x16x32_bf16 per 16-deep chunk (each lane group pairs
 // [bf16(hi_a), lo_a] with [lo_b, bf16(hi_b)] over its four kappa), FP32
 // accumulation; the tile is widened to FP64 when it is added into W.
-template <int FM, int FN, bool CORR>
+template <bool SW, int FM, int FN, bool CORR>
 __device__ __forceinline__ void wave_tile_split(const BSys &S, const BSplit &X,
-                                                int cl, int al, int be, int ga,
-                                                int o1, int o2, int mt, int nt,
-                                                double *Gwin, bool add,
-                                                int lane, double *xp) {
-  const int nb = S.nb;
+                                                const Sub &u, int cl, int r0,
+                                                int c0, double *Gwin, int lane) {
   const int64_t No = S.No, Nv = S.Nv, N2 = No * No, Kv = S.Kv, Ko = S.Ko;
   const int kk = lane >> 4, l16 = lane & 15;
-  int32_t ca[FN], cb[FN], cc[FN], cslot[FN], crr[FN];
-  bool cvalid[FN];
-  bool any = false;
-#pragma unroll
-  for (int g = 0; g < FN; g++) {
-    const int64_t n = (int64_t)nt * 16 * FN + g * 16 + l16;
-    const int t = (int)(n / No);
-    crr[g] = (int32_t)(n % No);
-    int64_t a, b, c, slot;
-    class_tuple(cl, al, be, ga, nb, o1, o2, t, a, b, c, slot);
-    const bool ok = t < nb && tuple_ok(Nv, a, b, c);
-    cvalid[g] = ok;
-    any |= ok;
-    if (!ok) { a = 0; b = 0; c = 0; crr[g] = 0; slot = 0; }
-    ca[g] = (int32_t)a; cb[g] = (int32_t)b; cc[g] = (int32_t)c;
-    cslot[g] = (int32_t)slot;
-  }
-  if (!__any(any)) return;
-
-  int64_t x1, x2;
-  class_pair(cl, al, be, ga, nb, o1, o2, x1, x2);
-  if (x1 >= Nv) x1 = Nv - 1;
-  if (x2 >= Nv) x2 = Nv - 1;
-  int32_t rowS[FM], rowW[FM];
-#pragma unroll
-  for (int f = 0; f < FM; f++) {
-    int64_t m = (int64_t)mt * 16 * FM + f * 16 + l16;
-    if (m >= N2) m = N2 - 1;
-    rowS[f] = (int32_t)m;
-    rowW[f] = (int32_t)(m / No + No * (m % No));
-  }
+  TileAt<FM, FN> at;
+  at.set((int)No, u, r0, c0, l16);
   f4 acc[FM][FN];
 #pragma unroll
   for (int f = 0; f < FM; f++)
 #pragma unroll
     for (int g = 0; g < FN; g++) acc[f][g] = f4{0.f, 0.f, 0.f, 0.f};
-  const float *aph[FM], *bph[FN];
-  const __bf16 *apc[FM], *bpc[FN];
+  uint32_t ao[FM], bo[FN];  // element offsets from the uniform bases
   f4 ah0[FM], bh0[FN], ah1[FM], bh1[FN];
   bf4 ac0[FM], bc0[FN], ac1[FM], bc1[FN];
 #define LOAD(AH, AC, BH, BC, KOFF)                                          \
   {                                                                         \
     _Pragma("unroll") for (int f = 0; f < FM; f++) {                        \
-      AH[f] = *(const f4 *)(aph[f] + (KOFF));                               \
-      if constexpr (CORR) AC[f] = *(const bf4 *)(apc[f] + (KOFF));         \
+      AH[f] = *(const f4 *)(aph + (KOFF) + ao[f]);                          \
+      if constexpr (CORR) AC[f] = *(const bf4 *)(apc + (KOFF) + ao[f]);     \
     }                                                                       \
     _Pragma("unroll") for (int g = 0; g < FN; g++) {                        \
-      BH[g] = *(const f4 *)(bph[g] + (KOFF));                               \
-      if constexpr (CORR) BC[g] = *(const bf4 *)(bpc[g] + (KOFF));         \
+      BH[g] = *(const f4 *)(bph + (KOFF) + bo[g]);                          \
+      if constexpr (CORR) BC[g] = *(const bf4 *)(bpc + (KOFF) + bo[g]);     \
     }                                                                       \
     __builtin_amdgcn_sched_barrier(0);                                      \
   }
@@ -323,8 +316,9 @@ __device__ __forceinline__ void wave_tile_split(const BSys &S, const BSplit &X,
     _Pragma("unroll") for (int s = 0; s < 4; s++)                           \
         _Pragma("unroll") for (int f = 0; f < FM; f++)                      \
             _Pragma("unroll") for (int g = 0; g < FN; g++) acc[f][g] =      \
-                __builtin_amdgcn_mfma_f32_16x16x4f32(AH[f][s], BH[g][s],    \
-                                                     acc[f][g], 0, 0, 0);   \
+                __builtin_amdgcn_mfma_f32_16x16x4f32(                       \
+                    SW ? BH[g][s] : AH[f][s], SW ? AH[f][s] : BH[g][s],     \
+                    acc[f][g], 0, 0, 0);                                    \
     if constexpr (CORR) {                                                   \
       bf8 ca_[FM], cb_[FN];                                                 \
       _Pragma("unroll") for (int f = 0; f < FM; f++) ca_[f] =               \
@@ -333,8 +327,9 @@ __device__ __forceinline__ void wave_tile_split(const BSys &S, const BSplit &X,
           corr_b(BH[g], BC[g]);                                             \
       _Pragma("unroll") for (int f = 0; f < FM; f++)                        \
           _Pragma("unroll") for (int g = 0; g < FN; g++) acc[f][g] =        \
-              __builtin_amdgcn_mfma_f32_16x16x32_bf16(ca_[f], cb_[g],       \
-                                                      acc[f][g], 0, 0, 0);  \
+              __builtin_amdgcn_mfma_f32_16x16x32_bf16(                      \
+                  SW ? cb_[g] : ca_[f], SW ? ca_[f] : cb_[g], acc[f][g], 0, \
+                  0, 0);                                                    \
     }                                                                       \
   }
   // per-segment pipelines: one pipeline across the segments (as in
@@ -343,26 +338,28 @@ __device__ __forceinline__ void wave_tile_split(const BSys &S, const BSplit &X,
 #pragma unroll 1
   for (int sg = 0; sg < 4; sg++) {
     const int64_t K_ = sg < 2 ? Kv : Ko;
-    const int64_t xa = (sg == 0 || sg == 3) ? x1 : x2;
-    const int64_t abase = xa * N2 * K_;
-    const float *Ah = (sg < 2 ? X.T3h : X.H3h) + abase;
-    const __bf16 *Ac = (const __bf16 *)(sg < 2 ? X.T3l : X.H3l) + abase;
+    const int64_t abase = ((sg == 0 || sg == 3) ? u.x1 : u.x2) * N2 * K_;
+    const float *aph = (sg < 2 ? X.T3h : X.H3h) + abase;
+    const __bf16 *apc = (const __bf16 *)(sg < 2 ? X.T3l : X.H3l) + abase;
 #pragma unroll
     for (int f = 0; f < FM; f++) {
-      const int64_t r = (int64_t)((sg & 1) ? rowW[f] : rowS[f]) * K_;
-      aph[f] = Ah + r + 4 * kk;
-      apc[f] = Ac + r + 4 * kk;
+      const uint32_t p = at.row[f] >> 16, q = at.row[f] & 0xffff;
+      ao[f] = (sg & 1 ? q + (uint32_t)No * p : p + (uint32_t)No * q) * (uint32_t)K_ + 4 * kk;
     }
+    int which;
+    const int64_t row0 = b_row(cl, sg, u.x1, u.x2, u.y0, 0, Nv, No, which);
+    const int64_t rstep =
+        b_row(cl, sg, u.x1, u.x2, u.y0 + 1, 0, Nv, No, which) - row0;
+    const float *bph =
+        (which == 0 ? X.V3h : which == 1 ? X.T2Nh : X.T2TNh) + row0 * K_;
+    const __bf16 *bpc =
+        (const __bf16 *)(which == 0 ? X.V3l : which == 1 ? X.T2Nl : X.T2TNl) +
+        row0 * K_;
 #pragma unroll
-    for (int g = 0; g < FN; g++) {
-      int64_t u, v;
-      const int wh = b_pair(cl, sg, ca[g], cb[g], cc[g], u, v);
-      const int64_t c = ((u + Nv * v) * No + crr[g]) * K_;
-      const float *Bh = wh == 0 ? X.V3h : wh == 1 ? X.T2Nh : X.T2TNh;
-      const uint16_t *Bc = wh == 0 ? X.V3l : wh == 1 ? X.T2Nl : X.T2TNl;
-      bph[g] = Bh + c + 4 * kk;
-      bpc[g] = (const __bf16 *)Bc + c + 4 * kk;
-    }
+    for (int g = 0; g < FN; g++)
+      bo[g] = ((at.col[g] >> 16) * (uint32_t)rstep + (at.col[g] & 0xffff)) *
+                  (uint32_t)K_ +
+              4 * kk;
     const int64_t last = K_ - KCHUNK;
     LOAD(ah0, ac0, bh0, bc0, 0);
     for (int64_t k0 = 0;; k0 += 2 * KCHUNK) {
@@ -377,8 +374,7 @@ __device__ __forceinline__ void wave_tile_split(const BSys &S, const BSplit &X,
 #undef LOAD
 #undef COMPUTE
 
-  store_tile<FM, FN, 4>(acc, cl, mt, nt, No, cvalid, cslot, crr, Gwin, add,
-                        lane, xp);
+  store_tile<SW, 4>(acc, at, u, cl, r0, c0, (int)No, Gwin, lane);
 }
 
 // Energy of tuple (a,b,c) from its W (order i + No j + No^2 k), by one
@@ -459,8 +455,9 @@ __global__ __launch_bounds__(256, 2) void batched_kernel(BatchedLaunch P) {
   __shared__ int task_sh;
   __shared__ double etup[512];
   __shared__ double tsing[4][3][BMAX_NO];
-  __shared__ double xpose[4][16 * 17];  // per-wave tile transposition
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  // uniform, so that a wave tile's place is worked out in scalar registers
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   double *Gwin = P.scratch + (int64_t)blockIdx.x * P.scratch_stride;
 #pragma unroll 1
   for (;;) {
@@ -478,28 +475,33 @@ __global__ __launch_bounds__(256, 2) void batched_kernel(BatchedLaunch P) {
     const int nb = S.nb, nb3 = nb * nb * nb;
     const int64_t No = S.No, N2 = No * No;
     const int fm = bfm(S.tile), fn = bfn(S.tile);
-    const int mtiles = (int)((N2 + 16 * fm - 1) / (16 * fm));
+    const int rfrags = (int)((N2 + 15) / 16);
+    const int mtiles = (rfrags + fm - 1) / fm;
     const int ntiles = (int)((nb * No + 16 * fn - 1) / (16 * fn));
     const int nsub = nb * nb * mtiles * ntiles;
 
 #pragma unroll 1
     for (int cl = 0; cl < 3; cl++) {
 #pragma unroll 1
-      for (int u = wave; u < nsub; u += 4) {
-        const int nt = u % ntiles, mt = (u / ntiles) % mtiles;
-        const int pair = u / (ntiles * mtiles);
-        const int o1 = pair / nb, o2 = pair % nb;
-        switch (S.tile) {
-#define TILE_CASE(V)                                                       \
-  case V:                                                                  \
-    if constexpr (PREC == ATRIP_FP64)                                      \
-      wave_tile<bfm(V), bfn(V)>(S, cl, T.al, T.be, T.ga, o1, o2, mt, nt,   \
-                                Gwin, cl > 0, lane, xpose[wave]);          \
-    else                                                                   \
-      wave_tile_split<bfm(V), bfn(V), PREC == ATRIP_SPLIT_FP32>(           \
-          S, X, cl, T.al, T.be, T.ga, o1, o2, mt, nt, Gwin, cl > 0, lane,  \
-          xpose[wave]);                                                    \
+      for (int q = wave; q < nsub; q += 4) {
+        const int nt = q % ntiles, mt = (q / ntiles) % mtiles;
+        const int pair = q / (ntiles * mtiles);
+        const Sub u = sub_work(S, T, cl, pair / nb, pair % nb);
+        const int r0 = mt * fm, c0 = nt * fn;
+        const int nc = (u.ncols + 15) / 16 - c0;
+        if (nc <= 0) continue;
+        const int v = fitting_tile(S.tile, min(fm, rfrags - r0), min(fn, nc));
+        // classes w and v with the MFMA's operands swapped (see store_tile)
+        switch (v + (cl == 2 ? N_BTILES : 0)) {
+#define TILE_CASE1(V, SW)                                                    \
+  case V + (SW ? 0 : N_BTILES):                                              \
+    if constexpr (PREC == ATRIP_FP64)                                        \
+      wave_tile<SW, bfm(V), bfn(V)>(S, u, cl, r0, c0, Gwin, lane);           \
+    else                                                                     \
+      wave_tile_split<SW, bfm(V), bfn(V), PREC == ATRIP_SPLIT_FP32>(         \
+          S, X, u, cl, r0, c0, Gwin, lane);                                  \
     break;
+#define TILE_CASE(V) TILE_CASE1(V, true) TILE_CASE1(V, false)
           TILE_CASE(0)
           TILE_CASE(1)
           TILE_CASE(2)
@@ -511,11 +513,14 @@ __global__ __launch_bounds__(256, 2) void batched_kernel(BatchedLaunch P) {
           TILE_CASE(8)
           TILE_CASE(9)
 #undef TILE_CASE
+#undef TILE_CASE1
           default:
             break;
         }
       }
-      __syncthreads();  // class done before the next adds to W
+      // the class is in memory before the next adds to it
+      __builtin_amdgcn_s_waitcnt(0);
+      __syncthreads();
     }
 
     // energies, one tuple per wave, each wave through its own slots: the

@@ -8,59 +8,6 @@
 
 namespace atrip_amd {
 
-// Column tuple of class `cl` for A-pair offsets (o1,o2) and third offset t;
-// slot is the tuple's position ((ta*nb + tb)*nb + tc) inside its window.
-__device__ inline void class_tuple(int cl, int64_t al, int64_t be, int64_t ga,
-                                   int nb, int o1, int o2, int t, int64_t &a,
-                                   int64_t &b, int64_t &c, int64_t &slot) {
-  if (cl == 0) {
-    a = al * nb + o1; b = be * nb + o2; c = ga * nb + t;
-    slot = ((int64_t)o1 * nb + o2) * nb + t;
-  } else if (cl == 1) {
-    a = al * nb + o1; b = be * nb + t; c = ga * nb + o2;
-    slot = ((int64_t)o1 * nb + t) * nb + o2;
-  } else {
-    a = al * nb + t; b = be * nb + o1; c = ga * nb + o2;
-    slot = ((int64_t)t * nb + o1) * nb + o2;
-  }
-}
-
-// B operand of segment sg of class cl for column tuple (a,b,c): returns the
-// array (0: V(xy) slabs, 1: -T(xy)[L,n], 2: -T(xy)[n,L]) and its pair (u,v).
-//   class w: P0 V(bc), P1 V(ac), H5 -TAC[L,k], H2 -TBC[L,k]
-//   class v: P3 V(cb), P5 V(ab), H1 -TAB[L,j], H4 -TBC[j,L]
-//   class u: P4 V(ca), P2 V(ba), H0 -TAB[i,L], H3 -TAC[i,L]
-__device__ inline int b_pair(int cl, int sg, int64_t a, int64_t b, int64_t c,
-                             int64_t &u, int64_t &v) {
-  if (cl == 0) {
-    if (sg == 0) { u = b; v = c; return 0; }
-    if (sg == 1) { u = a; v = c; return 0; }
-    if (sg == 2) { u = a; v = c; return 1; }
-    u = b; v = c; return 1;
-  }
-  if (cl == 1) {
-    if (sg == 0) { u = c; v = b; return 0; }
-    if (sg == 1) { u = a; v = b; return 0; }
-    if (sg == 2) { u = a; v = b; return 1; }
-    u = b; v = c; return 2;
-  }
-  if (sg == 0) { u = c; v = a; return 0; }
-  if (sg == 1) { u = b; v = a; return 0; }
-  if (sg == 2) { u = a; v = b; return 2; }
-  u = a; v = c; return 2;
-}
-
-// A-pair (x1, x2) of class cl: w (a,b), v (a,c), u (b,c).  The A operand of
-// segment 0 is T(x1) straight, 1 T(x2) swapped, 2 Vhhh(x2) straight,
-// 3 Vhhh(x1) swapped.
-__device__ inline void class_pair(int cl, int64_t al, int64_t be, int64_t ga,
-                                  int nb, int o1, int o2, int64_t &x1,
-                                  int64_t &x2) {
-  if (cl == 0) { x1 = al * nb + o1; x2 = be * nb + o2; }
-  else if (cl == 1) { x1 = al * nb + o1; x2 = ga * nb + o2; }
-  else { x1 = be * nb + o1; x2 = ga * nb + o2; }
-}
-
 // One workgroup's share of a launch over windows of eb x ec columns (see
 // BatchArgs): a class, an A-pair of its window and one tile of that pair's
 // GEMM.  The GEMM's columns are only those of valid tuples: the valid third
@@ -160,8 +107,12 @@ __device__ __forceinline__ int occupied(int64_t left, int w, int nw, int width,
 }
 
 // Row of segment sg's B operand at column (y, rr) of class cl with A-pair
-// (x1, x2), and its array (0: V(xy) slabs, 1: -T(xy)[L,n], 2: -T(xy)[n,L];
-// the pairs of b_pair, written by the pair and the third index).
+// (x1, x2), and its array (0: V(xy) slabs, 1: -T(xy)[L,n], 2: -T(xy)[n,L]).
+// By segment, with (a,b,c) the column's tuple:
+//   class w: P0 V(bc), P1 V(ac), H5 -TAC[L,k], H2 -TBC[L,k]
+//   class v: P3 V(cb), P5 V(ab), H1 -TAB[L,j], H4 -TBC[j,L]
+//   class u: P4 V(ca), P2 V(ba), H0 -TAB[i,L], H3 -TAC[i,L]
+// against T(x1) straight, T(x2) swapped, Vhhh(x2) straight, Vhhh(x1) swapped.
 __device__ __forceinline__ int64_t b_row(int cl, int sg, int32_t x1,
                                          int32_t x2, int32_t y, int32_t rr,
                                          int64_t Nv, int64_t No, int &which) {
@@ -180,14 +131,6 @@ inline int64_t doubles_grid(WindowArgs &W, int64_t No, int64_t mt_rows,
   W.ntiles = (int)((emax * No + nt_cols - 1) / nt_cols);
   const int64_t units = W.ea * W.eb + W.ea * W.ec + W.eb * W.ec;
   return (units + 7) / 8 * 8 * W.nw * W.mtiles * W.ntiles;
-}
-
-// W position (i,j,k) of GEMM element (row (p,q), column index rr).
-__device__ inline void class_out(int cl, int64_t p, int64_t q, int64_t rr,
-                                 int64_t &i, int64_t &j, int64_t &k) {
-  if (cl == 0) { i = p; j = q; k = rr; }       // "ij|k"
-  else if (cl == 1) { i = p; j = rr; k = q; }  // "ik|j"
-  else { i = rr; j = p; k = q; }               // "jk|i"
 }
 
 // Tile shapes (wave tile FM x FN fragments of 16x16, 2x2 waves) and the

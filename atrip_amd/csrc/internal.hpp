@@ -487,6 +487,20 @@ constexpr __host__ __device__ inline int bfn(int v) {
   return t[v];
 }
 
+// The smallest tile variant within `tile` holding its nr x nc fragments inside
+// the GEMM, for a tile at the edge.
+__host__ __device__ inline int fitting_tile(int tile, int nr, int nc) {
+  int best = bfm(tile) * bfn(tile), v = tile;
+#pragma unroll
+  for (int t = 0; t < N_BTILES; t++)
+    if (bfm(t) >= nr && bfm(t) <= bfm(tile) && bfn(t) >= nc &&
+        bfn(t) <= bfn(tile) && bfm(t) * bfn(t) < best) {
+      best = bfm(t) * bfn(t);
+      v = t;
+    }
+  return v;
+}
+
 // Split-FP32 operands of a system in a batched launch (h = FP32 values,
 // l = bf16(x - h); l unused by the FP32-only form).
 struct BSplit {
