@@ -1131,7 +1131,7 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
       ev.handed = true;
     }
     check(launch_slot_sums(fused && !s.cplx ? (const double *)wcube : nullptr,
-                           b.slots, n_triples(w_blocks(s.No)),
+                           b.slots, energy_parts(s.No, use_j),
                            (double *)e_slot, (double *)partials + 4 * nparts,
                            st),
           "slot sums kernel");

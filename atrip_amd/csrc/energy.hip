@@ -1,15 +1,17 @@
-// Fused singles + energy epilogue of the (T) hot path.
+// Singles + energy epilogue of the (T) hot path, from the three class buffers
+// the doubles kernels wrote (see internal.hpp for their layout; FP64, or FP32
+// for the forms with FP32 or bf16 products).
 //
-// wsum_kernel first sums the three class buffers the doubles kernel wrote
-// (each in its GEMM output order, see internal.hpp; FP64, or FP32 for the
-// single-precision-product forms) into W in FP64, (w + v) + u, re-laid out
-// as 8x8x8 cubes (w_cube).  It works on 16x16x16 bricks staged in LDS, so
-// every class is read along its own fastest index in full 128-byte lines and
-// every cube is written as one 4 KiB run.
+// energy_fused_kernel (a workgroup per block triple of a tuple) and
+// energy_small_kernel (small No: a wave or workgroup per tuple) sum the classes
+// to W in FP64 in LDS, (w + v) + u, and form the energies there; W is never
+// written to memory.  wsum_kernel and energy_kernel do it in two steps, W as
+// 8x8x8 cubes in between (w_cube); complex systems take their class sums from
+// the first.
 //
-// energy_kernel: one workgroup per tuple slot of a window batch.  Z = W +
-// singles is formed in registers (reference src/atrip/Equations.cxx:387-426, with Z copied from W
-// as in src/atrip/Atrip.cxx:899-906), and the energy of the tuple follows
+// Z = W + singles is formed in registers (reference
+// src/atrip/Equations.cxx:387-426, with Z copied from W as in
+// src/atrip/Atrip.cxx:899-906), and the energy of the tuple follows
 // get_energy_distinct / get_energy_same (src/atrip/Equations.cxx:101-238)
 // selected as src/atrip/Atrip.cxx:636-670 does.  The i>=j>=k points are
 // spread over the workgroup; each thread sums its points in a fixed order
@@ -140,6 +142,29 @@ __device__ __forceinline__ void orbit(int B1, int B2, int B3, int nbk,
   }
 }
 
+// A point's energy term from W at its permutations (A ijk, B ikj, C jik, D
+// jki, E kij, F kji; three of them, ijk, jki, kij, when two of a, b, c are
+// equal) and Z = W + singles there: get_energy_distinct / get_energy_same in
+// the reference's expression order.
+__device__ __forceinline__ double term_distinct(
+    double A, double B, double C, double D, double E, double F, double U,
+    double V, double W, double X, double Y, double Z, double denominator,
+    double fac) {
+  const double UXY = U + (X + Y), VWZ = V + (W + Z);
+  const double first = A * U + (B * V + (C * W + (D * X + (E * Y + F * Z))));
+  const double second = (UXY - 2.0 * VWZ) * (A + (D + E));
+  const double third = (VWZ - 2.0 * UXY) * (B + (C + F));
+  const double value = 3.0 * first + (second + third);
+  return ((2.0 * value) / denominator) * fac;
+}
+__device__ __forceinline__ double term_same(double A, double B, double C,
+                                            double U, double V, double W,
+                                            double denominator, double fac) {
+  const double UVW = U + (V + W);
+  const double value = 3.0 * ((A * U + B * V) + C * W) - (A + (B + C)) * UVW;
+  return ((2.0 * value) / denominator) * fac;
+}
+
 // Energy terms of the i>=j>=k points of block triple (B1, B2, B3) (edge 8)
 // of one tuple, two points per thread, added to e_acc (and, with the (cT)
 // W, to ect_acc).  The six permuted W cubes of the triple's orbit sit in
@@ -202,42 +227,21 @@ __device__ __forceinline__ void triple_points(
       const double U = Z(A, si, sj, sk), V = Z(B, si, sk, sj),
                    W = Z(C, sj, si, sk), X = Z(D, sj, sk, si),
                    Y = Z(E, sk, si, sj), Zz = Z(F, sk, sj, si);
-      const double UXY = U + (X + Y), VWZ = V + (W + Zz);
-      {
-        const double first =
-            A * U + (B * V + (C * W + (D * X + (E * Y + F * Zz))));
-        const double second = (UXY - 2.0 * VWZ) * (A + (D + E));
-        const double third = (VWZ - 2.0 * UXY) * (B + (C + F));
-        const double value = 3.0 * first + (second + third);
-        e_acc += ((2.0 * value) / denominator) * (facjk * facij);
-      }
-      if constexpr (HJ) {
-        const double A2 = J(0, o_ijk), B2 = J(1, o_ikj), C2 = J(2, o_jik),
-                     D2 = J(3, o_jki), E2 = J(4, o_kij), F2 = J(5, o_kji);
-        const double first =
-            A2 * U + (B2 * V + (C2 * W + (D2 * X + (E2 * Y + F2 * Zz))));
-        const double second = (UXY - 2.0 * VWZ) * (A2 + (D2 + E2));
-        const double third = (VWZ - 2.0 * UXY) * (B2 + (C2 + F2));
-        const double value = 3.0 * first + (second + third);
-        ect_acc += ((2.0 * value) / denominator) * (facjk * facij);
-      }
+      e_acc += term_distinct(A, B, C, D, E, F, U, V, W, X, Y, Zz, denominator,
+                             facjk * facij);
+      if constexpr (HJ)
+        ect_acc += term_distinct(J(0, o_ijk), J(1, o_ikj), J(2, o_jik),
+                                 J(3, o_jki), J(4, o_kij), J(5, o_kji), U, V, W,
+                                 X, Y, Zz, denominator, facjk * facij);
     } else {
       const double A = cube[alias[0]][o_ijk], B = cube[alias[3]][o_jki],
                    C = cube[alias[4]][o_kij];
       const double U = Z(A, si, sj, sk), V = Z(B, sj, sk, si),
                    W = Z(C, sk, si, sj);
-      const double UVW = U + (V + W);
-      {
-        const double value =
-            3.0 * ((A * U + B * V) + C * W) - (A + (B + C)) * UVW;
-        e_acc += ((2.0 * value) / denominator) * (facjk * facij);
-      }
-      if constexpr (HJ) {
-        const double A2 = J(0, o_ijk), B2 = J(3, o_jki), C2 = J(4, o_kij);
-        const double value =
-            3.0 * ((A2 * U + B2 * V) + C2 * W) - (A2 + (B2 + C2)) * UVW;
-        ect_acc += ((2.0 * value) / denominator) * (facjk * facij);
-      }
+      e_acc += term_same(A, B, C, U, V, W, denominator, facjk * facij);
+      if constexpr (HJ)
+        ect_acc += term_same(J(0, o_ijk), J(3, o_jki), J(4, o_kij), U, V, W,
+                             denominator, facjk * facij);
     }
   }
 }
@@ -434,9 +438,10 @@ void energy_kernel(EnergyParams P) {
 struct FusedParams {
   const void *G, *GJ;  // class buffers [3][slots][No^2 rows][NoP] (FP64 or FP32)
   const double *Tai, *VHH, *ei, *ea;
+  const uint32_t *points;
   WindowArgs win;
   double *e_part;  // [triple][slot][2]
-  int64_t No, Nv, N2, W3g, slots, ntri;
+  int64_t No, Nv, N2, W3g, slots, ntri, npoints;
   int nbk;
   double tai_sign;
 };
@@ -683,6 +688,191 @@ __global__ __launch_bounds__(256, HJ ? 2 : 4) void energy_fused_kernel(
 #undef ORBIT
 }
 
+// The same for small No: T threads do a whole tuple, a wave up to No = 8 and a
+// workgroup up to 16, NI pairs of elements of each class per thread.  By block
+// triples such a tuple took 1 or 4 workgroups of a few points each, whose time
+// was their setup, barriers and latencies, and half or more of the elements
+// they covered lay outside No; here every thread holds pairs that exist and W is
+// read once.  W sits in LDS at x + SY y + SZ z with odd strides, V and t whole.
+// Bound by HBM from No = 9 on: No=10, Nv=90 1.06 ms against 2.55 before (8.5 ns
+// a tuple, 38 KB of touched lines), No=16 2.98 against 3.42 (23.8 ns, 98 KB);
+// No=4, Nv=36 15 us against 52.
+template <typename GT, bool HJ, int T, int NI>
+__global__ __launch_bounds__(256) void energy_small_kernel(FusedParams P) {
+  extern __shared__ double lds[];
+  constexpr int S = 256 / T;  // tuples of a workgroup
+  const int tid = threadIdx.x, tl = tid % T;
+  const int sub = __builtin_amdgcn_readfirstlane(tid / T);
+  const int64_t gslot = (int64_t)blockIdx.x * S + sub;
+  if (gslot >= P.slots) return;
+  const int64_t Nv = P.Nv;
+  int64_t a, b, c;
+  if (!slot_tuple(P.win, (uint64_t)Nv, gslot, a, b, c)) {
+    if (tl < 2) P.e_part[2 * gslot + tl] = 0.0;
+    return;
+  }
+  // a tuple's threads are one wave, whose LDS accesses are in order, or the
+  // workgroup
+  auto sync = [] {
+    if constexpr (T == 64) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    } else {
+      __syncthreads();
+    }
+  };
+  const int no = (int)P.No, n2 = no * no;
+  const int SY = no | 1, SZ = (SY * no) | 1, CS = SZ * no;
+  double *cube = lds + sub * ((HJ ? 2 : 1) * CS + 3 * n2 + 4 * no);
+  double *cubeJ = cube + CS, *sV = cube + (HJ ? 2 : 1) * CS, *sT = sV + 3 * n2;
+
+  // element pairs (p, q, r), (p, q, r + 1) of the class buffers
+  const int H = (no + 1) / 2, count = n2 * H;
+  const float rH = 1.0f / (float)H, rN = 1.0f / (float)no;
+  uint32_t at[NI];
+  int pqr[NI];
+#pragma unroll
+  for (int it = 0; it < NI; it++) {
+    const int e = tl + T * it, x = e < count ? e : 0;
+    // (both quotients exact: they lie at least 1 / 32 from a whole number)
+    const int m = (int)(((float)x + 0.5f) * rH), r = 2 * (x - m * H);
+    const int q = (int)(((float)m + 0.5f) * rN), p = m - q * no;
+    at[it] = ((uint32_t)(((q >> 3) * P.nbk + (p >> 3)) * P.nbk + (r >> 3)) << 9) +
+             ((q & 7) << 6) + ((p & 7) << 3) + (r & 7);
+    pqr[it] = e < count ? p | q << 8 | r << 16 : -1;
+  }
+  typedef GT g2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+  for (int set = 0; set < (HJ ? 2 : 1); set++) {
+    const GT *Gs = (const GT *)(set ? P.GJ : P.G) + gslot * P.W3g;
+    g2 vals[3][NI];
+#pragma unroll
+    for (int cls = 0; cls < 3; cls++)
+#pragma unroll
+      for (int it = 0; it < NI; it++)
+        vals[cls][it] = *(const g2 *)(Gs + cls * P.slots * P.W3g + at[it]);
+    if (set == 0) {
+      const int v0 = tl < n2 ? tl : 0, x0 = tl < no ? tl : 0;
+      const double vbc = P.VHH[(b + Nv * c) * P.N2 + v0],
+                   vac = P.VHH[(a + Nv * c) * P.N2 + v0],
+                   vab = P.VHH[(a + Nv * b) * P.N2 + v0];
+      const double ta = P.Tai[a + Nv * x0], tb = P.Tai[b + Nv * x0],
+                   tc = P.Tai[c + Nv * x0], ex = P.ei[x0];
+      if (tl < n2) {
+        sV[tl] = vbc;
+        sV[n2 + tl] = vac;
+        sV[2 * n2 + tl] = vab;
+      }
+      if (tl < no) {
+        sT[tl] = P.tai_sign * ta;
+        sT[no + tl] = P.tai_sign * tb;
+        sT[2 * no + tl] = P.tai_sign * tc;
+        sT[3 * no + tl] = ex;
+      }
+    }
+    double *W = set ? cubeJ : cube;
+#pragma unroll
+    for (int cls = 0; cls < 3; cls++) {
+#pragma unroll
+      for (int it = 0; it < NI; it++) {
+        if (pqr[it] < 0) continue;
+        const int p = pqr[it] & 255, q = (pqr[it] >> 8) & 255, r = pqr[it] >> 16;
+        // (p, q, r) in W indices: w (i,j,k), v (i,k,j), u (j,k,i)
+        double *w = W + (cls == 0   ? p + SY * q + SZ * r
+                         : cls == 1 ? p + SY * r + SZ * q
+                                    : r + SY * p + SZ * q);
+        const int step = cls == 0 ? SZ : cls == 1 ? SY : 1;
+        const double x0 = (double)vals[cls][it][0], x1 = (double)vals[cls][it][1];
+        if (cls == 0) {
+          w[0] = x0;
+          if (r + 1 < no) w[step] = x1;
+        } else {
+          w[0] += x0;
+          if (r + 1 < no) w[step] += x1;
+        }
+      }
+      sync();
+    }
+  }
+
+  int distinct = 0;
+  if (a == b) distinct++;
+  if (b == c) distinct--;
+  const double epsabc = (P.ea[a] + P.ea[b]) + P.ea[c];
+  double e_acc = 0.0, ect_acc = 0.0;
+#pragma unroll 1
+  for (int pt = tl; pt < (int)P.npoints; pt += T) {
+    const uint32_t pk = P.points[pt];
+    const int i = pk & 1023, j = (pk >> 10) & 1023, k = pk >> 20;
+    const double *tA = sT, *tB = sT + no, *tC = sT + 2 * no, *sE = sT + 3 * no;
+    const double fac = (j == k ? 0.5 : 1.0) * (i == j ? 0.5 : 1.0);
+    const double denominator = epsabc - ((sE[i] + sE[j]) + sE[k]);
+    const int o_ijk = i + SY * j + SZ * k, o_ikj = i + SY * k + SZ * j,
+              o_jik = j + SY * i + SZ * k, o_jki = j + SY * k + SZ * i,
+              o_kij = k + SY * i + SZ * j, o_kji = k + SY * j + SZ * i;
+    // singles at a permutation (x,y,z): t_a[x] V^bc_yz + t_b[y] V^ac_xz
+    // + t_c[z] V^ab_xy
+    auto Z = [&](double wv, int x, int y, int z) {
+      double zz = wv + tA[x] * sV[y + no * z];
+      zz = zz + tB[y] * sV[n2 + x + no * z];
+      zz = zz + tC[z] * sV[2 * n2 + x + no * y];
+      return zz;
+    };
+    if (distinct == 0) {
+      const double A = cube[o_ijk], B = cube[o_ikj], C = cube[o_jik],
+                   D = cube[o_jki], E = cube[o_kij], F = cube[o_kji];
+      const double U = Z(A, i, j, k), V = Z(B, i, k, j), W = Z(C, j, i, k),
+                   X = Z(D, j, k, i), Y = Z(E, k, i, j), Zz = Z(F, k, j, i);
+      e_acc += term_distinct(A, B, C, D, E, F, U, V, W, X, Y, Zz, denominator, fac);
+      if constexpr (HJ)
+        ect_acc += term_distinct(cubeJ[o_ijk], cubeJ[o_ikj], cubeJ[o_jik],
+                                 cubeJ[o_jki], cubeJ[o_kij], cubeJ[o_kji], U, V,
+                                 W, X, Y, Zz, denominator, fac);
+    } else {
+      const double A = cube[o_ijk], B = cube[o_jki], C = cube[o_kij];
+      const double U = Z(A, i, j, k), V = Z(B, j, k, i), W = Z(C, k, i, j);
+      e_acc += term_same(A, B, C, U, V, W, denominator, fac);
+      if constexpr (HJ)
+        ect_acc += term_same(cubeJ[o_ijk], cubeJ[o_jki], cubeJ[o_kij], U, V, W,
+                             denominator, fac);
+    }
+  }
+  e_acc = wave_sum(e_acc);
+  ect_acc = wave_sum(ect_acc);
+  if constexpr (T == 256) {
+    __shared__ double red[2][4];
+    if ((tid & 63) == 0) {
+      red[0][tid >> 6] = e_acc;
+      red[1][tid >> 6] = ect_acc;
+    }
+    __syncthreads();
+    e_acc = (red[0][0] + red[0][1]) + (red[0][2] + red[0][3]);
+    ect_acc = (red[1][0] + red[1][1]) + (red[1][2] + red[1][3]);
+  }
+  if (tl == 0) {
+    P.e_part[2 * gslot] = e_acc;
+    P.e_part[2 * gslot + 1] = HJ ? ect_acc : e_acc;
+  }
+}
+
+template <typename GT, bool HJ>
+void launch_small(const FusedParams &P, hipStream_t st) {
+  const int no = (int)P.No, n2 = no * no, SZ = ((no | 1) * no) | 1;
+  const int T = no <= 8 ? 64 : 256, S = 256 / T;
+  const size_t lds = sizeof(double) * S * ((HJ ? 2 : 1) * SZ * no + 3 * n2 + 4 * no);
+  const int ni = (n2 * ((no + 1) / 2) + T - 1) / T;  // pairs per thread
+  const dim3 grid((unsigned)((P.slots + S - 1) / S));
+#define SMALL(TT, NI)                                                       \
+  if (T == TT && ni <= NI) {                                                \
+    hipLaunchKernelGGL((energy_small_kernel<GT, HJ, TT, NI>), grid, 256, lds, \
+                       st, P);                                              \
+    return;                                                                 \
+  }
+  SMALL(64, 1) SMALL(64, 2) SMALL(64, 4)
+  SMALL(256, 2) SMALL(256, 4) SMALL(256, 6) SMALL(256, 8)
+#undef SMALL
+}
+
 // Neumaier step on a (sum, compensation) pair.
 __device__ inline void nadd(double &s, double &c, double x) {
   const double t = s + x;
@@ -785,8 +975,10 @@ hipError_t launch_energy(const DevSystem &s, const BatchArgs &b,
                          double tai_sign, double *e_slot, double *scratch,
                          bool fused, hipStream_t st) {
   if (fused) {
-    const int64_t nbk = w_blocks(s.No), ntri = n_triples(nbk);
+    const int64_t nbk = w_blocks(s.No), ntri = energy_parts(s.No, GJ);
     FusedParams P;
+    P.points = s.points;
+    P.npoints = s.npoints;
     P.G = G;
     P.GJ = GJ;
     P.Tai = s.Tai;
@@ -805,6 +997,14 @@ hipError_t launch_energy(const DevSystem &s, const BatchArgs &b,
     P.tai_sign = tai_sign;
     const int64_t grid = (b.slots + 7) / 8 * 8 * ntri;
     if (grid <= 0) return hipSuccess;
+    if (small_energy(s.No, GJ)) {
+      if (grid > MAX_GRID) return hipErrorInvalidConfiguration;
+      if (g32)
+        GJ ? launch_small<float, true>(P, st) : launch_small<float, false>(P, st);
+      else
+        GJ ? launch_small<double, true>(P, st) : launch_small<double, false>(P, st);
+      return hipGetLastError();
+    }
     // (the kernel decodes its block id and class-buffer offsets in 32 bits)
     if (grid > MAX_GRID || g_elems(s.No) >= (int64_t(1) << 31))
       return hipErrorInvalidConfiguration;

@@ -122,6 +122,18 @@ __host__ __device__ inline int64_t n_triples(int64_t nbk) {
   return nbk * (nbk + 1) * (nbk + 2) / 6;
 }
 
+// Whether the fused epilogue does a tuple in one wave or workgroup: up to the No
+// whose W (two with (cT)) fits 64 KB of LDS; there it is the faster one at every
+// No (energies of No=4, Nv=36 52 -> 15 us, 10/90 2.55 -> 1.06 ms, 16/90 3.42
+// -> 2.98 in FP64, 3.06 -> 2.30 in bf16x3; (cT) 15/90 6.68 -> 5.45).
+__host__ __device__ inline bool small_energy(int64_t No, bool use_j) {
+  return No <= (use_j ? 15 : 16);
+}
+// Partial energies of a tuple in it: one, or one per block triple.
+__host__ __device__ inline int64_t energy_parts(int64_t No, bool use_j) {
+  return small_energy(No, use_j) ? 1 : n_triples(w_blocks(No));
+}
+
 // Device-resident system.  Pair-indexed arrays use the CTF pair order
 // p(x,y) = x + Nv*y.  The doubles operands, as rows times contraction index:
 //   T3  [x][p + No q][E < Kv]    = Tpphh[x,E,p,q]          (T(x) slices)
@@ -374,8 +386,8 @@ hipError_t launch_wsum(const DevSystem &s, const BatchArgs &b, const void *A,
 
 // Class sums and singles + energy epilogue.  fused: one kernel gathers each
 // block triple's W straight from the class buffers and writes the triple's
-// energies to scratch ([triple][slot][2], slots * n_triples * 2 doubles),
-// which launch_slot_sums adds up; otherwise the class-sum kernel writes W as
+// energies to scratch ([triple][slot][2], slots * energy_parts * 2 doubles),
+// which launch_slot_sums adds up (small No: a whole tuple at once); otherwise the class-sum kernel writes W as
 // cubes first (scratch: (GJ ? 2 : 1) * slots * w_cube(No) doubles) and
 // e_slot[2*slot + {0,1}] is written here.  Same W bits either way.
 hipError_t launch_energy(const DevSystem &s, const BatchArgs &b,
@@ -385,7 +397,7 @@ hipError_t launch_energy(const DevSystem &s, const BatchArgs &b,
 // Doubles of energy scratch per tuple slot (see launch_energy).
 inline int64_t energy_scratch_per_slot(int64_t No, bool use_j, bool cplx,
                                        bool fused) {
-  if (fused && !cplx) return 2 * n_triples(w_blocks(No));
+  if (fused && !cplx) return 2 * energy_parts(No, use_j);
   return (use_j ? 2 : 1) * (cplx ? 2 : 1) * w_cube(No);
 }
 

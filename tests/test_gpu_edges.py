@@ -43,3 +43,29 @@ def test_edge_tiles(hip_ctx, oracle, no, nv, window, precision):
         hip_ctx.set_option("tile", -1)
         hip_ctx.set_option("window", 0)
         hip_ctx.release(s)
+
+
+# The epilogue that does a whole tuple at once (No <= 16, with (cT) <= 15): one
+# pair of elements, odd and even No around the wave (8) and workgroup (16)
+# limits and the first No beyond them.  W is the same bits as in the cube
+# epilogue and the up to 969 terms of a tuple are added in another order:
+# within 969 roundings of 1.1e-16 of the sum of their magnitudes, bounded here
+# by 1e-12 of the largest tuple.
+@pytest.mark.parametrize("no", [1, 2, 3, 7, 8, 9, 14, 15, 16, 17])
+@pytest.mark.parametrize("precision", ["fp64", "bf16x3"])
+def test_small_epilogue(hip_ctx, no, precision):
+    nv = 13
+    n = nv * (nv + 1) * (nv + 2) // 6 - nv
+    for with_j in (False, True):
+        print("small epilogue", no, precision, with_j, flush=True)
+        s = hip_ctx.upload_synthetic(no, nv, 700 + no, with_j=with_j)
+        out = []
+        try:
+            for epi in (0, 1):
+                hip_ctx.set_option("epilogue", epi)
+                out.append(hip_ctx.tuple_energies(s, 0, n, precision, with_ct=True))
+        finally:
+            hip_ctx.set_option("epilogue", 0)
+            hip_ctx.release(s)
+        for x, y in zip(*out):
+            assert np.max(np.abs(x - y)) <= 1e-12 * np.max(np.abs(y))
