@@ -1114,7 +1114,7 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
     if (s.cplx)
       check(launch_energy_z(s, b, Gz, use_j ? GJz : nullptr,
                             ijkabc ? -1.0 : 1.0, (double *)e_slot,
-                            (double *)wcube, st),
+                            (double *)wcube, fused, st),
             "energy kernel (complex)");
     else
       check(launch_energy(s, b, G, GJ, g32, ijkabc ? -1.0 : 1.0,

@@ -129,7 +129,11 @@ __host__ __device__ inline int64_t n_triples(int64_t nbk) {
 __host__ __device__ inline bool small_energy(int64_t No, bool use_j) {
   return No <= (use_j ? 15 : 16);
 }
-// Partial energies of a tuple in it: one, or one per block triple.
+// The same for complex systems, whose two planes of W (four with (cT)) fit 160 KB.
+__host__ __device__ inline bool small_energy_z(int64_t No, bool use_j) {
+  return No <= (use_j ? 16 : 20);
+}
+// Partial energies of a real tuple in it: one, or one per block triple.
 __host__ __device__ inline int64_t energy_parts(int64_t No, bool use_j) {
   return small_energy(No, use_j) ? 1 : n_triples(w_blocks(No));
 }
@@ -398,16 +402,18 @@ hipError_t launch_energy(const DevSystem &s, const BatchArgs &b,
 inline int64_t energy_scratch_per_slot(int64_t No, bool use_j, bool cplx,
                                        bool fused) {
   if (fused && !cplx) return 2 * energy_parts(No, use_j);
+  if (fused && small_energy_z(No, use_j)) return 1;  // none needed
   return (use_j ? 2 : 1) * (cplx ? 2 : 1) * w_cube(No);
 }
 
 // Singles + energy of complex systems from the class-buffer sets of W's real
 // and imaginary plane; GJ null without (cT).
-// wcube: scratch of (GJ ? 4 : 2) * slots * w_cube(No) doubles.
+// fused: straight from the buffers where small_energy_z holds; otherwise by
+// cubes, wcube: scratch of (GJ ? 4 : 2) * slots * w_cube(No) doubles.
 hipError_t launch_energy_z(const DevSystem &s, const BatchArgs &b,
                            double *const G[2], double *const GJ[2],
                            double tai_sign, double *e_slot, double *wcube,
-                           hipStream_t st);
+                           bool fused, hipStream_t st);
 
 // Per window of a batch (nw windows of `per` slots), a compensated sum of
 // its slot energies in a fixed order: out[2 w] = sum, out[2 w + 1] =

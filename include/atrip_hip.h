@@ -227,9 +227,10 @@ int atrip_hip_tuple_energies(atrip_hip_ctx *ctx, int sys, int precision,
  *   "tile"    doubles-kernel tile variant: 0..7 for the FP64 kernel, 0..9
  *             for the FP32-product kernels (a variant a kernel lacks
  *             means automatic for it), -1 (default) = automatic
- *   "epilogue"  0 (default): fused class sums + energy per block triple;
- *               1: class sums written as W cubes first (complex systems
- *               always take this form)
+ *   "epilogue"  0 (default): fused class sums + energy, per tuple for small
+ *               No, else per block triple; 1: class sums written as W cubes
+ *               first (complex systems beyond No = 20, 16 with (cT), always
+ *               take this form)
  *   "serve_plain_no"  servers run requests with No at or above it through
  *               the plain class-GEMM path and the rest in the persistent
  *               batched launch (default 16; a bf16x3 server runs every

@@ -69,3 +69,23 @@ def test_small_epilogue(hip_ctx, no, precision):
             hip_ctx.release(s)
         for x, y in zip(*out):
             assert np.max(np.abs(x - y)) <= 1e-12 * np.max(np.abs(y))
+
+
+# The complex one (No <= 20, with (cT) <= 16), likewise; up to 1771 terms.
+@pytest.mark.parametrize("no", [1, 2, 3, 7, 8, 9, 15, 16, 17, 20, 21])
+def test_small_epilogue_complex(hip_ctx, no):
+    nv = 11
+    n = nv * (nv + 1) * (nv + 2) // 6 - nv
+    for with_j in (False, True):
+        print("small complex epilogue", no, with_j, flush=True)
+        s = hip_ctx.upload_synthetic_complex(no, nv, 800 + no, with_j=with_j)
+        out = []
+        try:
+            for epi in (0, 1):
+                hip_ctx.set_option("epilogue", epi)
+                out.append(hip_ctx.tuple_energies(s, 0, n, with_ct=True))
+        finally:
+            hip_ctx.set_option("epilogue", 0)
+            hip_ctx.release(s)
+        for x, y in zip(*out):
+            assert np.max(np.abs(x - y)) <= 1e-12 * np.max(np.abs(y))
