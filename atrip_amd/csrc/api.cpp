@@ -942,7 +942,7 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
     z.g = (size_t)((use_j ? 2 : 1) * nsets) * z.gsz;
     z.e_slot = (size_t)(2 * z.slots_max) * sizeof(double);
     z.wcube = (size_t)(z.slots_max * energy_scratch_per_slot(
-                                         s.No, use_j, s.cplx, fused)) *
+                                         s.No, use_j, g32, s.cplx, fused)) *
               sizeof(double);
     z.nbatch = (nsel + bw_ - 1) / bw_;
     z.partials = (size_t)(4 * z.nbatch * slot_partials(z.slots_max)) *
@@ -1131,7 +1131,7 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
       ev.handed = true;
     }
     check(launch_slot_sums(fused && !s.cplx ? (const double *)wcube : nullptr,
-                           b.slots, energy_parts(s.No, use_j),
+                           b.slots, energy_parts(s.No, use_j, g32),
                            (double *)e_slot, (double *)partials + 4 * nparts,
                            st),
           "slot sums kernel");

@@ -688,19 +688,21 @@ __global__ __launch_bounds__(256, HJ ? 2 : 4) void energy_fused_kernel(
 #undef ORBIT
 }
 
-// The same for small No: T threads do a whole tuple, a wave up to No = 8 and a
-// workgroup up to 16, NI pairs of elements of each class per thread.  By block
-// triples such a tuple took 1 or 4 workgroups of a few points each, whose time
-// was their setup, barriers and latencies, and half or more of the elements
-// they covered lay outside No; here every thread holds pairs that exist and W is
-// read once.  W sits in LDS at x + SY y + SZ z with odd strides, V and t whole.
-// Bound by HBM from No = 9 on: No=10, Nv=90 1.06 ms against 2.55 before (8.5 ns
-// a tuple, 38 KB of touched lines), No=16 2.98 against 3.42 (23.8 ns, 98 KB);
-// No=4, Nv=36 15 us against 52.
+// The same for small No: T threads do a whole tuple, a wave up to No = 8, four
+// up to 14 and eight up to 20, NI pairs of elements of each class per thread.
+// By block triples such a tuple took 1 to 10 workgroups of a few points each,
+// whose time was their setup, barriers and latencies, and half or more of the
+// elements they covered lay outside No; here every thread holds pairs that
+// exist and W is read once.  W sits in LDS at x + SY y + SZ z with odd strides, V
+// and t whole.  Bound by HBM from No = 9 on: No=10, Nv=90 8.5 ns a tuple for 38
+// KB of touched lines, No=16, Nv=80 21 ns for 98 KB; times before and after are
+// at small_energy, which chooses.  (No=14, 15, 16 in FP64 with four / eight
+// waves: 1.42 / 1.51, 2.0 / 1.83 ms at 14 and 16.)
 template <typename GT, bool HJ, int T, int NI>
-__global__ __launch_bounds__(256) void energy_small_kernel(FusedParams P) {
+__global__ __launch_bounds__(T < 256 ? 256 : T, HJ ? 2 : 4) void energy_small_kernel(
+    FusedParams P) {
   extern __shared__ double lds[];
-  constexpr int S = 256 / T;  // tuples of a workgroup
+  constexpr int S = T < 256 ? 256 / T : 1;  // tuples of a workgroup
   const int tid = threadIdx.x, tl = tid % T;
   const int sub = __builtin_amdgcn_readfirstlane(tid / T);
   const int64_t gslot = (int64_t)blockIdx.x * S + sub;
@@ -839,15 +841,18 @@ __global__ __launch_bounds__(256) void energy_small_kernel(FusedParams P) {
   }
   e_acc = wave_sum(e_acc);
   ect_acc = wave_sum(ect_acc);
-  if constexpr (T == 256) {
-    __shared__ double red[2][4];
+  if constexpr (T > 64) {
+    __shared__ double red[2][T / 64];
     if ((tid & 63) == 0) {
       red[0][tid >> 6] = e_acc;
       red[1][tid >> 6] = ect_acc;
     }
     __syncthreads();
-    e_acc = (red[0][0] + red[0][1]) + (red[0][2] + red[0][3]);
-    ect_acc = (red[1][0] + red[1][1]) + (red[1][2] + red[1][3]);
+    e_acc = ect_acc = 0.0;
+    for (int w = 0; w < T / 64; w++) {
+      e_acc += red[0][w];
+      ect_acc += red[1][w];
+    }
   }
   if (tl == 0) {
     P.e_part[2 * gslot] = e_acc;
@@ -856,21 +861,28 @@ __global__ __launch_bounds__(256) void energy_small_kernel(FusedParams P) {
 }
 
 template <typename GT, bool HJ>
-void launch_small(const FusedParams &P, hipStream_t st) {
+hipError_t launch_small(const FusedParams &P, hipStream_t st) {
   const int no = (int)P.No, n2 = no * no, SZ = ((no | 1) * no) | 1;
-  const int T = no <= 8 ? 64 : 256, S = 256 / T;
+  const int T = no <= 8 ? 64 : no <= 14 ? 256 : 512, S = T < 256 ? 256 / T : 1;
   const size_t lds = sizeof(double) * S * ((HJ ? 2 : 1) * SZ * no + 3 * n2 + 4 * no);
   const int ni = (n2 * ((no + 1) / 2) + T - 1) / T;  // pairs per thread
   const dim3 grid((unsigned)((P.slots + S - 1) / S));
 #define SMALL(TT, NI)                                                       \
   if (T == TT && ni <= NI) {                                                \
-    hipLaunchKernelGGL((energy_small_kernel<GT, HJ, TT, NI>), grid, 256, lds, \
-                       st, P);                                              \
-    return;                                                                 \
+    /* beyond the 64 KB every launch may have */                            \
+    hipError_t e = hipFuncSetAttribute(                                     \
+        (const void *)energy_small_kernel<GT, HJ, TT, NI>,                  \
+        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);              \
+    if (e != hipSuccess) return e;                                          \
+    hipLaunchKernelGGL((energy_small_kernel<GT, HJ, TT, NI>), grid,         \
+                       TT < 256 ? 256 : TT, lds, st, P);                    \
+    return hipGetLastError();                                               \
   }
   SMALL(64, 1) SMALL(64, 2) SMALL(64, 4)
-  SMALL(256, 2) SMALL(256, 4) SMALL(256, 6) SMALL(256, 8)
+  SMALL(256, 2) SMALL(256, 4) SMALL(256, 6)
+  SMALL(512, 4) SMALL(512, 6) SMALL(512, 8)
 #undef SMALL
+  return hipErrorInvalidConfiguration;
 }
 
 // Neumaier step on a (sum, compensation) pair.
@@ -975,7 +987,7 @@ hipError_t launch_energy(const DevSystem &s, const BatchArgs &b,
                          double tai_sign, double *e_slot, double *scratch,
                          bool fused, hipStream_t st) {
   if (fused) {
-    const int64_t nbk = w_blocks(s.No), ntri = energy_parts(s.No, GJ);
+    const int64_t nbk = w_blocks(s.No), ntri = energy_parts(s.No, GJ, g32);
     FusedParams P;
     P.points = s.points;
     P.npoints = s.npoints;
@@ -997,13 +1009,13 @@ hipError_t launch_energy(const DevSystem &s, const BatchArgs &b,
     P.tai_sign = tai_sign;
     const int64_t grid = (b.slots + 7) / 8 * 8 * ntri;
     if (grid <= 0) return hipSuccess;
-    if (small_energy(s.No, GJ)) {
+    if (small_energy(s.No, GJ, g32)) {
       if (grid > MAX_GRID) return hipErrorInvalidConfiguration;
       if (g32)
-        GJ ? launch_small<float, true>(P, st) : launch_small<float, false>(P, st);
-      else
-        GJ ? launch_small<double, true>(P, st) : launch_small<double, false>(P, st);
-      return hipGetLastError();
+        return GJ ? launch_small<float, true>(P, st)
+                  : launch_small<float, false>(P, st);
+      return GJ ? launch_small<double, true>(P, st)
+                : launch_small<double, false>(P, st);
     }
     // (the kernel decodes its block id and class-buffer offsets in 32 bits)
     if (grid > MAX_GRID || g_elems(s.No) >= (int64_t(1) << 31))

@@ -123,19 +123,22 @@ __host__ __device__ inline int64_t n_triples(int64_t nbk) {
 }
 
 // Whether the fused epilogue does a tuple in one wave or workgroup: up to the No
-// whose W (two with (cT)) fits 64 KB of LDS; there it is the faster one at every
-// No (energies of No=4, Nv=36 52 -> 15 us, 10/90 2.55 -> 1.06 ms, 16/90 3.42
-// -> 2.98 in FP64, 3.06 -> 2.30 in bf16x3; (cT) 15/90 6.68 -> 5.45).
-__host__ __device__ inline bool small_energy(int64_t No, bool use_j) {
-  return No <= (use_j ? 15 : 16);
+// whose W (two with (cT)) fits 160 KB of LDS, from FP64 buffers alone up to 18.
+// Energies by block triples -> by tuples, ms: FP64 No=4, Nv=36 .052 -> .015,
+// 10/90 2.55 -> 1.06, 16/80 2.32 -> 1.83, 18/80 5.58 -> 3.87, 20/80 5.82 -> 5.99
+// (one workgroup a CU, or spills); (cT) 20/60 4.93 -> 4.38; bf16x3 16/80 2.03
+// -> 1.48, 20/80 5.34 -> 3.06.
+__host__ __device__ inline bool small_energy(int64_t No, bool use_j, bool g32) {
+  return No <= (use_j || g32 ? 20 : 18);
 }
 // The same for complex systems, whose two planes of W (four with (cT)) fit 160 KB.
 __host__ __device__ inline bool small_energy_z(int64_t No, bool use_j) {
   return No <= (use_j ? 16 : 20);
 }
 // Partial energies of a real tuple in it: one, or one per block triple.
-__host__ __device__ inline int64_t energy_parts(int64_t No, bool use_j) {
-  return small_energy(No, use_j) ? 1 : n_triples(w_blocks(No));
+__host__ __device__ inline int64_t energy_parts(int64_t No, bool use_j,
+                                                bool g32) {
+  return small_energy(No, use_j, g32) ? 1 : n_triples(w_blocks(No));
 }
 
 // Device-resident system.  Pair-indexed arrays use the CTF pair order
@@ -399,9 +402,9 @@ hipError_t launch_energy(const DevSystem &s, const BatchArgs &b,
                          double tai_sign, double *e_slot, double *scratch,
                          bool fused, hipStream_t st);
 // Doubles of energy scratch per tuple slot (see launch_energy).
-inline int64_t energy_scratch_per_slot(int64_t No, bool use_j, bool cplx,
-                                       bool fused) {
-  if (fused && !cplx) return 2 * energy_parts(No, use_j);
+inline int64_t energy_scratch_per_slot(int64_t No, bool use_j, bool g32,
+                                       bool cplx, bool fused) {
+  if (fused && !cplx) return 2 * energy_parts(No, use_j, g32);
   if (fused && small_energy_z(No, use_j)) return 1;  // none needed
   return (use_j ? 2 : 1) * (cplx ? 2 : 1) * w_cube(No);
 }

@@ -45,13 +45,13 @@ def test_edge_tiles(hip_ctx, oracle, no, nv, window, precision):
         hip_ctx.release(s)
 
 
-# The epilogue that does a whole tuple at once (No <= 16, with (cT) <= 15): one
-# pair of elements, odd and even No around the wave (8) and workgroup (16)
-# limits and the first No beyond them.  W is the same bits as in the cube
-# epilogue and the up to 969 terms of a tuple are added in another order:
-# within 969 roundings of 1.1e-16 of the sum of their magnitudes, bounded here
-# by 1e-12 of the largest tuple.
-@pytest.mark.parametrize("no", [1, 2, 3, 7, 8, 9, 14, 15, 16, 17])
+# The epilogue that does a whole tuple at once (No <= 18, with (cT) or FP32
+# buffers <= 20): one pair of elements, odd and even No around the limits of a
+# wave (8) and of four (14), and the last No and the first beyond.  W is the same
+# bits as in the cube epilogue and the up to 1771 terms of a tuple are added in
+# another order: within 1771 roundings of 1.1e-16 of the sum of their
+# magnitudes, bounded here by 1e-12 of the largest tuple.
+@pytest.mark.parametrize("no", [1, 2, 3, 7, 8, 9, 14, 15, 16, 18, 19, 20, 21])
 @pytest.mark.parametrize("precision", ["fp64", "bf16x3"])
 def test_small_epilogue(hip_ctx, no, precision):
     nv = 13
