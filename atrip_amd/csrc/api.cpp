@@ -143,12 +143,8 @@ void atrip_amd::ensure_tri(atrip_hip_ctx *ctx, DevSystem &s) {
 namespace {
 
 double *dev_alloc(DevSystem &s, int64_t n, const char *what) {
-  void *p = nullptr;
-  const size_t bytes = (size_t)std::max<int64_t>(n, 1) * sizeof(double);
-  check(hipMalloc(&p, bytes), what);
-  s.allocations.push_back(p);
-  s.bytes += bytes;
-  return (double *)p;
+  return (double *)dev_bytes(s, (size_t)std::max<int64_t>(n, 1) * sizeof(double),
+                             what);
 }
 
 // The row-swapped copies of a system's FP64 A operands and the copies they
@@ -174,42 +170,50 @@ std::vector<SwapCopy> swap_copies(DevSystem &s) {
   return v;
 }
 
-// Allocates the row-swapped copies that fit; one that finds no memory stays
-// null and the kernels read the swapped rows from the straight array.
+// Allocates the row-swapped copies as one block if it fits; without memory they
+// stay null and the kernels read the swapped rows from the straight array.
 void alloc_swaps(DevSystem &s) {
-  for (const SwapCopy &c : swap_copies(s)) {
-    const size_t bytes =
-        (size_t)f64_elems(f64_geom_a(s.No, s.Nv, c.K)) * sizeof(double);
-    void *p = nullptr;
-    if (hipMalloc(&p, bytes) != hipSuccess) {
-      (void)hipGetLastError();
-      continue;
-    }
-    s.allocations.push_back(p);
-    s.bytes += bytes;
-    *c.copy = (double *)p;
+  const std::vector<SwapCopy> copies = swap_copies(s);
+  size_t bytes = 0;
+  for (const SwapCopy &c : copies)
+    bytes += (size_t)f64_elems(f64_geom_a(s.No, s.Nv, c.K)) * sizeof(double);
+  void *p = nullptr;
+  if (hipMalloc(&p, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return;
+  }
+  s.allocations.push_back(p);
+  s.bytes += bytes;
+  s.swaps = p;
+  s.swap_bytes = bytes;
+  char *at = (char *)p;
+  for (const SwapCopy &c : copies) {  // (whole 2 KB tiles: aligned)
+    *c.copy = (double *)at;
+    at += (size_t)f64_elems(f64_geom_a(s.No, s.Nv, c.K)) * sizeof(double);
   }
 }
 
-// Zeroes the FP64 operands of a system whose upload leaves their padding
-// unwritten.
+// Zeroes the arrays of a system whose upload leaves the padding of its FP64
+// operands unwritten.
 void clear_operands(DevSystem &s, hipStream_t st) {
-  auto zero = [&](double *x, bool a, int64_t K) {
-    if (!x) return;
-    const TriGeom g = a ? f64_geom_a(s.No, s.Nv, K) : f64_geom_b(s.No, s.Nv, K);
-    check(hipMemsetAsync(x, 0, (size_t)f64_elems(g) * sizeof(double), st),
-          "clear operands");
-  };
-  for (double *x : {s.T3, s.T3s, s.T3i, s.T3is}) zero(x, true, s.Kv);
-  for (double *x : {s.H3, s.H3s, s.H3J, s.H3Js, s.H3i, s.H3is, s.H3Ji, s.H3Jis})
-    zero(x, true, s.Ko);
-  for (double *x : {s.V3, s.V3J, s.V3i, s.V3Ji}) zero(x, false, s.Kv);
-  for (double *x : {s.T2N, s.T2TN, s.T2Ni, s.T2TNi}) zero(x, false, s.Ko);
+  if (s.store != 0) return;
+  check(hipMemsetAsync(s.block, 0, s.block_bytes, st), "clear operands");
+  if (s.swaps) check(hipMemsetAsync(s.swaps, 0, s.swap_bytes, st), "clear operands");
 }
 
+// Device memory of a system: while alloc_system lays it out a piece of its one
+// block (first counted, then placed), later allocations of their own.
 void *dev_bytes(DevSystem &s, size_t bytes, const char *what) {
+  bytes = std::max<size_t>(bytes, 1);
+  if (s.laying != DevSystem::NONE) {
+    const size_t at = s.block_bytes;
+    s.block_bytes += (bytes + 255) / 256 * 256;
+    if (s.laying == DevSystem::COUNT) return nullptr;
+    s.bytes += bytes;
+    return (char *)s.block + at;
+  }
   void *p = nullptr;
-  check(hipMalloc(&p, std::max<size_t>(bytes, 1)), what);
+  check(hipMalloc(&p, bytes), what);
   s.allocations.push_back(p);
   s.bytes += bytes;
   return p;
@@ -227,15 +231,14 @@ bool atrip_amd::drop_swap_copies(atrip_hip_ctx *ctx) {
   if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
   for (auto &kv : ctx->systems) {
     DevSystem &s = kv.second;
-    for (const SwapCopy &c : swap_copies(s)) {
-      if (!*c.copy) continue;
-      s.allocations.erase(std::find(s.allocations.begin(), s.allocations.end(),
-                                    (void *)*c.copy));
-      (void)hipFree(*c.copy);
-      *c.copy = nullptr;
-      s.bytes -= (uint64_t)f64_elems(f64_geom_a(s.No, s.Nv, c.K)) * sizeof(double);
-      any = true;
-    }
+    if (!s.swaps) continue;
+    for (const SwapCopy &c : swap_copies(s)) *c.copy = nullptr;
+    s.allocations.erase(
+        std::find(s.allocations.begin(), s.allocations.end(), s.swaps));
+    (void)hipFree(s.swaps);
+    s.swaps = nullptr;
+    s.bytes -= s.swap_bytes;
+    any = true;
   }
   return any;
 }
@@ -275,18 +278,9 @@ uint64_t atrip_amd::system_bytes(int64_t No, int64_t Nv, bool with_j,
 
 namespace {
 
-void alloc_system(atrip_hip_ctx *ctx, DevSystem &s, int64_t No, int64_t Nv,
-                  bool with_j, bool cplx = false) {
-  if (No < 1 || Nv < 1) throw Fail{"No and Nv must be positive"};
-  if (cplx && ctx->operand_store != 0)
-    throw Fail{"complex systems keep FP64 operands (operand_store 0)"};
-  if (No > 1023) throw Fail{"No > 1023 is not supported"};
-  s.No = No;
-  s.Nv = Nv;
-  s.Kv = pad16(Nv);
-  s.Ko = pad16(No);
-  const int64_t N2 = No * No, Nv2 = Nv * Nv;
-  s.store = ctx->operand_store;
+// The arrays of a system but its row-swapped copies.
+void lay_out(DevSystem &s, bool with_j, bool cplx) {
+  const int64_t No = s.No, Nv = s.Nv, N2 = No * No, Nv2 = Nv * Nv;
   // doubles operands: FP64, or only their split / FP32 / bf16x3 form
   auto operand = [&](double *&x, DevSystem::Split &sp, TriOp &tp,
                      const TriGeom &g, const char *what) {
@@ -342,41 +336,42 @@ void alloc_system(atrip_hip_ctx *ctx, DevSystem &s, int64_t No, int64_t Nv,
       s.H3Jin = dev_alloc(s, f64_elems(gh), "alloc -H3J (im)");
     }
   }
+  s.npoints = No * (No + 1) * (No + 2) / 6;
+  s.points = (uint32_t *)dev_bytes(s, (size_t)s.npoints * sizeof(uint32_t),
+                                   "alloc points");
+  s.aprefix = (uint64_t *)dev_bytes(s, (size_t)(Nv + 1) * sizeof(uint64_t),
+                                    "alloc prefix");
+}
+
+// One block holds all of a system's arrays: an allocation for each, with its
+// release, took a fifth of a small system's upload (No=10, Nv=50: upload and
+// release 930 -> 730 us with the two tables made on the device and no wait
+// between the tensors).
+void alloc_system(atrip_hip_ctx *ctx, DevSystem &s, int64_t No, int64_t Nv,
+                  bool with_j, bool cplx = false) {
+  if (No < 1 || Nv < 1) throw Fail{"No and Nv must be positive"};
+  if (cplx && ctx->operand_store != 0)
+    throw Fail{"complex systems keep FP64 operands (operand_store 0)"};
+  if (No > 1023) throw Fail{"No > 1023 is not supported"};
+  s.No = No;
+  s.Nv = Nv;
+  s.Kv = pad16(Nv);
+  s.Ko = pad16(No);
+  s.store = ctx->operand_store;
+  s.laying = DevSystem::COUNT;
+  lay_out(s, with_j, cplx);
+  check(hipMalloc(&s.block, s.block_bytes), "alloc system");
+  s.allocations.push_back(s.block);
+  s.block_bytes = 0;
+  s.laying = DevSystem::PLACE;
+  lay_out(s, with_j, cplx);
+  s.laying = DevSystem::NONE;
   if (s.store == 0 && ctx->operand_swaps) alloc_swaps(s);
-  // i >= j >= k points of the energy loops, packed 10 bits per index
-  std::vector<uint32_t> pts;
-  for (int64_t k = 0; k < No; k++)
-    for (int64_t j = k; j < No; j++)
-      for (int64_t i = j; i < No; i++)
-        pts.push_back((uint32_t)(i | (j << 10) | (k << 20)));
-  s.npoints = (int64_t)pts.size();
-  {
-    void *p = nullptr;
-    check(hipMalloc(&p, pts.size() * sizeof(uint32_t)), "alloc points");
-    s.allocations.push_back(p);
-    s.bytes += pts.size() * sizeof(uint32_t);
-    check(hipMemcpy(p, pts.data(), pts.size() * sizeof(uint32_t),
-                    hipMemcpyHostToDevice),
-          "upload points");
-    s.points = (uint32_t *)p;
-  }
-  // tuples with first index < a, for the canonical index
-  std::vector<uint64_t> pre(Nv + 1, 0);
-  for (int64_t a = 0; a < Nv; a++) {
-    const uint64_t m = (uint64_t)(Nv - a);
-    pre[a + 1] = pre[a] + m * (m + 1) / 2 - 1;
-  }
-  {
-    void *p = nullptr;
-    check(hipMalloc(&p, pre.size() * sizeof(uint64_t)), "alloc prefix");
-    s.allocations.push_back(p);
-    s.bytes += pre.size() * sizeof(uint64_t);
-    check(hipMemcpy(p, pre.data(), pre.size() * sizeof(uint64_t),
-                    hipMemcpyHostToDevice),
-          "upload prefix");
-    s.aprefix = (uint64_t *)p;
-  }
-  (void)ctx;
+}
+
+// The points and prefix tables (see launch_tables), after any clearing.
+void fill_tables(const DevSystem &s, hipStream_t st) {
+  check(launch_tables(s, st), "point and prefix tables");
 }
 
 // Where the values of a system's input tensors come from.  Values are in
@@ -476,33 +471,54 @@ struct ReaderSource : Source {
   }
 };
 
+// Device staging of an upload: one buffer, grown to the largest step of its
+// tensors (at most stage_kb, or one slab), given back at the end.
+struct Stage {
+  hipStream_t st;
+  void *p = nullptr;
+  size_t bytes = 0;
+  explicit Stage(hipStream_t s) : st(s) {}
+  Stage(const Stage &) = delete;
+  ~Stage() { drop(); }
+  void drop() {
+    if (!p) return;
+    (void)hipStreamSynchronize(st);  // the kernels that read it
+    (void)hipFree(p);
+    p = nullptr;
+    bytes = 0;
+  }
+  double *get(size_t need) {
+    if (need > bytes) {
+      drop();
+      check(hipMalloc(&p, need), "alloc staging");
+      bytes = need;
+    }
+    return (double *)p;
+  }
+};
+
 // Stage tensor t through a bounded device buffer (the context's stage_kb),
 // whole slabs of `slab` values of its slowest CTF index per step (n_slow
 // slabs; at least one slab per step), and hand each staged chunk to
-// `place(dev_chunk, first_slow, count_slow)`.
-template <typename P>
-void staged(atrip_hip_ctx *ctx, Source &src, int t, int64_t slab,
-            int64_t n_slow, P &&place) {
+// `place(dev_chunk, first_slow, count_slow)`.  A step's copy follows the kernels
+// that read the buffer before it on the stream.
+int64_t stage_slabs(const atrip_hip_ctx *ctx, int comp, int64_t slab,
+                    int64_t n_slow) {
   const int64_t budget = std::max<int64_t>(
-      1, ctx->stage_kb * 1024 / (int64_t)(sizeof(double) * src.comp));
-  int64_t per = std::max<int64_t>(1, budget / std::max<int64_t>(slab, 1));
-  per = std::min(per, n_slow);
-  void *stage = nullptr;
-  check(hipMalloc(&stage, (size_t)(per * slab * src.comp) * sizeof(double)),
-        "alloc staging");
-  try {
-    for (int64_t s0 = 0; s0 < n_slow; s0 += per) {
-      const int64_t cnt = std::min(per, n_slow - s0);
-      src.fetch(t, s0 * slab, cnt * slab, (double *)stage, ctx->stream);
-      place((const double *)stage, s0, cnt);
-      check(hipStreamSynchronize(ctx->stream), "relayout");
-    }
-  } catch (...) {
-    (void)hipStreamSynchronize(ctx->stream);
-    (void)hipFree(stage);
-    throw;
+      1, ctx->stage_kb * 1024 / (int64_t)(sizeof(double) * comp));
+  return std::min(std::max<int64_t>(1, budget / std::max<int64_t>(slab, 1)),
+                  n_slow);
+}
+template <typename P>
+void staged(atrip_hip_ctx *ctx, Stage &stage, Source &src, int t, int64_t slab,
+            int64_t n_slow, P &&place) {
+  const int64_t per = stage_slabs(ctx, src.comp, slab, n_slow);
+  double *buf = stage.get((size_t)(per * slab * src.comp) * sizeof(double));
+  for (int64_t s0 = 0; s0 < n_slow; s0 += per) {
+    const int64_t cnt = std::min(per, n_slow - s0);
+    src.fetch(t, s0 * slab, cnt * slab, buf, ctx->stream);
+    place((const double *)buf, s0, cnt);
   }
-  check(hipFree(stage), "free staging");
 }
 
 // A system that keeps only the split / FP32 / bf16x3 form of its doubles
@@ -564,7 +580,15 @@ void upload_tensors(atrip_hip_ctx *ctx, DevSystem &s, DevSystem *im,
   DevSystem *dst[2] = {&s, im};
   hipStream_t st = ctx->stream;
   clear_operands(s, st);
+  fill_tables(s, st);
   TempOperands tmp{s, st, {}};
+  Stage stage(st);
+  if (s.store == 0) {  // (beside no temporary operands)
+    auto need = [&](int64_t slab, int64_t n_slow) {
+      return stage_slabs(ctx, m, slab, n_slow) * slab * m * sizeof(double);
+    };
+    stage.get(std::max({need(Nv2 * No, No), need(N2 * No, Nv), need(Nv2 * Nv, No)}));
+  }
   tmp.add(s.T3, s.sT3, s.tT3, f64_geom_a(No, Nv, Kv));
   tmp.add(s.T2N, s.sT2N, s.tT2N, f64_geom_b(No, Nv, Ko));
   tmp.add(s.T2TN, s.sT2TN, s.tT2TN, f64_geom_b(No, Nv, Ko));
@@ -580,7 +604,7 @@ void upload_tensors(atrip_hip_ctx *ctx, DevSystem &s, DevSystem *im,
             what);
   };
   // Tabij {Nv,Nv,No,No}: slowest index j
-  staged(ctx, src, ATRIP_TENSOR_TABIJ, Nv2 * No, No,
+  staged(ctx, stage, src, ATRIP_TENSOR_TABIJ, Nv2 * No, No,
          [&](const double *c, int64_t j0, int64_t cj) {
            for (int part = 0; part < m; part++) {
              DevSystem &d = *dst[part];
@@ -606,7 +630,7 @@ void upload_tensors(atrip_hip_ctx *ctx, DevSystem &s, DevSystem *im,
            }
          });
   // Vabij {Nv,Nv,No,No}: VHH[pair][i + No j]
-  staged(ctx, src, ATRIP_TENSOR_VABIJ, Nv2 * No, No,
+  staged(ctx, stage, src, ATRIP_TENSOR_VABIJ, Nv2 * No, No,
          [&](const double *c, int64_t j0, int64_t cj) {
            for (int part = 0; part < m; part++)
              check(launch_transpose(c + part, dst[part]->VHH + j0 * No, 1,
@@ -616,7 +640,7 @@ void upload_tensors(atrip_hip_ctx *ctx, DevSystem &s, DevSystem *im,
          });
   // Vijka {No,No,No,Nv}: H3[x][row][L] = V[row,L,x]
   auto hhh = [&](int t, double *DevSystem::*arr, double *DevSystem::*arrs) {
-    staged(ctx, src, t, N2 * No, Nv,
+    staged(ctx, stage, src, t, N2 * No, Nv,
            [&](const double *c, int64_t x0, int64_t cx) {
              for (int part = 0; part < m; part++) {
                TileMap t, w;
@@ -630,7 +654,7 @@ void upload_tensors(atrip_hip_ctx *ctx, DevSystem &s, DevSystem *im,
   };
   // Vabci {Nv,Nv,Nv,No}: V3[pair][r][E] = V[pair,E,r]
   auto ppph = [&](int t, double *DevSystem::*arr) {
-    staged(ctx, src, t, Nv2 * Nv, No,
+    staged(ctx, stage, src, t, Nv2 * Nv, No,
            [&](const double *c, int64_t r0, int64_t cr) {
              for (int part = 0; part < m; part++) {
                TileMap t;
@@ -658,19 +682,27 @@ void upload_tensors(atrip_hip_ctx *ctx, DevSystem &s, DevSystem *im,
     tmp.convert();
   }
   // the small tensors whole (the reference's read_all, Atrip.cxx:176-181)
+  std::vector<std::vector<double>> kept;  // until the copies are done
   auto small = [&](int t, int64_t n, double *DevSystem::*arr, const char *what) {
-    std::vector<double> buf((size_t)(n * m)), part((size_t)n);
+    std::vector<double> buf((size_t)(n * m));
     src.host(t, 0, n, buf.data());
     for (int q = 0; q < m; q++) {
+      std::vector<double> part((size_t)n);
       for (int64_t e = 0; e < n; e++) part[e] = buf[e * m + q];
-      check(hipMemcpy(dst[q]->*arr, part.data(), (size_t)n * sizeof(double),
-                      hipMemcpyHostToDevice),
+      kept.push_back(std::move(part));
+      check(hipMemcpyAsync(dst[q]->*arr, kept.back().data(),
+                           (size_t)n * sizeof(double), hipMemcpyHostToDevice, st),
             what);
     }
   };
+  struct Done {  // no copy reads host memory or the stage after this returns
+    hipStream_t st;
+    ~Done() { (void)hipStreamSynchronize(st); }
+  } done{st};
   small(ATRIP_TENSOR_TAI, Nv * No, &DevSystem::Tai, "upload Tai");
   small(ATRIP_TENSOR_EI, No, &DevSystem::ei, "upload ei");
   small(ATRIP_TENSOR_EA, Nv, &DevSystem::ea, "upload ea");
+  check(hipStreamSynchronize(st), "upload");
 }
 
 // The imaginary planes of a complex system in the slots of the real ones
@@ -1356,6 +1388,7 @@ int atrip_hip_upload_synthetic_scaled(atrip_hip_ctx *ctx, int64_t No,
     DevSystem s;
     try {
       alloc_system(ctx, s, No, Nv, with_j != 0);
+      fill_tables(s, ctx->stream);
       check(launch_synth(s, seed, with_j != 0, ctx->stream, 0, scale),
             "synthetic fill");
       check(hipStreamSynchronize(ctx->stream), "synthetic fill");
@@ -1439,6 +1472,7 @@ int atrip_hip_upload_synthetic_complex(atrip_hip_ctx *ctx, int64_t No,
     DevSystem s;
     try {
       alloc_system(ctx, s, No, Nv, with_j != 0, true);
+      fill_tables(s, ctx->stream);
       check(launch_synth(s, seed, with_j != 0, ctx->stream), "synthetic fill");
       DevSystem v = imag_view(s);
       check(launch_synth(v, seed, with_j != 0, ctx->stream, ATRIP_SYN_IMAG),

@@ -197,6 +197,9 @@ struct DevSystem {
   uint64_t *aprefix = nullptr;            // tuples with first index < a
   uint64_t bytes = 0;
   std::vector<void *> allocations;
+  void *block = nullptr, *swaps = nullptr;  // all arrays; the swapped copies
+  size_t block_bytes = 0, swap_bytes = 0;
+  enum { NONE, COUNT, PLACE } laying = NONE;  // (see dev_bytes)
 };
 
 // bf16 of a float, round to nearest even (finite inputs).
@@ -418,6 +421,9 @@ hipError_t launch_energy_z(const DevSystem &s, const BatchArgs &b,
                            double tai_sign, double *e_slot, double *wcube,
                            bool fused, hipStream_t st);
 
+// The points table of a system (i >= j >= k, packed 10 bits per index, k
+// slowest) and its prefix table (tuples with a smaller first index).
+hipError_t launch_tables(const DevSystem &s, hipStream_t st);
 // Per window of a batch (nw windows of `per` slots), a compensated sum of
 // its slot energies in a fixed order: out[2 w] = sum, out[2 w + 1] =
 // compensation.

@@ -318,4 +318,29 @@ hipError_t launch_scale(const double *src, double *dst, int64_t n,
   return hipGetLastError();
 }
 
+// One thread per row (k, j) of points and per prefix entry.
+__global__ __launch_bounds__(256) void tables_kernel(uint32_t *points,
+                                                     uint64_t *prefix,
+                                                     int64_t No, int64_t Nv) {
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  auto tri = [](int64_t n) { return n * (n + 1) * (n + 2) / 6; };
+  if (t < No * No) {
+    const int64_t k = t / No, j = t % No, m = No - k, d = j - k;
+    if (d >= 0) {
+      // rows of smaller k, then rows k .. j - 1 of this k (m, m - 1, ... points)
+      uint32_t *at = points + (tri(No) - tri(m)) + d * m - d * (d - 1) / 2;
+      for (int64_t i = j; i < No; i++)
+        at[i - j] = (uint32_t)(i | (j << 10) | (k << 20));
+    }
+  }
+  if (t <= Nv) prefix[t] = (uint64_t)(tri(Nv) - tri(Nv - t) - t);
+}
+
+hipError_t launch_tables(const DevSystem &s, hipStream_t st) {
+  const int64_t n = std::max(s.No * s.No, s.Nv + 1);
+  hipLaunchKernelGGL(tables_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256),
+                     0, st, s.points, s.aprefix, s.No, s.Nv);
+  return hipGetLastError();
+}
+
 }  // namespace atrip_amd
