@@ -186,7 +186,9 @@ int atrip_hip_run_noalloc(atrip_hip_ctx *ctx, int sys, int precision,
  * needed): *nb the window edge (`window` 0 = automatic, as the context
  * option) and *fm x *fn the doubles kernel's wave tile in MFMA fragments
  * (16x16 FP64 fragments for ATRIP_FP64, 32x32 for the other forms), the
- * automatic pick of a context whose "tile" option is -1.  No counterpart in
+ * automatic pick of a context whose "tile" option is -1.  A range that is not
+ * the whole tuple space takes windows of its own, at most that edge in the first
+ * index.  No counterpart in
  * the reference, which has no tiles; for callers that size or schedule runs
  * from the plan.  Returns nonzero for No or Nv below 1, a window outside
  * 0..32 or an unknown precision. */
