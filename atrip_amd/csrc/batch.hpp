@@ -22,6 +22,8 @@ struct Win {
 // Windows (block triples of edge nb) holding at least one tuple, in
 // lexicographic order, with their tuple counts.
 std::vector<Win> windows_of(int64_t Nv, int nb);
+// Dispatch order of windows of these costs: largest first, ties in order.
+std::vector<int32_t> longest_first(const std::vector<double> &cost);
 // Modelled cycles of one full window on one workgroup.
 double window_cycles(int64_t No, int64_t Nv, int nb, int tile, int precision);
 // Window edge nb fits the scratch bound at this grid.

@@ -28,7 +28,6 @@
 #include <cmath>
 #include <deque>
 #include <map>
-#include <numeric>
 #include <string>
 #include <vector>
 
@@ -274,10 +273,7 @@ int step(atrip_hip_server *srv) {
     took.push_back({id, k});
   }
   if (!tasks.empty()) {
-    std::vector<int32_t> order(tasks.size());
-    std::iota(order.begin(), order.end(), 0);
-    std::stable_sort(order.begin(), order.end(),
-                     [&](int32_t x, int32_t y) { return cost[x] > cost[y]; });
+    const std::vector<int32_t> order = longest_first(cost);
     const LaunchOut out = retry_memory(ctx, [&] {
       std::vector<BSys> sys;
       std::vector<BSplit> split;
