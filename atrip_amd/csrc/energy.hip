@@ -872,7 +872,7 @@ hipError_t launch_small(const FusedParams &P, hipStream_t st) {
     /* beyond the 64 KB every launch may have */                            \
     hipError_t e = hipFuncSetAttribute(                                     \
         (const void *)energy_small_kernel<GT, HJ, TT, NI>,                  \
-        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);              \
+        hipFuncAttributeMaxDynamicSharedMemorySize, MAX_LDS);              \
     if (e != hipSuccess) return e;                                          \
     hipLaunchKernelGGL((energy_small_kernel<GT, HJ, TT, NI>), grid,         \
                        TT < 256 ? 256 : TT, lds, st, P);                    \

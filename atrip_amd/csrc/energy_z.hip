@@ -362,7 +362,7 @@ hipError_t launch_z_small(const EnergyZParams &P, hipStream_t st) {
     /* beyond the 64 KB every launch may have */                              \
     hipError_t e = hipFuncSetAttribute(                                       \
         (const void *)energy_z_small_kernel<HJ, TT, NI>,                      \
-        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);                \
+        hipFuncAttributeMaxDynamicSharedMemorySize, MAX_LDS);                \
     if (e != hipSuccess) return e;                                            \
     hipLaunchKernelGGL((energy_z_small_kernel<HJ, TT, NI>), grid,             \
                        TT < 256 ? 256 : TT, lds, st, P);                      \

@@ -131,6 +131,9 @@ __host__ __device__ inline int64_t n_triples(int64_t nbk) {
 __host__ __device__ inline bool small_energy(int64_t No, bool use_j, bool g32) {
   return No <= (use_j || g32 ? 20 : 18);
 }
+// Dynamic LDS those kernels are allowed (the same for every launch, so that
+// threads do not undo each other's); the largest use is 155,200 bytes.
+constexpr int MAX_LDS = 156 * 1024;
 // The same for complex systems, whose two planes of W (four with (cT)) fit 160 KB.
 __host__ __device__ inline bool small_energy_z(int64_t No, bool use_j) {
   return No <= (use_j ? 16 : 20);
