@@ -866,10 +866,11 @@ void drop_pending_events(atrip_hip_ctx *ctx) {
 
 // Runs every batch of windows intersecting [first, last).  When `sink` is
 // given it receives the per-slot energies of each batch.
-// A fixed device region a run may carve its scratch from (no allocation).
+// A fixed device region a run may carve its scratch from (no allocation), and
+// the bytes behind it that only the padding of class buffers may take.
 struct FixedScratch {
   void *base;
-  size_t bytes;
+  size_t bytes, pad;
 };
 
 // Which windows of the plan a run covers besides the tuple range: every
@@ -917,6 +918,18 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
   // select windows and count their tuples in range
   Windows win;
   win.ea = win.eb = win.ec = nb;
+  // Windows of the run's own, with edges (ea, eb, ec) of `win`, from the
+  // range's first index on.
+  const HostIndex hidx((uint64_t)s.Nv);
+  const int64_t a0 = hidx.first_of(first), a1 = hidx.first_of(last - 1);
+  auto own_windows = [&](int ea) {
+    win.origin.clear();
+    win.count.clear();
+    win.ea = ea;
+    for (int64_t a = a0; a <= a1; a += win.ea)
+      for (int64_t b = a0 + (a - a0) / win.eb * win.eb; b < s.Nv; b += win.eb)
+        for (int64_t c = b; c < s.Nv; c += win.ec) win.add(hidx, first, last, a, b, c);
+  };
   if (full) {
     const size_t nwin = plan.wcount.size();
     int64_t pair = -1, prev_a = -1, prev_b = -1;  // (alpha, beta) row index
@@ -938,25 +951,21 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
     // takes windows of its own: the first index of the range's tuples cut
     // evenly into blocks of at most the edge.  Blocks aligned as the plan's
     // left the window columns of the other first indices empty.
-    const HostIndex h((uint64_t)s.Nv);
-    const int64_t a0 = h.first_of(first), a1 = h.first_of(last - 1);
     const int64_t na = a1 - a0 + 1, blocks = (na + nb - 1) / nb;
-    win.ea = (int)((na + blocks - 1) / blocks);
-    for (int64_t a = a0; a <= a1; a += win.ea)
-      for (int64_t b = a0 + (a - a0) / win.eb * win.eb; b < s.Nv; b += win.eb)
-        for (int64_t c = b; c < s.Nv; c += win.ec) win.add(h, first, last, a, b, c);
+    own_windows((int)((na + blocks - 1) / blocks));
   }
   const std::vector<int32_t> &sel = win.origin;
   for (uint64_t c : win.count) res.tuples += c;
-  const int nsel = (int)win.count.size();
+  int nsel = (int)win.count.size();
   if (!nsel) return res;
   // Device scratch of the run: class buffers G (and those of the (cT)
   // pass; two planes each for complex systems), per-slot energies, the energy
   // kernels' scratch (per-triple partials, or W cubes for complex systems
   // and the cube epilogue), batch partials and the window list.  Taken from the context's buffers (grown
   // on demand), or carved out of a fixed region without any allocation
-  // (then the windows per launch shrink until the run fits).
-  const int64_t per = (int64_t)win.ea * win.eb * win.ec;  // slots of a window
+  // (then the windows per launch shrink until the run fits, and the window
+  // list and partials of a few launches at a time are held).
+  int64_t per = (int64_t)win.ea * win.eb * win.ec;  // slots of a window
   const int64_t W3 = g_elems(s.No);  // one tuple's class buffer
   const bool use_j = s.has_j;
   const int nsets = s.cplx ? 2 : 1;  // W's planes
@@ -965,21 +974,25 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
   struct Sizes {
     int64_t slots_max = 0;
     size_t gsz = 0, g = 0, e_slot = 0, wcube = 0, partials = 0, windows = 0;
-    int nbatch = 0;
+    int nbatch = 0, group = 0;  // launches; launches of one window list
   };
-  auto sizes = [&](int bw_) {
+  auto sizes = [&](int bw_, int64_t W3_) {
     Sizes z;
     z.slots_max = (int64_t)std::min(bw_, nsel) * per;
-    z.gsz = (size_t)(3 * z.slots_max * W3) * gelem;
+    z.gsz = (size_t)(3 * z.slots_max * W3_) * gelem;
     z.g = (size_t)((use_j ? 2 : 1) * nsets) * z.gsz;
     z.e_slot = (size_t)(2 * z.slots_max) * sizeof(double);
     z.wcube = (size_t)(z.slots_max * energy_scratch_per_slot(
                                          s.No, use_j, g32, s.cplx, fused)) *
               sizeof(double);
-    z.nbatch = (nsel + bw_ - 1) / bw_;
-    z.partials = (size_t)(4 * z.nbatch * slot_partials(z.slots_max)) *
-                 sizeof(double);
-    z.windows = sel.size() * sizeof(int32_t);
+    z.nbatch = z.group = (nsel + bw_ - 1) / bw_;
+    const size_t quads = (size_t)(4 * slot_partials(z.slots_max)) * sizeof(double),
+                 list = (size_t)(3 * bw_) * sizeof(int32_t);
+    if (fixed)
+      z.group = (int)std::min<size_t>(
+          z.nbatch, std::max<size_t>(1, (256 * 1024) / (quads + list)));
+    z.partials = z.group * quads;
+    z.windows = std::min(z.group * list, sel.size() * sizeof(int32_t));
     return z;
   };
   auto a256 = [](size_t x) { return (x + 255) / 256 * 256; };
@@ -1005,23 +1018,42 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
   if (fixed && kWinSums)
     throw Fail{"per-window sums are not an allocation-free run"};
   if (fixed) {
-    while (bw > 1 && total(sizes(bw)) > fixed->bytes) bw--;
-    z = sizes(bw);
-    if (total(z) > fixed->bytes) {
-      // largest window edge whose single window fits (class buffers, cubes
-      // and slot energies scale with edge^3)
-      const size_t per_slot = (z.g + z.wcube + z.e_slot) / (size_t)per;
-      const size_t rest = a256(z.partials) + a256(z.windows) + 3 * 256;
-      int fit = 0;
-      for (int e = nb - 1; e >= 1 && !fit; e--)
-        if ((size_t)e * e * e * per_slot + rest <= fixed->bytes) fit = e;
-      throw Fail{"run needs " + std::to_string(total(z)) +
-                 " bytes of scratch for one window of edge " +
-                 std::to_string(nb) + " at No=" + std::to_string(s.No) +
-                 "; the allocation-free entry point holds " +
-                 std::to_string(fixed->bytes) +
-                 (fit ? " (window edge " + std::to_string(fit) + " fits)"
-                      : " (no window edge fits this No)")};
+    while (bw > 1 && total(sizes(bw, W3)) > fixed->bytes) bw--;
+    z = sizes(bw, W3);
+    // What the region holds is counted in class buffers of GEMM order, rows
+    // padded to a line.  Blocks of 8^3 take more (2.8 times at No=17, 1.7 at
+    // 20), so a window that fits but for them is cut along its first index.
+    // Where the edge is 1 already, their padding has `pad`.
+    if (const size_t need = total(z); need > fixed->bytes) {
+      const Sizes zg = sizes(1, std::min(W3, g_row_elems(s.No, g32)));
+      const size_t per_slot = (zg.g + zg.wcube + zg.e_slot) / (size_t)per;
+      const size_t slab = (z.g + z.wcube + z.e_slot) / (size_t)win.ea;
+      const size_t limit = fixed->bytes + fixed->pad;
+      int ea = total(zg) > fixed->bytes
+                   ? 0
+                   : (int)std::min<size_t>(win.ea, limit / slab);
+      for (; ea >= 1; ea--) {
+        if (ea < win.ea) own_windows(ea);
+        per = (int64_t)win.ea * win.eb * win.ec;
+        nsel = (int)win.count.size();
+        z = sizes(1, W3);
+        if (total(z) <= limit) break;
+      }
+      if (ea < 1) {
+        // largest window edge whose single window fits (class buffers, cubes
+        // and slot energies scale with edge^3)
+        const size_t rest = a256(zg.partials) + a256(zg.windows) + 3 * 256;
+        int fit = 0;
+        for (int e = nb - 1; e >= 1 && !fit; e--)
+          if ((size_t)e * e * e * per_slot + rest <= fixed->bytes) fit = e;
+        throw Fail{"run needs " + std::to_string(need) +
+                   " bytes of scratch for one window of edge " +
+                   std::to_string(nb) + " at No=" + std::to_string(s.No) +
+                   "; the allocation-free entry point holds " +
+                   std::to_string(fixed->bytes) +
+                   (fit ? " (window edge " + std::to_string(fit) + " fits)"
+                        : " (no window edge fits this No)")};
+      }
     }
     char *p = (char *)fixed->base;
     Gbuf = p;
@@ -1032,12 +1064,9 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
     p += a256(z.wcube);
     partials = p;
     p += a256(z.partials);
-    d_sel = p;
-    check(hipMemcpyAsync(d_sel, sel.data(), z.windows, hipMemcpyHostToDevice,
-                         ctx->stream),
-          "upload windows");
+    d_sel = p;  // (filled by the launches)
   } else {
-    z = sizes(bw);
+    z = sizes(bw, W3);
     // the window list lives in a context buffer grown on demand (no
     // allocation and release per call); the copy is ordered on the stream
     // before the kernels that read it, and `sel` outlives it (the run
@@ -1062,7 +1091,7 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
         if (bw <= bw_least) throw;
         (void)hipGetLastError();
         bw = bw_least;
-        z = sizes(bw);
+        z = sizes(bw, W3);
       }
     }
     Gbuf = ctx->G;
@@ -1093,11 +1122,46 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
   void *G = Gbuf;
   void *GJ = use_j ? (void *)((char *)Gbuf + gsz) : nullptr;
   std::vector<double> host_slots;
+  // Neumaier over the partials in slot order
+  double s0 = 0, c0 = 0, s1 = 0, c1 = 0;
+  std::vector<double> part;
+  auto fetch_partials = [&] {
+    part.resize(4 * nparts);
+    check(hipMemcpyAsync(part.data(), (double *)partials,
+                         part.size() * sizeof(double), hipMemcpyDeviceToHost, st),
+          "download partials");
+  };
+  auto add_partials = [&] {
+    auto add = [](double &sum, double &comp, double x) {
+      const double t = sum + x;
+      comp += (std::fabs(sum) >= std::fabs(x)) ? (sum - t) + x : (x - t) + sum;
+      sum = t;
+    };
+    for (int64_t bi = 0; bi < nparts; bi++) {
+      add(s0, c0, part[4 * bi]);
+      add(s0, c0, part[4 * bi + 1]);
+      add(s1, c1, part[4 * bi + 2]);
+      add(s1, c1, part[4 * bi + 3]);
+    }
+    nparts = 0;
+  };
   for (int bi = 0; bi < nbatch; bi++) {
     BatchArgs b;
-    const int w0 = bi * bw;
+    const int w0 = bi * bw, listed = fixed ? bi / z.group * z.group * bw : 0;
+    if (fixed && w0 == listed) {
+      if (bi) {
+        fetch_partials();
+        check(hipStreamSynchronize(st), "run");
+        add_partials();
+      }
+      const int n = (int)std::min<int64_t>((int64_t)z.group * bw, nsel - w0);
+      check(hipMemcpyAsync(d_sel, sel.data() + 3 * (size_t)w0,
+                           (size_t)(3 * n) * sizeof(int32_t),
+                           hipMemcpyHostToDevice, st),
+            "upload windows");
+    }
     b.nw = std::min(bw, nsel - w0);
-    b.windows = (const int32_t *)d_sel + 3 * w0;
+    b.windows = (const int32_t *)d_sel + 3 * (w0 - listed);
     b.aprefix = s.aprefix;
     b.ea = win.ea;
     b.eb = win.eb;
@@ -1182,10 +1246,7 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
       sink(sel.data() + 3 * w0, b, host_slots);
     }
   }
-  std::vector<double> part(4 * nparts);
-  check(hipMemcpyAsync(part.data(), (double *)partials, part.size() * sizeof(double),
-                       hipMemcpyDeviceToHost, st),
-        "download partials");
+  fetch_partials();
   std::vector<double> wsums(kWinSums ? 2 * (size_t)nsel : 0);
   if (kWinSums)
     check(hipMemcpyAsync(wsums.data(), wsum_dev, wsz, hipMemcpyDeviceToHost,
@@ -1193,19 +1254,7 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
           "download window sums");
   check(hipStreamSynchronize(st), "run");
   if constexpr (kWinSums) sink.windows(wsums);
-  // Neumaier over the partials in slot order
-  double s0 = 0, c0 = 0, s1 = 0, c1 = 0;
-  auto add = [](double &sum, double &comp, double x) {
-    const double t = sum + x;
-    comp += (std::fabs(sum) >= std::fabs(x)) ? (sum - t) + x : (x - t) + sum;
-    sum = t;
-  };
-  for (int64_t bi = 0; bi < nparts; bi++) {
-    add(s0, c0, part[4 * bi]);
-    add(s0, c0, part[4 * bi + 1]);
-    add(s1, c1, part[4 * bi + 2]);
-    add(s1, c1, part[4 * bi + 3]);
-  }
+  add_partials();
   res.e = s0 + c0;
   res.ect = s1 + c1;
   // collect event timings
@@ -1262,11 +1311,11 @@ void atrip_amd::run_plan_windows(atrip_hip_ctx *ctx, int sys, int precision,
 
 void atrip_amd::run_fixed(atrip_hip_ctx *ctx, int sys, int precision,
                           int ijkabc, uint64_t first, uint64_t count,
-                          void *base, size_t bytes, double *energy,
-                          double *ct_energy) {
+                          void *base, size_t bytes, size_t pad,
+                          double *energy, double *ct_energy) {
   const uint64_t last =
       count == ~0ULL || first + count < first ? ~0ULL : first + count;
-  const FixedScratch fx{base, bytes};
+  const FixedScratch fx{base, bytes, pad};
   RunResult r = run_range(ctx, sys, precision, ijkabc, first, last, NoSink{},
                           WindowSel{}, &fx);
   *energy = ijkabc ? r.e : -r.e;

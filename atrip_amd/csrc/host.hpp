@@ -91,12 +91,17 @@ int guarded_memory(atrip_hip_ctx *ctx, F &&f) {
 // atrip_hip_run over [first, first + count) with every piece of device
 // scratch (class buffers, W cubes, slot energies, batch partials, window
 // list) carved out of [base, base + bytes): no device allocation, no timing
-// events.  The windows per launch shrink until a launch fits; a run whose
+// events.  The windows per launch shrink until a launch fits, and a window
+// that fits but for the padding of the class buffers' blocks is cut (with
+// edge 1 the padding takes up to `pad` bytes behind the region); a run whose
 // single window does not fit, or a mixed form whose operand copies are not
 // resident yet, throws Fail.  Writes the signed energies like atrip_hip_run.
 void run_fixed(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
                uint64_t first, uint64_t count, void *base, size_t bytes,
-               double *energy, double *ct_energy);
+               size_t pad, double *energy, double *ct_energy);
+// Bytes behind the allocation-free region: the most that a window of edge 1
+// counted as fitting it takes beyond it (No=233, FP32 products, cube epilogue).
+constexpr size_t NOALLOC_PAD_BYTES = 10u << 20;
 
 // Window edge of the plain path for system s: the "window" option, or
 // when it is 0 the automatic edge of the system's shape.

@@ -91,6 +91,12 @@ __host__ __device__ inline int64_t g_elems(int64_t No) {
   const int64_t n = w_blocks(No) * WCUBE;
   return n * n * n;
 }
+// Elements of it in GEMM order, each row padded to a 64-byte line: what the
+// allocation-free region is counted in.
+inline int64_t g_row_elems(int64_t No, bool g32) {
+  const int64_t q = g32 ? 16 : 8;
+  return No * No * ((No + q - 1) / q * q);
+}
 // Offset of a GEMM row and of a GEMM column in it.
 struct GLayout {
   uint32_t No, nbk, magic;  // magic: ceil(2^32 / No), exact for rows < No^2

@@ -23,7 +23,8 @@ using namespace atrip_amd;
 
 namespace {
 
-static __device__ __align__(256) unsigned char scratch[ATRIP_NOALLOC_SCRATCH_BYTES];
+static __device__ __align__(256) unsigned char
+    scratch[ATRIP_NOALLOC_SCRATCH_BYTES + NOALLOC_PAD_BYTES];
 
 constexpr int MAX_DEVICES = 64;
 std::mutex addr_mutex;
@@ -56,6 +57,7 @@ extern "C" int atrip_hip_run_noalloc(atrip_hip_ctx *ctx, int sys,
     check(hipSetDevice(ctx->device), "hipSetDevice");
     void *base = scratch_on(ctx->device);
     run_fixed(ctx, sys, precision, ijkabc, first, count, base,
-              (size_t)ATRIP_NOALLOC_SCRATCH_BYTES, energy, ct_energy);
+              (size_t)ATRIP_NOALLOC_SCRATCH_BYTES, (size_t)NOALLOC_PAD_BYTES,
+              energy, ct_energy);
   });
 }

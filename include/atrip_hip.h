@@ -158,7 +158,8 @@ int atrip_hip_run(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
                   uint64_t first, uint64_t count, double *energy,
                   double *ct_energy);
 
-/* Bytes of the fixed device region of atrip_hip_run_noalloc (per GPU). */
+/* Bytes of the fixed device region of atrip_hip_run_noalloc (per GPU; 10 MiB
+ * behind it are held for the padding of class buffers). */
 #define ATRIP_NOALLOC_SCRATCH_BYTES (256ull * 1024ull * 1024ull)
 
 /* atrip_hip_run without any device allocation.  No counterpart in the
@@ -173,9 +174,12 @@ int atrip_hip_run(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
  * launch shrink until a launch fits.  Fails with a clear error, before any
  * launch, when one window of the context's "window" edge needs more
  * (FP64 without (cT): No=40 fits edge 5, No=60 edge 3; the message names
- * the largest edge that fits), and for a mixed form whose operand copies are not
- * resident yet (upload with that operand_store, or run the form once
- * through atrip_hip_run).  No timing events are recorded.  Calls share the
+ * the largest edge that fits).  A window is counted with three class buffers
+ * per tuple of No^2 rows of No values, rounded up to 64 bytes; where the
+ * buffers' blocks of 8^3 values do not fit but that does (FP64 with (cT) at
+ * No=17..20, for one), the run takes windows of fewer first indices.  Fails
+ * too for a mixed form whose operand copies are not resident yet (upload with
+ * that operand_store, or run the form once through atrip_hip_run).  No timing events are recorded.  Calls share the
  * GPU's region: calls that overlap on one GPU (two threads, or contexts
  * on different streams of one device) race and give wrong results. */
 int atrip_hip_run_noalloc(atrip_hip_ctx *ctx, int sys, int precision,

@@ -103,3 +103,25 @@ def test_window_beyond_the_region_is_refused(ctx):
     (e, _), (e2, _) = _both(ctx, s)
     assert abs(e2 - e) <= 1e-12 * abs(e)
     ctx.release(s)
+
+
+# One window of these fits the region in GEMM order (No^2 rows of No values,
+# padded to 64 bytes), not in the 8^3 blocks of the class buffers: the run takes
+# windows of fewer first indices, or at edge 1 the bytes kept for the padding.
+# The same tuple energies in other groups: compensated sums, equal to rounding.
+@pytest.mark.parametrize("no,nv,precision,with_j,window", [
+    (12, 60, "fp64", True, 0), (17, 24, "fp64", True, 0), (20, 24, "fp64", True, 0),
+    (26, 24, "fp64", True, 0), (25, 20, "fp64", False, 8),
+    (41, 24, "bf16x3", False, 0), (42, 24, "split_fp32", False, 0),
+    (4, 70, "fp64", True, 32), (223, 2, "fp64", False, 1)])
+def test_window_cut_to_fit(ctx, no, nv, precision, with_j, window):
+    s = ctx.upload_synthetic(no, nv, 50 + no, with_j=with_j)
+    ctx.set_option("window", window)
+    n = nv * (nv + 1) * (nv + 2) // 6 - nv
+    for first, count in ((0, None), (1, None), (n // 3, n // 2)):
+        print("noalloc: cut", no, nv, precision, with_j, first, flush=True)
+        a, b = _both(ctx, s, precision, first=first, count=count)
+        assert a[0] != 0.0
+        for x, y in zip(a, b):
+            assert abs(x - y) <= 1e-12 * abs(x)
+    ctx.release(s)
