@@ -1002,10 +1002,11 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
   };
 
   // (a window of a range counts by its slots)
+  const int64_t least = ctx->batch > 0 ? ctx->batch : LEAST_BATCH;
   int bw = (int)std::min<int64_t>(
-      4096, std::max<int64_t>(1, ctx->batch * (int64_t)nb * nb * nb / per));
+      4096, std::max<int64_t>(1, least * (int64_t)nb * nb * nb / per));
   const int bw_least = bw;
-  if (!ctx->batch_set)
+  if (ctx->batch == 0)
     bw = std::max(bw, auto_batch((use_j ? 2 : 1) * nsets * 3 * W3 *
                                      (int64_t)gelem, per));
   void *Gbuf = nullptr, *e_slot = nullptr, *wcube = nullptr,
@@ -1629,9 +1630,9 @@ int atrip_hip_set_option(atrip_hip_ctx *ctx, const char *key, int64_t value) {
         throw Fail{"window must be in 0..32 (0: automatic)"};
       ctx->window = (int)value;
     } else if (k == "batch") {
-      if (value < 1 || value > 4096) throw Fail{"batch must be in 1..4096"};
+      if (value < 0 || value > 4096)
+        throw Fail{"batch must be in 0..4096 (0: automatic)"};
       ctx->batch = (int)value;
-      ctx->batch_set = true;
     } else if (k == "timing") {
       ctx->timing = value != 0;
     } else if (k == "tile") {

@@ -208,13 +208,14 @@ inline int auto_window(int64_t No, int64_t Nv) {
 
 // Windows per launch when the caller set none: as many as keep the launch's
 // class buffers (slot_bytes per tuple slot, `per` slots per window) within
-// LAUNCH_BYTES, at least the option's four.  Every launch ends in a partly
+// LAUNCH_BYTES, at least LEAST_BATCH of the plan's.  Every launch ends in a partly
 // filled chip and is followed by an epilogue that starts on an empty one, and
 // small systems are launch-bound: against four windows per launch, No=4,
 // Nv=36 takes 0.11 ms instead of 0.16, No=10, Nv=50 1.25 instead of 2.10,
 // No=16, Nv=120 42.5 instead of 45.6, No=26, Nv=308 (100,000 tuples) 160
 // instead of 174; beyond 2 GiB the gain is below 1 % (No=40 fits five
 // windows).
+constexpr int LEAST_BATCH = 4;
 constexpr int64_t LAUNCH_BYTES = (int64_t)2 << 30;
 inline int auto_batch(int64_t slot_bytes, int64_t per) {
   return (int)std::min<int64_t>(4096, LAUNCH_BYTES / (slot_bytes * per));

@@ -319,8 +319,7 @@ struct atrip_hip_ctx {
   int next_sys = 1;
   // options
   int window = 0;  // window edge; 0: automatic per system (auto_window)
-  int batch = 4;
-  bool batch_set = false;  // the caller chose `batch`
+  int batch = 0;   // windows per launch; 0: automatic (auto_batch)
   int timing = 0;
   int tile = -1;  // -1: chosen per system shape
   int operand_store = 0;  // store mode of the next uploads (DevSystem::store)

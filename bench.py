@@ -381,7 +381,7 @@ def main(argv=None):
     ap.add_argument("--precision", default="fp64",
                     choices=["fp64", "split_fp32", "fp32", "bf16x3"])
     ap.add_argument("--window", type=int, default=8)
-    ap.add_argument("--batch", type=int, default=4)
+    ap.add_argument("--batch", type=int, default=0)
     ap.add_argument("--tile", type=int, default=-1)
     ap.add_argument("--operand-store", type=int, default=0, choices=[0, 1, 2, 3],
                     help="operand store of the timed system: 0 FP64 (mixed "

@@ -226,9 +226,8 @@ int atrip_hip_tuple_energies(atrip_hip_ctx *ctx, int sys, int precision,
  *   "window"  block edge nb of the tuple windows (1..32); 0 (default):
  *             chosen per system shape (8 unless a modelled tile fit of
  *             edge 6 or 12 is 15 % better)
- *   "batch"   windows per launch (4 until set: then also as many more as
- *             keep the class buffers of a launch within 2 GiB, fewer where
- *             device memory is short)
+ *   "batch"   windows per launch (1..4096); 0 (default): as many as keep
+ *             the class buffers of a launch within 2 GiB, at least four
  *   "timing"  1: time every hot-kernel launch with HIP events
  *   "tile"    doubles-kernel tile variant: 0..7 for the FP64 kernel, 0..9
  *             for the FP32-product kernels (a variant a kernel lacks

@@ -26,3 +26,11 @@ def hip_ctx():
     ctx = hip.Context(0)
     yield ctx
     ctx.close()
+
+
+@pytest.fixture(autouse=True)
+def automatic_batch(request):
+    """Each test that uses the shared context starts with automatic launch
+    sizes, whatever an earlier one left."""
+    if "hip_ctx" in request.fixturenames:
+        request.getfixturevalue("hip_ctx").set_option("batch", 0)
