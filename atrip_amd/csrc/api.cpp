@@ -842,6 +842,20 @@ void ensure(void *&ptr, size_t &have, size_t need, const char *what) {
   have = need;
 }
 
+// Gives back the buffers a plain run's launches grow (not its window list).
+void drop_run_scratch(atrip_hip_ctx *ctx) {
+  if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
+  auto drop = [](double *&p, size_t &bytes) {
+    if (p) (void)hipFree(p);
+    p = nullptr;
+    bytes = 0;
+  };
+  drop(ctx->G, ctx->G_bytes);
+  drop(ctx->e_slot, ctx->e_slot_bytes);
+  drop(ctx->wcube, ctx->wcube_bytes);
+  drop(ctx->partials, ctx->partials_bytes);
+}
+
 struct RunResult {
   double e = 0, ect = 0;
   uint64_t tuples = 0;  // tuples computed
@@ -1088,9 +1102,11 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
                "alloc partials");
         break;
       } catch (const Fail &) {
-        // a device with little memory left: launches of the option's size
+        // a device with little memory left: launches of the least size, in
+        // buffers of their own (those the larger one had grown kept it out)
         if (bw <= bw_least) throw;
         (void)hipGetLastError();
+        drop_run_scratch(ctx);
         bw = bw_least;
         z = sizes(bw, W3);
       }
