@@ -226,9 +226,33 @@ void free_system(DevSystem &s) {
 
 }  // namespace
 
-bool atrip_amd::drop_swap_copies(atrip_hip_ctx *ctx) {
-  bool any = false;
+namespace {
+
+// Gives back the buffers a plain run's launches grow (not its window list).
+void drop_run_scratch(atrip_hip_ctx *ctx) {
   if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
+  auto drop = [](double *&p, size_t &bytes) {
+    if (p) (void)hipFree(p);
+    p = nullptr;
+    bytes = 0;
+  };
+  drop(ctx->G, ctx->G_bytes);
+  drop(ctx->e_slot, ctx->e_slot_bytes);
+  drop(ctx->wcube, ctx->wcube_bytes);
+  drop(ctx->partials, ctx->partials_bytes);
+}
+
+// The contexts of the process.  Whoever holds the mutex may wait for a
+// context's in_use; nobody takes it with an in_use held.
+std::mutex contexts_mutex;
+// (never destroyed: a context may be freed while the process ends)
+std::vector<atrip_hip_ctx *> &contexts = *new std::vector<atrip_hip_ctx *>;
+
+}  // namespace
+
+void atrip_amd::give_back(atrip_hip_ctx *ctx) {
+  std::lock_guard<std::mutex> use(ctx->in_use);
+  drop_run_scratch(ctx);  // (waits for the stream)
   for (auto &kv : ctx->systems) {
     DevSystem &s = kv.second;
     if (!s.swaps) continue;
@@ -238,9 +262,13 @@ bool atrip_amd::drop_swap_copies(atrip_hip_ctx *ctx) {
     (void)hipFree(s.swaps);
     s.swaps = nullptr;
     s.bytes -= s.swap_bytes;
-    any = true;
   }
-  return any;
+}
+
+void atrip_amd::give_back_others(atrip_hip_ctx *ctx) {
+  std::lock_guard<std::mutex> all(contexts_mutex);
+  for (atrip_hip_ctx *c : contexts)
+    if (c != ctx && c->device == ctx->device) give_back(c);
 }
 
 // Device bytes alloc_system takes for a system (the arrays below, the
@@ -842,18 +870,12 @@ void ensure(void *&ptr, size_t &have, size_t need, const char *what) {
   have = need;
 }
 
-// Gives back the buffers a plain run's launches grow (not its window list).
-void drop_run_scratch(atrip_hip_ctx *ctx) {
-  if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
-  auto drop = [](double *&p, size_t &bytes) {
-    if (p) (void)hipFree(p);
-    p = nullptr;
-    bytes = 0;
-  };
-  drop(ctx->G, ctx->G_bytes);
-  drop(ctx->e_slot, ctx->e_slot_bytes);
-  drop(ctx->wcube, ctx->wcube_bytes);
-  drop(ctx->partials, ctx->partials_bytes);
+// Makes a filled system resident; its handle.
+int add_system(atrip_hip_ctx *ctx, DevSystem &&s) {
+  std::lock_guard<std::mutex> use(ctx->in_use);
+  const int id = ctx->next_sys++;
+  ctx->systems.emplace(id, std::move(s));
+  return id;
 }
 
 struct RunResult {
@@ -901,6 +923,7 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
                     uint64_t first, uint64_t last, Sink &&sink,
                     const WindowSel &wsel = WindowSel{},
                     const FixedScratch *fixed = nullptr) {
+  std::lock_guard<std::mutex> use(ctx->in_use);
   drop_pending_events(ctx);
   DevSystem &s = get_sys(ctx, sys);
   WindowPlan &plan = get_plan(ctx, sys, s, wsel.nb);
@@ -1389,12 +1412,18 @@ int atrip_hip_create(int device, atrip_hip_ctx **out) {
     delete ctx;
     return rc;
   }
+  std::lock_guard<std::mutex> all(contexts_mutex);
+  contexts.push_back(ctx);
   *out = ctx;
   return 0;
 }
 
 int atrip_hip_destroy(atrip_hip_ctx *ctx) {
   if (!ctx) return 0;
+  {
+    std::lock_guard<std::mutex> all(contexts_mutex);
+    contexts.erase(std::find(contexts.begin(), contexts.end(), ctx));
+  }
   (void)hipSetDevice(ctx->device);
   if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
   for (auto &kv : ctx->systems) free_system(kv.second);
@@ -1432,9 +1461,7 @@ int atrip_hip_upload(atrip_hip_ctx *ctx, const atrip_sys_desc *desc,
       free_system(s);
       throw;
     }
-    const int id = ctx->next_sys++;
-    ctx->systems.emplace(id, std::move(s));
-    *sys = id;
+    *sys = add_system(ctx, std::move(s));
   });
 }
 
@@ -1462,9 +1489,7 @@ int atrip_hip_upload_synthetic_scaled(atrip_hip_ctx *ctx, int64_t No,
       free_system(s);
       throw;
     }
-    const int id = ctx->next_sys++;
-    ctx->systems.emplace(id, std::move(s));
-    *sys = id;
+    *sys = add_system(ctx, std::move(s));
   });
 }
 
@@ -1490,9 +1515,7 @@ int atrip_hip_upload_complex(atrip_hip_ctx *ctx, const atrip_sys_desc *desc,
       free_system(s);
       throw;
     }
-    const int id = ctx->next_sys++;
-    ctx->systems.emplace(id, std::move(s));
-    *sys = id;
+    *sys = add_system(ctx, std::move(s));
   });
 }
 
@@ -1523,9 +1546,7 @@ int atrip_hip_upload_stream(atrip_hip_ctx *ctx, int64_t No, int64_t Nv,
       free_system(s);
       throw;
     }
-    const int id = ctx->next_sys++;
-    ctx->systems.emplace(id, std::move(s));
-    *sys = id;
+    *sys = add_system(ctx, std::move(s));
   });
 }
 
@@ -1549,14 +1570,13 @@ int atrip_hip_upload_synthetic_complex(atrip_hip_ctx *ctx, int64_t No,
       free_system(s);
       throw;
     }
-    const int id = ctx->next_sys++;
-    ctx->systems.emplace(id, std::move(s));
-    *sys = id;
+    *sys = add_system(ctx, std::move(s));
   });
 }
 
 int atrip_hip_release(atrip_hip_ctx *ctx, int sys) {
   return guarded(ctx, [&] {
+    std::lock_guard<std::mutex> use(ctx->in_use);
     DevSystem &s = get_sys(ctx, sys);
     check(hipStreamSynchronize(ctx->stream), "sync");
     free_system(s);
@@ -1733,6 +1753,7 @@ int atrip_hip_reset_stats(atrip_hip_ctx *ctx) {
 int atrip_hip_sys_info(atrip_hip_ctx *ctx, int sys, int64_t *No, int64_t *Nv,
                        uint64_t *n_tup, uint64_t *device_bytes) {
   return guarded(ctx, [&] {
+    std::lock_guard<std::mutex> use(ctx->in_use);
     DevSystem &s = get_sys(ctx, sys);
     if (No) *No = s.No;
     if (Nv) *Nv = s.Nv;

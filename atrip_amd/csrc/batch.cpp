@@ -368,6 +368,7 @@ int atrip_hip_batch_run(atrip_hip_ctx *ctx, const int *systems, int nsys,
       throw Fail{"bad system list"};
     check_batched_precision(precision);
     check(hipSetDevice(ctx->device), "hipSetDevice");
+    std::lock_guard<std::mutex> use(ctx->in_use);
     const int grid =
         ctx->batch_grid ? ctx->batch_grid : default_grid(ctx, precision);
     std::vector<BSys> sys;
@@ -426,6 +427,7 @@ int atrip_hip_batch_tune(atrip_hip_ctx *ctx, const int *systems, int nsys,
     if (mode != 0 && mode != 1) throw Fail{"mode must be 0 or 1"};
     check_batched_precision(precision);
     check(hipSetDevice(ctx->device), "hipSetDevice");
+    std::lock_guard<std::mutex> use(ctx->in_use);
     const int grid =
         ctx->batch_grid ? ctx->batch_grid : default_grid(ctx, precision);
     // one representative system per shape

@@ -59,28 +59,35 @@ void check_precision(const DevSystem &s, int precision);
 // (`swaps`: with the row-swapped copies of the FP64 store).
 uint64_t system_bytes(int64_t No, int64_t Nv, bool with_j, int store,
                       bool swaps = true);
-// Frees the row-swapped copies of a context's FP64 systems (the kernels then
-// read the straight arrays); whether there were any.
-bool drop_swap_copies(atrip_hip_ctx *ctx);
-// f(), again without the row-swapped copies (of the resident systems and of
-// the one an upload is making) when the device ran out of memory: they are a
-// convenience and never cost a call its memory.  f leaves nothing behind when
-// it throws.
+// Frees what a context holds but can do without: the row-swapped copies of
+// its FP64 systems (the kernels then read the straight arrays) and the buffers
+// of a plain run (the next one takes them again).  Waits for the device work
+// of a call that another thread is in.
+void give_back(atrip_hip_ctx *ctx);
+// The same for every other context of the process on ctx's device.
+void give_back_others(atrip_hip_ctx *ctx);
+// f(), again when the device ran out of memory, without the row-swapped copies
+// (of the resident systems and of the one an upload is making) and grown
+// buffers of this context and then of the other ones on the device: they are
+// a convenience and never cost a call its memory.  f leaves nothing behind when
+// it throws, and holds no context's in_use then.
 template <typename F>
 auto retry_memory(atrip_hip_ctx *ctx, F &&f) {
-  try {
-    return f();
-  } catch (const Fail &x) {
-    if (x.msg.find("out of memory") == std::string::npos) throw;
-    (void)hipGetLastError();
-    drop_swap_copies(ctx);
-  }
-  struct Without {
+  struct Swaps {
     atrip_hip_ctx *ctx;
     bool was;
-    ~Without() { ctx->operand_swaps = was; }
-  } w{ctx, ctx->operand_swaps};
-  ctx->operand_swaps = false;
+    ~Swaps() { ctx->operand_swaps = was; }
+  } swaps{ctx, ctx->operand_swaps};
+  for (auto *more : {give_back, give_back_others}) {
+    try {
+      return f();
+    } catch (const Fail &x) {
+      if (x.msg.find("out of memory") == std::string::npos) throw;
+    }
+    (void)hipGetLastError();
+    ctx->operand_swaps = false;
+    more(ctx);
+  }
   return f();
 }
 template <typename F>

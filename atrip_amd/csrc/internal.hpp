@@ -6,6 +6,7 @@
 #include <array>
 #include <cstdint>
 #include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -327,6 +328,10 @@ struct atrip_hip_ctx {
   int epilogue = 0;  // 0: fused class sums + energy, 1: W cubes first
   int serve_plain_no = 16;  // served requests with No >= this: plain path
   int64_t stage_kb = 4 << 20;  // device staging of host uploads (KiB)
+  // Held while device work of a call uses the systems' arrays and the scratch
+  // below, so that a call of another context may give back what this one can
+  // do without (give_back); never while a callback of the caller runs.
+  std::mutex in_use;
   // scratch, grown on demand
   double *G = nullptr;       // class buffers [ncls][slots][g_elems(No)]
   size_t G_bytes = 0;

@@ -275,6 +275,7 @@ int step(atrip_hip_server *srv) {
   if (!tasks.empty()) {
     const std::vector<int32_t> order = longest_first(cost);
     const LaunchOut out = retry_memory(ctx, [&] {
+      std::lock_guard<std::mutex> use(ctx->in_use);
       std::vector<BSys> sys;
       std::vector<BSplit> split;
       for (size_t q = 0; q < owners.size(); q++) {

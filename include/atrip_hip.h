@@ -12,7 +12,11 @@
  * error convention (src/atrip/Acc.hpp:95-107, src/atrip/HIP.hpp:31-42).
  *
  * A context is bound to one device and is not thread-safe: use one host
- * thread per context (the serving loop owns its own context).
+ * thread per context (the serving loop owns its own context).  A call that
+ * finds no device memory takes back what its context, and then the other
+ * contexts of the process on that device, hold only for speed (grown launch
+ * buffers, the row-swapped copies of FP64 systems), waiting for their current
+ * run; results stay the same bits.
  */
 #ifndef ATRIP_HIP_H
 #define ATRIP_HIP_H

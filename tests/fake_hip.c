@@ -1,18 +1,25 @@
 /* A host-memory stand-in for the HIP runtime calls of libatrip_hip.so, for tests
  * of its memory handling on the CPU: allocations come from host memory up to a
- * limit, copies are copies, kernels do nothing (so energies are zero). */
+ * limit, copies are copies, kernels take a settable time and do nothing (so
+ * energies are zero). */
+#include <pthread.h>
 #include <stdint.h>
 #include <stdlib.h>
 #include <string.h>
+#include <unistd.h>
 
 enum { OK = 0, OUT_OF_MEMORY = 2, MAX_BLOCKS = 4096 };
 static struct { void *p; size_t n; } block[MAX_BLOCKS];
 static size_t limit = SIZE_MAX, used;
 
+static pthread_mutex_t lock = PTHREAD_MUTEX_INITIALIZER;
+static unsigned launch_us;
+
 void fake_set_limit(size_t bytes) { limit = bytes; }
 size_t fake_used(void) { return used; }
+void fake_set_launch_us(unsigned us) { launch_us = us; }
 
-int hipMalloc(void **p, size_t n) {
+static int take(void **p, size_t n) {
   *p = NULL;
   if (n > limit || used > limit - n) return OUT_OF_MEMORY;
   for (int q = 0; q < MAX_BLOCKS; q++)
@@ -25,7 +32,7 @@ int hipMalloc(void **p, size_t n) {
     }
   return OUT_OF_MEMORY;
 }
-int hipFree(void *p) {
+static int give(void *p) {
   for (int q = 0; q < MAX_BLOCKS && p; q++)
     if (block[q].p == p) {
       used -= block[q].n;
@@ -34,6 +41,18 @@ int hipFree(void *p) {
       return OK;
     }
   return p ? 1 : OK;
+}
+int hipMalloc(void **p, size_t n) {
+  pthread_mutex_lock(&lock);
+  const int e = take(p, n);
+  pthread_mutex_unlock(&lock);
+  return e;
+}
+int hipFree(void *p) {
+  pthread_mutex_lock(&lock);
+  const int e = give(p);
+  pthread_mutex_unlock(&lock);
+  return e;
 }
 int hipHostMalloc(void **p, size_t n, unsigned flags) {
   (void)flags;
@@ -76,6 +95,7 @@ int hipGetLastError(void) { return OK; }
 typedef struct { unsigned x, y, z; } dims;
 int hipLaunchKernel(const void *f, dims g, dims b, void **a, size_t l, void *s) {
   (void)f; (void)g; (void)b; (void)a; (void)l; (void)s;
+  if (launch_us) usleep(launch_us);
   return OK;
 }
 int __hipPushCallConfiguration(dims g, dims b, size_t l, void *s) {

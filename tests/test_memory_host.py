@@ -49,3 +49,72 @@ fake.fake_set_limit(fake.fake_used() + 2140 * 10**6)
 ctx.run(s)
 assert fake.fake_used() < 2140 * 10**6
 """)
+
+
+# `full`: bytes of a No=12, Nv=48 system, `swaps` of them (3.5 MB) its
+# row-swapped copies; a run of it grows launch buffers of more than 1 GiB
+SIZES = """
+probe = hip.Context(0)
+before = fake.fake_used()
+p = probe.upload_synthetic(12, 48, 1)
+full = fake.fake_used() - before
+probe.run(p)
+grown = fake.fake_used() - before - full
+assert grown > GiB
+probe.close()
+assert fake.fake_used() == before
+swaps = 8 * 48 * 144 * (48 + 16)
+"""
+
+
+def test_upload_takes_back_what_its_context_grew(fake):
+    _run(fake, SIZES + """
+ctx = hip.Context(0)
+a = ctx.upload_synthetic(12, 48, 1)
+ctx.run(a)
+fake.fake_set_limit(fake.fake_used() + full // 2)
+b = ctx.upload_synthetic(12, 48, 2)
+ctx.run(b)
+""")
+
+
+def test_upload_takes_back_what_another_context_holds(fake):
+    # room for the second system only without its own copies and without the
+    # first's copies or launch buffers
+    _run(fake, SIZES + """
+for run in (False, True):
+    one, two = hip.Context(0), hip.Context(0)
+    a = one.upload_synthetic(12, 48, 1)
+    assert one.sys_info(a)["bytes"] > full - swaps
+    if run:
+        one.run(a)
+    fake.fake_set_limit(fake.fake_used() + full - swaps - 10**6)
+    b = two.upload_synthetic(12, 48, 2)
+    assert one.sys_info(a)["bytes"] <= full - swaps
+    fake.fake_set_limit(1 << 40)
+    one.run(a)
+    two.run(b)
+    two.close()
+    one.close()
+""")
+
+
+def test_waits_for_a_run_of_another_context(fake):
+    # the other context's run has 0.2 s to go when the upload finds no memory
+    _run(fake, SIZES + """
+import threading, time
+one, two = hip.Context(0), hip.Context(0)
+a = one.upload_synthetic(12, 48, 1)
+one.run(a)
+fake.fake_set_limit(fake.fake_used() + full - swaps - 10**6)
+fake.fake_set_launch_us(100000)
+ended = []
+t = threading.Thread(target=lambda: (one.run(a), ended.append(time.time())))
+t.start()
+time.sleep(0.1)
+b = two.upload_synthetic(12, 48, 2)
+t.join()
+assert one.sys_info(a)["bytes"] <= full - swaps
+one.run(a)
+two.run(b)
+""")
