@@ -436,7 +436,7 @@ void energy_kernel(EnergyParams P) {
 // 39.8 with one instance per orbit type and for triples inside the range,
 // 40.8 / 36.8 with the LDS strides below; No=60, Nv=240 131 / 119 -> 95 / 83.
 struct FusedParams {
-  const void *G, *GJ;  // class buffers [3][slots][No^2 rows][NoP] (FP64 or FP32)
+  const void *G, *GJ;  // class buffers [3][slots][g_elems(No)] (FP64 or FP32)
   const double *Tai, *VHH, *ei, *ea;
   const uint32_t *points;
   WindowArgs win;
@@ -736,7 +736,7 @@ __global__ __launch_bounds__(T < 256 ? 256 : T, HJ ? 2 : 4) void energy_small_ke
 #pragma unroll
   for (int it = 0; it < NI; it++) {
     const int e = tl + T * it, x = e < count ? e : 0;
-    // (both quotients exact: they lie at least 1 / 32 from a whole number)
+    // (both quotients exact: they lie at least 1 / 40 from a whole number)
     const int m = (int)(((float)x + 0.5f) * rH), r = 2 * (x - m * H);
     const int q = (int)(((float)m + 0.5f) * rN), p = m - q * no;
     at[it] = ((uint32_t)(((q >> 3) * P.nbk + (p >> 3)) * P.nbk + (r >> 3)) << 9) +
@@ -880,7 +880,9 @@ hipError_t launch_small(const FusedParams &P, hipStream_t st) {
   }
   SMALL(64, 1) SMALL(64, 2) SMALL(64, 4)
   SMALL(256, 2) SMALL(256, 4) SMALL(256, 6)
-  SMALL(512, 4) SMALL(512, 6) SMALL(512, 8)
+  SMALL(512, 4) SMALL(512, 6)
+  // (No = 19, 20: with (cT) or FP32 buffers only, see small_energy)
+  if constexpr (HJ || std::is_same_v<GT, float>) SMALL(512, 8)
 #undef SMALL
   return hipErrorInvalidConfiguration;
 }

@@ -368,7 +368,9 @@ hipError_t launch_z_small(const EnergyZParams &P, hipStream_t st) {
                        TT < 256 ? 256 : TT, lds, st, P);                      \
     return hipGetLastError();                                                 \
   }
-  SMALL(64, 1) SMALL(64, 4) SMALL(512, 2) SMALL(512, 4) SMALL(512, 8)
+  SMALL(64, 1) SMALL(64, 4) SMALL(512, 2) SMALL(512, 4)
+  // (No = 17..20: without (cT) only, see small_energy_z)
+  if constexpr (!HJ) SMALL(512, 8)
 #undef SMALL
   return hipErrorInvalidConfiguration;
 }
