@@ -1126,11 +1126,13 @@ RunResult run_range(atrip_hip_ctx *ctx, int sys, int precision, int ijkabc,
         break;
       } catch (const Fail &) {
         // a device with little memory left: launches of the least size, in
-        // buffers of their own (those the larger one had grown kept it out)
-        if (bw <= bw_least) throw;
+        // buffers of their own (those the larger one had grown kept it out),
+        // and when nothing is left to take back (retry_memory) of fewer windows:
+        // blocks of 8^3 can take more than four windows in GEMM order did
+        if (bw == 1 || (bw <= bw_least && ctx->operand_swaps)) throw;
         (void)hipGetLastError();
         drop_run_scratch(ctx);
-        bw = bw_least;
+        bw = bw > bw_least ? bw_least : bw / 2;
         z = sizes(bw, W3);
       }
     }

@@ -118,3 +118,20 @@ assert one.sys_info(a)["bytes"] <= full - swaps
 one.run(a)
 two.run(b)
 """)
+
+
+def test_fewer_windows_where_four_do_not_fit(fake):
+    # No=9, edge 16: 12288 class buffers of 4096 values for one window of 4096
+    # tuples, 403 MB (four in GEMM order, 9^2 rows of 16: 510 MB)
+    _run(fake, """
+ctx = hip.Context(0)
+ctx.set_option("window", 16)
+s = ctx.upload_synthetic(9, 48, 1)
+for batch in (0, 4):
+    ctx.set_option("batch", batch)
+    fake.fake_set_limit(fake.fake_used() + 512 * 10**6)
+    ctx.run(s)
+    fake.fake_set_limit(fake.fake_used() + 10**9)
+    ctx.run(s, first=10, count=20000)
+    fake.fake_set_limit(1 << 40)
+""")
