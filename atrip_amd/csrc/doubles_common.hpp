@@ -133,13 +133,16 @@ inline int64_t doubles_grid(WindowArgs &W, int64_t No, int64_t mt_rows,
   return (units + 7) / 8 * 8 * W.nw * W.mtiles * W.ntiles;
 }
 
-// Tile shapes (wave tile FM x FN fragments of 16x16, 2x2 waves) and the
-// fraction of peak each reaches per useful tile element on MI355X in FP64:
-// 5x5 at No=40, Nv=400; 4x2, 4x4, 3x3, 4x5 and 5x4 relative to it from
-// whole-system runs at No=26/Nv=308, 31/270, 38/204 and 20/183, each divided
-// by its padded-grid fraction (5x4 measured 4 % above 5x5 there, entered
-// equal to it, since no shape measured both at full use); 2x2 and 2x4 from
-// an earlier kernel at No=40.
+// Tile shapes (FM x FN fragments of 16x16 of each of 2x2 waves; 5x5, 4x5 and
+// 5x4 run as 4x2 waves of half the rows) and the rate of each per useful
+// tile element in FP64, as fitted to kernels that computed a tile's padding and
+// the columns of tuples that do not exist (whole-system runs at No=20, 26, 31,
+// 38 and 40; 2x2 and 2x4 older still).  The present kernels compute neither.
+// Their rates, in TFLOP/s of the doubles kernel over a sample of the whole
+// space at edge 8, as picked / with 4x4: No=20, Nv=183 54.0 (5x5) / 55.0, 26/308
+// 52.3 (5x4) / 55.2, 31/270 55.5 (5x4) / 59.2, 38/204 55.3 (4x5) / 56.1, 40/400
+// (edge 12) 65.6 (5x5) / 66.8, where the same tile timed twice differs by 3 %.
+// The table stands until it is fitted anew; host tests hold its picks.
 constexpr int N_TILES = 8;
 __host__ __device__ inline int tile_fm(int t) {
   const int v[N_TILES] = {2, 4, 2, 4, 3, 5, 4, 5};
@@ -154,8 +157,8 @@ inline double tile_rate(int t) {
   return v[t];
 }
 
-// Automatic tile: best measured rate times the useful fraction of the padded
-// M = No^2 by N = nb*No tile grid.
+// Automatic tile: best of the rates above times the useful fraction of the
+// padded M = No^2 by N = nb*No tile grid.
 inline int pick_tile(int tile, int64_t No, int nb) {
   if (tile >= 0 && tile < N_TILES) return tile;
   double best = -1.0;
@@ -176,11 +179,14 @@ inline int pick_tile(int tile, int64_t No, int nb) {
 
 // Automatic window edge of the plain path: the doubles GEMMs of a window
 // have N = nb No columns, so the edge sets how much of the last column tile
-// is padding.  Each candidate edge is scored by its best tile's modelled
+// is empty.  Each candidate edge is scored by its best tile's modelled
 // rate (pick_tile's model) times the share of valid tuples in the windows;
 // an edge other than 8 is taken only when it scores 15 % above 8 (the
-// model's own error).  Measured in FP64 on MI355X: No=26, Nv=308 runs at
-// 40.6 TFLOP/s with edge 6 against 33.2 with edge 8; No=40 and No=60 keep 8.
+// model's own error).  The model charges empty columns as the earlier kernels
+// paid for them (No=26, Nv=308: 40.6 TFLOP/s with edge 6, its pick, 33.2 with 8).
+// With the present ones edges 6, 8 and 12 lie within 5 % there (51.6, 52.3, 53.9)
+// and within 7 % at No=20, 31 and 38 but for edge 6 at No=20 and 38 (11 % and
+// 8 % below 8).
 inline int auto_window(int64_t No, int64_t Nv) {
   auto score = [&](int nb) {
     const int t = pick_tile(-1, No, nb);
@@ -213,8 +219,9 @@ inline int auto_window(int64_t No, int64_t Nv) {
 // small systems are launch-bound: against four windows per launch, No=4,
 // Nv=36 takes 0.11 ms instead of 0.16, No=10, Nv=50 1.25 instead of 2.10,
 // No=16, Nv=120 42.5 instead of 45.6, No=26, Nv=308 (100,000 tuples) 160
-// instead of 174; beyond 2 GiB the gain is below 1 % (No=40 fits five
-// windows).
+// instead of 174; beyond 2 GiB the gain is below 1 %.  (LEAST_BATCH windows
+// pass 2 GiB from No=33 in FP64: 3.1 GB at No=40, where five fit in FP32, and
+// 12.9 GB at No=60; twice that with (cT).)
 constexpr int LEAST_BATCH = 4;
 constexpr int64_t LAUNCH_BYTES = (int64_t)2 << 30;
 inline int auto_batch(int64_t slot_bytes, int64_t per) {
